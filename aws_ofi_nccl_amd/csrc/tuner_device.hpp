@@ -36,7 +36,6 @@ enum { PROTO_LL = 0, PROTO_LL128 = 1, PROTO_SIMPLE = 2, NUM_PROTOS = 3 };
 
 constexpr int kNumPlatforms = 4;
 constexpr int kNumShapes = 3; /* ranks == 8*nodes, 2*nodes, nodes */
-constexpr int kMaxVertices = 20;
 constexpr uint32_t kAllAllowed = (1u << (NUM_ALGOS * NUM_PROTOS)) - 1;
 
 __host__ __device__ inline bool allowed(uint32_t mask, int algo, int proto)
@@ -263,12 +262,23 @@ struct pt_t {
 	double x, y;
 };
 
+typedef double double4_t __attribute__((ext_vector_type(4)));
+
+/* one edge of a polygon, from the vertex before it (the last one for a polygon's first) to vertex `b` */
+struct edge_t {
+	pt_t a, b;
+};
+
+/* The polygons of one (platform, shape, collective): consecutive in `poly`, their edges -- at most 64 --
+ * consecutive in `edges`.  polys == 0: no regions. */
+struct region_set_t {
+	uint16_t first_poly, polys, first_edge, edges;
+};
+
 struct region_tables_t {
-	/* [platform][shape][coll] -> first polygon / count (0 when no regions) */
-	int32_t set_first[kNumPlatforms][kNumShapes][NUM_FUNCS];
-	int32_t set_count[kNumPlatforms][kNumShapes][NUM_FUNCS];
-	const int32_t *poly; /* per polygon {algo, proto, first_vertex, num_vertices} */
-	const pt_t *verts;   /* log2 space */
+	region_set_t set[kNumPlatforms][kNumShapes][NUM_FUNCS];
+	const int32_t *poly; /* per polygon {algo, proto, first_edge, num_edges} */
+	const edge_t *edges; /* log2 space */
 	const double *bbox;  /* per polygon {min_x, max_x, min_y, max_y} as is_inside_region finds them */
 	pt_t far_point;      /* log2 of (2*max size, 2*max ranks) */
 };
@@ -320,59 +330,97 @@ __device__ inline double seg_distance(pt_t x, pt_t y0, pt_t y1, double eps)
 }
 
 /*
- * Certain-answer forms of the two per-edge tests.  Each evaluates the quotient of `intersect`
- * with an approximate reciprocal (hardware estimate plus one Newton step: relative error below
- * 1e-12 against the 1e-5 margins used here) and says whether the exact code's answer is already
- * certain from it.  They are straight-line code -- no branch, no division, no square root -- so
- * the walk over a polygon's edges can overlap the arithmetic of several edges; a point for which
- * any edge is not certain (a quotient near one of the thresholds, a degenerate edge, a foot point
- * close to the edge) is run again through the exact code above, so results are the exact code's.
+ * Certain-answer forms of the two per-edge tests, from the signs of cross products: no division, no
+ * square root, no branch.  With P the point, F the far end of its ray and A, B the edge's ends,
+ *
+ *   side_a, side_b = (A - P) x (F - P), (B - P) x (F - P)     which side of the ray's line A and B lie on
+ *   side_p, side_f = (P - A) x (B - A), (F - A) x (B - A)     which side of the edge's line P and F lie on
+ *
+ * `intersect`'s quotients are a = side_a / (side_a - side_b) and b = side_p / (side_p - side_f).
+ * Coordinates are logarithms to base 2 of 64-bit numbers, so a cross product is below 2e4 and is
+ * computed to 1e-11: with |side_a| and |side_b| above kSure = 1e-4, a is outside [0, 1] by 5e-9 when the
+ * signs agree and inside (eps, 1 - eps) by as much when they differ (eps is 1e-10), and the same holds
+ * for b.  What is not certain goes through the exact code above, so results are the exact code's.
  */
-__device__ __forceinline__ double approx_rcp(double d)
+constexpr double kSure = 1e-4;
+
+struct edge_sides_t {
+	double side_a, side_b, side_p;
+};
+
+__device__ __forceinline__ edge_sides_t edge_sides(pt_t p, pt_t ray, pt_t a, pt_t b)
 {
-	double r = __builtin_amdgcn_rcp(d);
-	return r * (2.0 - d * r);
+	const pt_t pa = vsub(a, p), pb = vsub(b, p);
+	return edge_sides_t{ vcross(pa, ray), vcross(pb, ray), vcross(pb, pa) };
 }
 
-/* |a - t| far beyond what the approximate quotient can be off by */
-__device__ __forceinline__ bool clear_of(double a, double t)
+/* n / d < t as the exact code's rounded quotient compares, d > 0; `sure` is cleared when n and t * d are too
+ * close to tell without dividing (their rounding errors and the quotient's are below 4e-16 of either) */
+__device__ __forceinline__ bool quotient_below(double n, double d, double t, bool &sure)
 {
-	return fabs(a - t) > 1e-5 * (1.0 + fabs(a));
+	const double gap = n - t * d;
+	sure &= fabs(gap) > 1e-15 * (fabs(n) + d);
+	return gap < 0;
 }
 
-/* Whether intersect(x0, x0 + dx, y0, y1, eps, nullptr) == 1; `certain` is cleared when only the
- * exact quotient can tell. */
-__device__ __forceinline__ bool crosses_edge(pt_t x0, pt_t dx, pt_t y0, pt_t y1, double eps, bool &certain)
+/* intersect(x0, x1, y0, y1, eps, nullptr) == 1.  Grid points sit on the lines of many edges (rank counts that
+ * are powers of two), where the quotients are 0 or 1 to the last bit and the signs are not certain; comparing
+ * products instead of quotients answers those too, and the two divisions are left for what is within
+ * rounding of a threshold. */
+__device__ __forceinline__ bool intersects(pt_t x0, pt_t x1, pt_t y0, pt_t y1, double eps)
 {
-	const pt_t dy = vsub(y1, y0);
-	const double d = vcross(dy, dx);
-	const bool parallel = fabs(d) < eps; /* the exact code answers 0 */
-	const double r = approx_rcp(parallel ? 1.0 : d);
-	const double a = (vcross(x0, dx) - vcross(y0, dx)) * r;
-	const double b = (vcross(x0, dy) - vcross(y0, dy)) * r;
-	const bool a_clear = clear_of(a, 0.0) && clear_of(a, 1.0);
-	const bool b_clear = clear_of(b, 0.0) && clear_of(b, 1.0);
-	const bool a_in = a > 0.0 && a < 1.0; /* with a_clear: inside (eps, 1 - eps); else beyond -eps or 1 + eps */
-	const bool b_in = b > 0.0 && b < 1.0;
-	certain &= parallel | (a_clear & (!a_in | b_clear));
-	return !parallel && a_in && b_in;
+	const pt_t dx = vsub(x1, x0), dy = vsub(y1, y0);
+	const double d = vcross(dy, dx), n = vcross(x0, dx) - vcross(y0, dx), m = vcross(x0, dy) - vcross(y0, dy);
+	if (fabs(d) < eps) {
+		return false;
+	}
+	const double s = d < 0 ? -1.0 : 1.0, D = fabs(d);
+	bool sure = true;
+	/* eps <= a <= 1 - eps and 0 <= b <= 1 (what lies beyond -eps or 1 + eps lies beyond these too; a
+	 * quotient's sign is exact) */
+	const bool inside = !quotient_below(s * n, D, eps, sure) && quotient_below(s * n, D, 1 - eps, sure) &&
+			    s * m >= 0 && quotient_below(s * m, D, 1.0, sure);
+	return sure ? inside : intersect(x0, x1, y0, y1, eps, nullptr) == 1;
 }
 
-/* false only when seg_distance(x, y0, y1, eps) is certainly not below eps */
-__device__ __forceinline__ bool may_touch_edge(pt_t x, pt_t y0, pt_t y1, double eps)
+/* `crossing` is intersect(p, far, a, b, eps, nullptr) == 1 wherever `crossing_certain` */
+__device__ __forceinline__ bool crossing_certain(const edge_sides_t &s, double side_f)
 {
-	const pt_t dy = vsub(y1, y0);
-	pt_t x1;
-	x1.x = x.x + dy.y;
-	x1.y = x.y - dy.x;
-	const pt_t dx = vsub(x1, x);
-	const double d = vcross(dy, dx);
-	const bool degenerate = fabs(d) < eps; /* the exact code leaves the foot point unset here */
-	const double a = (vcross(x, dx) - vcross(y0, dx)) * approx_rcp(degenerate ? 1.0 : d);
-	const pt_t s = { y0.x + a * dy.x - x.x, y0.y + a * dy.y - x.y };
-	/* the foot point computed exactly differs from this one by ~1e-12 (1 + |a|)(1 + |dy|) at most */
-	const double far = 1e-4 * (1.0 + fabs(a)) * (1.0 + fabs(dy.x) + fabs(dy.y));
-	return degenerate || !(vdot(s, s) > far * far);
+	const bool apart = (s.side_a > 0) != (s.side_b > 0);
+	return fmin(fabs(s.side_a), fabs(s.side_b)) > kSure &&
+	       (!apart || fmin(fabs(s.side_p), fabs(side_f)) > kSure);
+}
+__device__ __forceinline__ bool crossing(const edge_sides_t &s, double side_f)
+{
+	return (s.side_a > 0) != (s.side_b > 0) && (s.side_p > 0) != (side_f > 0);
+}
+
+/* Whether seg_distance(p, a, b, eps) < eps.  |side_p| is the
+ * distance to the edge's line times the edge's length, `along` the foot point's place on the edge times the
+ * length squared.  Distances come out to 1e-11 here and to 1e-13 in the exact code (edges are at least
+ * kMinEdge long), so a distance beyond 2 eps, or a foot point beyond an end by 1e-6 of the length, is a no.
+ * With the foot point as far inside the ends, a point on the side the exact code's perpendicular does not lead
+ * to the edge from is a no however close it is (its second quotient is below 0: `m` has that quotient's sign
+ * by the same operations), and one on the line or on the other side within half an eps is a yes.  What is
+ * left goes through the exact code, as does an edge of length 0 (some polygons list their first vertex
+ * again). */
+constexpr double kMinEdge = 0.04;
+__device__ __forceinline__ bool touches_edge(pt_t p, pt_t a, pt_t b, const edge_sides_t &s, double eps)
+{
+	const pt_t d = vsub(b, a);
+	const double along = vdot(vsub(p, a), d), len2 = vdot(d, d), ends = 1e-6 * len2;
+	const double far2 = s.side_p * s.side_p, eps2 = eps * eps * len2;
+	const double m = vcross(p, d) - vcross(a, d);
+	const bool within = along > ends && along < len2 - ends;
+	const bool no = far2 > 4.0 * eps2 || along < -ends || along > len2 + ends || (within && m > 0);
+	const bool yes = within && m <= 0 && far2 < 0.25 * eps2;
+	return yes || (!no && seg_distance(p, a, b, eps) < eps);
+}
+
+/* A point with |side_p| beyond this is farther than kSure from the edge's line: touches_edge is false */
+__device__ __forceinline__ double touch_reach(pt_t a, pt_t b)
+{
+	return kSure * (fabs(b.x - a.x) + fabs(b.y - a.y));
 }
 
 /* The bounds is_inside_region computes (:177-196): selections only, so the host can do it
@@ -393,86 +441,55 @@ __host__ __device__ inline void region_bounds(const pt_t *v, int n, double out[4
 	out[3] = max_y;
 }
 
-/* is_inside_region, :159-221; `bounds` is region_bounds of the same polygon */
-__device__ __forceinline__ int inside_region(pt_t point, const pt_t *v, int n, const double *bounds,
-					      pt_t far_point)
+/* The edges of polygon i of a set as bits of a wavefront's lanes (edge e of the set is lane e's) */
+__device__ __forceinline__ uint64_t edge_lanes(int first_edge, int count)
 {
-	const double eps = 1e-10;
-	const double min_x = bounds[0], max_x = bounds[1], min_y = bounds[2], max_y = bounds[3];
-	/* The reference looks for a point on an edge first (result 0) and rejects by bounding
-	 * box second (result -1).  A point more than 1e-6 outside the box cannot be within
-	 * 1e-10 of an edge -- edges lie inside the box, and the foot of the perpendicular may
-	 * leave the segment by at most eps times its length -- so for such a point the second
-	 * answer is known without looking at the edges.  Most polygons are dismissed here. */
-	const double margin = 1e-6;
-	if (point.x < min_x - margin || point.x > max_x + margin || point.y < min_y - margin ||
-	    point.y > max_y + margin) {
-		return -1;
-	}
-	/* One branch-free walk over the edges (at most 20, one bit each) serves both of the
-	 * reference's loops, the on-edge search (:168-175) and the crossing count (:207-219); the
-	 * edges whose answer it could not be certain of are then put through the exact code. */
-	const pt_t ray = vsub(far_point, point);
-	uint32_t touch = 0, unsure = 0;
-	int crosses = 0;
-	pt_t a = v[n - 1];
-#pragma unroll 4
-	for (int i = 0; i < n; i++) { /* edge (i - 1, i): the same edges, starting from the closing one */
-		const pt_t b = v[i];
-		bool certain = true;
-		const bool crossing = crosses_edge(point, ray, a, b, eps, certain);
-		touch |= (uint32_t)may_touch_edge(point, a, b, eps) << i;
-		unsure |= (uint32_t)!certain << i;
-		crosses += (crossing & certain) ? 1 : 0;
-		a = b;
-	}
-	while (touch != 0) {
-		const int i = __ffs(touch) - 1;
-		touch &= touch - 1;
-		if (seg_distance(point, v[i == 0 ? n - 1 : i - 1], v[i], eps) < eps) {
-			return 0;
-		}
-	}
-	if (point.x < min_x || point.x > max_x || point.y < min_y || point.y > max_y) {
-		return -1;
-	}
-	while (unsure != 0) {
-		const int i = __ffs(unsure) - 1;
-		unsure &= unsure - 1;
-		if (intersect(point, far_point, v[i == 0 ? n - 1 : i - 1], v[i], eps, nullptr) == 1) {
-			crosses++;
-		}
-	}
-	return (crosses & 1) ? 1 : -1;
+	return (count >= 64 ? ~0ull : (1ull << count) - 1ull) << first_edge;
 }
 
-/* calculateChunkSizeTreeLL128, :1883-1938 (constants: include/internal/tuner/nccl_defaults.h) */
-__device__ inline uint64_t chunk_tree_ll128(uint64_t message_size, int nChannels, int log2_nnodes)
+/* is_inside_region's bounding-box test (:159-221) */
+__device__ __forceinline__ bool in_bounds(pt_t p, const double *b, double margin)
+{
+	return !(p.x < b[0] - margin || p.x > b[1] + margin || p.y < b[2] - margin || p.y > b[3] + margin);
+}
+
+/*
+ * calculateChunkSizeTreeLL128, :1883-1938 (constants: include/internal/tuner/nccl_defaults.h), for the
+ * three channel counts its caller tries.  The chunk only ever takes the values kChunkLadder -- it starts
+ * at 640 threads x 120 elements x 8 bytes x 15/16 and is halved while the message has too few chunks for
+ * the tree's depth -- so every division is by a constant, the ladder's quotients do not wait for each
+ * other, and the payload of a rung (whole 1920-byte grains, 480 elements to 2048 bytes) is a
+ * constant too.  Messages are at most 32 MiB here.
+ */
+constexpr uint32_t kChunkLadder[6] = { 576000, 288000, 144000, 72000, 36000, 18000 };
+constexpr uint64_t chunk_payload(uint32_t chunk)
+{
+	const uint32_t grain = 32 * 8 / 16 * 15 * 8; /* 1920 bytes */
+	const uint32_t nelem = chunk / grain * (grain / 4);
+	return (uint64_t)((nelem + 479) / 480) * 256 * 8;
+}
+
+template <uint32_t CHANNELS>
+__device__ __forceinline__ uint64_t chunk_tree_ll128(uint32_t message_size, int log2_nnodes)
 {
 	const int ppn = 8;
-	const uint64_t STEPS = 8, ELEMS_PER_THREAD = 120, MAX_NTHREADS = 640;
-	const uint64_t LINEELEMS = 16, DATAELEMS = 15, WARP = 32, SHMEM_ELEMS = 8;
-
-	uint64_t buffSize = ELEMS_PER_THREAD * MAX_NTHREADS * STEPS * 8;
-	uint64_t chunkSize = buffSize / STEPS;
-	chunkSize = (chunkSize / LINEELEMS) * DATAELEMS;
-	double nSteps = 1 + log2_nnodes + 0.1 * ppn;
-
-	while ((double)(message_size / ((uint64_t)nChannels * chunkSize)) < nSteps * 64 / ppn &&
-	       chunkSize > 131072) {
-		chunkSize /= 2;
+	const double nSteps = 1 + log2_nnodes + 0.1 * ppn;
+	const double deep = nSteps * 64 / ppn, shallow = nSteps * 16 / ppn;
+	int rung = 0;
+#pragma unroll
+	for (int k = 0; k < 3; k++) { /* while chunk > 131072 */
+		rung += rung == k && (double)(message_size / (CHANNELS * kChunkLadder[k])) < deep;
 	}
-	while ((double)(message_size / ((uint64_t)nChannels * chunkSize)) < nSteps * 16 / ppn &&
-	       chunkSize > 32768) {
-		chunkSize /= 2;
+#pragma unroll
+	for (int k = 0; k < 5; k++) { /* while chunk > 32768 */
+		rung += rung == k && (double)(message_size / (CHANNELS * kChunkLadder[k])) < shallow;
 	}
-	uint64_t grainSize = WARP * SHMEM_ELEMS / LINEELEMS * DATAELEMS * 8;
-	chunkSize = (chunkSize / grainSize) * grainSize;
-	uint64_t elementsPerGrain = grainSize / 4;
-	uint64_t nelem = (chunkSize / grainSize) * elementsPerGrain;
-	uint64_t WireWordPerSlice = WARP * SHMEM_ELEMS;
-	uint64_t DataEltPerSlice = (WireWordPerSlice - WireWordPerSlice / LINEELEMS) * 2;
-	return (uint64_t)(ceil((double)nelem / (double)DataEltPerSlice) * (double)WireWordPerSlice * 8.0);
+	uint64_t payload = chunk_payload(kChunkLadder[0]);
+#pragma unroll
+	for (int k = 1; k < 6; k++) {
+		payload = rung == k ? chunk_payload(kChunkLadder[k]) : payload;
+	}
+	return payload;
 }
 
 __device__ __forceinline__ int log2i_nodes(uint64_t nodes)
@@ -482,45 +499,18 @@ __device__ __forceinline__ int log2i_nodes(uint64_t nodes)
 }
 
 /* Which polygon set answers for (platform, collective, ranks per node): shape selection as in
- * the per-platform init functions (:302,:485,:675,:768,:878,...).  count 0: no regions. */
-__host__ __device__ __forceinline__ void region_set(const region_tables_t &t, int platform, int coll, uint64_t ranks,
-					    uint64_t nodes, int &first, int &count)
+ * the per-platform init functions (:302,:485,:675,:768,:878,...).  The host looks it up: kernels get
+ * the set. */
+inline region_set_t region_set(const region_tables_t &t, int platform, int coll, uint64_t ranks, uint64_t nodes)
 {
-	first = 0;
-	count = 0;
 	int shape = -1;
 	if (ranks == 8 * nodes) shape = 0;
 	else if (ranks == 2 * nodes && platform == OFI_AMD_PLATFORM_P5_P5E) shape = 1;
 	else if (ranks == nodes) shape = 2;
-	if (platform < 0 || platform >= kNumPlatforms || shape < 0 || coll < 0 || coll >= NUM_FUNCS ||
-	    t.set_count[platform][shape][coll] <= 0) {
-		return;
+	if (platform < 0 || platform >= kNumPlatforms || shape < 0 || coll < 0 || coll >= NUM_FUNCS) {
+		return region_set_t{};
 	}
-	first = t.set_first[platform][shape][coll];
-	count = t.set_count[platform][shape][coll];
-}
-
-/* The loop of region_get_coll_info_internal_v3 (:2106-2128) over one set: the first polygon that
- * holds the point (inside or on an edge) wins.  Regions whose (algo, proto) bit is clear in
- * `mask` are passed over: for v3 those are the cells NCCL marked -1 or that lie beyond numAlgo /
- * numProto (:2109-2114); for v2 PAT and, without NVLS support, NVLS tree (:2023-2030).
- * poly: 4 ints per polygon, its vertex index relative to `verts`; bounds: 4 doubles per polygon.
- * The arrays may live in global memory or in LDS. */
-__device__ __forceinline__ int region_pick(const int32_t *poly, const double *bounds, const pt_t *verts,
-					    int count, pt_t p, uint32_t mask, pt_t far_point, int &a, int &pr)
-{
-	int in_out = -1;
-	a = -1;
-	pr = -1;
-	for (int i = 0; i < count && in_out < 0; i++) {
-		a = poly[i * 4 + 0];
-		pr = poly[i * 4 + 1];
-		if (!allowed(mask, a, pr)) {
-			continue;
-		}
-		in_out = inside_region(p, &verts[poly[i * 4 + 2]], poly[i * 4 + 3], &bounds[i * 4], far_point);
-	}
-	return in_out;
+	return t.set[platform][shape][coll];
 }
 
 /* The nChannels override of the chosen region (:2135-2153), -1 when there is none. */
@@ -531,16 +521,11 @@ __device__ __forceinline__ int region_channels(int platform, uint64_t size, uint
 	if (platform == OFI_AMD_PLATFORM_P6 && size >= 4 * 1024 * 1024 && size <= 32 * 1024 * 1024 &&
 	    algorithm == ALGO_TREE && protocol == PROTO_LL128 && nodes * 8 == ranks) { /* :2140-2146 */
 		const int log2_nnodes = log2i_nodes(nodes);
-		const int channels[3] = { 16, 24, 32 };
-		int best = 0;
-		uint64_t max_chunk = 0;
-		for (int c = 0; c < 3; c++) { /* calculateBestNChannelTree, :1955-1971 */
-			uint64_t payload = chunk_tree_ll128(size, channels[c], log2_nnodes);
-			if (payload > max_chunk || (payload == max_chunk && channels[c] > best)) {
-				max_chunk = payload;
-				best = channels[c];
-			}
-		}
+		/* calculateBestNChannelTree, :1955-1971: the largest payload, the most channels when they tie */
+		const uint32_t bytes = (uint32_t)size;
+		const uint64_t with16 = chunk_tree_ll128<16>(bytes, log2_nnodes), with24 = chunk_tree_ll128<24>(bytes, log2_nnodes),
+			       with32 = chunk_tree_ll128<32>(bytes, log2_nnodes);
+		const int best = with32 >= with24 && with32 >= with16 ? 32 : (with24 >= with16 ? 24 : 16);
 		nchannels = best;
 	}
 	if (platform == OFI_AMD_PLATFORM_P6 && size <= 32 * 1024 * 1024 && algorithm == ALGO_PAT &&
@@ -551,29 +536,6 @@ __device__ __forceinline__ int region_channels(int platform, uint64_t size, uint
 		else if (size <= nodes * 65536 * 2) nchannels = 2;
 	}
 	return nchannels;
-}
-
-/* region_get_coll_info_internal_v3, :2070-2157, for one point with the tables in global memory.
- * p = (log2 bytes, log2 ranks) as transform_log2 gives them. */
-__device__ inline void region_choose(const region_tables_t &t, int platform, int coll, uint64_t size,
-				     uint64_t ranks, uint64_t nodes, pt_t p, uint32_t mask,
-				     int &algorithm, int &protocol, int &nchannels)
-{
-	algorithm = -1;
-	protocol = -1;
-	nchannels = -1;
-	int first, count;
-	region_set(t, platform, coll, ranks, nodes, first, count);
-	if (count <= 0 || nodes <= 2) {
-		return;
-	}
-	int a, pr;
-	if (region_pick(&t.poly[first * 4], &t.bbox[first * 4], t.verts, count, p, mask, t.far_point, a, pr) < 0) {
-		return;
-	}
-	algorithm = a;
-	protocol = pr;
-	nchannels = region_channels(platform, size, ranks, nodes, a, pr);
 }
 
 /* region_get_chunk_size_internal, :2276-2306, with chunkSizeTuningTreeLL128P5en

@@ -32,6 +32,10 @@ struct grid_dims_t {
 	const double *log2_nodes; /* log2((double)nodes[i]) from the host's libm */
 	const double *log2_sizes; /* per size index: transform_log2 of the byte count */
 	const double *log2_ranks; /* per (node, ppn): transform_log2 of the rank count */
+	/* tiles of the region grid: 2^tile_shift node counts x 2^(6 - tile_shift) sizes, a wavefront each */
+	uint32_t tile_shift, tiles_n, tiles_s;
+	const double2 *size_span; /* per tile row: smallest and largest log2_sizes */
+	const double2 *rank_span; /* per (tile column, ppn): smallest and largest log2_ranks */
 };
 
 /*
@@ -146,102 +150,241 @@ __global__ __launch_bounds__(256) void model_grid_kernel(grid_dims_t g,
 	}
 }
 
-constexpr int kMaxSetPolys = 8;  /* polygons of one (platform, shape, collective) set */
-constexpr int kMaxSetVerts = 64; /* their vertices together */
+constexpr int kMaxSetEdges = 64; /* of one (platform, shape, collective) set: one per lane */
 constexpr uint32_t kRegionBlock = 64; /* threads per workgroup of the region kernel: one wavefront */
+constexpr uint64_t kMostRuns = 65535; /* of one launch: gridDim.y */
 constexpr uint32_t kXcds = 8;         /* workgroup w of a launch runs on XCD w mod 8, each with its own L2 */
-static_assert(kRegionBlock >= (uint32_t)kMaxSetVerts && kRegionBlock >= (uint32_t)kMaxSetPolys * 4,
-	      "one thread per staged vertex and per staged polygon word");
+static_assert(kRegionBlock >= (uint32_t)kMaxSetEdges, "one lane per edge of a set");
+
+/* One (platform entry, collective, ranks per node) of a region grid: where its points go and which
+ * polygons answer for it (region_set, looked up by the host: ranks = nodes * ppn, so the shape is a
+ * function of ppn). */
+struct region_run_t {
+	uint32_t entry, ci, pi, ppn;
+	uint32_t first_poly, first_edge;
+	uint32_t counts;   /* edges << 16 | polygons; 0: no regions.  Whole words: they come through the scalar cache */
+	int32_t platform;
+};
+
+
+/* What a whole tile knows about one edge of its polygon set */
+struct tile_edge_t {
+	bool crossed;  /* the ray of every point of the tile crosses it, and certainly so (crossing_certain) */
+	bool by_point; /* some points' rays may cross it and some may not: each point looks for itself */
+	bool near;     /* a point of the tile may lie on it */
+};
 
 /*
- * One thread per point.  A workgroup (one wavefront) works on 64 points of one (collective,
- * ranks per node) pair -- `blocks_per_run` chunks make up the pair's n_sizes x n_nodes points,
- * node count fastest -- because the polygon set depends on that pair alone: the set (at most 8 polygons, 64 vertices, with their bounds) is copied into LDS
- * once and every lane then walks the same polygons out of LDS instead of chasing them through
- * global memory, and workgroups of pairs without regions leave after one table lookup.
+ * Edge e against the tile [lo.x, hi.x] x [lo.y, hi.y].  The sides of edge_sides are affine in the
+ * point, so over the tile each lies between its values at the four corners: when those are all beyond
+ * kTileSure on one side, every point's certain answer is the same.  The ends of most edges lie
+ * outside the narrow fan of rays between a tile and the far point.
+ */
+constexpr double kTileSure = 1e-3; /* > kSure */
+__device__ __forceinline__ tile_edge_t tile_edge(const edge_t &e, pt_t lo, pt_t hi, pt_t far, double side_f)
+{
+	const pt_t d = vsub(e.b, e.a), fa = vsub(e.a, far), fb = vsub(e.b, far);
+	bool a_pos = true, a_neg = true, b_pos = true, b_neg = true, p_pos = true, p_neg = true;
+	const double beside = kTileSure * (1.0 + fabs(d.x) + fabs(d.y));
+	bool left = true, right = true; /* the whole tile on one side of the edge's line, and not close to it */
+#pragma unroll
+	for (int k = 0; k < 4; k++) {
+		const pt_t c = { (k & 1) ? hi.x : lo.x, (k & 2) ? hi.y : lo.y };
+		const pt_t fc = vsub(c, far);
+		const double sa = vcross(fc, fa), sb = vcross(fc, fb), sp = vcross(vsub(c, e.a), d);
+		a_pos &= sa > kTileSure, a_neg &= sa < -kTileSure;
+		b_pos &= sb > kTileSure, b_neg &= sb < -kTileSure;
+		p_pos &= sp > kTileSure, p_neg &= sp < -kTileSure;
+		left &= sp > beside, right &= sp < -beside;
+	}
+	const bool f_pos = side_f > kTileSure, f_neg = side_f < -kTileSure;
+	const bool together = (a_pos && b_pos) || (a_neg && b_neg);
+	const bool apart = (a_pos && b_neg) || (a_neg && b_pos);
+	const bool between = (p_pos && f_neg) || (p_neg && f_pos);
+	const bool beyond = (p_pos && f_pos) || (p_neg && f_neg);
+	tile_edge_t r;
+	r.crossed = apart && between;
+	r.by_point = !(together || (apart && (between || beyond)));
+	bool near = !(left || right); /* &= : no branches between the comparisons */
+	near &= fmin(e.a.x, e.b.x) <= hi.x + kTileSure;
+	near &= fmax(e.a.x, e.b.x) >= lo.x - kTileSure;
+	near &= fmin(e.a.y, e.b.y) <= hi.y + kTileSure;
+	near &= fmax(e.a.y, e.b.y) >= lo.y - kTileSure;
+	r.near = near;
+	return r;
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane)
+{
+	const uint64_t bits = (uint64_t)__double_as_longlong(v);
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, lane);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), lane);
+	return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+/* all lanes when m is not 0, else none */
+__device__ __forceinline__ uint64_t every(uint64_t m)
+{
+	return m != 0 ? ~0ull : 0ull;
+}
+
+/* The points of a wavefront against one edge, a bit per point: whether its ray crosses the edge, and whether
+ * that is certain (crossing, crossing_certain). */
+struct point_edge_t {
+	uint64_t crossing, sure;
+};
+__device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64_t f_positive, uint64_t f_sure)
+{
+	const uint64_t apart = __ballot(s.side_a > 0) ^ __ballot(s.side_b > 0);
+	point_edge_t r;
+	r.crossing = apart & (__ballot(s.side_p > 0) ^ f_positive);
+	r.sure = __ballot(fabs(s.side_a) > kSure) & __ballot(fabs(s.side_b) > kSure) &
+		 (~apart | (__ballot(fabs(s.side_p) > kSure) & f_sure));
+	return r;
+}
+
+/*
+ * One thread per point.  A workgroup (one wavefront) works on a tile of neighbouring sizes and node
+ * counts of one (collective, ranks per node) pair, because the polygon set depends on that pair
+ * alone.  The launch is bound by arithmetic (chains of fp64 operations), so a wavefront first
+ * works out, one edge per lane, what its whole tile has in common about each edge of the set
+ * (tile_edge); the points then only look at the edges about which they differ -- those with an end in the
+ * fan of rays from the tile to the far point, and those the tile touches -- read out of the
+ * lanes that hold them.  A tile has one such edge at the median and 20 at the most; every edge for every
+ * point, with quotients, took 40-42 us for 1.02 M points of four platforms (560 sizes, 38 node counts),
+ * this takes 12.0: 5 us of it are the dispatch of 16,896 wavefronts, the rest the time of the
+ * tiles with the most edges, which is why their turns count instructions (two edges a turn, for
+ * shorter chains of dependent operations, was slower: 13.3).
  *
- * In the output the ranks-per-node index runs fastest, so a wavefront's 64 records lie 4 x
- * n_ppn bytes apart and the records between them belong to the same chunk's other
+ * In the output the ranks-per-node index runs fastest, so a wavefront's records lie 4 x
+ * n_ppn bytes apart and the records between them belong to the same tile's other
  * ranks-per-node values, i.e. to other workgroups.  Those workgroups are given numbers that
  * are equal mod 8: they run on the same XCD, their partial writes to a cache line meet in that
  * XCD's L2 and leave it as one line (measured: 4.7 MB written for 4.7 MB of records; with the
- * workgroups of a chunk on different XCDs every L2 wrote its quarter of each line, 18.9 MB).
- * Giving a thread all ranks-per-node values of its point, or a workgroup four wavefronts that
- * share an LDS staging buffer, writes the same 4.7 MB but makes the units of work four times
- * coarser, and the launch, which lasts as long as its most loaded SIMD, 15-18 % longer than
- * with single-wavefront units.
+ * workgroups of a tile on different XCDs every L2 wrote its quarter of each line, 18.9 MB).
  */
-__global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t g, region_tables_t t,
-							    const int32_t *__restrict__ platforms,
-							    uint32_t points_per_platform, uint32_t blocks_per_run,
-							    const uint2 *__restrict__ order, int8_t *__restrict__ choice)
+__global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t g, const int32_t *__restrict__ polys,
+							    const double *__restrict__ bboxes,
+							    const edge_t *__restrict__ edges, pt_t far_point,
+							    const region_run_t *__restrict__ runs,
+							    uint32_t points_per_platform, int8_t *__restrict__ choice)
 {
-	__shared__ int32_t s_poly[kMaxSetPolys * 4];
-	__shared__ double s_bounds[kMaxSetPolys * 4];
-	__shared__ pt_t s_verts[kMaxSetVerts];
-
-	/* blockIdx.x = k * 8 + x (a one-dimensional grid, so x is the XCD).  order[k] names a
-	 * (platform entry, group, pi): chunk 8 * group + x' of the collectives' chunks,
-	 * ranks-per-node index pi -- whatever the order, the workgroups of one chunk and platform
-	 * entry share x.  The host lists the triples by falling cost (polygons of the pair's set):
-	 * the long workgroups start first and the short ones fill the end of the launch, and
-	 * workgroups of equal cost are neighbours in launch order, which the dispatcher deals to
-	 * the CUs of an XCD in turn.  (In (entry, group, pi) order, or scattered by a fixed stride,
-	 * the pairs with many regions recur at periods that keep meeting the same CUs: 74-78 us
-	 * against 54 us.) */
-	const uint32_t x = blockIdx.x % kXcds;
-	const uint2 item = order[blockIdx.x / kXcds];
-	const uint32_t entry = item.x;
-	const uint32_t pi = item.y % g.n_ppn;
-	const uint32_t group = item.y / g.n_ppn;
-	/* which of a group's eight chunks an XCD takes rotates with the platform entry: the chunks
-	 * differ in cost (collective, size range), and an XCD that kept the same ones for every
+	/* blockIdx.y names a run, blockIdx.x = 8 * group + x the tiles 8 * group .. 8 * group + 7 of it, of
+	 * which XCD x takes one (workgroups are dealt to the XCDs in launch order, and gridDim.x is a
+	 * multiple of 8).  The host lists the runs by falling cost (edges of the pair's set): the long
+	 * workgroups start first and the short ones fill the end of the launch. */
+	const uint32_t lane = threadIdx.x;
+	const region_run_t run = runs[blockIdx.y];
+	/* which of a group's eight tiles an XCD takes rotates with the platform entry: the tiles
+	 * differ in cost (size range), and an XCD that kept the same ones for every
 	 * entry would keep the same share of the long ones */
-	const uint32_t chunk = group * kXcds + (x + entry) % kXcds;
-	if (chunk >= blocks_per_run * g.n_colls) {
+	const uint32_t tile = (blockIdx.x & ~(kXcds - 1u)) + (blockIdx.x + run.entry) % kXcds;
+	if (tile >= g.tiles_n * g.tiles_s) {
 		return; /* padding of the last group */
 	}
-	const uint32_t ci = chunk / blocks_per_run;
-	const uint32_t in_run = (chunk - ci * blocks_per_run) * kRegionBlock + threadIdx.x;
-	const int platform = platforms[entry];
-	const int coll = g.colls[ci];
-	const uint32_t ppn = g.ppn[pi];
+	const uint32_t n_polys = run.counts & 0xffffu, n_edges = run.counts >> 16;
+	const uint32_t ts = tile / g.tiles_n, tn = tile - ts * g.tiles_n;
+	const uint32_t at_n = (tn << g.tile_shift) + (lane & ((1u << g.tile_shift) - 1u));
+	const uint32_t at_s = ts * (64u >> g.tile_shift) + (lane >> g.tile_shift);
+	const bool live = at_n < g.n_nodes && at_s < g.n_sizes;
+	/* lanes beyond the axes' ends stand on the tile's last point */
+	const uint32_t ni = min(at_n, g.n_nodes - 1u), si = min(at_s, g.n_sizes - 1u);
 
-	/* ranks = nodes * ppn with nodes >= 1: the shape is a function of ppn */
-	int first, count;
-	region_set(t, platform, coll, ppn, 1, first, count);
-	if (count > 0) {
-		const int v0 = t.poly[first * 4 + 2];
-		const int v_end = t.poly[(first + count - 1) * 4 + 2] + t.poly[(first + count - 1) * 4 + 3];
-		if ((int)threadIdx.x < count * 4) {
-			const int32_t w = t.poly[first * 4 + threadIdx.x];
-			s_poly[threadIdx.x] = (threadIdx.x & 3u) == 2u ? w - v0 : w; /* vertex index within the set */
-			s_bounds[threadIdx.x] = t.bbox[first * 4 + threadIdx.x];
+	int algorithm = -1, protocol = -1, nchannels = -1;
+	if (n_polys > 0) {
+		/* everything the wavefront needs is asked for at once: its edge and, in the first lanes, a
+		 * polygon's words and bounds; the loop below reads them out of the lanes */
+		const uint32_t my_poly = run.first_poly + min(lane, n_polys - 1u);
+		const int4 pw = reinterpret_cast<const int4 *>(polys)[my_poly];
+		const double4_t box = reinterpret_cast<const double4_t *>(bboxes)[my_poly];
+		/* lane e's edge; lanes beyond the set's edges take its last one and are masked out below */
+		const edge_t mine = edges[run.first_edge + min(lane, n_edges - 1u)];
+		const uint64_t nodes = g.nodes[ni];
+		const uint64_t size = g.sizes[si];
+		const pt_t at = { g.log2_sizes[si], g.log2_ranks[ni * g.n_ppn + run.pi] };
+		const double2 sx = g.size_span[ts], sy = g.rank_span[tn * g.n_ppn + run.pi];
+
+		const double eps = 1e-10;
+		const double mine_f = vcross(vsub(far_point, mine.a), vsub(mine.b, mine.a));
+		const double mine_reach = touch_reach(mine.a, mine.b);
+		const tile_edge_t te = tile_edge(mine, pt_t{ sx.x, sy.x }, pt_t{ sx.y, sy.y }, far_point, mine_f);
+		/* From here on conditions are masks of lanes in scalar registers -- lanes standing for edges, polygons
+		 * or points -- and the logic between them is scalar: no branch over lanes but the rare ones. */
+		const uint64_t all = edge_lanes(0, (int)n_edges);
+		const uint64_t crossed = __ballot(te.crossed) & all, by_point = __ballot(te.by_point) & all,
+			       near = __ballot(te.near) & all;
+		const uint64_t f_positive = __ballot(mine_f > 0), f_sure = __ballot(fabs(mine_f) > kSure);
+		/* The reference looks for a point on an edge first (result 0) and rejects by bounding
+		 * box second (result -1).  A point more than 1e-6 outside the box cannot be within
+		 * 1e-10 of an edge -- edges lie inside the box, and the foot of the perpendicular may
+		 * leave the segment by at most eps times its length -- so for such a point the second
+		 * answer is known without looking at the edges. */
+		const double margin = 1e-6;
+		const uint64_t apart_polys = __ballot(sx.x > box.y + margin) | __ballot(sx.y < box.x - margin) |
+					     __ballot(sy.x > box.w + margin) | __ballot(sy.y < box.z - margin);
+		const uint64_t whole_polys = __ballot(sx.x >= box.x) & __ballot(sx.y <= box.y) & __ballot(sy.x >= box.z) &
+					     __ballot(sy.y <= box.w);
+		const pt_t ray = vsub(far_point, at);
+		uint64_t open = __ballot(live) & __ballot(nodes > 2); /* the points still without a region */
+		for (uint64_t todo = edge_lanes(0, (int)n_polys) & ~apart_polys; todo != 0 && open != 0; todo &= todo - 1) {
+			const int i = __builtin_ctzll(todo);
+			uint64_t asks = open, in_box = ~0ull;
+			if (!((whole_polys >> i) & 1u)) {
+				const double x0 = lane_value(box.x, i), x1 = lane_value(box.y, i);
+				const double y0 = lane_value(box.z, i), y1 = lane_value(box.w, i);
+				asks &= __ballot(at.x >= x0 - margin) & __ballot(at.x <= x1 + margin) & __ballot(at.y >= y0 - margin) &
+					__ballot(at.y <= y1 + margin);
+				in_box = __ballot(at.x >= x0) & __ballot(at.x <= x1) & __ballot(at.y >= y0) & __ballot(at.y <= y1);
+				if (asks == 0) {
+					continue;
+				}
+			}
+			const uint64_t of_poly = edge_lanes(__builtin_amdgcn_readlane(pw.z, i) - (int)run.first_edge,
+							    __builtin_amdgcn_readlane(pw.w, i));
+			uint64_t odd = (__popcll(crossed & of_poly) & 1) ? ~0ull : 0ull; /* points with an odd number of crossings */
+			uint64_t touching = 0;
+			for (uint64_t left = (by_point | near) & of_poly; left != 0; left &= left - 1) {
+				const int e = __builtin_ctzll(left);
+				const uint64_t bit = left & -left;
+				const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
+				const pt_t b = { lane_value(mine.b.x, e), lane_value(mine.b.y, e) };
+				const edge_sides_t s = edge_sides(at, ray, a, b);
+				uint64_t unsure = 0, reached = 0;
+				if ((by_point & bit) != 0) {
+					const point_edge_t pe = point_edge(s, every(f_positive & bit), every(f_sure & bit));
+					unsure = asks & ~pe.sure;
+					odd ^= pe.crossing & ~unsure;
+				}
+				if ((near & bit) != 0) {
+					reached = asks & __ballot(fabs(s.side_p) <= lane_value(mine_reach, e));
+				}
+				if ((unsure | reached) != 0) {
+					bool c = false, t = false;
+					if ((unsure >> lane) & 1u) {
+						c = intersects(at, far_point, a, b, eps);
+					}
+					if ((reached >> lane) & 1u) {
+						t = touches_edge(at, a, b, s, eps);
+					}
+					odd ^= __ballot(c);
+					touching |= __ballot(t);
+				}
+			}
+			const uint64_t hit = asks & (touching | (odd & in_box));
+			const int a = __builtin_amdgcn_readlane(pw.x, i), pr = __builtin_amdgcn_readlane(pw.y, i);
+			algorithm = (hit >> lane) & 1u ? a : algorithm;
+			protocol = (hit >> lane) & 1u ? pr : protocol;
+			open &= ~hit;
 		}
-		if ((int)threadIdx.x < v_end - v0) {
-			s_verts[threadIdx.x] = t.verts[v0 + threadIdx.x];
+		if (algorithm >= 0) {
+			nchannels = region_channels(run.platform, size, nodes * run.ppn, nodes, algorithm, protocol);
 		}
-		__syncthreads();
 	}
-	if (in_run >= g.n_sizes * g.n_nodes) {
+	if (!live) {
 		return;
 	}
-	const uint32_t ni = in_run % g.n_nodes;
-	const uint32_t si = in_run / g.n_nodes;
-	const uint32_t p = ((ci * g.n_sizes + si) * g.n_nodes + ni) * g.n_ppn + pi; /* output order */
-
-	const uint64_t nodes = g.nodes[ni];
-	int algorithm = -1, protocol = -1, nchannels = -1;
-	if (count > 0 && nodes > 2) {
-		int a, pr;
-		const pt_t at = { g.log2_sizes[si], g.log2_ranks[ni * g.n_ppn + pi] };
-		if (region_pick(s_poly, s_bounds, s_verts, count, at, kAllAllowed, t.far_point, a, pr) >= 0) {
-			algorithm = a;
-			protocol = pr;
-			nchannels = region_channels(platform, g.sizes[si], nodes * ppn, nodes, a, pr);
-		}
-	}
-	const uint64_t idx = (uint64_t)entry * points_per_platform + p;
+	const uint32_t p = ((run.ci * g.n_sizes + si) * g.n_nodes + ni) * g.n_ppn + run.pi; /* output order */
+	const uint64_t idx = (uint64_t)run.entry * points_per_platform + p;
 	/* {int8 algorithm, int8 protocol, int16 nchannels} as one 4-byte store */
 	reinterpret_cast<uint32_t *>(choice)[idx] = ((uint32_t)(uint8_t)(int8_t)algorithm) |
 						     ((uint32_t)(uint8_t)(int8_t)protocol << 8) |
@@ -295,19 +438,46 @@ int upload(const std::vector<T> &host, T **dev)
 	return 0;
 }
 
+/* puts v's elements behind what `to` holds, on a 16-byte boundary; where they begin */
+template <typename T>
+size_t append(std::vector<uint8_t> &to, const std::vector<T> &v)
+{
+	const size_t at = (to.size() + 15) / 16 * 16;
+	to.resize(at + v.size() * sizeof(T));
+	std::memcpy(to.data() + at, v.data(), v.size() * sizeof(T));
+	return at;
+}
+
+/* log2 of the node counts per tile: of 4, 8 and 16 the one that leaves the fewest lanes idle at the
+ * end of the axis, 8 x 8 when they tie (a square tile has the narrowest fan of rays) */
+uint32_t pick_tile_shift(uint32_t n_nodes)
+{
+	uint32_t best = 3;
+	for (const uint32_t shift : { 2u, 4u }) {
+		const uint32_t padded = (n_nodes + (1u << shift) - 1) >> shift << shift;
+		const uint32_t padded_best = (n_nodes + (1u << best) - 1) >> best << best;
+		best = padded < padded_best ? shift : best;
+	}
+	return best;
+}
+
+/* smallest and largest of v[k * stride + at], k in [from, to) */
+double2 span_of(const double *v, uint32_t from, uint32_t to, uint32_t stride, uint32_t at)
+{
+	double2 span = { v[(size_t)from * stride + at], v[(size_t)from * stride + at] };
+	for (uint32_t k = from + 1; k < to; k++) {
+		span.x = std::min(span.x, v[(size_t)k * stride + at]);
+		span.y = std::max(span.y, v[(size_t)k * stride + at]);
+	}
+	return span;
+}
+
 int build_region_tables(region_tables_t *t)
 {
 	std::vector<int32_t> poly;
-	std::vector<pt_t> verts;
+	std::vector<edge_t> edges;
 	std::vector<double> bounds;
-	for (int p = 0; p < kNumPlatforms; p++) {
-		for (int s = 0; s < kNumShapes; s++) {
-			for (int c = 0; c < NUM_FUNCS; c++) {
-				t->set_first[p][s][c] = 0;
-				t->set_count[p][s][c] = 0;
-			}
-		}
-	}
+	std::memset(t->set, 0, sizeof(t->set));
 	const pt_t z = { kTunerMaxSize, kTunerMaxRanks };
 	for (int s = 0; s < OFI_REGION_NUM_SETS; s++) {
 		const int *set = ofi_region_sets[s];
@@ -320,21 +490,17 @@ int build_region_tables(region_tables_t *t)
 			const double *r = ofi_region_exts[set[5] + e];
 			ext[e] = extend(pt_t{ r[0], r[1] }, pt_t{ r[2], r[3] }, z);
 		}
-		t->set_first[set[0]][shape][set[2]] = (int32_t)(poly.size() / 4);
-		t->set_count[set[0]][shape][set[2]] = set[4];
-		const size_t set_first_vertex = verts.size();
-		if (set[4] > kMaxSetPolys) {
-			return -EINVAL;
-		}
+		const size_t first_poly = poly.size() / 4, first_edge = edges.size();
 		for (int q = 0; q < set[4]; q++) {
 			const int *pd = ofi_region_polys[set[3] + q];
-			if (pd[3] < 2 || pd[3] > kMaxVertices) {
+			if (pd[3] < 2) {
 				return -EINVAL;
 			}
 			poly.push_back(pd[0]);
 			poly.push_back(pd[1]);
-			poly.push_back((int32_t)verts.size());
+			poly.push_back((int32_t)edges.size());
 			poly.push_back(pd[3]);
+			std::vector<pt_t> verts;
 			for (int v = 0; v < pd[3]; v++) {
 				const int *kind = ofi_region_vert_kind[pd[2] + v];
 				const double *xy = ofi_region_vert_xy[pd[2] + v];
@@ -348,31 +514,41 @@ int build_region_tables(region_tables_t *t)
 				verts.push_back(to_log2(pt)); /* set_regions, :236-247 */
 			}
 			double b[4];
-			region_bounds(&verts[verts.size() - pd[3]], pd[3], b);
+			region_bounds(verts.data(), pd[3], b);
 			bounds.insert(bounds.end(), b, b + 4);
+			for (int k = 0; k < pd[3]; k++) {
+				const edge_t e = { verts[k == 0 ? pd[3] - 1 : k - 1], verts[k] };
+				const double length = std::hypot(e.b.x - e.a.x, e.b.y - e.a.y);
+				if (length != 0 && length < kMinEdge) {
+					return -EINVAL; /* the certain-answer tests rely on it */
+				}
+				edges.push_back(e);
+			}
 		}
-		if (verts.size() - set_first_vertex > (size_t)kMaxSetVerts) {
-			return -EINVAL; /* the grid kernel keeps one set in LDS */
+		if (edges.size() - first_edge > (size_t)kMaxSetEdges || edges.size() > 65535 || set[4] > kMaxSetEdges) {
+			return -EINVAL; /* the kernels keep one edge (and one polygon) of a set per lane */
 		}
+		t->set[set[0]][shape][set[2]] = region_set_t{ (uint16_t)first_poly, (uint16_t)set[4], (uint16_t)first_edge,
+							      (uint16_t)(edges.size() - first_edge) };
 	}
 	t->far_point = to_log2(pt_t{ 2.0 * kTunerMaxSize, 2.0 * kTunerMaxRanks });
 	int32_t *d_poly = nullptr;
-	pt_t *d_verts = nullptr;
+	edge_t *d_edges = nullptr;
 	double *d_bounds = nullptr;
 	int rc = upload(poly, &d_poly);
 	if (rc == 0) {
-		rc = upload(verts, &d_verts);
+		rc = upload(edges, &d_edges);
 	}
 	if (rc == 0) {
 		rc = upload(bounds, &d_bounds);
 	}
 	if (rc != 0) {
 		(void)hipFree(d_poly);
-		(void)hipFree(d_verts);
+		(void)hipFree(d_edges);
 		return rc;
 	}
 	t->poly = d_poly;
-	t->verts = d_verts;
+	t->edges = d_edges;
 	t->bbox = d_bounds;
 	return 0;
 }
@@ -422,23 +598,17 @@ struct ofi_amd_tuner_plan {
 	region_tables_t t;
 	uint64_t points;
 	uint64_t cells;
-	/* owned device allocations */
-	int32_t *d_colls, *d_algos;
-	uint64_t *d_sizes, *d_nodes;
-	uint32_t *d_ppn;
-	double *d_log2_nodes, *d_log2_sizes, *d_log2_ranks;
-	/* per-call variant / platform staging (device) */
+	void *d_axes; /* owned: what g's pointers point into */
+	/* per-call staging (device): the variants, and the runs of the platform list */
 	ofi_amd_tuner_variant_t *d_variants;
-	int32_t *d_platforms;
-	uint32_t variants_cap, platforms_cap;
-	/* what d_variants currently holds, so that an unchanged list is not uploaded again */
+	region_run_t *d_runs;
+	uint32_t variants_cap;
+	uint64_t runs_cap;
+	/* what they currently hold, so that an unchanged list is not uploaded again */
 	std::vector<ofi_amd_tuner_variant_t> h_variants;
 	std::vector<int32_t> h_platforms;
-	/* region launch order for the current platform list (see region_choice_kernel) */
 	std::vector<int32_t> h_colls;
 	std::vector<uint32_t> h_ppn;
-	uint2 *d_order;
-	uint64_t order_cap;
 };
 
 using namespace ofi_amd;
@@ -450,17 +620,9 @@ int ofi_amd_tuner_plan_destroy(ofi_amd_tuner_plan_t *plan)
 	if (!plan) {
 		return -EINVAL;
 	}
-	(void)hipFree(plan->d_colls);
-	(void)hipFree(plan->d_algos);
-	(void)hipFree(plan->d_sizes);
-	(void)hipFree(plan->d_nodes);
-	(void)hipFree(plan->d_ppn);
-	(void)hipFree(plan->d_log2_nodes);
-	(void)hipFree(plan->d_log2_sizes);
-	(void)hipFree(plan->d_log2_ranks);
+	(void)hipFree(plan->d_axes);
 	(void)hipFree(plan->d_variants);
-	(void)hipFree(plan->d_platforms);
-	(void)hipFree(plan->d_order);
+	(void)hipFree(plan->d_runs);
 	delete plan;
 	return 0;
 }
@@ -522,14 +684,35 @@ int ofi_amd_tuner_plan_create(const int32_t *colls, uint32_t n_colls, const uint
 		log2_sizes[i] = log2_coord((double)sizes[i]);
 	}
 
-	rc = upload(std::vector<int32_t>(colls, colls + n_colls), &plan->d_colls);
-	if (rc == 0) rc = upload(std::vector<int32_t>(algos, algos + n_algos), &plan->d_algos);
-	if (rc == 0) rc = upload(std::vector<uint64_t>(sizes, sizes + n_sizes), &plan->d_sizes);
-	if (rc == 0) rc = upload(std::vector<uint64_t>(nodes, nodes + n_nodes), &plan->d_nodes);
-	if (rc == 0) rc = upload(std::vector<uint32_t>(ppn, ppn + n_ppn), &plan->d_ppn);
-	if (rc == 0) rc = upload(log2_nodes, &plan->d_log2_nodes);
-	if (rc == 0) rc = upload(log2_sizes, &plan->d_log2_sizes);
-	if (rc == 0) rc = upload(log2_ranks, &plan->d_log2_ranks);
+	/* tiles of the region grid and the span of coordinates of each */
+	const uint32_t tile_shift = pick_tile_shift(n_nodes);
+	const uint32_t per_col = 1u << tile_shift, per_row = 64u >> tile_shift;
+	const uint32_t tiles_n = (n_nodes + per_col - 1) / per_col, tiles_s = (n_sizes + per_row - 1) / per_row;
+	std::vector<double2> size_span(tiles_s), rank_span((size_t)tiles_n * n_ppn);
+	for (uint32_t k = 0; k < tiles_s; k++) {
+		size_span[k] = span_of(log2_sizes.data(), k * per_row, std::min(n_sizes, (k + 1) * per_row), 1, 0);
+	}
+	for (uint32_t k = 0; k < tiles_n; k++) {
+		for (uint32_t j = 0; j < n_ppn; j++) {
+			rank_span[(size_t)k * n_ppn + j] =
+				span_of(log2_ranks.data(), k * per_col, std::min(n_nodes, (k + 1) * per_col), n_ppn, j);
+		}
+	}
+
+	/* one allocation and one copy for all of it */
+	grid_dims_t &g = plan->g;
+	std::vector<uint8_t> axes;
+	const size_t at_spans = append(axes, size_span), at_rank_spans = append(axes, rank_span);
+	const size_t at_sizes = append(axes, std::vector<uint64_t>(sizes, sizes + n_sizes));
+	const size_t at_nodes = append(axes, std::vector<uint64_t>(nodes, nodes + n_nodes));
+	const size_t at_log2_nodes = append(axes, log2_nodes), at_log2_sizes = append(axes, log2_sizes);
+	const size_t at_log2_ranks = append(axes, log2_ranks);
+	const size_t at_colls = append(axes, std::vector<int32_t>(colls, colls + n_colls));
+	const size_t at_algos = append(axes, std::vector<int32_t>(algos, algos + n_algos));
+	const size_t at_ppn = append(axes, std::vector<uint32_t>(ppn, ppn + n_ppn));
+	uint8_t *d_axes = nullptr;
+	rc = upload(axes, &d_axes);
+	plan->d_axes = d_axes;
 	if (rc != 0) {
 		ofi_amd_tuner_plan_destroy(plan);
 		return rc;
@@ -542,20 +725,24 @@ int ofi_amd_tuner_plan_create(const int32_t *colls, uint32_t n_colls, const uint
 		ofi_amd_tuner_plan_destroy(plan);
 		return -ENOMEM;
 	}
-	grid_dims_t &g = plan->g;
 	g.n_colls = n_colls;
 	g.n_sizes = n_sizes;
 	g.n_nodes = n_nodes;
 	g.n_ppn = n_ppn;
 	g.n_algos = n_algos;
-	g.colls = plan->d_colls;
-	g.sizes = plan->d_sizes;
-	g.nodes = plan->d_nodes;
-	g.ppn = plan->d_ppn;
-	g.algos = plan->d_algos;
-	g.log2_nodes = plan->d_log2_nodes;
-	g.log2_sizes = plan->d_log2_sizes;
-	g.log2_ranks = plan->d_log2_ranks;
+	g.colls = reinterpret_cast<const int32_t *>(d_axes + at_colls);
+	g.sizes = reinterpret_cast<const uint64_t *>(d_axes + at_sizes);
+	g.nodes = reinterpret_cast<const uint64_t *>(d_axes + at_nodes);
+	g.ppn = reinterpret_cast<const uint32_t *>(d_axes + at_ppn);
+	g.algos = reinterpret_cast<const int32_t *>(d_axes + at_algos);
+	g.log2_nodes = reinterpret_cast<const double *>(d_axes + at_log2_nodes);
+	g.log2_sizes = reinterpret_cast<const double *>(d_axes + at_log2_sizes);
+	g.log2_ranks = reinterpret_cast<const double *>(d_axes + at_log2_ranks);
+	g.tile_shift = tile_shift;
+	g.tiles_n = tiles_n;
+	g.tiles_s = tiles_s;
+	g.size_span = reinterpret_cast<const double2 *>(d_axes + at_spans);
+	g.rank_span = reinterpret_cast<const double2 *>(d_axes + at_rank_spans);
 	plan->points = (uint64_t)n_colls * n_sizes * n_nodes * n_ppn;
 	plan->cells = plan->points * n_algos * NUM_PROTOS;
 	*out = plan;
@@ -649,67 +836,50 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 		return -EINVAL;
 	}
 	const uint32_t points = (uint32_t)plan->points;
-	const uint64_t run_len = (uint64_t)plan->g.n_sizes * plan->g.n_nodes;
-	const uint64_t blocks_per_run = (run_len + kRegionBlock - 1) / kRegionBlock;
-	const uint64_t n_chunks = blocks_per_run * plan->g.n_colls;
-	const uint64_t n_groups = (n_chunks + kXcds - 1) / kXcds;
-	const uint64_t per_entry = n_groups * plan->g.n_ppn;
-	const uint64_t per_xcd = per_entry * n_platforms;
-	const uint64_t blocks = per_xcd * kXcds;
+	const uint64_t tiles = (uint64_t)plan->g.tiles_n * plan->g.tiles_s;
+	const uint64_t groups = (tiles + kXcds - 1) / kXcds;
+	const uint64_t n_runs = (uint64_t)n_platforms * plan->g.n_colls * plan->g.n_ppn;
+	const uint64_t blocks = groups * n_runs * kXcds;
 	if (blocks == 0 || blocks > 0x7fffffffull) {
 		return -EINVAL;
 	}
 
 	hipStream_t s = as_stream(stream);
-	if (n_platforms > plan->platforms_cap || per_xcd > plan->order_cap) {
+	if (n_runs > plan->runs_cap) {
 		OFI_AMD_HIP_TRY(hipStreamSynchronize(s));
-		(void)hipFree(plan->d_platforms);
-		(void)hipFree(plan->d_order);
-		plan->d_platforms = nullptr;
-		plan->d_order = nullptr;
-		plan->platforms_cap = 0;
-		plan->order_cap = 0;
+		(void)hipFree(plan->d_runs);
+		plan->d_runs = nullptr;
+		plan->runs_cap = 0;
 		plan->h_platforms.clear();
-		OFI_AMD_HIP_TRY(hipMalloc((void **)&plan->d_platforms, sizeof(int32_t) * n_platforms));
-		plan->platforms_cap = n_platforms;
-		OFI_AMD_HIP_TRY(hipMalloc((void **)&plan->d_order, sizeof(uint2) * per_xcd));
-		plan->order_cap = per_xcd;
+		OFI_AMD_HIP_TRY(hipMalloc((void **)&plan->d_runs, sizeof(region_run_t) * n_runs));
+		plan->runs_cap = n_runs;
 	}
 	try {
 		if (plan->h_platforms.size() != n_platforms ||
 		    std::memcmp(plan->h_platforms.data(), platforms, sizeof(int32_t) * n_platforms) != 0) {
 			plan->h_platforms.clear(); /* stays empty if an upload fails: the next call uploads again */
-			/* launch order: (entry, group, pi) by falling number of polygons in the pair's set; a
-			 * group that straddles two collectives counts as the costlier one */
-			struct item_t {
-				int32_t cost;
-				uint2 v;
-			};
-			std::vector<item_t> items;
-			items.reserve(per_xcd);
+			std::vector<region_run_t> runs;
+			runs.reserve(n_runs);
 			for (uint32_t pi = 0; pi < plan->g.n_ppn; pi++) {
-				for (uint64_t group = 0; group < n_groups; group++) {
-					const uint64_t last = std::min<uint64_t>(group * kXcds + kXcds - 1, n_chunks - 1);
-					const int32_t c0 = plan->h_colls[group * kXcds / blocks_per_run];
-					const int32_t c1 = plan->h_colls[last / blocks_per_run];
+				for (uint32_t ci = 0; ci < plan->g.n_colls; ci++) {
 					for (uint32_t e = 0; e < n_platforms; e++) {
-						int first, count0, count1;
-						region_set(plan->t, platforms[e], c0, plan->h_ppn[pi], 1, first, count0);
-						region_set(plan->t, platforms[e], c1, plan->h_ppn[pi], 1, first, count1);
-						items.push_back({ std::max(count0, count1),
-								  make_uint2(e, (uint32_t)(group * plan->g.n_ppn + pi)) });
+						region_run_t run = {};
+						run.entry = e;
+						run.ci = ci;
+						run.pi = pi;
+						run.ppn = plan->h_ppn[pi];
+						run.platform = platforms[e];
+						const region_set_t set = region_set(plan->t, run.platform, plan->h_colls[ci], run.ppn, 1);
+						run.first_poly = set.first_poly;
+						run.first_edge = set.first_edge;
+						run.counts = (uint32_t)set.edges << 16 | set.polys;
+						runs.push_back(run);
 					}
 				}
 			}
-			std::stable_sort(items.begin(), items.end(),
-					 [](const item_t &a, const item_t &b) { return a.cost > b.cost; });
-			std::vector<uint2> order(items.size());
-			for (size_t i = 0; i < items.size(); i++) {
-				order[i] = items[i].v;
-			}
-			OFI_AMD_HIP_TRY(hipMemcpyAsync(plan->d_platforms, platforms, sizeof(int32_t) * n_platforms,
-						       hipMemcpyHostToDevice, s));
-			OFI_AMD_HIP_TRY(hipMemcpyAsync(plan->d_order, order.data(), sizeof(uint2) * order.size(),
+			std::stable_sort(runs.begin(), runs.end(),
+					 [](const region_run_t &a, const region_run_t &b) { return a.counts > b.counts; });
+			OFI_AMD_HIP_TRY(hipMemcpyAsync(plan->d_runs, runs.data(), sizeof(region_run_t) * runs.size(),
 						       hipMemcpyHostToDevice, s));
 			OFI_AMD_HIP_TRY(hipStreamSynchronize(s));
 			plan->h_platforms.assign(platforms, platforms + n_platforms);
@@ -718,8 +888,12 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 		plan->h_platforms.clear();
 		return -ENOMEM;
 	}
-	hipLaunchKernelGGL(region_choice_kernel, dim3((uint32_t)blocks), dim3(kRegionBlock), 0, s, plan->g, plan->t,
-			   plan->d_platforms, points, (uint32_t)blocks_per_run, plan->d_order, d_choice);
+	for (uint64_t at = 0; at < n_runs; at += kMostRuns) {
+		const uint32_t here = (uint32_t)(n_runs - at < kMostRuns ? n_runs - at : kMostRuns);
+		hipLaunchKernelGGL(region_choice_kernel, dim3((uint32_t)(groups * kXcds), here), dim3(kRegionBlock), 0, s, plan->g,
+				   plan->t.poly, plan->t.bbox, plan->t.edges, plan->t.far_point, plan->d_runs + at, points,
+				   d_choice);
+	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -211,6 +211,28 @@ def test_region_grid_shapes_around_the_workgroup_size(lib, oracle, gpu, n_sizes,
         lib.ofi_amd_tuner_plan_destroy(plan)
 
 
+@pytest.mark.parametrize("n_nodes", [3, 4, 5, 8, 9, 13, 16, 17])
+def test_region_tiles_on_edges_and_unsorted_axes(lib, oracle, gpu, n_nodes):
+    """Points on polygon edges and vertices (rank counts that are powers of two, sizes at vertices), the
+    axes in order and shuffled: a tile's span of coordinates then covers anything from a point to the whole
+    plane, with every way an edge can lie to it, and each tile width (4, 8, 16 node counts) gets a
+    remainder."""
+    rng = np.random.default_rng(n_nodes)
+    nodes = np.array(([4, 8, 16, 32, 64, 128, 256, 512, 3, 5, 12, 24, 48, 96, 192, 2, 1])[:n_nodes], dtype=np.uint64)
+    sizes = np.array([1, 1 << 15, 1 << 17, 196608, 786432, 3145728, 4 << 20, 4718592, 8 << 20, 13107200, 29884416,
+                      31457280, 32 << 20, 33554433, 129499136, 1 << 30, 107374182399, 107374182400, 107374182401], dtype=np.uint64)
+    colls, ppn = np.array([4, 2, 3], dtype=np.int32), np.array([8, 1, 2], dtype=np.uint32)
+    for order in (lambda a: np.sort(a), rng.permutation):
+        s, n = order(sizes), order(nodes)
+        plan = make_plan(lib, colls, s, n, ppn, np.array([1], dtype=np.int32))
+        want = oracle_region_grid(oracle, [0, 1, 2, 3], colls, s, n, ppn)
+        got = run_region(lib, plan, [0, 1, 2, 3], (4, 3, len(s), len(n), 3))
+        mism = np.argwhere((got != want).any(axis=-1))
+        assert len(mism) == 0, mism[:10]
+        assert (want[..., 0] >= 0).any()
+        lib.ofi_amd_tuner_plan_destroy(plan)
+
+
 def test_region_grid_on_changing_platform_lists(lib, oracle, gpu):
     """One plan, platform lists that grow, shrink and change in place: the launch order the plan keeps
     for a list (which entry, chunk and ranks-per-node value each workgroup takes) is rebuilt whenever
