@@ -10,23 +10,20 @@
  *   small_rail_i = (rr_small + #{j < i : size_j <  max_small}) mod R
  *   start_rail_i = (rr      + sum{j < i : size_j >= max_small} n_j) mod R
  *
- * Launches on one stream:
- *   1. stripe_count_kernel  per-tile totals of (small count, stripe count), each
- *                           reduced mod R (only the residues matter); snapshots the
- *                           two counters of *state as the batch's seed
- *   2. stripe_scan_kernel   (batches of more than kInlineTiles tiles only) one
- *                           workgroup scans the tile totals and writes the new
- *                           counters back
- *   3. stripe_emit_kernel   re-reads the tile, scans inside the workgroup with
- *                           wavefront shuffles, builds the 96-byte stripe rows in
- *                           LDS and writes them out as coalesced 16-byte stores.
- *                           Up to kInlineTiles tiles every workgroup sums the
- *                           totals of the tiles before it by itself (at most 16 KiB
- *                           from L2) instead of waiting for a scan launch, and the
- *                           last workgroup writes the new counters back.
- * A tile is 512 messages for batches up to 2^21 messages and 1024 beyond.
+ * Three forms, by the size of the batch:
+ *   up to kDirectBatch messages, one launch: every workgroup adds up the messages before
+ *   its tile by itself, from their sizes (at most 48 KiB out of the L2);
+ *   up to kSmallBatch, two launches: stripe_count_kernel leaves each tile's totals of
+ *   (small count, stripe count), reduced mod R (only the residues matter), and
+ *   stripe_emit_kernel, whose workgroups add up the totals of the tiles before them (at most
+ *   48 KiB), builds the 96-byte stripe rows in LDS and writes them out as coalesced 16-byte
+ *   stores;
+ *   beyond, the same two launches with larger tiles, and a level of totals above the tiles', for
+ *   every kPart messages.
+ * The count launch snapshots the two counters of *state as the batch's seed, the workgroup of the
+ * last tile writes the new ones back.
  *
- * HBM traffic per message: 8 B read twice + 4 B + 96 B written.
+ * HBM traffic per message: 8 B read twice (once in the one-launch form) + 4 B + 96 B written.
  */
 #include <mutex>
 #include <unordered_map>
@@ -38,64 +35,62 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kThreads = 256;
-/* Messages per workgroup = kThreads * PASSES.  Small batches want many small tiles (the
- * launch is short, so ramp-up and tail dominate: 1,000,000 messages take 22.2 us with two
- * passes per workgroup against 24.4 with four); large ones want somewhat longer workgroups
- * (16,000,000: 322-325 us with three or four passes, 332-334 with two, six or eight). */
-#ifndef OFI_STRIPE_PASSES_SMALL
-#define OFI_STRIPE_PASSES_SMALL 2
-#endif
-#ifndef OFI_STRIPE_PASSES_LARGE
-#define OFI_STRIPE_PASSES_LARGE 4
-#endif
-constexpr uint32_t kPassesSmall = OFI_STRIPE_PASSES_SMALL, kPassesLarge = OFI_STRIPE_PASSES_LARGE;
-constexpr uint64_t kSmallBatch = 1ull << 21;
-constexpr uint32_t kScanThreads = 1024;
-constexpr uint32_t kScanPer = 8; /* tiles per thread and round of the scan kernel */
+/* One-launch form: tiles of 256 messages.  Between 6000 and 7000 messages the workgroups' own look at
+ * everything before them comes to cost what the second launch does (4.3 against 6.2 us at 1000 messages, 4.8
+ * against 5.7 at 4000, 6.2 against 5.7 at 8000). */
+constexpr uint32_t kDirectTile = 256;
+constexpr uint64_t kDirectBatch = 6144;
+static_assert(4 * kDirectBatch <= 65536, "packed sums of a whole batch: up to 4 stripes a message, and the seed");
+/* Two-launch form: tiles of 512 messages, counted by 256 threads and written by 512 (21.5 us per 1,000,000
+ * messages, 39.0 per 2,000,000; 256 threads twice 21.6 and 40.2, 128 threads four times 23.9 and 43.5). */
+constexpr uint32_t kTile = 512;
+constexpr uint32_t kCountThreads = 256;
+constexpr uint64_t kSmallBatch = 6ull << 20;
+/* Beyond: tiles of 1024 messages, a workgroup of 1024 threads each, one to a CU (its rows fill 96 KiB of
+ * LDS).  Once the output is larger than the last-level cache the rate of a write-only launch depends on how
+ * narrow the front is on which the chip writes: 1.5 GB in pieces of 24 KiB from six workgroups a CU
+ * goes at 5.4 TB/s, in 48 KiB pieces from one workgroup a CU at 6.8.  16,000,000 messages take 276 us
+ * like this, 314 with four passes of 256 messages, six workgroups a CU; 5,000,000 take 99.7 and, in
+ * tiles of 512, 95.0, 7,000,000 take 130.8 and 132.6: the line lies between. */
+constexpr uint32_t kBigTile = 1024;
+constexpr uint32_t kBlockTiles = 4; /* tiles that share a block total: a workgroup of the count kernel */
+/* ... in parts of 2^24 messages, chained through *state.  The sizes of a part, 128 MiB, are still in the
+ * last-level cache when the emit launch reads them again; in one part, 60,000,000 messages took
+ * 1294 us, in parts 1056. */
+constexpr uint64_t kPart = 1ull << 24;
+constexpr uint32_t kMaxTiles = (uint32_t)(kPart / kBigTile), kMaxBlocks = kMaxTiles / kBlockTiles;
+static_assert(kSmallBatch / kTile <= kMaxTiles && kMaxBlocks <= 4 * kBigTile && kMaxTiles <= 1u << 14,
+	      "room for every tile, one 16-byte load a thread, sums of residues below 2^16");
 constexpr uint64_t kMaxBatch = 1ull << 28;
-/* residues are < 4, so packed 16-bit sums over this many tiles cannot overflow */
-#ifndef OFI_STRIPE_INLINE_TILES
-#define OFI_STRIPE_INLINE_TILES 4096
-#endif
-constexpr uint32_t kInlineTiles = OFI_STRIPE_INLINE_TILES;
-#ifndef OFI_STRIPE_NT_STORES
-#define OFI_STRIPE_NT_STORES 1
-#endif
 
 struct params_t {
 	uint64_t max_small;
-	uint64_t min_stripe;
+	uint64_t stripes[3];    /* 1, 2 and 3 times the minimum stripe size, at most 2^64 - 1 */
 	uint64_t align;
-	int32_t min_stripe_shift; /* log2 when a power of two, else -1 */
-	int32_t align_shift;
+	int32_t align_shift;    /* log2 when a power of two, else -1 */
 	uint32_t num_rails;
 	uint32_t stripe_counts; /* get_num_stripes for this rail count, 4 bits per requested count 1..4 */
 	uint32_t mod_magic;     /* 65536 / num_rails + 1, see mod_rails */
 };
 
-__device__ __forceinline__ uint64_t div_by(uint64_t x, uint64_t d, int32_t shift)
-{
-	return shift >= 0 ? (x >> shift) : (x / d);
-}
-
 /* NCCL_OFI_DIV_CEIL, include/nccl_ofi_math.h:23-26 */
 __device__ __forceinline__ uint64_t div_ceil_by(uint64_t x, uint64_t d, int32_t shift)
 {
-	return x == 0 ? 0 : 1 + div_by(x - 1, d, shift);
+	return x == 0 ? 0 : 1 + (shift >= 0 ? ((x - 1) >> shift) : ((x - 1) / d));
 }
 
 /* get_num_stripes, src/nccl_ofi_scheduler.cpp:47-64: the request, capped to the rail count,
  * goes down to the largest count >= 2 that divides the rail count and stays as it is when there
- * is none (3 rails: 2 stays 2).  At most 4 rails, so the loop is a 16-entry table. */
+ * is none (3 rails: 2 stays 2).  At most 4 rails, so the loop is a 16-entry table, and the request --
+ * the size divided by the minimum stripe, rounded up -- needs three comparisons and no division: a
+ * division per message made the count kernels 15 KB of code and a third of their time. */
 constexpr uint64_t kStripeCounts = 0x4221332122211111ull; /* 16 bits per rail count, 4 per request */
 
 __device__ __forceinline__ uint32_t num_stripes(uint64_t size, const params_t &p)
 {
-	uint64_t want = div_ceil_by(size, p.min_stripe, p.min_stripe_shift);
-	uint32_t n = (uint32_t)(want < p.num_rails ? want : p.num_rails);
-	n = n > 1 ? n : 1;
-	return (p.stripe_counts >> (4u * (n - 1u))) & 7u;
+	uint32_t n = (size > p.stripes[0]) + (size > p.stripes[1]) + (size > p.stripes[2]);
+	n = n < p.num_rails ? n : p.num_rails - 1u;
+	return (p.stripe_counts >> (4u * n)) & 7u;
 }
 
 /* x mod num_rails for x < 16384, by multiply and shift (checked exhaustively for 1..4 rails) */
@@ -104,36 +99,35 @@ __device__ __forceinline__ uint32_t mod_rails(uint32_t x, const params_t &p)
 	return x - p.num_rails * ((x * p.mod_magic) >> 16);
 }
 
-/* Thresholds come from the device-resident state; a power-of-two divisor becomes a
- * shift.  False when the state is unusable (rails outside 1..4, zero stripe size). */
 __device__ __forceinline__ int32_t log2_if_pow2_dev(uint64_t v)
 {
 	return (v != 0 && (v & (v - 1)) == 0) ? (int32_t)(__ffsll((unsigned long long)v) - 1) : -1;
 }
 
+/* Thresholds come from the device-resident state.  False when the state is unusable (rails outside
+ * 1..4, zero stripe size). */
 __device__ __forceinline__ bool load_params(const ofi_amd_sched_state_t *st, uint64_t align,
 					    params_t &p)
 {
 	p.max_small = st->max_small_msg_size;
-	p.min_stripe = st->min_stripe_size;
+	const uint64_t m = st->min_stripe_size;
+	p.stripes[0] = m;
+	p.stripes[1] = m > ~0ull / 2 ? ~0ull : 2 * m;
+	p.stripes[2] = m > ~0ull / 3 ? ~0ull : 3 * m;
 	p.align = align;
-	p.min_stripe_shift = log2_if_pow2_dev(p.min_stripe);
 	p.align_shift = log2_if_pow2_dev(align);
 	p.num_rails = (uint32_t)st->num_rails;
 	p.stripe_counts = (uint32_t)(kStripeCounts >> (16u * ((p.num_rails - 1u) & 3u))) & 0xffffu;
 	p.mod_magic = 65536u / (p.num_rails ? p.num_rails : 1u) + 1u;
-	return st->num_rails >= 1 && st->num_rails <= OFI_AMD_MAX_NUM_RAILS && p.min_stripe != 0;
+	return st->num_rails >= 1 && st->num_rails <= OFI_AMD_MAX_NUM_RAILS && m != 0;
 }
 
 /* packed (small count << 16 | stripe count) contribution of one message */
 __device__ __forceinline__ uint32_t contribution(uint64_t size, const params_t &p, uint32_t &n_out)
 {
-	if (size < p.max_small) {
-		n_out = 1;
-		return 1u << 16;
-	}
-	n_out = num_stripes(size, p);
-	return n_out;
+	const bool small = size < p.max_small;
+	n_out = small ? 1u : num_stripes(size, p);
+	return small ? 1u << 16 : n_out;
 }
 
 /* Inclusive sum over the 64 lanes with lane-to-lane moves inside the vector unit: shifts by 1,
@@ -150,38 +144,40 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, uint32_t)
 	return v;
 }
 
-/* Which tile a workgroup takes.  Workgroups are dealt to the 8 XCDs in turn; with tile =
- * workgroup number every XCD writes one tile's rows (96 KiB) out of every eight, with runs of
- * 16 consecutive tiles per XCD each of them writes 1.5 MiB at a stretch.  Once the output no
- * longer fits the last-level cache the longer stretches are faster (5,000,000 messages: 110.6 ->
- * 102.9 us, 16,000,000: 324.6 -> 305.9 us; runs of 4, 64, 256 or an eighth of the batch per XCD:
- * 307-312 us), below that they are slower (1,000,000: 22.4 -> 24.1 us, 4,200,000: 91.3 -> 97.0
- * us), so they are used from 4.5 Mi messages on.  The grid is rounded up to whole rounds; a
- * workgroup whose tile does not exist leaves at once. */
-constexpr uint32_t kXcdRunShift = 4;
-constexpr uint64_t kXcdRunBatch = 9ull << 19;
-__device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t wg, uint32_t run_shift)
+/* residues mod R of a packed pair whose halves are the true sums */
+__device__ __forceinline__ uint32_t residues(uint32_t packed, uint32_t num_rails)
 {
-	/* XCDs take runs of 2^run_shift consecutive tiles in turn */
-	const uint32_t x = wg & 7u, t = wg >> 3;
-	return ((((t >> run_shift) << 3) + x) << run_shift) + (t & ((1u << run_shift) - 1u));
+	return (((packed >> 16) % num_rails) << 16) | ((packed & 0xffffu) % num_rails);
 }
 
-template <uint32_t PASSES>
-__global__ __launch_bounds__(kThreads) void stripe_count_kernel(
+__device__ __forceinline__ uint32_t wave_sum_of(uint32_t v)
+{
+	v = wave_inclusive_scan(v, 0);
+	return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+/* The batch's seed: *state's counters as they are before the emit launch's last workgroup moves them on */
+__device__ __forceinline__ uint32_t batch_seed(const ofi_amd_sched_state_t *state, uint32_t num_rails)
+{
+	return ((state->rr_small_counter % num_rails) << 16) | (state->rr_counter % num_rails);
+}
+
+/* Totals of one tile of kTile messages per workgroup */
+__global__ __launch_bounds__(kCountThreads) void stripe_count_kernel(
 	const uint64_t *__restrict__ sizes, uint32_t n, const ofi_amd_sched_state_t *__restrict__ state,
 	uint64_t align, uint32_t *__restrict__ tile_totals, uint32_t *__restrict__ seed0,
 	uint32_t *__restrict__ err)
 {
-	__shared__ uint32_t wave_sum[kThreads / 64];
+	constexpr uint32_t kPer = kTile / kCountThreads;
+	__shared__ uint32_t wave_sum[kCountThreads / 64];
 	/* the tile's sizes are requested before anything waits for the state, so a workgroup pays
 	 * one memory latency, not two */
-	const uint32_t base = blockIdx.x * (kThreads * PASSES);
-	uint64_t size_of[PASSES];
+	const uint32_t base = blockIdx.x * kTile;
+	uint64_t size_of[kPer];
 #pragma unroll
-	for (uint32_t pass = 0; pass < PASSES; pass++) {
-		const uint32_t i = base + pass * kThreads + threadIdx.x;
-		size_of[pass] = i < n ? sizes[i] : 0;
+	for (uint32_t j = 0; j < kPer; j++) {
+		const uint32_t i = base + j * kCountThreads + threadIdx.x;
+		size_of[j] = i < n ? sizes[i] : 0;
 	}
 	params_t p;
 	if (!load_params(state, align, p)) {
@@ -191,288 +187,271 @@ __global__ __launch_bounds__(kThreads) void stripe_count_kernel(
 		return;
 	}
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
-		*seed0 = ((state->rr_small_counter % p.num_rails) << 16) | (state->rr_counter % p.num_rails);
+		*seed0 = batch_seed(state, p.num_rails);
 	}
 	uint32_t acc = 0;
 #pragma unroll
-	for (uint32_t pass = 0; pass < PASSES; pass++) {
+	for (uint32_t j = 0; j < kPer; j++) {
 		uint32_t k;
-		const uint32_t c = contribution(size_of[pass], p, k);
-		acc += base + pass * kThreads + threadIdx.x < n ? c : 0u;
+		const uint32_t c = contribution(size_of[j], p, k);
+		acc += base + j * kCountThreads + threadIdx.x < n ? c : 0u;
 	}
-#pragma unroll
-	for (uint32_t d = 32; d > 0; d >>= 1) {
-		acc += __shfl_xor(acc, d, 64);
-	}
+	acc = wave_sum_of(acc);
 	if ((threadIdx.x & 63u) == 0) {
 		wave_sum[threadIdx.x >> 6] = acc;
 	}
 	__syncthreads();
 	if (threadIdx.x == 0) {
-		const uint32_t t = wave_sum[0] + wave_sum[1] + wave_sum[2] + wave_sum[3];
-		tile_totals[blockIdx.x] = (((t >> 16) % p.num_rails) << 16) | ((t & 0xffffu) % p.num_rails);
+		tile_totals[blockIdx.x] = residues(wave_sum[0] + wave_sum[1] + wave_sum[2] + wave_sum[3], p.num_rails);
 	}
 }
 
-/* One workgroup: exclusive scan of the tile totals.  tile_prefix[t] holds the two
- * rail seeds of tile t (already reduced mod R); *state gets the final counters. */
-__global__ __launch_bounds__(kScanThreads) void stripe_scan_kernel(
-	const uint32_t *__restrict__ tile_totals, uint32_t num_tiles,
-	ofi_amd_sched_state_t *__restrict__ state, uint32_t *__restrict__ tile_prefix,
-	uint32_t *__restrict__ err)
+/* The same for the large form: a wavefront per tile of kBigTile messages, every load of it in flight at
+ * once, and the sum of the workgroup's tiles beside them. */
+__global__ __launch_bounds__(64 * kBlockTiles) void stripe_count_big_kernel(
+	const uint64_t *__restrict__ sizes, uint32_t n, const ofi_amd_sched_state_t *__restrict__ state,
+	uint64_t align, uint32_t *__restrict__ tile_totals, uint32_t *__restrict__ block_totals,
+	uint32_t *__restrict__ seed0, uint32_t *__restrict__ err)
 {
-	__shared__ uint32_t wave_small[kScanThreads / 64];
-	__shared__ uint32_t wave_big[kScanThreads / 64];
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	if (state->num_rails < 1 || state->num_rails > OFI_AMD_MAX_NUM_RAILS ||
-	    state->min_stripe_size == 0) {
-		if (threadIdx.x == 0) {
+	constexpr uint32_t kPer = kBigTile / 64;
+	__shared__ uint32_t wave_total[kBlockTiles];
+	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const uint32_t tile = blockIdx.x * kBlockTiles + wave;
+	const uint64_t base = (uint64_t)tile * kBigTile;
+	uint64_t size_of[kPer];
+#pragma unroll
+	for (uint32_t j = 0; j < kPer; j++) {
+		const uint64_t i = base + j * 64u + lane;
+		size_of[j] = i < n ? sizes[i] : 0;
+	}
+	params_t p;
+	if (!load_params(state, align, p)) {
+		if (blockIdx.x == 0 && threadIdx.x == 0) {
 			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE);
 		}
 		return;
 	}
-	const uint32_t num_rails = (uint32_t)state->num_rails;
-	/* totals can reach 2^28 each, so the two sums are scanned unpacked */
-	uint32_t carry_small = state->rr_small_counter % num_rails;
-	uint32_t carry_big = state->rr_counter % num_rails;
-
-	/* eight consecutive tiles per thread and round: 16 M messages are one round, so the kernel
-	 * waits for memory once */
-	for (uint32_t start = 0; start < num_tiles; start += kScanThreads * kScanPer) {
-		const uint32_t t0 = start + threadIdx.x * kScanPer;
-		const bool whole = t0 + kScanPer <= num_tiles;
-		uint32_t v[kScanPer];
-		if (whole) {
-			const u32x4 lo = *reinterpret_cast<const u32x4 *>(tile_totals + t0);
-			const u32x4 hi = *reinterpret_cast<const u32x4 *>(tile_totals + t0 + 4);
-			v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w;
-			v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
-		} else {
-#pragma unroll
-			for (uint32_t j = 0; j < kScanPer; j++) {
-				v[j] = t0 + j < num_tiles ? tile_totals[t0 + j] : 0;
-			}
-		}
-		uint32_t s = 0, b = 0;
-#pragma unroll
-		for (uint32_t j = 0; j < kScanPer; j++) {
-			s += v[j] >> 16;
-			b += v[j] & 0xffffu;
-		}
-		uint32_t inc_s = wave_inclusive_scan(s, lane);
-		uint32_t inc_b = wave_inclusive_scan(b, lane);
-		if (lane == 63) {
-			wave_small[wave] = inc_s;
-			wave_big[wave] = inc_b;
-		}
-		__syncthreads();
-		uint32_t off_s = 0, off_b = 0, tot_s = 0, tot_b = 0;
-		for (uint32_t w = 0; w < kScanThreads / 64; w++) {
-			uint32_t ws = wave_small[w], wb = wave_big[w];
-			if (w < wave) {
-				off_s += ws;
-				off_b += wb;
-			}
-			tot_s += ws;
-			tot_b += wb;
-		}
-		uint32_t run_s = carry_small + off_s + inc_s - s;
-		uint32_t run_b = carry_big + off_b + inc_b - b;
-		uint32_t out[kScanPer];
-#pragma unroll
-		for (uint32_t j = 0; j < kScanPer; j++) {
-			out[j] = ((run_s % num_rails) << 16) | (run_b % num_rails);
-			run_s += v[j] >> 16;
-			run_b += v[j] & 0xffffu;
-		}
-		if (whole) {
-			*reinterpret_cast<u32x4 *>(tile_prefix + t0) = u32x4{ out[0], out[1], out[2], out[3] };
-			*reinterpret_cast<u32x4 *>(tile_prefix + t0 + 4) = u32x4{ out[4], out[5], out[6], out[7] };
-		} else {
-#pragma unroll
-			for (uint32_t j = 0; j < kScanPer; j++) {
-				if (t0 + j < num_tiles) {
-					tile_prefix[t0 + j] = out[j];
-				}
-			}
-		}
-		carry_small = (carry_small + tot_s) % num_rails;
-		carry_big = (carry_big + tot_b) % num_rails;
-		__syncthreads();
+	if (blockIdx.x == 0 && threadIdx.x == 0) {
+		*seed0 = batch_seed(state, p.num_rails);
 	}
+	uint32_t acc = 0;
+#pragma unroll
+	for (uint32_t j = 0; j < kPer; j++) {
+		uint32_t k;
+		const uint32_t c = contribution(size_of[j], p, k);
+		acc += base + j * 64u + lane < n ? c : 0u;
+	}
+	acc = residues(wave_sum_of(acc), p.num_rails);
+	if (lane == 0) {
+		wave_total[wave] = acc;
+		if (base < n) {
+			tile_totals[tile] = acc;
+		}
+	}
+	__syncthreads();
 	if (threadIdx.x == 0) {
-		state->rr_small_counter = carry_small;
-		state->rr_counter = carry_big;
+		uint32_t t = 0;
+#pragma unroll
+		for (uint32_t w = 0; w < kBlockTiles; w++) {
+			t += wave_total[w];
+		}
+		block_totals[blockIdx.x] = residues(t, p.num_rails);
 	}
 }
 
-/* INLINE: tile_prefix holds the per-tile totals (residues) and *seed0 the batch's seed;
- * otherwise tile_prefix holds each tile's finished seed. */
-template <bool INLINE, uint32_t PASSES>
-__global__ __launch_bounds__(kThreads) void stripe_emit_kernel(
+/* Where a tile's seed comes from: the sizes before it (DIRECT), the totals of the tiles before it (TILES), or
+ * the totals of the blocks of tiles before its block and of the tiles before it in its block (BLOCKS) */
+enum stripe_form { DIRECT, TILES, BLOCKS };
+
+template <stripe_form FORM, uint32_t THREADS>
+__global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	const uint64_t *__restrict__ sizes, uint32_t n, ofi_amd_sched_state_t *__restrict__ state,
-	uint64_t align, const uint32_t *__restrict__ tile_prefix, const uint32_t *__restrict__ seed0,
-	uint32_t num_tiles, uint32_t xcd_run_shift, uint32_t *__restrict__ num_xfers, u32x4 *__restrict__ xfers)
+	uint64_t align, const uint32_t *__restrict__ totals, const uint32_t *__restrict__ block_totals,
+	uint32_t *__restrict__ seed0, uint32_t num_tiles, uint32_t *__restrict__ num_xfers, u32x4 *__restrict__ xfers,
+	uint32_t *__restrict__ err)
 {
-	/* 256 rows of 96 bytes = 6 x 16 B each */
-	__shared__ u32x4 rows[kThreads * 6];
-	__shared__ uint32_t wave_sum[kThreads / 64];
+	constexpr uint32_t kWaves = THREADS / 64;
+	/* THREADS rows of 96 bytes = 6 x 16 B each */
+	__shared__ u32x4 rows[THREADS * 6];
+	__shared__ uint32_t wave_sum[kWaves], seed_sum[kWaves];
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	const uint32_t tile = tile_of_workgroup(blockIdx.x, xcd_run_shift);
-	if (tile >= num_tiles) {
-		return;
-	}
-	const uint32_t base = tile * (kThreads * PASSES);
-	/* every pass's size is requested up front: the passes below then run out of registers
-	 * instead of each waiting for its own load */
-	uint64_t size_of[PASSES];
+	const uint32_t tile = blockIdx.x, base = tile * THREADS, i = base + threadIdx.x;
+	const bool live = i < n;
+	const uint64_t size = live ? __builtin_nontemporal_load(&sizes[i]) : 0;
+	uint32_t acc = 0;
+	/* DIRECT: the first messages before the tile, requested along with its own */
+	constexpr uint32_t kAhead = 16;
+	uint64_t before[kAhead];
+	auto look_ahead = [&](uint32_t i0) {
 #pragma unroll
-	for (uint32_t pass = 0; pass < PASSES; pass++) {
-		const uint32_t i = base + pass * kThreads + threadIdx.x;
-		size_of[pass] = i < n ? __builtin_nontemporal_load(&sizes[i]) : 0;
+		for (uint32_t j = 0; j < kAhead; j++) {
+			const uint32_t at = i0 + j * THREADS + threadIdx.x;
+			before[j] = at < base ? sizes[at] : 0;
+		}
+	};
+	if (FORM == DIRECT) {
+		look_ahead(0);
+	} else {
+		/* sums of residues: packed halves, below 2^14 words of at most 3 each */
+		if (FORM == TILES) {
+			/* A word a thread and turn: the later a tile, the later its workgroup starts to write, and
+			 * the launch is faster for it (1,000,000 messages: 21.6 us; with four 16-byte loads in
+			 * flight, so that all start at once, 22.8). */
+			for (uint32_t t = threadIdx.x; t < tile; t += THREADS) {
+				acc += totals[t];
+			}
+		}
+		if (FORM == BLOCKS) {
+			/* at most kMaxBlocks words: one 16-byte load a thread, the words beyond the last masked out */
+			const uint32_t blocks = tile / kBlockTiles, at = threadIdx.x * 4u;
+			if (at < blocks) {
+				const u32x4 v = *reinterpret_cast<const u32x4 *>(block_totals + at);
+				acc = v.x + (at + 1 < blocks ? v.y : 0) + (at + 2 < blocks ? v.z : 0) + (at + 3 < blocks ? v.w : 0);
+			}
+			acc += threadIdx.x < tile % kBlockTiles ? totals[blocks * kBlockTiles + threadIdx.x] : 0;
+		}
 	}
 	params_t p;
 	if (!load_params(state, align, p)) {
+		if (FORM == DIRECT && tile == 0 && threadIdx.x == 0) {
+			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE);
+		}
 		return;
 	}
 	const uint32_t R = p.num_rails;
-
-	uint32_t seed;
-	if (INLINE) {
-		/* sum of the totals of the tiles before this one (packed halves, no overflow) */
-		uint32_t acc = 0;
-		for (uint32_t t = threadIdx.x; t < tile; t += kThreads) {
-			acc += tile_prefix[t];
-		}
+	if (FORM == DIRECT) {
+		for (uint32_t i0 = 0; i0 < base;) {
 #pragma unroll
-		for (uint32_t d = 32; d > 0; d >>= 1) {
-			acc += __shfl_xor(acc, d, 64);
-		}
-		if (lane == 0) {
-			wave_sum[wave] = acc;
-		}
-		__syncthreads();
-		acc = wave_sum[0] + wave_sum[1] + wave_sum[2] + wave_sum[3] + *seed0;
-		__syncthreads();
-		seed = (((acc >> 16) % R) << 16) | ((acc & 0xffffu) % R);
-	} else {
-		seed = tile_prefix[tile];
-	}
-	uint32_t carry_small = seed >> 16, carry_big = seed & 0xffffu; /* both < R */
-
-#pragma unroll
-	for (uint32_t pass = 0; pass < PASSES; pass++) {
-		const uint32_t first = base + pass * kThreads;
-		if (first >= n) {
-			break;
-		}
-		const uint32_t i = first + threadIdx.x;
-		const bool live = i < n;
-		const uint64_t size = size_of[pass];
-		uint32_t k = 0;
-		const uint32_t c = live ? contribution(size, p, k) : 0;
-
-		uint32_t inc = wave_inclusive_scan(c, lane);
-		if (lane == 63) {
-			wave_sum[wave] = inc;
-		}
-		__syncthreads();
-		uint32_t off = 0, tot = 0;
-#pragma unroll
-		for (uint32_t w = 0; w < kThreads / 64; w++) {
-			uint32_t ws = wave_sum[w];
-			off += (w < wave) ? ws : 0;
-			tot += ws;
-		}
-		const uint32_t excl = off + inc - c;
-
-		/* set_schedule_by_threshold, src/nccl_ofi_scheduler.cpp:77-133 */
-		const bool small = (c >> 16) != 0;
-		uint32_t rail = mod_rails(small ? carry_small + (excl >> 16) : carry_big + (excl & 0xffffu), p);
-		uint64_t max_stripe = size;
-		if (!small) {
-			/* (size - 1) / k: k is 1, 2 or 4 unless there are three rails */
-			uint64_t whole = size == 0 ? 0 : (size - 1) >> (k >> 1);
-			if (R == 3) {
-				whole = k == 3 ? (size == 0 ? 0 : (size - 1) / 3) : whole;
+			for (uint32_t j = 0; j < kAhead; j++) {
+				uint32_t k;
+				const uint32_t c = contribution(before[j], p, k);
+				acc += i0 + j * THREADS + threadIdx.x < base ? c : 0u;
 			}
-			const uint64_t per = size == 0 ? 0 : 1 + whole;
-			max_stripe = div_ceil_by(per, p.align, p.align_shift) * p.align;
+			i0 += THREADS * kAhead;
+			if (i0 < base) {
+				look_ahead(i0);
+			}
 		}
-		/* k stripes of max_stripe cover the message, so `left` is 0 from stripe k on and the
-		 * length of an unused entry comes out as 0 by itself; lanes past the end have k = 0 */
-		uint64_t left = size, offset = 0;
-		u32x4 *row = &rows[threadIdx.x * 6];
-		uint64_t f[12]; /* 4 x {rail word, offset, msg_size} */
-#pragma unroll
-		for (uint32_t s = 0; s < 4; s++) {
-			const bool used = s < k;
-			const uint64_t stripe = left < max_stripe ? left : max_stripe;
-			f[3 * s + 0] = used ? rail : 0; /* rail_id in the low 16 bits, padding zero */
-			f[3 * s + 1] = used ? offset : 0;
-			f[3 * s + 2] = stripe;
-			offset += stripe;
-			left -= stripe;
-			rail = rail + 1 == R ? 0 : rail + 1;
-		}
-#pragma unroll
-		for (uint32_t q = 0; q < 6; q++) {
-			u32x4 v;
-			v.x = (uint32_t)f[2 * q];
-			v.y = (uint32_t)(f[2 * q] >> 32);
-			v.z = (uint32_t)f[2 * q + 1];
-			v.w = (uint32_t)(f[2 * q + 1] >> 32);
-			row[q] = v;
-		}
-		if (live) {
-			num_xfers[i] = k;
-		}
-		__syncthreads();
-
-		/* coalesced write-out of the tile's rows */
-		const uint32_t valid = (n - first) < kThreads ? (n - first) : kThreads;
-		u32x4 *out = xfers + (uint64_t)first * 6;
-		for (uint32_t v = threadIdx.x; v < valid * 6; v += kThreads) {
-#if OFI_STRIPE_NT_STORES
-			__builtin_nontemporal_store(rows[v], &out[v]);
-#else
-			out[v] = rows[v];
-#endif
-		}
-
-		carry_small = mod_rails(carry_small + (tot >> 16), p);
-		carry_big = mod_rails(carry_big + (tot & 0xffffu), p);
-		__syncthreads();
 	}
-	if (INLINE && tile == num_tiles - 1 && threadIdx.x == 0) {
+	acc = wave_sum_of(acc);
+	uint32_t k = 0;
+	const uint32_t c = live ? contribution(size, p, k) : 0;
+	const uint32_t inc = wave_inclusive_scan(c, lane);
+	if (lane == 0) {
+		seed_sum[wave] = acc;
+	}
+	if (lane == 63) {
+		wave_sum[wave] = inc;
+	}
+	const uint32_t seed = FORM == DIRECT ? batch_seed(state, R) : *seed0;
+	__syncthreads();
+	uint32_t before_tile = seed, off = 0, tot = 0;
+#pragma unroll
+	for (uint32_t w = 0; w < kWaves; w++) {
+		const uint32_t ws = wave_sum[w];
+		off += (w < wave) ? ws : 0;
+		tot += ws;
+		before_tile += seed_sum[w];
+	}
+	const uint32_t carry_small = (before_tile >> 16) % R, carry_big = (before_tile & 0xffffu) % R;
+	const uint32_t excl = off + inc - c;
+
+	/* set_schedule_by_threshold, src/nccl_ofi_scheduler.cpp:77-133 */
+	const bool small = (c >> 16) != 0;
+	uint32_t rail = mod_rails(small ? carry_small + (excl >> 16) : carry_big + (excl & 0xffffu), p);
+	uint64_t max_stripe = size;
+	if (!small) {
+		/* (size - 1) / k: k is 1, 2 or 4 unless there are three rails */
+		uint64_t whole = size == 0 ? 0 : (size - 1) >> (k >> 1);
+		if (R == 3) {
+			whole = k == 3 ? (size == 0 ? 0 : (size - 1) / 3) : whole;
+		}
+		const uint64_t per = size == 0 ? 0 : 1 + whole;
+		max_stripe = div_ceil_by(per, p.align, p.align_shift) * p.align;
+	}
+	/* k stripes of max_stripe cover the message, so `left` is 0 from stripe k on and the
+	 * length of an unused entry comes out as 0 by itself; lanes past the end have k = 0 */
+	uint64_t left = size, offset = 0;
+	u32x4 *row = &rows[threadIdx.x * 6];
+	uint64_t f[12]; /* 4 x {rail word, offset, msg_size} */
+#pragma unroll
+	for (uint32_t s = 0; s < 4; s++) {
+		const bool used = s < k;
+		const uint64_t stripe = left < max_stripe ? left : max_stripe;
+		f[3 * s + 0] = used ? rail : 0; /* rail_id in the low 16 bits, padding zero */
+		f[3 * s + 1] = used ? offset : 0;
+		f[3 * s + 2] = stripe;
+		offset += stripe;
+		left -= stripe;
+		rail = rail + 1 == R ? 0 : rail + 1;
+	}
+#pragma unroll
+	for (uint32_t q = 0; q < 6; q++) {
+		u32x4 v;
+		v.x = (uint32_t)f[2 * q];
+		v.y = (uint32_t)(f[2 * q] >> 32);
+		v.z = (uint32_t)f[2 * q + 1];
+		v.w = (uint32_t)(f[2 * q + 1] >> 32);
+		row[q] = v;
+	}
+	if (live) {
+		num_xfers[i] = k;
+	}
+	__syncthreads();
+
+	/* coalesced write-out of the tile's rows */
+	const uint32_t valid = (n - base) < THREADS ? (n - base) : THREADS;
+	u32x4 *out = xfers + (uint64_t)base * 6;
+	for (uint32_t v = threadIdx.x; v < valid * 6; v += THREADS) {
+		__builtin_nontemporal_store(rows[v], &out[v]);
+	}
+
+	if (threadIdx.x != 0) {
+		return;
+	}
+	const uint32_t after_small = mod_rails(carry_small + (tot >> 16), p);
+	const uint32_t after_big = mod_rails(carry_big + (tot & 0xffffu), p);
+	if (FORM == DIRECT && num_tiles > 1) {
+		/* Every workgroup has read the counters, so they may only be moved on when all are done:
+		 * each adds itself to the arrival word (low half), the last tile's with the carries behind
+		 * it (high half), and whoever is last puts them in place and leaves the word at zero. */
+		const uint32_t mine = 1u + (tile == num_tiles - 1 ? (after_small << 16) | (after_big << 20) : 0u);
+		const uint32_t all = mine + __hip_atomic_fetch_add(seed0, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		if ((all & 0xffffu) == num_tiles) {
+			__hip_atomic_store(seed0, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			state->rr_small_counter = (all >> 16) & 3u;
+			state->rr_counter = (all >> 20) & 3u;
+		}
+	} else if (tile == num_tiles - 1) {
 		/* the carries after the last tile are the counters the next batch starts from;
 		 * nobody reads them any more in this launch (the seed was snapshotted) */
-		state->rr_small_counter = carry_small;
-		state->rr_counter = carry_big;
+		state->rr_small_counter = after_small;
+		state->rr_counter = after_big;
 	}
 }
 
-/* Scratch for tile totals / prefixes, one per stream (launches on one stream are ordered, so
- * they can share; launches on different streams may overlap and must not), grown on demand. */
-struct workspace_t {
-	uint32_t *totals = nullptr;
-	uint32_t *prefix = nullptr; /* prefix[capacity] is the seed word */
-	uint32_t tiles = 0;
-};
+/* Scratch of the batches of one stream: launches on one stream are ordered, so they can share; launches on
+ * different streams may overlap and must not.  Layout in 32-bit words: the arrival word of the one-launch
+ * form, which is zero between batches, and the seed word of the others, on 128-byte lines of
+ * their own; then the block totals; then the tile totals. */
+constexpr uint32_t kArrivalWord = 0, kSeedWord = 32, kBlockWords = 64;
+constexpr uint32_t kTileWords = kBlockWords + kMaxBlocks;
+constexpr uint32_t kScratchWords = kTileWords + kMaxTiles;
 std::mutex g_ws_lock;
-std::unordered_map<void *, workspace_t> g_ws_by_stream;
+std::unordered_map<void *, uint32_t *> g_ws_by_stream;
+
+__global__ __launch_bounds__(64) void stripe_scratch_kernel(uint32_t *__restrict__ words)
+{
+	words[threadIdx.x] = 0;
+}
 
 /*
  * The same scratch for callers that may not allocate: one array per GPU, part of the loaded
- * code object, held until the process ends.  Layout in 32-bit words:
- * [0, kNoAllocTiles) tile totals, [kNoAllocTiles, 2 * kNoAllocTiles) tile prefixes, then the
- * seed word.  kNoAllocMaxBatch messages need kNoAllocTiles tiles of 1024.  In host code the
+ * code object (which starts at zero), held until the process ends.  In host code the
  * array's name is only a handle for hipGetSymbolAddress; kernels get the address it returns.
  */
 constexpr uint64_t kNoAllocMaxBatch = 1ull << 26;
-constexpr uint32_t kNoAllocTiles = (uint32_t)(kNoAllocMaxBatch / (kThreads * kPassesLarge));
-static_assert(kNoAllocTiles >= kInlineTiles, "small batches use up to kInlineTiles tiles of 512");
-static __device__ __align__(256) __attribute__((used)) uint32_t scratch[2 * kNoAllocTiles + 64];
+static __device__ __align__(256) __attribute__((used)) uint32_t scratch[kScratchWords];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_lock;
@@ -517,29 +496,35 @@ int scratch_of_current_device(uint32_t **out)
 	return 0;
 }
 
-uint32_t pick_passes(uint64_t n)
+uint32_t tiles_of(uint64_t n, uint32_t tile)
 {
-	return n <= kSmallBatch ? kPassesSmall : kPassesLarge;
+	return (uint32_t)((n + tile - 1) / tile);
 }
 
-template <uint32_t PASSES>
-void launch_batch(hipStream_t s, uint32_t tiles, const uint64_t *d_sizes, uint32_t n,
-		  ofi_amd_sched_state_t *d_state, uint64_t align, uint32_t *totals, uint32_t *prefix,
-		  uint32_t *seed0, uint32_t *d_num_xfers, u32x4 *d_xfers, uint32_t *err)
+void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_amd_sched_state_t *d_state, uint64_t align,
+		  uint32_t *words, uint32_t *d_num_xfers, u32x4 *d_xfers, uint32_t *err)
 {
-	hipLaunchKernelGGL(stripe_count_kernel<PASSES>, dim3(tiles), dim3(kThreads), 0, s, d_sizes, n, d_state,
-			   align, totals, seed0, err);
-	const uint32_t xcd_run_shift = n >= kXcdRunBatch ? kXcdRunShift : 0u;
-	const uint32_t xcd_run = 1u << xcd_run_shift;
-	const uint32_t emit_grid = (tiles + 8u * xcd_run - 1u) / (8u * xcd_run) * (8u * xcd_run);
-	if (tiles <= kInlineTiles) {
-		hipLaunchKernelGGL((stripe_emit_kernel<true, PASSES>), dim3(emit_grid), dim3(kThreads), 0, s, d_sizes, n,
-				   d_state, align, totals, seed0, tiles, xcd_run_shift, d_num_xfers, d_xfers);
-	} else {
-		hipLaunchKernelGGL(stripe_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, totals, tiles, d_state,
-				   prefix, err);
-		hipLaunchKernelGGL((stripe_emit_kernel<false, PASSES>), dim3(emit_grid), dim3(kThreads), 0, s, d_sizes, n,
-				   d_state, align, prefix, seed0, tiles, xcd_run_shift, d_num_xfers, d_xfers);
+	uint32_t *seed0 = words + kSeedWord, *blocks = words + kBlockWords, *totals = words + kTileWords;
+	if (total <= kDirectBatch) {
+		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kDirectTile);
+		hipLaunchKernelGGL((stripe_emit_kernel<DIRECT, kDirectTile>), dim3(tiles), dim3(kDirectTile), 0, s, d_sizes, n,
+				   d_state, align, nullptr, nullptr, words + kArrivalWord, tiles, d_num_xfers, d_xfers, err);
+		return;
+	}
+	if (total <= kSmallBatch) {
+		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kTile);
+		hipLaunchKernelGGL(stripe_count_kernel, dim3(tiles), dim3(kCountThreads), 0, s, d_sizes, n, d_state, align, totals,
+				   seed0, err);
+		hipLaunchKernelGGL((stripe_emit_kernel<TILES, kTile>), dim3(tiles), dim3(kTile), 0, s, d_sizes, n, d_state, align,
+				   totals, nullptr, seed0, tiles, d_num_xfers, d_xfers, err);
+		return;
+	}
+	for (uint64_t at = 0; at < total; at += kPart) {
+		const uint32_t n = (uint32_t)(total - at < kPart ? total - at : kPart), tiles = tiles_of(n, kBigTile);
+		hipLaunchKernelGGL(stripe_count_big_kernel, dim3(tiles_of(tiles, kBlockTiles)), dim3(64 * kBlockTiles), 0, s,
+				   d_sizes + at, n, d_state, align, totals, blocks, seed0, err);
+		hipLaunchKernelGGL((stripe_emit_kernel<BLOCKS, kBigTile>), dim3(tiles), dim3(kBigTile), 0, s, d_sizes + at, n,
+				   d_state, align, totals, blocks, seed0, tiles, d_num_xfers + at, d_xfers + 6 * at, err);
 	}
 }
 
@@ -594,38 +579,17 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
 		return -ENOMEM;
 	}
 
-	const uint32_t passes = pick_passes(n);
-	const uint32_t tiles = (uint32_t)((n + kThreads * passes - 1) / (kThreads * passes));
 	hipStream_t s = as_stream(stream);
 	try {
 		/* held until the launches are queued: two threads submitting to one stream share its
 		 * scratch, and their count/emit pairs must not interleave */
 		std::lock_guard<std::mutex> g(g_ws_lock);
-		workspace_t &ws = g_ws_by_stream[stream];
-		if (tiles > ws.tiles) {
-			uint32_t want = tiles < 4096 ? 4096 : tiles;
-			uint32_t *a = nullptr, *b = nullptr;
-			OFI_AMD_HIP_TRY(hipMalloc((void **)&a, sizeof(uint32_t) * want));
-			if (hipMalloc((void **)&b, sizeof(uint32_t) * (want + 1)) != hipSuccess) {
-				(void)hipFree(a);
-				return -ENOMEM;
-			}
-			/* the older buffers may still be in use by launches queued on this stream */
-			(void)hipStreamSynchronize(s);
-			(void)hipFree(ws.totals);
-			(void)hipFree(ws.prefix);
-			ws.totals = a;
-			ws.prefix = b;
-			ws.tiles = want;
+		uint32_t *&words = g_ws_by_stream[stream];
+		if (!words) {
+			OFI_AMD_HIP_TRY(hipMalloc((void **)&words, sizeof(uint32_t) * kScratchWords));
+			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(1), dim3(64), 0, s, words);
 		}
-		uint32_t *seed0 = ws.prefix + ws.tiles;
-		if (passes == kPassesSmall) {
-			launch_batch<kPassesSmall>(s, tiles, d_sizes, (uint32_t)n, d_state, align, ws.totals, ws.prefix,
-						   seed0, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
-		} else {
-			launch_batch<kPassesLarge>(s, tiles, d_sizes, (uint32_t)n, d_state, align, ws.totals, ws.prefix,
-						   seed0, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
-		}
+		launch_batch(s, d_sizes, n, d_state, align, words, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
 	} catch (...) {
 		return -ENOMEM;
 	}
@@ -639,20 +603,19 @@ int ofi_amd_sched_stream_release(void *stream)
 	if (rc != 0) {
 		return rc;
 	}
-	workspace_t ws;
+	uint32_t *words = nullptr;
 	{
 		std::lock_guard<std::mutex> g(g_ws_lock);
 		auto it = g_ws_by_stream.find(stream);
 		if (it == g_ws_by_stream.end()) {
 			return 0; /* nothing was ever allocated for it */
 		}
-		ws = it->second;
+		words = it->second;
 		g_ws_by_stream.erase(it);
 	}
 	/* launches queued on the stream may still read the scratch */
 	OFI_AMD_HIP_TRY(hipStreamSynchronize(as_stream(stream)));
-	(void)hipFree(ws.totals);
-	(void)hipFree(ws.prefix);
+	(void)hipFree(words);
 	return 0;
 }
 
@@ -685,18 +648,8 @@ int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *
 	if (rc != 0) {
 		return rc;
 	}
-	uint32_t *totals = base, *prefix = base + kNoAllocTiles, *seed0 = base + 2 * kNoAllocTiles;
-
-	const uint32_t passes = pick_passes(n);
-	const uint32_t tiles = (uint32_t)((n + kThreads * passes - 1) / (kThreads * passes));
-	hipStream_t s = as_stream(stream);
-	if (passes == kPassesSmall) {
-		launch_batch<kPassesSmall>(s, tiles, d_sizes, (uint32_t)n, d_state, align, totals, prefix, seed0,
-					   d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
-	} else {
-		launch_batch<kPassesLarge>(s, tiles, d_sizes, (uint32_t)n, d_state, align, totals, prefix, seed0,
-					   d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
-	}
+	launch_batch(as_stream(stream), d_sizes, n, d_state, align, base, d_num_xfers,
+		     reinterpret_cast<u32x4 *>(d_xfers), err);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -121,7 +121,7 @@ typedef struct {
 int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
 			uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
 			void *stream);
-/* ofi_amd_sched_batch keeps a few KiB of device scratch per stream it has been called with
+/* ofi_amd_sched_batch keeps some 80 KiB of device scratch per stream it has been called with
  * (the reference's scheduler keeps a freelist per instance, src/nccl_ofi_scheduler.cpp:135-190).
  * A caller that destroys a stream hands the scratch back first: waits for the stream, frees. */
 int ofi_amd_sched_stream_release(void *stream);
@@ -131,12 +131,13 @@ int ofi_amd_sched_stream_release(void *stream);
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
  * reference.  Same arguments, same results and the same kernels; the tile totals and prefixes
  * that ofi_amd_sched_batch keeps in a per-stream allocation live here in a fixed array inside
- * the library's device code (about 512 KiB per GPU, held until the process ends), so the call
+ * the library's device code (about 80 KiB per GPU, held until the process ends), so the call
  * allocates and frees nothing.  n <= 2^26 messages per call, -E2BIG beyond.  Call
  * ofi_amd_gpu_init() once beforehand (it allocates the asynchronous error word and looks up
  * the array's address on every GPU); -ENXIO otherwise.  All calls on one GPU share that GPU's
  * array: calls that overlap there -- different streams, or two threads -- race; order them.
- * Nothing in the array has to start at zero: a call writes every word before it reads it.
+ * One word of the array is zero between calls, as it is when the code is loaded; every other word a call
+ * writes before it reads it.
  */
 int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
 				uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,

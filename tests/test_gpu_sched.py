@@ -68,6 +68,57 @@ def test_parity_random(lib, oracle, gpu, n, rails, min_stripe, max_small, seeds)
     assert (st.max_small_msg_size, st.min_stripe_size, st.num_rails) == (max_small, min_stripe, rails)
 
 
+@pytest.mark.parametrize("n", [8191, 8192, 8193, 8704, 9 << 19, (9 << 19) + 1, (9 << 19) + 4097, 5_000_001])
+@pytest.mark.parametrize("rails,min_stripe,max_small", [(4, 131072, 64), (3, 100000, 5000)])
+def test_batches_around_the_forms_of_the_launch(lib, oracle, gpu, n, rails, min_stripe, max_small):
+    """The largest batch of the one-launch form, of the form with tiles of 512 and the smallest ones of the
+    next, with whole and ragged tiles and blocks of tiles; twice in a row, so that the second one starts
+    from what the first left in the state and in the scratch."""
+    sizes = synthetic.stripe_sizes(n + rails, n)
+    sizes[::5] = sizes[::5] % np.uint64(200)
+    d_state = dev_state(rails, min_stripe, max_small, (1, 0))
+    seeds = (1, 0)
+    for _ in range(2):
+        want_num, want_xf, ost = _oracle.sched_batch(oracle, sizes, rails, min_stripe, max_small, seeds)
+        rc, num, xf = gpu_batch(lib, d_state, sizes)
+        assert rc == 0
+        assert np.array_equal(num, want_num) and np.array_equal(xf, want_xf)
+        st = read_state(d_state)
+        seeds = (ost.rr_small_counter, ost.rr_counter)
+        assert (st.rr_small_counter, st.rr_counter) == seeds
+
+
+@pytest.mark.parametrize("min_stripe", [1, (1 << 62) - 1, 1 << 62, (1 << 63) + 5, (1 << 64) - 1])
+def test_stripe_sizes_whose_multiples_do_not_fit_64_bits(lib, oracle, gpu, min_stripe):
+    sizes = np.array([0, 1, 2, 3, 4, 5, 64, (1 << 62) - 1, 1 << 62, (1 << 62) + 1, (1 << 63) - 1, 1 << 63, (1 << 63) + 6,
+                      3 << 62, (3 << 62) - 3, (3 << 62) - 2, (1 << 64) - 130, (1 << 64) - 2, (1 << 64) - 1], dtype=np.uint64)
+    want_num, want_xf, _ = _oracle.sched_batch(oracle, sizes, 4, min_stripe, 0, (0, 2))
+    rc, num, xf = gpu_batch(lib, dev_state(4, min_stripe, 0, (0, 2)), sizes)
+    assert rc == 0 and np.array_equal(num, want_num) and np.array_equal(xf, want_xf)
+
+
+def test_a_batch_of_more_than_2_26_messages_equals_its_parts(lib, gpu):
+    """Beyond 2^26 messages sixteen tiles make a block instead of four: the batch against the same
+    messages in parts of the size the other tests cover, chained through the state, compared on the GPU."""
+    n, part = (1 << 26) + 1025, 4_000_000
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    d_sizes = torch.randint(0, 1 << 20, (n,), generator=gen, device="cuda")
+    whole, parts = dev_state(4, 131072, 64, (3, 1)), dev_state(4, 131072, 64, (3, 1))
+    d_num = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    d_xf = torch.full((n * 12,), -1, dtype=torch.int64, device="cuda")
+    p_num, p_xf = torch.empty(part, dtype=torch.int32, device="cuda"), torch.empty(part * 12, dtype=torch.int64, device="cuda")
+    assert lib.ofi_amd_sched_batch(whole.data_ptr(), d_sizes.data_ptr(), n, 128, d_num.data_ptr(), d_xf.data_ptr(),
+                                   _gpu.stream()) == 0
+    for at in range(0, n, part):
+        k = min(part, n - at)
+        assert lib.ofi_amd_sched_batch(parts.data_ptr(), d_sizes.data_ptr() + 8 * at, k, 128, p_num.data_ptr(),
+                                       p_xf.data_ptr(), _gpu.stream()) == 0
+        assert torch.equal(d_num[at:at + k], p_num[:k]) and torch.equal(d_xf[12 * at:12 * (at + k)], p_xf[:12 * k])
+    assert torch.equal(whole, parts)
+    assert lib.ofi_amd_sched_stream_release(_gpu.stream()) == 0
+
+
 @pytest.mark.parametrize("n", [1, 2, 511, 513, 70001, 3_000_001])
 def test_sizes_array_at_an_odd_eight_byte_offset(lib, oracle, gpu, n):
     """The sizes array only has to be 8-byte aligned."""
