@@ -1,13 +1,18 @@
 /*
- * Signal delivery on the GPU: a batch of folded signal work items becomes one launch of
- * 64-bit device-scope atomic adds on the counters in HBM.
+ * Signal delivery on the GPU: a batch of signal work items becomes one launch of 64-bit
+ * device-scope atomic adds on the counters in HBM.
  *
  * The reference updates each counter from a CPU worker thread through GDRCopy -- a PCIe
  * read and a PCIe write per slot (apply_signal_work, src/rdma/gin/nccl_ofi_gin.cpp:
  * 1193-1256) -- and therefore folds a batch by slot first to save round trips
- * (apply_and_complete, :1425-1479).  With the adds executed next to the memory the fold
- * is unnecessary for speed and, additions being commutative, for the result: N items on
- * one slot leave it at the same value as the reference's single +sum write.
+ * (apply_and_complete, :1425-1479).  Here a workgroup folds its items in an LDS table keyed
+ * by the counter's address and adds each sum once: additions are commutative, so every
+ * counter ends at the value that N single adds leave.
+ *
+ * What bounds it: adds to one 64-byte line of counters follow each other at 12 ns, whatever
+ * their XCD, so a batch on few counters is a queue at the memory (262,144 items on one counter
+ * 3148 us, on 64 counters 311 us, on 262,144 counters 14 us, items in HBM); items in pinned host
+ * memory come over the host link (32 B each, 8 MiB in 155 us at 54 GB/s).
  */
 #include "common.hpp"
 #include "ofi_amd_hotpath.h"
@@ -16,6 +21,7 @@ namespace {
 
 constexpr uint32_t kMaxRegions = 16;
 constexpr uint32_t kMaxApplyPost = 65536; /* items one workgroup applies in front of a flush read */
+constexpr uint32_t kProbes = 4;           /* entries of the fold an item looks at */
 
 struct regions_t {
 	uint64_t base[kMaxRegions];
@@ -24,64 +30,151 @@ struct regions_t {
 	uint32_t n;
 };
 
-__device__ __forceinline__ void apply_one(const ofi_amd_gin_signal_work_t &w, const regions_t &regions,
-					  uint32_t *__restrict__ rejected)
+/* What a workgroup keeps in LDS: the regions, indexed per lane, and the fold of its items. */
+template <uint32_t kSlots> struct fold_t {
+	unsigned long long key[kSlots]; /* address of a counter; 0: free */
+	unsigned long long sum[kSlots];
+	uint64_t base[kMaxRegions], size[kMaxRegions];
+	uint64_t *counters[kMaxRegions];
+};
+
+/* before any item; the caller waits for the workgroup afterwards */
+template <uint32_t kSlots>
+__device__ __forceinline__ void fold_begin(fold_t<kSlots> &f, const regions_t &regions, uint32_t threads)
 {
-	uint64_t *slot = nullptr;
-	/* The window is found by its base; the counter by its address inside the window, which may
-	 * continue through the regions listed next while each begins where the one before it ends
-	 * (a window backed by several allocations: the reference looks the segment up by address
-	 * too, ensure_signal_seg, src/rdma/gin/nccl_ofi_gin.cpp:1038-1122, 1156-1166). */
-	for (uint32_t r = 0; r < regions.n; r++) {
-		if (w.base != regions.base[r]) {
-			continue;
-		}
-		uint64_t off = w.offset;
-		for (uint32_t k = r;; k++) {
-			if (off <= regions.size[k] && regions.size[k] - off >= 8) {
-				slot = regions.counters[k] + (off >> 3);
-				break;
-			}
-			if (off < regions.size[k] || k + 1 >= regions.n ||
-			    regions.base[k + 1] != regions.base[k] + regions.size[k]) {
-				break; /* a counter across the end of a segment, or past the window */
-			}
-			off -= regions.size[k];
-		}
-		break;
+	for (uint32_t i = threadIdx.x; i < kSlots; i += threads) {
+		f.key[i] = 0;
+		f.sum[i] = 0;
 	}
-	if (slot == nullptr || (w.offset & 7u) != 0) {
+	if (threadIdx.x < kMaxRegions) {
+		f.base[threadIdx.x] = regions.base[threadIdx.x];
+		f.size[threadIdx.x] = regions.size[threadIdx.x];
+		f.counters[threadIdx.x] = regions.counters[threadIdx.x];
+	}
+}
+
+/* The counter of a work item, nullptr if it has none.  The window is found by its base; the
+ * counter by its address inside the window, which may continue through the regions listed next
+ * while each begins where the one before it ends (a window backed by several allocations: the
+ * reference looks the segment up by address too, ensure_signal_seg,
+ * src/rdma/gin/nccl_ofi_gin.cpp:1038-1122, 1156-1166).  The bases are compared straight through
+ * (they sit in scalar registers, the first match wins); only what follows differs from lane to
+ * lane and is read from LDS.  A loop that left at the match walked the regions once per
+ * distinct base of a wavefront, with a dependent load each: 4096 items a workgroup over 16
+ * regions took 24 us. */
+template <uint32_t kSlots>
+__device__ __forceinline__ uint64_t *slot_of(const fold_t<kSlots> &f, const regions_t &regions, uint64_t base,
+					     uint64_t offset)
+{
+	uint32_t r = kMaxRegions;
+#pragma unroll
+	for (int k = (int)kMaxRegions - 1; k >= 0; k--) {
+		r = (uint32_t)k < regions.n && base == regions.base[k] ? (uint32_t)k : r;
+	}
+	if (r == kMaxRegions || (offset & 7u) != 0) {
+		return nullptr;
+	}
+	for (uint64_t off = offset;; r++) {
+		const uint64_t size = f.size[r];
+		if (off <= size && size - off >= 8) {
+			return f.counters[r] + (off >> 3);
+		}
+		if (off < size || r + 1 >= regions.n || f.base[r + 1] != f.base[r] + size) {
+			return nullptr; /* a counter across the end of a segment, or past the window */
+		}
+		off -= size;
+	}
+}
+
+/* One item into the fold; past kProbes entries taken by other counters it goes to its own
+ * directly.  Relaxed: ordering against the payload is the put-before-signal protocol's business
+ * (the reference uses a relaxed fetch_add on its host path for the same reason, :1209). */
+template <uint32_t kSlots>
+__device__ __forceinline__ void fold_item(fold_t<kSlots> &f, const regions_t &regions, uint64_t base, uint64_t offset,
+					  uint64_t value, uint32_t *__restrict__ rejected)
+{
+	uint64_t *slot = slot_of(f, regions, base, offset);
+	if (slot == nullptr) {
 		if (rejected) {
 			atomicAdd(rejected, 1u);
 		}
 		return;
 	}
-	/* relaxed: ordering against the payload is the put-before-signal protocol's business
-	 * (the reference uses a relaxed fetch_add on its host path for the same reason, :1209) */
-	__hip_atomic_fetch_add(slot, w.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	const unsigned long long key = (unsigned long long)reinterpret_cast<uintptr_t>(slot);
+	uint32_t h = ((uint32_t)(key >> 3) * 0x9e3779b1u) >> (32 - __builtin_ctz(kSlots));
+	for (uint32_t probe = 0; probe < kProbes; probe++) {
+		unsigned long long at = __hip_atomic_load(&f.key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+		if (at == 0) {
+			at = atomicCAS(&f.key[h], 0ull, key);
+			at = at == 0 ? key : at;
+		}
+		if (at == key) {
+			__hip_atomic_fetch_add(&f.sum[h], (unsigned long long)value, __ATOMIC_RELAXED,
+					       __HIP_MEMORY_SCOPE_WORKGROUP);
+			return;
+		}
+		h = (h + 1) & (kSlots - 1);
+	}
+	__hip_atomic_fetch_add(slot, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(256) void gin_signal_apply_kernel(
+/* the sums onto the counters; after the workgroup has met behind its last item */
+template <uint32_t kSlots> __device__ __forceinline__ void fold_end(fold_t<kSlots> &f, uint32_t threads)
+{
+	for (uint32_t i = threadIdx.x; i < kSlots; i += threads) {
+		if (f.key[i] != 0) {
+			__hip_atomic_fetch_add(reinterpret_cast<uint64_t *>(f.key[i]), (uint64_t)f.sum[i], __ATOMIC_RELAXED,
+					       __HIP_MEMORY_SCOPE_AGENT);
+		}
+	}
+}
+
+template <uint32_t kThreads, uint32_t kItems, uint32_t kSlots>
+__global__ __launch_bounds__(kThreads) void gin_signal_apply_kernel(
 	const ofi_amd_gin_signal_work_t *__restrict__ work, uint32_t n, regions_t regions,
 	uint32_t *__restrict__ rejected)
 {
-	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-	if (i < n) {
-		apply_one(work[i], regions, rejected);
+	__shared__ __align__(16) fold_t<kSlots> f;
+	uint64_t base[kItems], offset[kItems], value[kItems];
+	const uint32_t first = blockIdx.x * (kThreads * kItems) + threadIdx.x;
+#pragma unroll
+	for (uint32_t k = 0; k < kItems; k++) { /* every item of a thread in flight at once */
+		const ofi_amd_gin_signal_work_t *w = work + min(first + k * kThreads, n - 1u);
+		base[k] = w->base;
+		offset[k] = w->offset;
+		value[k] = w->value;
 	}
+	fold_begin(f, regions, kThreads);
+	__syncthreads();
+#pragma unroll
+	for (uint32_t k = 0; k < kItems; k++) {
+		if (first + k * kThreads < n) {
+			fold_item(f, regions, base[k], offset[k], value[k], rejected);
+		}
+	}
+	__syncthreads();
+	fold_end(f, kThreads);
 }
 
 /* The adds of a batch and the flush read behind them in one launch of one workgroup: every
  * thread's adds have been performed at the memory before the workgroup meets, and only then is
  * the flush buffer read back into the host's slots -- what two launches order by the kernel
  * boundary between them. */
-__global__ __launch_bounds__(256) void gin_signal_apply_post_kernel(
+constexpr uint32_t kPostThreads = 256, kPostSlots = 1024;
+__global__ __launch_bounds__(kPostThreads) void gin_signal_apply_post_kernel(
 	const ofi_amd_gin_signal_work_t *__restrict__ work, uint32_t n, regions_t regions,
 	uint32_t *__restrict__ rejected, const uint64_t *__restrict__ flush_buf, uint64_t *__restrict__ slots,
 	uint32_t num_rails)
 {
-	for (uint32_t i = threadIdx.x; i < n; i += 256u) {
-		apply_one(work[i], regions, rejected);
+	__shared__ __align__(16) fold_t<kPostSlots> f;
+	if (n != 0) {
+		fold_begin(f, regions, kPostThreads);
+		__syncthreads();
+		for (uint32_t i = threadIdx.x; i < n; i += kPostThreads) {
+			fold_item(f, regions, work[i].base, work[i].offset, work[i].value, rejected);
+		}
+		__syncthreads();
+		fold_end(f, kPostThreads);
 	}
 	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
 	__syncthreads();
@@ -112,6 +205,16 @@ static int pack_regions(const ofi_amd_gin_signal_region_t *regions, uint32_t n_r
 	return 0;
 }
 
+static bool in_host_memory(const void *p)
+{
+	hipPointerAttribute_t attr;
+	if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+		(void)hipGetLastError();
+		return false;
+	}
+	return attr.type == hipMemoryTypeHost;
+}
+
 extern "C" int ofi_amd_gin_signal_apply(const ofi_amd_gin_signal_work_t *d_work, uint32_t n,
 					const ofi_amd_gin_signal_region_t *regions, uint32_t n_regions,
 					uint32_t *d_rejected, void *stream)
@@ -127,8 +230,36 @@ extern "C" int ofi_amd_gin_signal_apply(const ofi_amd_gin_signal_work_t *d_work,
 	if (!d_work || pack_regions(regions, n_regions, &r) != 0) {
 		return -EINVAL;
 	}
-	hipLaunchKernelGGL(gin_signal_apply_kernel, dim3((n + 255u) / 256u), dim3(256), 0, as_stream(stream),
-			   d_work, n, r, d_rejected);
+	/* Items per workgroup.  More items fold further, fewer spread the lookups over more CUs; times
+	 * in us with a launch per item before the fold / with 256, 512, 1024 x 2, 1024 x 4 items.
+	 *   1000 items in host memory, 1 counter           15.3 / 4.0  4.4  5.0  6.0
+	 *   1000 items in host memory, 8192 counters        5.6 / 4.5  4.9  5.9  6.8
+	 *   16384 items in host memory, 64 counters        24.8 / 16.8 14.3 13.1 13.4
+	 *   16384 items in host memory, 8192 counters      15.3 / 13.9 13.8 16.3 20.2
+	 *   262144 items in HBM, 64 counters                311 / 166  90   25.9 16.5
+	 *   262144 items in HBM, 8192 counters             16.8 / 16.0 15.8 16.5 18.0
+	 *   262144 items in HBM, 262144 counters           14.3 / 14.6 14.6 16.5 18.0
+	 * so 256 up to 4096 items, then 512, and 2048 or 4096 for long batches on few counters (one to 64 items or more).  Long
+	 * batches in host memory take those too: the link is read faster from 64 CUs than from all of
+	 * them (262144 items over 8192 counters 187 / 188 187 179 160). */
+	uint64_t counters = 0;
+	for (uint32_t i = 0; i < n_regions; i++) {
+		counters += r.size[i] / 8;
+	}
+	const bool large = n > 32768u && (counters <= n / 64u || in_host_memory(d_work));
+	auto launch = [&](auto kernel, uint32_t threads, uint32_t items) {
+		hipLaunchKernelGGL(kernel, dim3((n - 1u) / (threads * items) + 1u), dim3(threads), 0, as_stream(stream),
+				   d_work, n, r, d_rejected);
+	};
+	if (n <= 4096u) {
+		launch(gin_signal_apply_kernel<256, 1, 512>, 256, 1);
+	} else if (!large) {
+		launch(gin_signal_apply_kernel<512, 1, 1024>, 512, 1);
+	} else if (n <= 131072u) {
+		launch(gin_signal_apply_kernel<1024, 2, 4096>, 1024, 2);
+	} else {
+		launch(gin_signal_apply_kernel<1024, 4, 4096>, 1024, 4);
+	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -210,6 +210,42 @@ def test_windows_backed_by_several_segments(lib, oracle, gpu):
         assert np.array_equal(got[:-1], h) and got[-1] == 0
 
 
+@pytest.mark.parametrize("pinned", [False, True])
+@pytest.mark.parametrize("n,slots", [(4096, 600), (4097, 3), (4097, 40000), (32768, 3), (32769, 1), (32769, 5000),
+                                     (131072, 4097), (131073, 1), (131073, 70001)])
+def test_workgroup_folds_at_their_edges(lib, gpu, n, slots, pinned):
+    """Batches on both sides of every size at which the launch changes its items per workgroup, on few
+    counters (one entry of the fold takes a workgroup's every item) and on more than the fold holds;
+    a window that goes on in the next region, and one item in eight without a counter.  Sums modulo
+    2^64 and the count of refused items are exact."""
+    rng = np.random.default_rng(n + slots)
+    cut = (slots + 1) // 2
+    work = np.zeros(n, dtype=work_array([(0,) * 6]).dtype)
+    kind = rng.integers(0, 32, n)
+    slot = rng.integers(0, slots, n).astype(np.uint64)
+    work["base"], work["offset"] = SIG_BASE, 8 * slot
+    work["value"] = rng.integers(0, 1 << 63, n).astype(np.uint64) * np.uint64(2) + np.uint64(1)
+    work["base"][kind == 0] += np.uint64(8)                       # no such window
+    work["offset"][kind == 1] += np.uint64(4)                     # not a counter's address
+    work["offset"][kind == 2] = np.uint64(8 * slots)              # past the window
+    work["offset"][kind == 3] = np.uint64((1 << 64) - 8)
+    want = rng.integers(0, 1 << 63, slots).astype(np.uint64)
+    d_counters = _gpu.to_dev(want.copy())
+    ok = kind > 3
+    np.add.at(want, slot[ok].astype(np.int64), work["value"][ok])
+    pieces = [(0, cut)] + ([(cut, slots)] if slots > cut else [])
+    regs = (m.GinSignalRegion * len(pieces))(*[
+        m.GinSignalRegion(SIG_BASE + 8 * a, 8 * (b - a), d_counters.data_ptr() + 8 * a) for a, b in pieces])
+    words = torch.from_numpy(work.view(np.int64))
+    d_work = words.pin_memory() if pinned else words.cuda()
+    rejected = torch.zeros(1, dtype=torch.int32, device="cuda")
+    assert lib.ofi_amd_gin_signal_apply(ctypes.c_void_p(d_work.data_ptr()), n, regs, len(pieces),
+                                        ctypes.c_void_p(rejected.data_ptr()), _gpu.stream()) == 0
+    _gpu.sync()
+    assert np.array_equal(_gpu.to_host(d_counters, np.uint64), want)
+    assert int(rejected.item()) == int((~ok).sum())
+
+
 def test_work_items_in_pinned_host_memory(lib, oracle, gpu):
     """The proxy writes work items into pinned host memory and launches straight from there."""
     n = 5000
