@@ -340,41 +340,68 @@ __global__ __launch_bounds__(64 * kTableWaves) void copy_table_kernel(const uint
 }
 
 /*
- * The same table with one wavefront per 8 KiB piece of an entry instead of per entry: entry e is
- * pieces [e * pieces_per_entry, (e + 1) * pieces_per_entry), and a wavefront whose piece lies
- * beyond its entry's length leaves at once.  Consecutive wavefronts then sweep long entries
- * densely, 8 KiB each, instead of each streaming through its own entry (1 GiB copied 8 KiB per
- * wavefront: 5.65 TB/s read + written, 256 KiB per wavefront: 5.17), and the XCDs take runs of
- * 128 consecutive pieces (1 MiB) in turn (5.82 TB/s; runs of 4 or 16: 5.5-5.7).
+ * The same table with one wavefront per 8 KiB piece of an entry instead of per entry: entry e has
+ * the `per` piece numbers from e * per on, and a wavefront whose piece lies beyond its entry's
+ * length leaves at once.  Consecutive wavefronts then sweep long entries densely, 8 KiB each,
+ * instead of each streaming through its own entry (1 GiB copied 8 KiB per wavefront: 5.65 TB/s read
+ * + written, 256 KiB per wavefront: 5.17), and the XCDs take runs of about 128 consecutive pieces (1 MiB)
+ * in turn (5.82 TB/s; runs of 4 or 16: 5.5-5.7).
+ *
+ * A table of mixed lengths consists mostly of pieces that do not exist (lengths log-uniform in
+ * 8 B..1 MiB: 11 of an entry's 128 pieces do), and how those that do are dealt out counts:
+ * - Workgroups are handed out at about 4.5 a nanosecond, whatever they hold: 262,144 wavefronts that
+ *   leave at once take 56 us singly and 15 us by fours.  244 entries of 8 B..64 MiB: 538 us
+ *   singly, 435 us by fours.  By fours a dense copy is as fast as singly; by eights a sparse one is slower
+ *   (2048 entries of 8 B..1 MiB 84 us against 76).
+ * - Workgroups are dealt to the XCDs, and inside one to the shader engines, in turn.  With a power of two of
+ *   pieces to an entry the first, always present pieces of all entries fall to the same few of them.  So
+ *   `per` is odd, or an odd number of runs, each of an odd number of workgroups, and the four
+ *   wavefronts of a workgroup take pieces a quarter of a run apart (copy_pieces_map says from when
+ *   on).  442 entries of 64 KiB..4 MiB: 204 -> 180 us; 16,384 of 8 B..64 KiB: 59 -> 48 us; 10,088
+ *   of 8 B..512 KiB 200 -> 183 us.
+ * - The table may lie in host memory, a link's round trip away.  Its three words are asked for together,
+ *   not the addresses once the length is known (7 entries of 4-8 KiB: 5.6 -> 4.1 us).
+ * All told, tables in host memory, other buffers at every launch: 2048 entries of 8 B..1 MiB 78 -> 76 us (4.9 of
+ * the 5.4 TB/s read + written of one plain copy of those bytes), 16,384 of 8 B..64 KiB 69 -> 48 us.
  */
 constexpr uint32_t kPieceBytes = kRows * 1024u;
-constexpr uint32_t kPieceRunShift = 7;
-__global__ __launch_bounds__(64) void copy_table_pieces_kernel(const uint64_t *__restrict__ src_addr,
-							       const uint64_t *__restrict__ dst_addr,
-							       const uint32_t *__restrict__ len, uint32_t n,
-							       uint32_t pieces_per_entry, uint32_t max_len,
-							       uint32_t *__restrict__ err)
+constexpr uint32_t kPieceWaves = 4;
+constexpr uint32_t kRunPieces = 128;
+struct piece_map_t {
+	uint32_t per;         /* piece numbers of an entry: at least those of the longest one */
+	uint32_t run_blocks;  /* workgroups of a run */
+	uint32_t wave_stride; /* piece numbers between two wavefronts of a workgroup, and ... */
+	uint32_t block_stride; /* ... between two workgroups of a run */
+};
+__global__ __launch_bounds__(64 * kPieceWaves) void copy_table_pieces_kernel(const uint64_t *__restrict__ src_addr,
+									     const uint64_t *__restrict__ dst_addr,
+									     const uint32_t *__restrict__ len, uint32_t n,
+									     piece_map_t map, uint32_t max_len,
+									     uint32_t *__restrict__ err)
 {
-	const uint32_t lane = threadIdx.x;
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const uint32_t xcd = blockIdx.x % kXcds, turn = blockIdx.x / kXcds;
-	const uint32_t g = ((((turn >> kPieceRunShift) * kXcds) + xcd) << kPieceRunShift) +
-			   (turn & ((1u << kPieceRunShift) - 1u));
-	const uint32_t e = g / pieces_per_entry, piece = g - e * pieces_per_entry;
+	const uint32_t run = turn / map.run_blocks, block = turn - run * map.run_blocks;
+	const uint32_t g = (run * kXcds + xcd) * map.run_blocks * kPieceWaves + wave * map.wave_stride +
+			   block * map.block_stride;
+	const uint32_t e = g / map.per, piece = g - e * map.per;
 	if (e >= n) {
 		return;
 	}
 	const uint32_t stated = len[e];
+	const uint64_t src = src_addr[e], dst = dst_addr[e];
+	/* all three are in hand from here on: the compiler would move the addresses behind the test of the length */
+	__asm__ volatile("" : : "s"(stated), "s"(src), "s"(dst));
 	if (piece == 0 && stated > max_len && lane == 0) {
 		atomicOr(err, ofi_amd::ASYNC_ERR_COPY_LENGTH); /* longer than the caller said: the rest stays uncopied */
 	}
 	const uint32_t bytes = min(stated, max_len);
 	const uint64_t off = (uint64_t)piece * kPieceBytes;
-	if (off >= bytes) {
-		return;
+	if (off < bytes) {
+		copy_any(reinterpret_cast<const uint8_t *>(src + off), reinterpret_cast<uint8_t *>(dst + off),
+			 min((uint32_t)(bytes - off), kPieceBytes), lane);
 	}
-	const uint32_t here = bytes - off < kPieceBytes ? (uint32_t)(bytes - off) : kPieceBytes;
-	copy_any(reinterpret_cast<const uint8_t *>(src_addr[e] + off), reinterpret_cast<uint8_t *>(dst_addr[e] + off),
-		 here, lane);
 }
 
 __global__ __launch_bounds__(256) void flush_read_kernel(const uint8_t *__restrict__ arena,
@@ -399,6 +426,34 @@ __global__ __launch_bounds__(64) void flush_post_kernel(const uint64_t *__restri
 							uint64_t *__restrict__ slots, uint32_t num_rails)
 {
 	ofi_amd::flush_post_lanes(flush_buf, slots, num_rails, threadIdx.x);
+}
+
+/*
+ * How the pieces of a table are dealt out, by the pieces of its longest entry (`pieces`: of all entries
+ * if they were all that long).  Few pieces: neighbours in a workgroup, whose table words then share cache lines
+ * (5818 entries of up to 4 pieces 11.0 us, a quarter of a run apart 13.8).  1024 and more: an entry has
+ * a run for every XCD and spreads by itself (64 entries of 16-32 MiB 578 us, padded 582).
+ * Between the two as the kernel's comment says.  Tables so large that the padding might exceed what one launch
+ * can number (2^32 work-items) go without it.
+ */
+constexpr uint32_t kFewPieces = 8, kManyPieces = 1024;
+constexpr uint64_t kMostPadded = 1ull << 24;
+piece_map_t copy_pieces_map(uint32_t per, uint64_t pieces)
+{
+	piece_map_t m = { per, kRunPieces / kPieceWaves, 1, kPieceWaves };
+	if (per < kFewPieces || per >= kManyPieces || pieces > kMostPadded) {
+		return m;
+	}
+	if (per <= kRunPieces) {
+		m.per = per | 1u;
+	} else {
+		const uint32_t runs = ((per + kRunPieces - 1) / kRunPieces) | 1u;
+		m.run_blocks = ((per + runs * kPieceWaves - 1) / (runs * kPieceWaves)) | 1u;
+		m.per = runs * m.run_blocks * kPieceWaves;
+	}
+	m.wave_stride = m.run_blocks;
+	m.block_stride = 1;
+	return m;
 }
 
 } // namespace
@@ -510,17 +565,20 @@ int ofi_amd_copy_table_pieces(const uint64_t *d_src_addr, const uint64_t *d_dst_
 		return -EINVAL;
 	}
 	const uint64_t pieces_per_entry = max_len == 0 ? 1 : ((uint64_t)max_len + kPieceBytes - 1) / kPieceBytes;
-	const uint64_t round = (uint64_t)kXcds << kPieceRunShift; /* whole rounds over the XCDs */
-	const uint64_t blocks = ((uint64_t)n * pieces_per_entry + round - 1) / round * round;
-	if (blocks > 0x7fffffffull) {
-		return -E2BIG; /* more pieces than one launch has workgroups: split the table */
+	const uint64_t least = (uint64_t)kXcds * kRunPieces;
+	const uint64_t pieces = ((uint64_t)n * pieces_per_entry + least - 1) / least * least;
+	if (pieces > 0x7fffffffull) {
+		return -E2BIG; /* split the table */
 	}
 	uint32_t *err = async_error_word();
 	if (!err) {
 		return -ENOMEM;
 	}
-	hipLaunchKernelGGL(copy_table_pieces_kernel, dim3((uint32_t)blocks), dim3(64), 0, as_stream(stream), d_src_addr,
-			   d_dst_addr, d_len, n, (uint32_t)pieces_per_entry, max_len, err);
+	const piece_map_t map = copy_pieces_map((uint32_t)pieces_per_entry, pieces);
+	const uint64_t round = (uint64_t)kXcds * map.run_blocks * kPieceWaves; /* whole rounds over the XCDs */
+	const uint64_t blocks = ((uint64_t)n * map.per + round - 1) / round * (kXcds * map.run_blocks);
+	hipLaunchKernelGGL(copy_table_pieces_kernel, dim3((uint32_t)blocks), dim3(64 * kPieceWaves), 0, as_stream(stream),
+			   d_src_addr, d_dst_addr, d_len, n, map, max_len, err);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -210,8 +210,8 @@ int ofi_amd_copy_table(const uint64_t *d_src_addr, const uint64_t *d_dst_addr, c
  * entry rather than per entry, so that a few long RDMA writes (a rendezvous message's
  * stripes: one fi_writedata per rail, src/nccl_ofi_rdma.cpp:2447-2479) are swept by the whole chip
  * instead of by one wavefront each, and the caller need not cut them.  max_len >= every
- * d_len[i]; the launch has n * ceil(max_len / 8192) wavefronts (-E2BIG beyond 2^31 - 1: split
- * the table), those past the end of their entry leave at once.  An entry longer than max_len
+ * d_len[i]; the launch has a wavefront for each of n * ceil(max_len / 8192) pieces, and up to twice as many
+ * (-E2BIG beyond 2^31 - 1 pieces: split the table); those past the end of their entry leave at once.  An entry longer than max_len
  * is copied up to exactly max_len bytes (nothing of it when max_len is 0) and reported through
  * ofi_amd_async_error_fetch (bit 3).
  */

@@ -322,3 +322,32 @@ def test_bad_arguments(lib, gpu):
     assert lib.ofi_amd_gin_loopback_run(rings, 1, *args, 1, 0, 0, 0, 1, 10, None, ctypes.byref(stats)) == -22
     assert lib.ofi_amd_gin_loopback_run(rings, 1, *args, 1, 5000, 64, 0, 1, 10, None, ctypes.byref(stats)) == -22
     lib.ofi_amd_gin_rings_destroy(rings)
+
+
+@pytest.mark.parametrize("pieces,n", [(1, 9), (7, 40), (8, 40), (9, 257), (127, 37), (128, 8), (129, 41), (257, 9),
+                                      (1023, 10), (1024, 10), (2049, 1)])
+def test_every_piece_of_a_mixed_table_is_dealt_out_once(lib, gpu, pieces, n):
+    """The piece numbering changes with the pieces of the longest entry (few, up to a run, several runs, a
+    run for every XCD): lengths from nothing to exactly that many pieces, at any alignment, in a table
+    in pinned host memory, guard bytes between the destinations."""
+    rng = np.random.default_rng(pieces)
+    max_len = pieces * 8192
+    lens = np.minimum((2.0 ** (rng.random(n) * np.log2(max_len))).astype(np.uint32), max_len)
+    lens[n // 2], lens[0] = max_len, max_len if n == 1 else 0
+    room = lens.astype(np.int64) + rng.integers(1, 70, n)
+    dst_off = np.cumsum(room) - room
+    src_off = rng.integers(0, 64, n)
+    src = rng.integers(0, 256, max_len + 64, dtype=np.uint8)
+    want = np.full(int(room.sum()) + 64, 0x77, dtype=np.uint8)
+    for s, d, l in zip(src_off, dst_off, lens):
+        want[d:d + int(l)] = src[s:s + int(l)]
+    d_src = _gpu.to_dev(src)
+    d_dst = torch.full((len(want),), 0x77, dtype=torch.uint8, device="cuda")
+    t_src = torch.from_numpy(src_off + d_src.data_ptr()).pin_memory()
+    t_dst = torch.from_numpy(dst_off + d_dst.data_ptr()).pin_memory()
+    t_len = torch.from_numpy(lens.view(np.int32)).pin_memory()
+    assert lib.ofi_amd_copy_table_pieces(t_src.data_ptr(), t_dst.data_ptr(), t_len.data_ptr(), n, max_len,
+                                         _gpu.stream()) == 0
+    _gpu.sync()
+    assert np.array_equal(d_dst.cpu().numpy(), want)
+    assert _gpu.fetch_async_errors(lib) == 0
