@@ -445,6 +445,38 @@ __global__ __launch_bounds__(64) void stripe_scratch_kernel(uint32_t *__restrict
 	words[threadIdx.x] = 0;
 }
 
+/* Scratch for stream s with its arrival word at zero before anything queued on s from here on.  A stream that is
+ * being captured would only record the clearing launch, and batches called before the first replay would count
+ * from whatever the memory held: there it runs on a stream of its own and is waited for. */
+int new_scratch(hipStream_t s, uint32_t **out)
+{
+	uint32_t *words = nullptr;
+	OFI_AMD_HIP_TRY(hipMalloc((void **)&words, sizeof(uint32_t) * kScratchWords));
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	hipError_t e = hipStreamIsCapturing(s, &capture);
+	if (e == hipSuccess && capture == hipStreamCaptureStatusNone) {
+		hipLaunchKernelGGL(stripe_scratch_kernel, dim3(1), dim3(64), 0, s, words);
+		e = hipGetLastError();
+	} else {
+		hipStream_t own = nullptr;
+		e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+		if (e == hipSuccess) {
+			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(1), dim3(64), 0, own, words);
+			e = hipGetLastError();
+			const hipError_t waited = hipStreamSynchronize(own);
+			e = e == hipSuccess ? waited : e;
+			(void)hipStreamDestroy(own);
+		}
+	}
+	if (e != hipSuccess) {
+		(void)hipGetLastError();
+		(void)hipFree(words);
+		return ofi_amd::errno_of(e);
+	}
+	*out = words;
+	return 0;
+}
+
 /*
  * The same scratch for callers that may not allocate: one array per GPU, part of the loaded
  * code object (which starts at zero), held until the process ends.  In host code the
@@ -586,8 +618,10 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
 		std::lock_guard<std::mutex> g(g_ws_lock);
 		uint32_t *&words = g_ws_by_stream[stream];
 		if (!words) {
-			OFI_AMD_HIP_TRY(hipMalloc((void **)&words, sizeof(uint32_t) * kScratchWords));
-			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(1), dim3(64), 0, s, words);
+			rc = new_scratch(s, &words);
+			if (rc != 0) {
+				return rc;
+			}
 		}
 		launch_batch(s, d_sizes, n, d_state, align, words, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
 	} catch (...) {

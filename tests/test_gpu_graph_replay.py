@@ -141,3 +141,49 @@ def test_graph_of_hot_path_launches_replays_exactly(lib, oracle, gpu):
             counters += per_replay
         assert np.array_equal(_gpu.to_host(d_cnt, np.uint64), counters), replay
     assert _gpu.fetch_async_errors(lib) == 0
+
+
+def test_batch_first_called_while_its_stream_is_captured(lib, oracle, gpu):
+    """The scratch of a stream is made by the call that the stream is being captured in (a capture mode that lets a
+    call allocate): batches called before the first replay, the replay and batches after it all match the oracle,
+    whatever the memory held.  1000 messages is the one-launch form, whose workgroups count themselves."""
+    s = torch.cuda.Stream()
+    sp = ctypes.c_void_p(s.cuda_stream)
+    assert lib.ofi_amd_sched_stream_release(sp) == 0
+    # memory of the scratch's size, left dirty for the allocator to hand out again
+    dirty = [torch.full((20608,), -1, dtype=torch.int32, device="cuda") for _ in range(8)]
+    torch.cuda.synchronize()
+    del dirty
+    torch.cuda.empty_cache()
+    n = 1000
+    sizes = synthetic.stripe_sizes(6, n)
+    st = m.SchedState(2, 1, 64, 131072, 4, 0)
+    d_state = _gpu.to_dev(np.frombuffer(bytes(st), dtype=np.uint8).copy())
+    d_sizes = _gpu.to_dev(sizes)
+    d_num = torch.zeros(n, dtype=torch.int32, device="cuda")
+    d_xf = torch.zeros(n * 12, dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+
+    def call():
+        return lib.ofi_amd_sched_batch(d_state.data_ptr(), d_sizes.data_ptr(), n, 128, d_num.data_ptr(), d_xf.data_ptr(), sp)
+
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s, capture_error_mode="relaxed"):
+        rc = call()
+    if rc != 0:
+        pytest.skip("this runtime refuses allocations during a capture: %d" % rc)
+    seeds = (2, 1)
+    for step in ("call", "replay", "call", "replay"):
+        if step == "call":
+            assert call() == 0
+        else:
+            with torch.cuda.stream(s):
+                g.replay()
+        s.synchronize()
+        want_num, want_xf, ost = _oracle.sched_batch(oracle, sizes, 4, 131072, 64, seeds)
+        assert np.array_equal(_gpu.to_host(d_num, np.uint32), want_num), step
+        assert np.array_equal(_gpu.to_host(d_xf, np.uint64).reshape(n, 4, 3), want_xf), step
+        now = m.SchedState.from_buffer_copy(d_state.cpu().numpy().tobytes())
+        seeds = (ost.rr_small_counter, ost.rr_counter)
+        assert (now.rr_small_counter, now.rr_counter) == seeds, step
+    assert lib.ofi_amd_sched_stream_release(sp) == 0

@@ -68,12 +68,13 @@ def test_parity_random(lib, oracle, gpu, n, rails, min_stripe, max_small, seeds)
     assert (st.max_small_msg_size, st.min_stripe_size, st.num_rails) == (max_small, min_stripe, rails)
 
 
-@pytest.mark.parametrize("n", [8191, 8192, 8193, 8704, 9 << 19, (9 << 19) + 1, (9 << 19) + 4097, 5_000_001])
+@pytest.mark.parametrize("n", [255, 257, 4097, 6143, 6144, 6145, 6656, 6 << 20, (6 << 20) + 1, (6 << 20) + 4097, (1 << 24) + 1])
 @pytest.mark.parametrize("rails,min_stripe,max_small", [(4, 131072, 64), (3, 100000, 5000)])
 def test_batches_around_the_forms_of_the_launch(lib, oracle, gpu, n, rails, min_stripe, max_small):
-    """The largest batch of the one-launch form, of the form with tiles of 512 and the smallest ones of the
-    next, with whole and ragged tiles and blocks of tiles; twice in a row, so that the second one starts
-    from what the first left in the state and in the scratch."""
+    """Batches of the one-launch form up to its largest (6144), of the form with tiles of 512 up to its largest
+    (6 Mi) and the smallest ones of the next, with whole and ragged tiles and blocks of tiles and a second
+    part of one message; twice in a row, so that the second one starts from what the first left in the
+    state and in the scratch."""
     sizes = synthetic.stripe_sizes(n + rails, n)
     sizes[::5] = sizes[::5] % np.uint64(200)
     d_state = dev_state(rails, min_stripe, max_small, (1, 0))
@@ -98,8 +99,8 @@ def test_stripe_sizes_whose_multiples_do_not_fit_64_bits(lib, oracle, gpu, min_s
 
 
 def test_a_batch_of_more_than_2_26_messages_equals_its_parts(lib, gpu):
-    """Beyond 2^26 messages sixteen tiles make a block instead of four: the batch against the same
-    messages in parts of the size the other tests cover, chained through the state, compared on the GPU."""
+    """Five parts of 2^24 messages, the last one ragged: the batch against the same messages in batches of the
+    form with tiles of 512, chained through the state, compared on the GPU."""
     n, part = (1 << 26) + 1025, 4_000_000
     gen = torch.Generator(device="cuda")
     gen.manual_seed(5)
