@@ -32,8 +32,11 @@ struct grid_dims_t {
 	const double *log2_nodes; /* log2((double)nodes[i]) from the host's libm */
 	const double *log2_sizes; /* per size index: transform_log2 of the byte count */
 	const double *log2_ranks; /* per (node, ppn): transform_log2 of the rank count */
-	/* tiles of the region grid: 2^tile_shift node counts x 2^(6 - tile_shift) sizes, a wavefront each */
-	uint32_t tile_shift, tiles_n, tiles_s;
+};
+
+/* tiles of the region grid: 2^shift_n node counts x 2^shift_s sizes, a wavefront each */
+struct tiling_t {
+	uint32_t shift_n, shift_s, tiles_n, tiles_s;
 	const double2 *size_span; /* per tile row: smallest and largest log2_sizes */
 	const double2 *rank_span; /* per (tile column, ppn): smallest and largest log2_ranks */
 };
@@ -254,7 +257,8 @@ __device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64
  * point, with quotients, took 40-42 us for 1.02 M points of four platforms (560 sizes, 38 node counts),
  * this takes 12.0: 5 us of it are the dispatch of 16,896 wavefronts, the rest the time of the
  * tiles with the most edges, which is why their turns count instructions (two edges a turn, for
- * shorter chains of dependent operations, was slower: 13.3).
+ * shorter chains of dependent operations, was slower: 13.3).  A grid of few points is the time of such a
+ * tile alone, and takes smaller ones (pick_tiling).
  *
  * In the output the ranks-per-node index runs fastest, so a wavefront's records lie 4 x
  * n_ppn bytes apart and the records between them belong to the same tile's other
@@ -263,7 +267,7 @@ __device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64
  * XCD's L2 and leave it as one line (measured: 4.7 MB written for 4.7 MB of records; with the
  * workgroups of a tile on different XCDs every L2 wrote its quarter of each line, 18.9 MB).
  */
-__global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t g, const int32_t *__restrict__ polys,
+__global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t g, tiling_t t, const int32_t *__restrict__ polys,
 							    const double *__restrict__ bboxes,
 							    const edge_t *__restrict__ edges, pt_t far_point,
 							    const region_run_t *__restrict__ runs,
@@ -279,15 +283,16 @@ __global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t
 	 * differ in cost (size range), and an XCD that kept the same ones for every
 	 * entry would keep the same share of the long ones */
 	const uint32_t tile = (blockIdx.x & ~(kXcds - 1u)) + (blockIdx.x + run.entry) % kXcds;
-	if (tile >= g.tiles_n * g.tiles_s) {
+	if (tile >= t.tiles_n * t.tiles_s) {
 		return; /* padding of the last group */
 	}
 	const uint32_t n_polys = run.counts & 0xffffu, n_edges = run.counts >> 16;
-	const uint32_t ts = tile / g.tiles_n, tn = tile - ts * g.tiles_n;
-	const uint32_t at_n = (tn << g.tile_shift) + (lane & ((1u << g.tile_shift) - 1u));
-	const uint32_t at_s = ts * (64u >> g.tile_shift) + (lane >> g.tile_shift);
-	const bool live = at_n < g.n_nodes && at_s < g.n_sizes;
-	/* lanes beyond the axes' ends stand on the tile's last point */
+	const uint32_t ts = tile / t.tiles_n, tn = tile - ts * t.tiles_n;
+	const uint32_t tile_points = 1u << (t.shift_n + t.shift_s), point = min(lane, tile_points - 1u);
+	const uint32_t at_n = (tn << t.shift_n) + (point & ((1u << t.shift_n) - 1u));
+	const uint32_t at_s = (ts << t.shift_s) + (point >> t.shift_n);
+	const bool live = lane < tile_points && at_n < g.n_nodes && at_s < g.n_sizes;
+	/* lanes beyond the tile's points and the axes' ends stand on the last point there is */
 	const uint32_t ni = min(at_n, g.n_nodes - 1u), si = min(at_s, g.n_sizes - 1u);
 
 	int algorithm = -1, protocol = -1, nchannels = -1;
@@ -302,7 +307,7 @@ __global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t
 		const uint64_t nodes = g.nodes[ni];
 		const uint64_t size = g.sizes[si];
 		const pt_t at = { g.log2_sizes[si], g.log2_ranks[ni * g.n_ppn + run.pi] };
-		const double2 sx = g.size_span[ts], sy = g.rank_span[tn * g.n_ppn + run.pi];
+		const double2 sx = t.size_span[ts], sy = t.rank_span[tn * g.n_ppn + run.pi];
 
 		const double eps = 1e-10;
 		const double mine_f = vcross(vsub(far_point, mine.a), vsub(mine.b, mine.a));
@@ -448,7 +453,7 @@ size_t append(std::vector<uint8_t> &to, const std::vector<T> &v)
 	return at;
 }
 
-/* log2 of the node counts per tile: of 4, 8 and 16 the one that leaves the fewest lanes idle at the
+/* log2 of the node counts per tile of 64 points: of 4, 8 and 16 the one that leaves the fewest lanes idle at the
  * end of the axis, 8 x 8 when they tie (a square tile has the narrowest fan of rays) */
 uint32_t pick_tile_shift(uint32_t n_nodes)
 {
@@ -459,6 +464,47 @@ uint32_t pick_tile_shift(uint32_t n_nodes)
 		best = padded < padded_best ? shift : best;
 	}
 	return best;
+}
+
+/*
+ * Tilings a plan keeps, by falling size: 64, 16 (4 x 4), 8 (2 node counts x 4 sizes) and 4 points (2 x 2) to a
+ * tile.  The points of a smaller tile differ about fewer edges, so its wavefront is done sooner, at the price of
+ * more wavefronts, each of which costs 0.2 ns of dispatch and works out its edges' sides anew.
+ */
+constexpr int kTilings = 4;
+void tile_shifts(uint32_t n_nodes, uint32_t shift_n[kTilings], uint32_t shift_s[kTilings])
+{
+	shift_n[0] = pick_tile_shift(n_nodes);
+	shift_s[0] = 6 - shift_n[0];
+	shift_n[1] = shift_s[1] = 2;
+	shift_n[2] = 1, shift_s[2] = 2;
+	shift_n[3] = shift_s[3] = 1;
+}
+
+/*
+ * The smallest tiles that make at most kMostTiles, which the chip holds at once.  Times in us with tiles of 64 / 16 /
+ * 8 / 4 points and, in brackets, the tiles these make (3 collectives, 4 values of ranks per node):
+ *   35 sizes, 11 node counts, 4 platforms      14.2 / 10.2 / 8.4 / 7.4  [ 480, 1296, 2592, 5184]
+ *   70 sizes, 11 node counts, 2 platforms      14.4 /  8.2 / 7.0 / 6.2  [ 432, 1296, 2592, 5040]
+ *   140 sizes, 27 node counts, 1 platform       8.1 /  6.2 / 5.7 / 5.9  [ 840, 2940, 5880, 11760]
+ *   35 sizes, 38 node counts, 4 platforms      11.8 /  8.7 / 9.4 / 9.8  [1200, 4320, 8208, 16416]
+ *   140 sizes, 11 node counts, 4 platforms     10.6 /  8.4 / 7.8 / 9.7  [1728, 5040, 10080, 20160]
+ *   160 sizes, 27 node counts, 3 platforms      5.3 /  6.5 / 7.1 / 13   [2880, 10080, 20160, 40320]
+ *   140 sizes, 38 node counts, 4 platforms      9.0 / 10.9 / 12.7 / 23  [4320, 16800, 31920, 63840]
+ */
+constexpr uint64_t kMostTiles = 6000;
+uint64_t tiling_tiles(const tiling_t &t)
+{
+	return (uint64_t)t.tiles_n * t.tiles_s;
+}
+
+const tiling_t &pick_tiling(const tiling_t tilings[kTilings], uint64_t n_runs)
+{
+	int i = kTilings - 1;
+	while (i > 0 && n_runs * tiling_tiles(tilings[i]) > kMostTiles) {
+		i--;
+	}
+	return tilings[i];
 }
 
 /* smallest and largest of v[k * stride + at], k in [from, to) */
@@ -596,9 +642,10 @@ int device_region_tables(region_tables_t *out)
 struct ofi_amd_tuner_plan {
 	grid_dims_t g;
 	region_tables_t t;
+	tiling_t tilings[kTilings];
 	uint64_t points;
 	uint64_t cells;
-	void *d_axes; /* owned: what g's pointers point into */
+	void *d_axes; /* owned: what g's and the tilings' pointers point into */
 	/* per-call staging (device): the variants, and the runs of the platform list */
 	ofi_amd_tuner_variant_t *d_variants;
 	region_run_t *d_runs;
@@ -684,25 +731,31 @@ int ofi_amd_tuner_plan_create(const int32_t *colls, uint32_t n_colls, const uint
 		log2_sizes[i] = log2_coord((double)sizes[i]);
 	}
 
-	/* tiles of the region grid and the span of coordinates of each */
-	const uint32_t tile_shift = pick_tile_shift(n_nodes);
-	const uint32_t per_col = 1u << tile_shift, per_row = 64u >> tile_shift;
-	const uint32_t tiles_n = (n_nodes + per_col - 1) / per_col, tiles_s = (n_sizes + per_row - 1) / per_row;
-	std::vector<double2> size_span(tiles_s), rank_span((size_t)tiles_n * n_ppn);
-	for (uint32_t k = 0; k < tiles_s; k++) {
-		size_span[k] = span_of(log2_sizes.data(), k * per_row, std::min(n_sizes, (k + 1) * per_row), 1, 0);
-	}
-	for (uint32_t k = 0; k < tiles_n; k++) {
-		for (uint32_t j = 0; j < n_ppn; j++) {
-			rank_span[(size_t)k * n_ppn + j] =
-				span_of(log2_ranks.data(), k * per_col, std::min(n_nodes, (k + 1) * per_col), n_ppn, j);
-		}
-	}
-
 	/* one allocation and one copy for all of it */
 	grid_dims_t &g = plan->g;
 	std::vector<uint8_t> axes;
-	const size_t at_spans = append(axes, size_span), at_rank_spans = append(axes, rank_span);
+	/* the tilings of the region grid and the span of coordinates of each tile */
+	size_t at_spans[kTilings], at_rank_spans[kTilings];
+	uint32_t shift_n[kTilings], shift_s[kTilings];
+	tile_shifts(n_nodes, shift_n, shift_s);
+	for (int i = 0; i < kTilings; i++) {
+		const uint32_t per_col = 1u << shift_n[i], per_row = 1u << shift_s[i];
+		tiling_t &t = plan->tilings[i];
+		t = { shift_n[i], shift_s[i], (n_nodes + per_col - 1) >> shift_n[i], (n_sizes + per_row - 1) >> shift_s[i],
+		      nullptr, nullptr };
+		std::vector<double2> size_span(t.tiles_s), rank_span((size_t)t.tiles_n * n_ppn);
+		for (uint32_t k = 0; k < t.tiles_s; k++) {
+			size_span[k] = span_of(log2_sizes.data(), k * per_row, std::min(n_sizes, (k + 1) * per_row), 1, 0);
+		}
+		for (uint32_t k = 0; k < t.tiles_n; k++) {
+			for (uint32_t j = 0; j < n_ppn; j++) {
+				rank_span[(size_t)k * n_ppn + j] =
+					span_of(log2_ranks.data(), k * per_col, std::min(n_nodes, (k + 1) * per_col), n_ppn, j);
+			}
+		}
+		at_spans[i] = append(axes, size_span);
+		at_rank_spans[i] = append(axes, rank_span);
+	}
 	const size_t at_sizes = append(axes, std::vector<uint64_t>(sizes, sizes + n_sizes));
 	const size_t at_nodes = append(axes, std::vector<uint64_t>(nodes, nodes + n_nodes));
 	const size_t at_log2_nodes = append(axes, log2_nodes), at_log2_sizes = append(axes, log2_sizes);
@@ -738,11 +791,10 @@ int ofi_amd_tuner_plan_create(const int32_t *colls, uint32_t n_colls, const uint
 	g.log2_nodes = reinterpret_cast<const double *>(d_axes + at_log2_nodes);
 	g.log2_sizes = reinterpret_cast<const double *>(d_axes + at_log2_sizes);
 	g.log2_ranks = reinterpret_cast<const double *>(d_axes + at_log2_ranks);
-	g.tile_shift = tile_shift;
-	g.tiles_n = tiles_n;
-	g.tiles_s = tiles_s;
-	g.size_span = reinterpret_cast<const double2 *>(d_axes + at_spans);
-	g.rank_span = reinterpret_cast<const double2 *>(d_axes + at_rank_spans);
+	for (int i = 0; i < kTilings; i++) {
+		plan->tilings[i].size_span = reinterpret_cast<const double2 *>(d_axes + at_spans[i]);
+		plan->tilings[i].rank_span = reinterpret_cast<const double2 *>(d_axes + at_rank_spans[i]);
+	}
 	plan->points = (uint64_t)n_colls * n_sizes * n_nodes * n_ppn;
 	plan->cells = plan->points * n_algos * NUM_PROTOS;
 	*out = plan;
@@ -836,9 +888,9 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 		return -EINVAL;
 	}
 	const uint32_t points = (uint32_t)plan->points;
-	const uint64_t tiles = (uint64_t)plan->g.tiles_n * plan->g.tiles_s;
-	const uint64_t groups = (tiles + kXcds - 1) / kXcds;
 	const uint64_t n_runs = (uint64_t)n_platforms * plan->g.n_colls * plan->g.n_ppn;
+	const tiling_t &tiling = pick_tiling(plan->tilings, n_runs);
+	const uint64_t groups = (tiling_tiles(tiling) + kXcds - 1) / kXcds;
 	const uint64_t blocks = groups * n_runs * kXcds;
 	if (blocks == 0 || blocks > 0x7fffffffull) {
 		return -EINVAL;
@@ -891,7 +943,7 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 	for (uint64_t at = 0; at < n_runs; at += kMostRuns) {
 		const uint32_t here = (uint32_t)(n_runs - at < kMostRuns ? n_runs - at : kMostRuns);
 		hipLaunchKernelGGL(region_choice_kernel, dim3((uint32_t)(groups * kXcds), here), dim3(kRegionBlock), 0, s, plan->g,
-				   plan->t.poly, plan->t.bbox, plan->t.edges, plan->t.far_point, plan->d_runs + at, points,
+				   tiling, plan->t.poly, plan->t.bbox, plan->t.edges, plan->t.far_point, plan->d_runs + at, points,
 				   d_choice);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());

@@ -233,6 +233,27 @@ def test_region_tiles_on_edges_and_unsorted_axes(lib, oracle, gpu, n_nodes):
         lib.ofi_amd_tuner_plan_destroy(plan)
 
 
+@pytest.mark.parametrize("repeats,n_sizes,n_nodes", [(1, 19, 17), (3, 19, 17), (5, 19, 17), (10, 19, 17), (1, 1, 1), (1, 18, 16),
+                                                     (11, 16, 15), (30, 9, 3)])
+def test_region_tiles_of_every_size(lib, oracle, gpu, repeats, n_sizes, n_nodes):
+    """The more entries a platform list has, the larger the tiles: 4, 8, 16 and 64 points for 1, 3, 5 and 10 times
+    the four platforms on 19 x 17 points, which leave every kind of tile a remainder on both axes.  Points
+    on polygon edges and vertices, shuffled axes."""
+    rng = np.random.default_rng(repeats + n_sizes)
+    nodes = np.array([4, 8, 16, 32, 64, 128, 256, 512, 3, 5, 12, 24, 48, 96, 192, 2, 1][:n_nodes], dtype=np.uint64)
+    sizes = np.array([1 << 30, 1, 1 << 15, 1 << 17, 196608, 786432, 3145728, 4 << 20, 4718592, 8 << 20, 13107200, 29884416,
+                      31457280, 32 << 20, 33554433, 129499136, 107374182399, 107374182400, 107374182401][:n_sizes], dtype=np.uint64)
+    colls, ppn = np.array([4, 2, 3], dtype=np.int32), np.array([8, 1, 2], dtype=np.uint32)
+    nodes, sizes = rng.permutation(nodes), rng.permutation(sizes)
+    plan = make_plan(lib, colls, sizes, nodes, ppn, np.array([1], dtype=np.int32))
+    want = oracle_region_grid(oracle, [0, 1, 2, 3], colls, sizes, nodes, ppn)
+    for times in (repeats, 1):
+        got = run_region(lib, plan, [0, 1, 2, 3] * times, (4 * times, 3, n_sizes, n_nodes, 3))
+        mism = np.argwhere((got != np.concatenate([want] * times)).any(axis=-1))
+        assert len(mism) == 0, (times, mism[:10])
+    lib.ofi_amd_tuner_plan_destroy(plan)
+
+
 def test_region_grid_on_changing_platform_lists(lib, oracle, gpu):
     """One plan, platform lists that grow, shrink and change in place: the launch order the plan keeps
     for a list (which entry, chunk and ranks-per-node value each workgroup takes) is rebuilt whenever
