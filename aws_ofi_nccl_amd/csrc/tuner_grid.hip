@@ -154,10 +154,13 @@ __global__ __launch_bounds__(256) void model_grid_kernel(grid_dims_t g,
 }
 
 constexpr int kMaxSetEdges = 64; /* of one (platform, shape, collective) set: one per lane */
-constexpr uint32_t kRegionBlock = 64; /* threads per workgroup of the region kernel: one wavefront */
+/* Wavefronts per workgroup of the region kernel: two in launches of more than kMostTiles tiles, whose workgroups
+ * take as long to hand out as to work off (560 sizes x 38 node counts of four platforms 11.2 -> 10.8 us, 280 x 38 9.6
+ * -> 9.0; four wavefronts 10.9), one in smaller ones, where two gain nothing. */
+constexpr uint32_t kMostRegionWaves = 2;
 constexpr uint64_t kMostRuns = 65535; /* of one launch: gridDim.y */
 constexpr uint32_t kXcds = 8;         /* workgroup w of a launch runs on XCD w mod 8, each with its own L2 */
-static_assert(kRegionBlock >= (uint32_t)kMaxSetEdges, "one lane per edge of a set");
+static_assert(kMaxSetEdges <= 64, "one lane per edge of a set");
 
 /* One (platform entry, collective, ranks per node) of a region grid: where its points go and which
  * polygons answer for it (region_set, looked up by the host: ranks = nodes * ppn, so the shape is a
@@ -247,7 +250,7 @@ __device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64
 }
 
 /*
- * One thread per point.  A workgroup (one wavefront) works on a tile of neighbouring sizes and node
+ * One thread per point.  A wavefront works on a tile of neighbouring sizes and node
  * counts of one (collective, ranks per node) pair, because the polygon set depends on that pair
  * alone.  The launch is bound by arithmetic (chains of fp64 operations), so a wavefront first
  * works out, one edge per lane, what its whole tile has in common about each edge of the set
@@ -267,7 +270,7 @@ __device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64
  * XCD's L2 and leave it as one line (measured: 4.7 MB written for 4.7 MB of records; with the
  * workgroups of a tile on different XCDs every L2 wrote its quarter of each line, 18.9 MB).
  */
-__global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t g, tiling_t t, const int32_t *__restrict__ polys,
+__global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(grid_dims_t g, tiling_t t, const int32_t *__restrict__ polys,
 							    const double *__restrict__ bboxes,
 							    const edge_t *__restrict__ edges, pt_t far_point,
 							    const region_run_t *__restrict__ runs,
@@ -275,14 +278,15 @@ __global__ __launch_bounds__(kRegionBlock) void region_choice_kernel(grid_dims_t
 {
 	/* blockIdx.y names a run, blockIdx.x = 8 * group + x the tiles 8 * group .. 8 * group + 7 of it, of
 	 * which XCD x takes one (workgroups are dealt to the XCDs in launch order, and gridDim.x is a
-	 * multiple of 8).  The host lists the runs by falling cost (edges of the pair's set): the long
+	 * multiple of 8); a second wavefront takes its tile from the other half of the groups.  The host lists the runs by falling cost (edges of the pair's set): the long
 	 * workgroups start first and the short ones fill the end of the launch. */
-	const uint32_t lane = threadIdx.x;
+	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const region_run_t run = runs[blockIdx.y];
 	/* which of a group's eight tiles an XCD takes rotates with the platform entry: the tiles
 	 * differ in cost (size range), and an XCD that kept the same ones for every
 	 * entry would keep the same share of the long ones */
-	const uint32_t tile = (blockIdx.x & ~(kXcds - 1u)) + (blockIdx.x + run.entry) % kXcds;
+	const uint32_t group = (blockIdx.x + wave * gridDim.x) / kXcds;
+	const uint32_t tile = group * kXcds + (blockIdx.x + run.entry) % kXcds;
 	if (tile >= t.tiles_n * t.tiles_s) {
 		return; /* padding of the last group */
 	}
@@ -940,9 +944,11 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 		plan->h_platforms.clear();
 		return -ENOMEM;
 	}
+	const uint32_t waves = n_runs * tiling_tiles(tiling) > kMostTiles ? kMostRegionWaves : 1;
+	const uint32_t grid_x = (uint32_t)((groups + waves - 1) / waves * kXcds);
 	for (uint64_t at = 0; at < n_runs; at += kMostRuns) {
 		const uint32_t here = (uint32_t)(n_runs - at < kMostRuns ? n_runs - at : kMostRuns);
-		hipLaunchKernelGGL(region_choice_kernel, dim3((uint32_t)(groups * kXcds), here), dim3(kRegionBlock), 0, s, plan->g,
+		hipLaunchKernelGGL(region_choice_kernel, dim3(grid_x, here), dim3(64 * waves), 0, s, plan->g,
 				   tiling, plan->t.poly, plan->t.bbox, plan->t.edges, plan->t.far_point, plan->d_runs + at, points,
 				   d_choice);
 	}

@@ -234,15 +234,18 @@ def test_region_tiles_on_edges_and_unsorted_axes(lib, oracle, gpu, n_nodes):
 
 
 @pytest.mark.parametrize("repeats,n_sizes,n_nodes", [(1, 19, 17), (3, 19, 17), (5, 19, 17), (10, 19, 17), (1, 1, 1), (1, 18, 16),
-                                                     (11, 16, 15), (30, 9, 3)])
+                                                     (11, 16, 15), (30, 9, 3), (90, 19, 3), (20, 19, 17),
+                                                     (12, 60, 17)])
 def test_region_tiles_of_every_size(lib, oracle, gpu, repeats, n_sizes, n_nodes):
     """The more entries a platform list has, the larger the tiles: 4, 8, 16 and 64 points for 1, 3, 5 and 10 times
-    the four platforms on 19 x 17 points, which leave every kind of tile a remainder on both axes.  Points
-    on polygon edges and vertices, shuffled axes."""
+    the four platforms on 19 x 17 points, which leave every kind of tile a remainder on both axes; then two
+    wavefronts a workgroup, on one, two and three groups of tiles.  Points on polygon edges and vertices, shuffled
+    axes."""
     rng = np.random.default_rng(repeats + n_sizes)
     nodes = np.array([4, 8, 16, 32, 64, 128, 256, 512, 3, 5, 12, 24, 48, 96, 192, 2, 1][:n_nodes], dtype=np.uint64)
-    sizes = np.array([1 << 30, 1, 1 << 15, 1 << 17, 196608, 786432, 3145728, 4 << 20, 4718592, 8 << 20, 13107200, 29884416,
-                      31457280, 32 << 20, 33554433, 129499136, 107374182399, 107374182400, 107374182401][:n_sizes], dtype=np.uint64)
+    sizes = np.resize(np.array([1 << 30, 1, 1 << 15, 1 << 17, 196608, 786432, 3145728, 4 << 20, 4718592, 8 << 20, 13107200,
+                                29884416, 31457280, 32 << 20, 33554433, 129499136, 107374182399, 107374182400,
+                                107374182401], dtype=np.uint64), n_sizes)
     colls, ppn = np.array([4, 2, 3], dtype=np.int32), np.array([8, 1, 2], dtype=np.uint32)
     nodes, sizes = rng.permutation(nodes), rng.permutation(sizes)
     plan = make_plan(lib, colls, sizes, nodes, ppn, np.array([1], dtype=np.int32))
