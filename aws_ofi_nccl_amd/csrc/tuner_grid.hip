@@ -258,17 +258,18 @@ __device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64
  * fan of rays from the tile to the far point, and those the tile touches -- read out of the
  * lanes that hold them.  A tile has one such edge at the median and 20 at the most; every edge for every
  * point, with quotients, took 40-42 us for 1.02 M points of four platforms (560 sizes, 38 node counts),
- * this takes 12.0: 5 us of it are the dispatch of 16,896 wavefronts, the rest the time of the
+ * this takes 10.8, a part of it the handing out of 16,896 wavefronts (kMostRegionWaves), the rest the time of the
  * tiles with the most edges, which is why their turns count instructions (two edges a turn, for
- * shorter chains of dependent operations, was slower: 13.3).  A grid of few points is the time of such a
+ * shorter chains of dependent operations, was slower: 13.3 against then 12.0).  A grid of few points is the time of such a
  * tile alone, and takes smaller ones (pick_tiling).
  *
  * In the output the ranks-per-node index runs fastest, so a wavefront's records lie 4 x
  * n_ppn bytes apart and the records between them belong to the same tile's other
  * ranks-per-node values, i.e. to other workgroups.  Those workgroups are given numbers that
  * are equal mod 8: they run on the same XCD, their partial writes to a cache line meet in that
- * XCD's L2 and leave it as one line (measured: 4.7 MB written for 4.7 MB of records; with the
- * workgroups of a tile on different XCDs every L2 wrote its quarter of each line, 18.9 MB).
+ * XCD's L2 and leave it as one line (64 grids of 140 sizes x 11 node counts: 7.1 MB written for 4.7 MB of
+ * records, the rest lines that tiles side by side share; with the workgroups of a tile on different XCDs every
+ * L2 wrote its quarter of each line, 18.9 MB).
  */
 __global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(grid_dims_t g, tiling_t t, const int32_t *__restrict__ polys,
 							    const double *__restrict__ bboxes,
