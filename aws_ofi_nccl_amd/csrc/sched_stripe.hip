@@ -12,7 +12,8 @@
  *
  * Three forms, by the size of the batch:
  *   up to kDirectBatch messages, one launch: every workgroup adds up the messages before
- *   its tile by itself, from their sizes (at most 48 KiB out of the L2);
+ *   its tile by itself, from their sizes (at most 48 KiB out of the L2); beyond one tile not in a
+ *   batch that is being captured into a graph (launch_batch says why);
  *   up to kSmallBatch, two launches: stripe_count_kernel leaves each tile's totals of
  *   (small count, stripe count), reduced mod R (only the residues matter), and
  *   stripe_emit_kernel, whose workgroups add up the totals of the tiles before them (at most
@@ -21,10 +22,11 @@
  *   beyond, the same two launches with larger tiles, and a level of totals above the tiles', for
  *   every kPart messages.
  * The count launch snapshots the two counters of *state as the batch's seed, the workgroup of the
- * last tile writes the new ones back.
+ * last tile writes the new ones back; in the one-launch form the workgroup that is done last does.
  *
  * HBM traffic per message: 8 B read twice (once in the one-launch form) + 4 B + 96 B written.
  */
+#include <atomic>
 #include <mutex>
 #include <unordered_map>
 
@@ -267,8 +269,8 @@ template <stripe_form FORM, uint32_t THREADS>
 __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	const uint64_t *__restrict__ sizes, uint32_t n, ofi_amd_sched_state_t *__restrict__ state,
 	uint64_t align, const uint32_t *__restrict__ totals, const uint32_t *__restrict__ block_totals,
-	uint32_t *__restrict__ seed0, uint32_t num_tiles, uint32_t *__restrict__ num_xfers, u32x4 *__restrict__ xfers,
-	uint32_t *__restrict__ err)
+	uint32_t *__restrict__ seed0, uint32_t *__restrict__ arrival_ahead, uint32_t num_tiles,
+	uint32_t *__restrict__ num_xfers, u32x4 *__restrict__ xfers, uint32_t *__restrict__ err)
 {
 	constexpr uint32_t kWaves = THREADS / 64;
 	/* THREADS rows of 96 bytes = 6 x 16 B each */
@@ -413,8 +415,12 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	const uint32_t after_big = mod_rails(carry_big + (tot & 0xffffu), p);
 	if (FORM == DIRECT && num_tiles > 1) {
 		/* Every workgroup has read the counters, so they may only be moved on when all are done:
-		 * each adds itself to the arrival word (low half), the last tile's with the carries behind
-		 * it (high half), and whoever is last puts them in place and leaves the word at zero. */
+		 * each adds itself to the batch's arrival word (low half), the last tile's with the carries
+		 * behind it (high half), and whoever is last puts them in place and leaves the word at zero.
+		 * A later batch's word is cleared on the way, whatever is in it (kArrivalWords). */
+		if (tile == 0) {
+			__hip_atomic_store(arrival_ahead, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		}
 		const uint32_t mine = 1u + (tile == num_tiles - 1 ? (after_small << 16) | (after_big << 20) : 0u);
 		const uint32_t all = mine + __hip_atomic_fetch_add(seed0, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		if ((all & 0xffffu) == num_tiles) {
@@ -431,37 +437,62 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 }
 
 /* Scratch of the batches of one stream: launches on one stream are ordered, so they can share; launches on
- * different streams may overlap and must not.  Layout in 32-bit words: the arrival word of the one-launch
- * form, which is zero between batches, and the seed word of the others, on 128-byte lines of
- * their own; then the block totals; then the tile totals. */
-constexpr uint32_t kArrivalWord = 0, kSeedWord = 32, kBlockWords = 64;
+ * different streams may overlap and must not.  Layout in 32-bit words: the arrival words of the one-launch
+ * form; the seed word of the others, on a 128-byte line of its own; then the block totals; then the
+ * tile totals.
+ *
+ * A batch of the one-launch form takes the next arrival word round the ring, finds it at zero and leaves it at
+ * zero, and clears the word half a ring ahead.  So batches that overlap on one scratch, against the rule, do not
+ * count in each other's word, and a word that such a mistake (more than half a ring apart) or a launch
+ * that never ran to its end has left with a count is at zero again when its turn comes: the damage
+ * does not outlast the ring.  With one word for all batches a leftover count spoiled the counters of every
+ * later small batch. */
+constexpr uint32_t kArrivalWords = 1024;
+constexpr uint32_t kSeedWord = kArrivalWords, kBlockWords = kSeedWord + 32;
 constexpr uint32_t kTileWords = kBlockWords + kMaxBlocks;
 constexpr uint32_t kScratchWords = kTileWords + kMaxTiles;
+static_assert((kArrivalWords & (kArrivalWords - 1)) == 0 && kBlockWords % 32 == 0, "a ring; block totals on a line");
+struct scratch_t {
+	uint32_t *words = nullptr;
+	std::atomic<uint32_t> turn{ 0 }; /* of the next batch that counts arrivals */
+};
 std::mutex g_ws_lock;
-std::unordered_map<void *, uint32_t *> g_ws_by_stream;
+std::unordered_map<void *, scratch_t> g_ws_by_stream;
 
-__global__ __launch_bounds__(64) void stripe_scratch_kernel(uint32_t *__restrict__ words)
+constexpr uint32_t kClearThreads = 256;
+__global__ __launch_bounds__(kClearThreads) void stripe_scratch_kernel(uint32_t *__restrict__ words)
 {
-	words[threadIdx.x] = 0;
+	words[blockIdx.x * kClearThreads + threadIdx.x] = 0;
 }
 
-/* Scratch for stream s with its arrival word at zero before anything queued on s from here on.  A stream that is
+/* also where the runtime cannot say: the null stream while another one is captured */
+bool being_captured(hipStream_t s)
+{
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	if (hipStreamIsCapturing(s, &capture) != hipSuccess) {
+		(void)hipGetLastError();
+		return true;
+	}
+	return capture != hipStreamCaptureStatusNone;
+}
+
+/* Scratch for stream s with its arrival words at zero before anything queued on s from here on.  A stream that is
  * being captured would only record the clearing launch, and batches called before the first replay would count
  * from whatever the memory held: there it runs on a stream of its own and is waited for. */
 int new_scratch(hipStream_t s, uint32_t **out)
 {
 	uint32_t *words = nullptr;
 	OFI_AMD_HIP_TRY(hipMalloc((void **)&words, sizeof(uint32_t) * kScratchWords));
-	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-	hipError_t e = hipStreamIsCapturing(s, &capture);
-	if (e == hipSuccess && capture == hipStreamCaptureStatusNone) {
-		hipLaunchKernelGGL(stripe_scratch_kernel, dim3(1), dim3(64), 0, s, words);
+	hipError_t e = hipSuccess;
+	if (!being_captured(s)) {
+		hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kArrivalWords / kClearThreads), dim3(kClearThreads), 0, s, words);
 		e = hipGetLastError();
 	} else {
 		hipStream_t own = nullptr;
 		e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
 		if (e == hipSuccess) {
-			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(1), dim3(64), 0, own, words);
+			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kArrivalWords / kClearThreads), dim3(kClearThreads), 0, own,
+					   words);
 			e = hipGetLastError();
 			const hipError_t waited = hipStreamSynchronize(own);
 			e = e == hipSuccess ? waited : e;
@@ -487,11 +518,11 @@ static __device__ __align__(256) __attribute__((used)) uint32_t scratch[kScratch
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_lock;
-uint32_t *g_scratch_ptr[kMaxDevices]; /* device address of `scratch` on each GPU, once looked up */
+scratch_t g_scratch[kMaxDevices]; /* words: device address of `scratch` on each GPU, once looked up */
 
-/* Device address of the current GPU's copy of `scratch` as ofi_amd_gpu_init() has recorded it;
- * no runtime call that could allocate.  -ENXIO when the address has not been looked up. */
-int cached_scratch_of_current_device(uint32_t **out)
+/* The current GPU's copy of `scratch` as ofi_amd_gpu_init() has recorded it; no runtime call that
+ * could allocate.  -ENXIO when its address has not been looked up. */
+int cached_scratch_of_current_device(scratch_t **out)
 {
 	int dev = -1;
 	OFI_AMD_HIP_TRY(hipGetDevice(&dev));
@@ -499,16 +530,16 @@ int cached_scratch_of_current_device(uint32_t **out)
 		return -ENODEV;
 	}
 	std::lock_guard<std::mutex> g(g_scratch_lock);
-	if (!g_scratch_ptr[dev]) {
+	if (!g_scratch[dev].words) {
 		return -ENXIO;
 	}
-	*out = g_scratch_ptr[dev];
+	*out = &g_scratch[dev];
 	return 0;
 }
 
 /* Device address of the current GPU's copy of `scratch` (each GPU has its own), looked up on
  * first use: set-up only. */
-int scratch_of_current_device(uint32_t **out)
+int look_up_scratch_of_current_device()
 {
 	int dev = -1;
 	OFI_AMD_HIP_TRY(hipGetDevice(&dev));
@@ -516,15 +547,14 @@ int scratch_of_current_device(uint32_t **out)
 		return -ENODEV;
 	}
 	std::lock_guard<std::mutex> g(g_scratch_lock);
-	if (!g_scratch_ptr[dev]) {
+	if (!g_scratch[dev].words) {
 		void *p = nullptr;
 		OFI_AMD_HIP_TRY(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
 		if (!p) {
 			return -EIO;
 		}
-		g_scratch_ptr[dev] = static_cast<uint32_t *>(p);
+		g_scratch[dev].words = static_cast<uint32_t *>(p);
 	}
-	*out = g_scratch_ptr[dev];
 	return 0;
 }
 
@@ -533,14 +563,20 @@ uint32_t tiles_of(uint64_t n, uint32_t tile)
 	return (uint32_t)((n + tile - 1) / tile);
 }
 
+/* A batch that is being captured goes the two-launch way from its second tile on, all of whose scratch is
+ * written before it is read: a replay would come back to the arrival word it was captured with, and its stream's
+ * other batches may meanwhile be anywhere round the ring. */
 void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_amd_sched_state_t *d_state, uint64_t align,
-		  uint32_t *words, uint32_t *d_num_xfers, u32x4 *d_xfers, uint32_t *err)
+		  scratch_t &scratch, uint32_t *d_num_xfers, u32x4 *d_xfers, uint32_t *err)
 {
+	uint32_t *words = scratch.words;
 	uint32_t *seed0 = words + kSeedWord, *blocks = words + kBlockWords, *totals = words + kTileWords;
-	if (total <= kDirectBatch) {
+	if (total <= kDirectTile || (total <= kDirectBatch && !being_captured(s))) {
 		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kDirectTile);
+		const uint32_t turn = tiles > 1 ? scratch.turn.fetch_add(1, std::memory_order_relaxed) : 0u;
 		hipLaunchKernelGGL((stripe_emit_kernel<DIRECT, kDirectTile>), dim3(tiles), dim3(kDirectTile), 0, s, d_sizes, n,
-				   d_state, align, nullptr, nullptr, words + kArrivalWord, tiles, d_num_xfers, d_xfers, err);
+				   d_state, align, nullptr, nullptr, words + turn % kArrivalWords,
+				   words + (turn + kArrivalWords / 2) % kArrivalWords, tiles, d_num_xfers, d_xfers, err);
 		return;
 	}
 	if (total <= kSmallBatch) {
@@ -548,7 +584,7 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 		hipLaunchKernelGGL(stripe_count_kernel, dim3(tiles), dim3(kCountThreads), 0, s, d_sizes, n, d_state, align, totals,
 				   seed0, err);
 		hipLaunchKernelGGL((stripe_emit_kernel<TILES, kTile>), dim3(tiles), dim3(kTile), 0, s, d_sizes, n, d_state, align,
-				   totals, nullptr, seed0, tiles, d_num_xfers, d_xfers, err);
+				   totals, nullptr, seed0, nullptr, tiles, d_num_xfers, d_xfers, err);
 		return;
 	}
 	for (uint64_t at = 0; at < total; at += kPart) {
@@ -556,7 +592,7 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 		hipLaunchKernelGGL(stripe_count_big_kernel, dim3(tiles_of(tiles, kBlockTiles)), dim3(64 * kBlockTiles), 0, s,
 				   d_sizes + at, n, d_state, align, totals, blocks, seed0, err);
 		hipLaunchKernelGGL((stripe_emit_kernel<BLOCKS, kBigTile>), dim3(tiles), dim3(kBigTile), 0, s, d_sizes + at, n,
-				   d_state, align, totals, blocks, seed0, tiles, d_num_xfers + at, d_xfers + 6 * at, err);
+				   d_state, align, totals, blocks, seed0, nullptr, tiles, d_num_xfers + at, d_xfers + 6 * at, err);
 	}
 }
 
@@ -571,12 +607,11 @@ int sched_noalloc_setup()
 	OFI_AMD_HIP_TRY(hipGetDevice(&before));
 	int rc = 0;
 	for (int dev = 0; dev < count && dev < kMaxDevices && rc == 0; dev++) {
-		uint32_t *p = nullptr;
 		if (hipSetDevice(dev) != hipSuccess) {
 			rc = -ENODEV;
 			break;
 		}
-		rc = scratch_of_current_device(&p);
+		rc = look_up_scratch_of_current_device();
 	}
 	(void)hipSetDevice(before);
 	return rc;
@@ -616,14 +651,14 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
 		/* held until the launches are queued: two threads submitting to one stream share its
 		 * scratch, and their count/emit pairs must not interleave */
 		std::lock_guard<std::mutex> g(g_ws_lock);
-		uint32_t *&words = g_ws_by_stream[stream];
-		if (!words) {
-			rc = new_scratch(s, &words);
+		scratch_t &scratch = g_ws_by_stream[stream];
+		if (!scratch.words) {
+			rc = new_scratch(s, &scratch.words);
 			if (rc != 0) {
 				return rc;
 			}
 		}
-		launch_batch(s, d_sizes, n, d_state, align, words, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
+		launch_batch(s, d_sizes, n, d_state, align, scratch, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
 	} catch (...) {
 		return -ENOMEM;
 	}
@@ -644,7 +679,7 @@ int ofi_amd_sched_stream_release(void *stream)
 		if (it == g_ws_by_stream.end()) {
 			return 0; /* nothing was ever allocated for it */
 		}
-		words = it->second;
+		words = it->second.words;
 		g_ws_by_stream.erase(it);
 	}
 	/* launches queued on the stream may still read the scratch */
@@ -677,12 +712,12 @@ int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *
 	if (!err) {
 		return -ENXIO; /* ofi_amd_gpu_init() allocates it; this call must not */
 	}
-	uint32_t *base = nullptr;
-	rc = cached_scratch_of_current_device(&base); /* -ENXIO: ofi_amd_gpu_init() looks the address up; this call must not */
+	scratch_t *scratch = nullptr;
+	rc = cached_scratch_of_current_device(&scratch); /* -ENXIO: ofi_amd_gpu_init() looks the address up; this call must not */
 	if (rc != 0) {
 		return rc;
 	}
-	launch_batch(as_stream(stream), d_sizes, n, d_state, align, base, d_num_xfers,
+	launch_batch(as_stream(stream), d_sizes, n, d_state, align, *scratch, d_num_xfers,
 		     reinterpret_cast<u32x4 *>(d_xfers), err);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;

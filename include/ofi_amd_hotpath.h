@@ -123,7 +123,9 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
 			void *stream);
 /* ofi_amd_sched_batch keeps some 80 KiB of device scratch per stream it has been called with
  * (the reference's scheduler keeps a freelist per instance, src/nccl_ofi_scheduler.cpp:135-190).
- * A caller that destroys a stream hands the scratch back first: waits for the stream, frees. */
+ * A caller that destroys a stream hands the scratch back first: waits for the stream, frees.
+ * A batch captured into a graph keeps the scratch of the stream it was captured on: replays are
+ * ordered with each other and with that stream's batches of more than 6144 messages. */
 int ofi_amd_sched_stream_release(void *stream);
 
 /*
@@ -135,9 +137,10 @@ int ofi_amd_sched_stream_release(void *stream);
  * allocates and frees nothing.  n <= 2^26 messages per call, -E2BIG beyond.  Call
  * ofi_amd_gpu_init() once beforehand (it allocates the asynchronous error word and looks up
  * the array's address on every GPU); -ENXIO otherwise.  All calls on one GPU share that GPU's
- * array: calls that overlap there -- different streams, or two threads -- race; order them.
- * One word of the array is zero between calls, as it is when the code is loaded; every other word a call
- * writes before it reads it.
+ * array: calls that overlap there -- different streams, or two threads -- race; order them.  What
+ * an overlap spoils is the batches that took part in it, not later ones.  A call writes every word of the
+ * array before it reads it, but for 1024 words that small batches count in: those are zero between
+ * calls, as they are when the code is loaded, and calls clear them again by turns.
  */
 int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
 				uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,

@@ -1,0 +1,208 @@
+/*
+ * The launches of libofi_amd_hotpath.so with a stand-in for the HIP runtime: this program defines the runtime
+ * functions the library calls, so the library's host code runs without a GPU and every launch is seen with its
+ * grid and its arguments.  argv[1] names the part to run.
+ */
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include <cxxabi.h>
+#include <hip/hip_runtime_api.h>
+
+#include "ofi_amd_hotpath.h"
+
+#define CHECK(cond)                                                                  \
+	do {                                                                         \
+		if (!(cond)) {                                                       \
+			std::printf("%s:%d: %s\n", __FILE__, __LINE__, #cond);       \
+			std::exit(1);                                                \
+		}                                                                    \
+	} while (0)
+
+namespace {
+
+struct launch_t {
+	std::string kernel; /* demangled, with its template arguments */
+	dim3 grid, block;
+	void **args;
+	hipStream_t stream;
+	template <typename T> T arg(int i) const { return *static_cast<T *>(args[i]); }
+};
+
+std::map<const void *, std::string> &kernels()
+{
+	static std::map<const void *, std::string> m;
+	return m;
+}
+
+std::function<void(const launch_t &)> on_launch = [](const launch_t &) {};
+hipError_t capture_answer = hipSuccess;
+hipStreamCaptureStatus capture_status = hipStreamCaptureStatusNone;
+struct config_t {
+	dim3 grid, block;
+	size_t shared;
+	hipStream_t stream;
+} pushed;
+
+} // namespace
+
+extern "C" {
+
+/* nothing but malloc behind them */
+hipError_t hipMalloc(void **p, size_t n) { return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDriverGetVersion(int *v) { *v = 1; return hipSuccess; }
+hipError_t hipRuntimeGetVersion(int *v) { *v = 1; return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = reinterpret_cast<hipStream_t>(0x70); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipGetSymbolAddress(void **p, const void *)
+{
+	static uint32_t array[1u << 18];
+	*p = array;
+	return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status)
+{
+	*status = capture_status;
+	return capture_answer;
+}
+
+void **__hipRegisterFatBinary(const void *) { static void *module; return &module; }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *, void *, int *)
+{
+	int status = 0;
+	char *plain = abi::__cxa_demangle(name, nullptr, nullptr, &status);
+	kernels()[host] = plain ? plain : name;
+	std::free(plain);
+}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shared, hipStream_t stream)
+{
+	pushed = { grid, block, shared, stream };
+	return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hipStream_t *stream)
+{
+	*grid = pushed.grid, *block = pushed.block, *shared = pushed.shared, *stream = pushed.stream;
+	return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t, hipStream_t stream)
+{
+	on_launch({ kernels()[f], grid, block, args, stream });
+	return hipSuccess;
+}
+
+} /* extern "C" */
+
+namespace {
+
+/*
+ * The arrival words of small striping batches.  The stand-in counts as the kernel does: every tile adds one to
+ * the batch's word, whoever makes it the number of tiles sets it to zero and moves the counters on, and
+ * the word named beside it is cleared.  A batch that finds a count in its word moves the
+ * counters on too early, or not at all.
+ */
+struct arrivals_t {
+	std::vector<uint32_t *> words; /* of the batches so far */
+	int spoiled = 0, two_launch = 0;
+	void operator()(const launch_t &l)
+	{
+		two_launch += l.kernel.find("stripe_count_kernel") != std::string::npos;
+		if (l.kernel.find("stripe_emit_kernel<((anonymous namespace)::stripe_form)0") == std::string::npos) {
+			if (l.kernel.find("stripe_scratch_kernel") != std::string::npos) {
+				std::memset(l.arg<uint32_t *>(0), 0, 4ull * l.grid.x * l.block.x);
+			}
+			return;
+		}
+		uint32_t *word = l.arg<uint32_t *>(6), *ahead = l.arg<uint32_t *>(7);
+		const uint32_t tiles = l.grid.x;
+		if (tiles == 1) {
+			return;
+		}
+		spoiled += *word != 0;
+		*ahead = 0;
+		for (uint32_t t = 0; t < tiles; t++) {
+			*word = *word + 1 == tiles ? 0 : *word + 1;
+		}
+		words.push_back(word);
+	}
+};
+
+int striping()
+{
+	using batch_t = int (*)(ofi_amd_sched_state_t *, const uint64_t *, uint64_t, uint64_t, uint32_t *, ofi_amd_xfer_info_t *,
+				void *);
+	ofi_amd_sched_state_t state = {};
+	uint64_t sizes[1] = {};
+	uint32_t num[1];
+	ofi_amd_xfer_info_t xfers[4];
+	void *stream = reinterpret_cast<void *>(0x40);
+	for (const batch_t batch : { &ofi_amd_sched_batch, &ofi_amd_sched_batch_noalloc }) {
+		arrivals_t seen;
+		on_launch = std::ref(seen);
+		auto small = [&](uint64_t n) { CHECK(batch(&state, sizes, n, 128, num, xfers, stream) == 0); };
+		/* no two of 512 batches in a row count in one word, and each finds its own at zero */
+		for (int i = 0; i < 5000; i++) {
+			small(257 + (i * 97) % 5888);
+		}
+		CHECK(seen.words.size() == 5000 && seen.spoiled == 0 && seen.two_launch == 0);
+		for (size_t i = 0; i + 512 <= seen.words.size(); i++) {
+			CHECK(std::set<uint32_t *>(&seen.words[i], &seen.words[i] + 512).size() == 512);
+		}
+		/* a count left in every word, by whatever went wrong: the batches after it soon find zero again */
+		for (uint32_t *w : std::set<uint32_t *>(seen.words.begin(), seen.words.end())) {
+			*w = 4;
+		}
+		for (int i = 0; i < 512; i++) {
+			small(1000);
+		}
+		seen.spoiled = 0;
+		for (int i = 0; i < 5000; i++) {
+			small(1000);
+		}
+		CHECK(seen.spoiled == 0);
+		/* a captured batch comes back to the scratch it was captured with: it counts in no word */
+		const size_t before = seen.words.size();
+		capture_status = hipStreamCaptureStatusActive;
+		small(257);
+		small(6144);
+		capture_status = hipStreamCaptureStatusNone;
+		capture_answer = hipErrorStreamCaptureImplicit;
+		small(1000);
+		capture_answer = hipSuccess;
+		CHECK(seen.words.size() == before && seen.two_launch == 3);
+		small(256); /* one tile */
+		CHECK(seen.words.size() == before && seen.two_launch == 3);
+	}
+	CHECK(ofi_amd_sched_stream_release(stream) == 0);
+	return 0;
+}
+
+} // namespace
+
+int main(int argc, char **argv)
+{
+	const std::map<std::string, int (*)()> parts = { { "striping", striping } };
+	CHECK(argc == 2 && parts.count(argv[1]) && ofi_amd_gpu_init() == 0);
+	const int rc = parts.at(argv[1])();
+	std::printf("%s: ok\n", argv[1]);
+	return rc;
+}

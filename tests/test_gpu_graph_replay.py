@@ -187,3 +187,48 @@ def test_batch_first_called_while_its_stream_is_captured(lib, oracle, gpu):
         seeds = (ost.rr_small_counter, ost.rr_counter)
         assert (now.rr_small_counter, now.rr_counter) == seeds, step
     assert lib.ofi_amd_sched_stream_release(sp) == 0
+
+
+def test_small_batch_replayed_on_another_stream_beside_its_own_streams_batches(lib, oracle, gpu):
+    """A small batch captured on one stream and replayed on another while the first stream runs small batches of
+    its own (one launch each, with the same scratch): both schedulers' results and counters match the
+    oracle at the end of every round, and so does the next round."""
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    sp = ctypes.c_void_p(s.cuda_stream)
+    cases = []
+    for n, seeds in ((3001, (2, 1)), (5000, (0, 3))):
+        sizes = synthetic.stripe_sizes(n, n)
+        d_state = _gpu.to_dev(np.frombuffer(bytes(m.SchedState(*seeds, 64, 131072, 4, 0)), dtype=np.uint8).copy())
+        cases.append(dict(n=n, seeds=seeds, sizes=sizes, d_state=d_state, d_sizes=_gpu.to_dev(sizes),
+                          d_num=torch.zeros(n, dtype=torch.int32, device="cuda"),
+                          d_xf=torch.zeros(n * 12, dtype=torch.int64, device="cuda")))
+    torch.cuda.synchronize()
+
+    def call(c):
+        assert lib.ofi_amd_sched_batch(c["d_state"].data_ptr(), c["d_sizes"].data_ptr(), c["n"], 128, c["d_num"].data_ptr(),
+                                       c["d_xf"].data_ptr(), sp) == 0
+
+    captured, direct = cases
+    call(direct)                                    # the stream's scratch is there before the capture
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s, capture_error_mode="relaxed"):
+        call(captured)
+    times = {3001: 0, 5000: 1}
+    for _ in range(3):
+        for _ in range(20):
+            with torch.cuda.stream(t):
+                g.replay()
+            call(direct)
+        times = {n: k + 20 for n, k in times.items()}
+        torch.cuda.synchronize()
+        for c in cases:
+            ost = c["seeds"]
+            for _ in range(times[c["n"]]):
+                want_num, want_xf, st = _oracle.sched_batch(oracle, c["sizes"], 4, 131072, 64, ost)
+                ost = (st.rr_small_counter, st.rr_counter)
+            assert np.array_equal(_gpu.to_host(c["d_num"], np.uint32), want_num)
+            assert np.array_equal(_gpu.to_host(c["d_xf"], np.uint64).reshape(c["n"], 4, 3), want_xf)
+            now = m.SchedState.from_buffer_copy(c["d_state"].cpu().numpy().tobytes())
+            assert (now.rr_small_counter, now.rr_counter) == ost
+    assert lib.ofi_amd_sched_stream_release(sp) == 0

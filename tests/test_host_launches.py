@@ -1,0 +1,37 @@
+"""What the library launches, without a GPU: the built library runs against a stand-in for the HIP runtime
+(tests/host/launch_driver.cpp) that sees every launch's grid and arguments and can refuse a call."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIBDIR = os.path.join(ROOT, "aws_ofi_nccl_amd", "lib")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    if not shutil.which("g++"):
+        pytest.skip("no host compiler")
+    if not os.path.exists(os.path.join(LIBDIR, "libofi_amd_hotpath.so")):
+        from aws_ofi_nccl_amd import build
+        build.build_library()
+    exe = os.path.join(tmp_path_factory.mktemp("launches"), "launch_driver")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "host", "launch_driver.cpp"),
+                    "-rdynamic", "-L", LIBDIR, "-l:libofi_amd_hotpath.so", "-Wl,-rpath," + LIBDIR, "-Wl,-rpath,/opt/rocm/lib",
+                    "-Wl,--allow-shlib-undefined", "-o", exe], check=True)
+    return exe
+
+
+def run(driver, part):
+    proc = subprocess.run([driver, part], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert proc.returncode == 0 and part + ": ok" in proc.stdout, proc.stdout[-4000:]
+
+
+def test_small_striping_batches_never_meet_a_count_left_by_another(driver):
+    """The one-launch form of striping counts its workgroups in a word of the scratch: consecutive batches use
+    different words, a count left in one is gone before its turn comes again, and a batch that is captured
+    counts in none."""
+    run(driver, "striping")

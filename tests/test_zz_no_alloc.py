@@ -114,3 +114,29 @@ def test_noalloc_rejects_oversized_batch(lib, gpu):
                                          d.data_ptr(), _gpu.stream())
     assert rc == -7                                            # -E2BIG, nothing launched
     _gpu.sync()
+
+
+def test_small_batches_that_overlapped_leave_nothing_behind(lib, oracle, gpu):
+    """Small batches of two schedulers on two streams that nobody ordered, as the callers should have: whatever
+    becomes of those, later batches on the same scratch match the oracle."""
+    assert lib.ofi_amd_gpu_init() == 0
+    n = 6144
+    d_sizes = _gpu.to_dev(synthetic.stripe_sizes(31, n))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = [(dev_state(4, 131072, 64, (1, 2)), torch.zeros(n, dtype=torch.int32, device="cuda"),
+             torch.zeros(n * 12, dtype=torch.int64, device="cuda")) for _ in streams]
+    torch.cuda.synchronize()
+    for k in range(100):
+        for s, (d_state, d_num, d_xf) in zip(streams, outs):
+            assert lib.ofi_amd_sched_batch_noalloc(d_state.data_ptr(), d_sizes.data_ptr(), n - 256 * (k % 20), 128,
+                                                   d_num.data_ptr(), d_xf.data_ptr(), ctypes.c_void_p(s.cuda_stream)) == 0
+    torch.cuda.synchronize()
+    d_state, seeds = dev_state(4, 131072, 64, (3, 1)), (3, 1)
+    for k in (257, 1000, 6144, 2001):
+        sizes = synthetic.stripe_sizes(k, k)
+        got = run(lib.ofi_amd_sched_batch_noalloc, d_state, _gpu.to_dev(sizes), k)
+        want_num, want_xf, ost = _oracle.sched_batch(oracle, sizes, 4, 131072, 64, seeds)
+        assert np.array_equal(got[0], want_num) and np.array_equal(got[1], want_xf), k
+        st = m.SchedState.from_buffer_copy(got[2])
+        seeds = (ost.rr_small_counter, ost.rr_counter)
+        assert (st.rr_small_counter, st.rr_counter) == seeds, k
