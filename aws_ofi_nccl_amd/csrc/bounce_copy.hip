@@ -433,11 +433,15 @@ __global__ __launch_bounds__(64) void flush_post_kernel(const uint64_t *__restri
  * if they were all that long).  Few pieces: neighbours in a workgroup, whose table words then share cache lines
  * (5818 entries of up to 4 pieces 11.0 us, a quarter of a run apart 13.8).  1024 and more: an entry has
  * a run for every XCD and spreads by itself (64 entries of 16-32 MiB 578 us, padded 582).
- * Between the two as the kernel's comment says.  Tables so large that the padding might exceed what one launch
- * can number (2^32 work-items) go without it.
+ * Between the two as the kernel's comment says.  Tables of more than kMostPadded pieces go without the padding,
+ * which is less than as much again, so that a launch always stays below what it can number.
  */
 constexpr uint32_t kFewPieces = 8, kManyPieces = 1024;
 constexpr uint64_t kMostPadded = 1ull << 24;
+/* The pieces of one launch, in whole rounds over the XCDs: 2^32 work-items are one too many for a launch. */
+constexpr uint64_t kMostPieces = (1ull << 26) - kXcds * kRunPieces;
+static_assert(kMostPieces * 64 < 1ull << 32 && 2 * kMostPadded + kXcds * 2 * kRunPieces <= kMostPieces,
+	      "a launch, padded or not");
 piece_map_t copy_pieces_map(uint32_t per, uint64_t pieces)
 {
 	piece_map_t m = { per, kRunPieces / kPieceWaves, 1, kPieceWaves };
@@ -566,19 +570,23 @@ int ofi_amd_copy_table_pieces(const uint64_t *d_src_addr, const uint64_t *d_dst_
 	}
 	const uint64_t pieces_per_entry = max_len == 0 ? 1 : ((uint64_t)max_len + kPieceBytes - 1) / kPieceBytes;
 	const uint64_t least = (uint64_t)kXcds * kRunPieces;
-	const uint64_t pieces = ((uint64_t)n * pieces_per_entry + least - 1) / least * least;
-	if (pieces > 0x7fffffffull) {
+	if (((uint64_t)n * pieces_per_entry + least - 1) / least * least > 0x7fffffffull) {
 		return -E2BIG; /* split the table */
 	}
 	uint32_t *err = async_error_word();
 	if (!err) {
 		return -ENOMEM;
 	}
-	const piece_map_t map = copy_pieces_map((uint32_t)pieces_per_entry, pieces);
-	const uint64_t round = (uint64_t)kXcds * map.run_blocks * kPieceWaves; /* whole rounds over the XCDs */
-	const uint64_t blocks = ((uint64_t)n * map.per + round - 1) / round * (kXcds * map.run_blocks);
-	hipLaunchKernelGGL(copy_table_pieces_kernel, dim3((uint32_t)blocks), dim3(64 * kPieceWaves), 0, as_stream(stream),
-			   d_src_addr, d_dst_addr, d_len, n, map, max_len, err);
+	/* a launch for every kMostPieces pieces: at least 127 entries each, however long */
+	const uint32_t part = (uint32_t)(kMostPieces / pieces_per_entry);
+	for (uint32_t at = 0; at < n; at += part) {
+		const uint32_t here = n - at < part ? n - at : part;
+		const piece_map_t map = copy_pieces_map((uint32_t)pieces_per_entry, here * pieces_per_entry);
+		const uint64_t round = (uint64_t)kXcds * map.run_blocks * kPieceWaves; /* whole rounds over the XCDs */
+		const uint64_t blocks = ((uint64_t)here * map.per + round - 1) / round * (kXcds * map.run_blocks);
+		hipLaunchKernelGGL(copy_table_pieces_kernel, dim3((uint32_t)blocks), dim3(64 * kPieceWaves), 0,
+				   as_stream(stream), d_src_addr + at, d_dst_addr + at, d_len + at, here, map, max_len, err);
+	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -208,8 +208,8 @@ extern "C" int ofi_amd_gin_loopback_run(ofi_amd_gin_rings_t *r, uint64_t ops_per
 		}
 		int e = 0;
 		if (b.n_copy) {
-			/* one table entry per write, every 8 KiB of it a wavefront of its own; a launch holds
-			 * at most 2^31 - 1 wavefronts, so a table with very long entries goes in parts */
+			/* one table entry per write, every 8 KiB of it a wavefront of its own; a call takes
+			 * at most 2^31 - 1 of those pieces, so a table with very long entries goes in parts */
 			const uint64_t per_entry = ((uint64_t)b.max_len + 8191u) / 8192u;
 			const uint64_t most = per_entry ? (0x7fff0000ull / per_entry) : b.n_copy;
 			const uint32_t part = most < 1 ? 1u : (most < b.n_copy ? (uint32_t)most : b.n_copy);

@@ -247,7 +247,7 @@ struct ofi_amd_netfab {
 		}
 		int rc = 0;
 		if (g.n_copy) {
-			/* a launch holds at most 2^31 - 1 wavefronts, one per 8 KiB of the longest entry */
+			/* a call takes at most 2^31 - 1 pieces, one per 8 KiB of the longest entry */
 			const uint64_t per_entry = ((uint64_t)g.max_len + 8191u) / 8192u;
 			const uint64_t most = per_entry ? 0x7fff0000ull / per_entry : g.n_copy;
 			const uint32_t part = most < 1 ? 1u : (most < g.n_copy ? (uint32_t)most : g.n_copy);

@@ -213,10 +213,12 @@ int ofi_amd_copy_table(const uint64_t *d_src_addr, const uint64_t *d_dst_addr, c
  * entry rather than per entry, so that a few long RDMA writes (a rendezvous message's
  * stripes: one fi_writedata per rail, src/nccl_ofi_rdma.cpp:2447-2479) are swept by the whole chip
  * instead of by one wavefront each, and the caller need not cut them.  max_len >= every
- * d_len[i]; the launch has a wavefront for each of n * ceil(max_len / 8192) pieces, and up to twice as many
- * (-E2BIG beyond 2^31 - 1 pieces: split the table); those past the end of their entry leave at once.  An entry longer than max_len
- * is copied up to exactly max_len bytes (nothing of it when max_len is 0) and reported through
- * ofi_amd_async_error_fetch (bit 3).
+ * d_len[i]; a wavefront is launched for each of n * ceil(max_len / 8192) pieces, and some more: the
+ * pieces of an entry may be padded to up to twice as many, and a launch has whole rounds of at least 1024
+ * wavefronts.  Those without a piece leave at once.  -E2BIG where the pieces, rounded up to 1024, are more
+ * than 2^31 - 1: split the table (one launch takes 2^26 - 1024 of them, a larger table several).  An entry
+ * longer than max_len is copied up to exactly max_len bytes (nothing of it when max_len is 0) and reported
+ * through ofi_amd_async_error_fetch (bit 3).
  */
 int ofi_amd_copy_table_pieces(const uint64_t *d_src_addr, const uint64_t *d_dst_addr, const uint32_t *d_len,
 			      uint32_t n, uint32_t max_len, void *stream);

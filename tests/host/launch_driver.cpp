@@ -3,6 +3,7 @@
  * functions the library calls, so the library's host code runs without a GPU and every launch is seen with its
  * grid and its arguments.  argv[1] names the part to run.
  */
+#include <cerrno>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -43,6 +44,7 @@ std::map<const void *, std::string> &kernels()
 }
 
 std::function<void(const launch_t &)> on_launch = [](const launch_t &) {};
+hipError_t last_error = hipSuccess;
 hipError_t capture_answer = hipSuccess;
 hipStreamCaptureStatus capture_status = hipStreamCaptureStatusNone;
 struct config_t {
@@ -68,7 +70,12 @@ hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipDriverGetVersion(int *v) { *v = 1; return hipSuccess; }
 hipError_t hipRuntimeGetVersion(int *v) { *v = 1; return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError()
+{
+	const hipError_t e = last_error;
+	last_error = hipSuccess;
+	return e;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = reinterpret_cast<hipStream_t>(0x70); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
@@ -106,6 +113,10 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
 }
 hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t, hipStream_t stream)
 {
+	/* what HIP supports: fewer than 2^32 work-items along each dimension */
+	if ((uint64_t)grid.x * block.x >> 32 || (uint64_t)grid.y * block.y >> 32 || (uint64_t)grid.z * block.z >> 32) {
+		return last_error = hipErrorInvalidConfiguration;
+	}
 	on_launch({ kernels()[f], grid, block, args, stream });
 	return hipSuccess;
 }
@@ -196,13 +207,62 @@ int striping()
 	return 0;
 }
 
+/*
+ * Copy tables by pieces of 8 KiB: every table up to 2^31 - 1 pieces is launched, within the limits of a launch,
+ * every entry in one launch and with a wavefront for each of its pieces; larger ones are refused with nothing launched.
+ */
+int pieces()
+{
+	struct map_t {
+		uint32_t per, run_blocks, wave_stride, block_stride;
+	};
+	uint64_t *const src = reinterpret_cast<uint64_t *>(0x1000000), *const dst = reinterpret_cast<uint64_t *>(0x80000000000);
+	uint32_t *const len = reinterpret_cast<uint32_t *>(0x70000000000);
+	const uint32_t mib = 1u << 20;
+	struct table_t {
+		uint32_t n, max_len;
+		int rc;
+	};
+	const table_t tables[] = {
+		{ 1, 0, 0 }, { 1, 8192, 0 }, { 1, ~0u, 0 }, { 127, ~0u, 0 }, { 128, ~0u, 0 }, { 4095, ~0u, 0 },
+		/* a launch group with one write of 128 MiB: 2^26 pieces */
+		{ 4096, 128 * mib, 0 }, { 4095, 128 * mib, 0 }, { 4096, 64 * mib, 0 }, { 8192, 64 * mib - 8192, 0 },
+		{ (1u << 24) - 1, 8192, 0 }, { 1u << 24, 8192, 0 }, { (1u << 26) - 1024, 8192, 0 }, { (1u << 26) - 1023, 8192, 0 },
+		{ 1u << 26, 8192, 0 }, { 1u << 30, 8192, 0 }, { 1u << 20, 129 * 8192, 0 }, { 1u << 17, 129 * 8192, 0 },
+		{ 1u << 21, 8 * 8192, 0 }, { 130055, 129 * 8192, 0 }, { 4096, ~0u, -E2BIG }, { 1u << 20, ~0u, -E2BIG },
+	};
+	for (const table_t &t : tables) {
+		uint64_t covered = 0, launches = 0;
+		on_launch = [&](const launch_t &l) {
+			const uint32_t n = l.arg<uint32_t>(3);
+			const map_t map = l.arg<map_t>(4);
+			CHECK(l.arg<uint64_t *>(0) == src + covered && l.arg<uint64_t *>(1) == dst + covered &&
+			      l.arg<uint32_t *>(2) == len + covered && l.arg<uint32_t>(5) == t.max_len);
+			CHECK((uint64_t)map.per * 8192 >= t.max_len && l.block.x == 256 && l.grid.y * l.grid.z == 1);
+			/* whole runs for each of the 8 XCDs, their pieces numbered without a gap, enough of them */
+			CHECK(l.grid.x % (8 * map.run_blocks) == 0 && (uint64_t)l.grid.x * 4 >= (uint64_t)n * map.per);
+			CHECK((map.wave_stride == 1 && map.block_stride == 4) ||
+			      (map.wave_stride == map.run_blocks && map.block_stride == 1));
+			covered += n;
+			launches++;
+		};
+		const int rc = ofi_amd_copy_table_pieces(src, dst, len, t.n, t.max_len, nullptr);
+		if (rc != t.rc || covered != (rc == 0 ? t.n : 0)) {
+			std::printf("n %u max_len %u: %d, %llu of the entries in %llu launches\n", t.n, t.max_len, rc,
+				    (unsigned long long)covered, (unsigned long long)launches);
+			return 1;
+		}
+	}
+	return 0;
+}
+
 } // namespace
 
 int main(int argc, char **argv)
 {
-	const std::map<std::string, int (*)()> parts = { { "striping", striping } };
+	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "pieces", pieces } };
 	CHECK(argc == 2 && parts.count(argv[1]) && ofi_amd_gpu_init() == 0);
 	const int rc = parts.at(argv[1])();
-	std::printf("%s: ok\n", argv[1]);
+	std::printf("%s: %s\n", argv[1], rc == 0 ? "ok" : "failed");
 	return rc;
 }

@@ -351,3 +351,27 @@ def test_every_piece_of_a_mixed_table_is_dealt_out_once(lib, gpu, pieces, n):
     _gpu.sync()
     assert np.array_equal(d_dst.cpu().numpy(), want)
     assert _gpu.fetch_async_errors(lib) == 0
+
+
+@pytest.mark.parametrize("n,max_len", [(4097, 128 << 20), ((1 << 26) // 130 + 3, 129 * 8192)])
+def test_a_table_of_more_pieces_than_one_launch_takes(lib, gpu, n, max_len):
+    """A launch numbers fewer than 2^26 pieces; this table has more, short entries all of them, and its last ones are
+    copied by a launch of their own."""
+    rng = np.random.default_rng(n)
+    lens = rng.integers(0, 24, n).astype(np.uint32)
+    dst_off = 25 * np.arange(n, dtype=np.int64)
+    src = rng.integers(0, 256, 64, dtype=np.uint8)
+    src_off = rng.integers(0, 40, n)
+    want = np.full(25 * n, 0x77, dtype=np.uint8)
+    cols = np.arange(25)
+    rows = np.where(cols < lens[:, None], src[np.minimum(src_off[:, None] + cols, 63)], 0x77).astype(np.uint8)
+    want[:] = rows.reshape(-1)
+    d_src = _gpu.to_dev(src)
+    d_dst = torch.full((len(want),), 0x77, dtype=torch.uint8, device="cuda")
+    t_src, t_dst = (_gpu.to_dev(a) for a in (src_off + d_src.data_ptr(), dst_off + d_dst.data_ptr()))
+    t_len = _gpu.to_dev(lens)
+    assert lib.ofi_amd_copy_table_pieces(t_src.data_ptr(), t_dst.data_ptr(), t_len.data_ptr(), n, max_len,
+                                         _gpu.stream()) == 0
+    _gpu.sync()
+    assert np.array_equal(d_dst.cpu().numpy(), want)
+    assert _gpu.fetch_async_errors(lib) == 0

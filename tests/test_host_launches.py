@@ -35,3 +35,9 @@ def test_small_striping_batches_never_meet_a_count_left_by_another(driver):
     different words, a count left in one is gone before its turn comes again, and a batch that is captured
     counts in none."""
     run(driver, "striping")
+
+
+def test_copy_tables_of_many_pieces_stay_within_what_a_launch_can_number(driver):
+    """A launch holds fewer than 2^32 work-items: tables beyond go in several, up to the documented 2^31 - 1
+    pieces, and every entry is in exactly one of them."""
+    run(driver, "pieces")
