@@ -27,8 +27,9 @@
  * HBM traffic per message: 8 B read twice (once in the one-launch form) + 4 B + 96 B written.
  */
 #include <atomic>
+#include <map>
 #include <mutex>
-#include <unordered_map>
+#include <tuple>
 
 #include "common.hpp"
 #include "ofi_amd_hotpath.h"
@@ -456,8 +457,22 @@ struct scratch_t {
 	uint32_t *words = nullptr;
 	std::atomic<uint32_t> turn{ 0 }; /* of the next batch that counts arrivals */
 };
+/* The stream behind a handle: a created stream has its own, but the null stream's stands for another
+ * stream on each GPU, and hipStreamPerThread for another one in each thread besides. */
+using stream_key_t = std::tuple<void *, int, uint64_t>;
+int key_of_stream(void *stream, stream_key_t *key)
+{
+	static std::atomic<uint64_t> threads{ 0 };
+	static thread_local const uint64_t this_thread = ++threads;
+	int dev = -1;
+	if (stream == nullptr || stream == hipStreamLegacy || stream == hipStreamPerThread) {
+		OFI_AMD_HIP_TRY(hipGetDevice(&dev));
+	}
+	*key = { stream, dev, stream == hipStreamPerThread ? this_thread : 0 };
+	return 0;
+}
 std::mutex g_ws_lock;
-std::unordered_map<void *, scratch_t> g_ws_by_stream;
+std::map<stream_key_t, scratch_t> g_ws_by_stream;
 
 constexpr uint32_t kClearThreads = 256;
 __global__ __launch_bounds__(kClearThreads) void stripe_scratch_kernel(uint32_t *__restrict__ words)
@@ -647,11 +662,16 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
 	}
 
 	hipStream_t s = as_stream(stream);
+	stream_key_t key;
+	rc = key_of_stream(stream, &key);
+	if (rc != 0) {
+		return rc;
+	}
 	try {
 		/* held until the launches are queued: two threads submitting to one stream share its
 		 * scratch, and their count/emit pairs must not interleave */
 		std::lock_guard<std::mutex> g(g_ws_lock);
-		scratch_t &scratch = g_ws_by_stream[stream];
+		scratch_t &scratch = g_ws_by_stream[key];
 		if (!scratch.words) {
 			rc = new_scratch(s, &scratch.words);
 			if (rc != 0) {
@@ -672,10 +692,15 @@ int ofi_amd_sched_stream_release(void *stream)
 	if (rc != 0) {
 		return rc;
 	}
+	stream_key_t key;
+	rc = key_of_stream(stream, &key);
+	if (rc != 0) {
+		return rc;
+	}
 	uint32_t *words = nullptr;
 	{
 		std::lock_guard<std::mutex> g(g_ws_lock);
-		auto it = g_ws_by_stream.find(stream);
+		auto it = g_ws_by_stream.find(key);
 		if (it == g_ws_by_stream.end()) {
 			return 0; /* nothing was ever allocated for it */
 		}

@@ -123,7 +123,9 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
 			void *stream);
 /* ofi_amd_sched_batch keeps some 80 KiB of device scratch per stream it has been called with
  * (the reference's scheduler keeps a freelist per instance, src/nccl_ofi_scheduler.cpp:135-190).
- * A caller that destroys a stream hands the scratch back first: waits for the stream, frees.
+ * The null stream has scratch on each GPU, hipStreamPerThread on each GPU and for each thread.
+ * A caller that destroys a stream, or a thread that ends after calls on hipStreamPerThread, hands
+ * the scratch back first: waits for the stream, frees.
  * A batch captured into a graph keeps the scratch of the stream it was captured on: replays are
  * ordered with each other and with that stream's batches of more than 6144 messages. */
 int ofi_amd_sched_stream_release(void *stream);

@@ -12,6 +12,7 @@
 #include <map>
 #include <set>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include <cxxabi.h>
@@ -45,6 +46,7 @@ std::map<const void *, std::string> &kernels()
 
 std::function<void(const launch_t &)> on_launch = [](const launch_t &) {};
 hipError_t last_error = hipSuccess;
+int device = 0;
 hipError_t capture_answer = hipSuccess;
 hipStreamCaptureStatus capture_status = hipStreamCaptureStatusNone;
 struct config_t {
@@ -66,7 +68,7 @@ hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
 hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
-hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = device; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipDriverGetVersion(int *v) { *v = 1; return hipSuccess; }
 hipError_t hipRuntimeGetVersion(int *v) { *v = 1; return hipSuccess; }
@@ -208,6 +210,52 @@ int striping()
 }
 
 /*
+ * The scratch of a batch belongs to one stream: hipStreamPerThread is another stream in each thread, the null stream on
+ * each GPU, whatever their handles say; other handles are one stream whichever thread calls.
+ */
+int streams()
+{
+	ofi_amd_sched_state_t state = {};
+	uint64_t sizes[1] = {};
+	uint32_t num[1];
+	ofi_amd_xfer_info_t xfers[4];
+	/* the tile totals of a batch in the two-launch form */
+	auto scratch_on = [&](void *stream) {
+		uint32_t *totals = nullptr;
+		on_launch = [&](const launch_t &l) {
+			if (l.kernel.find("stripe_count_kernel") != std::string::npos) {
+				totals = l.arg<uint32_t *>(4);
+			}
+		};
+		CHECK(ofi_amd_sched_batch(&state, sizes, 10000, 128, num, xfers, stream) == 0 && totals);
+		return totals;
+	};
+	auto in_another_thread = [&](void *stream) {
+		uint32_t *totals = nullptr;
+		std::thread([&] { totals = scratch_on(stream); }).join();
+		return totals;
+	};
+	void *const made = reinterpret_cast<void *>(0x40), *const per_thread = hipStreamPerThread;
+	CHECK(scratch_on(made) == in_another_thread(made));
+	CHECK(scratch_on(nullptr) == in_another_thread(nullptr));
+	uint32_t *const mine = scratch_on(per_thread), *const null0 = scratch_on(nullptr);
+	CHECK(mine == scratch_on(per_thread) && mine != scratch_on(made) && mine != null0);
+	uint32_t *const other = in_another_thread(per_thread), *const third = in_another_thread(per_thread);
+	CHECK(other != mine && third != mine && third != other);
+	device = 1;
+	CHECK(scratch_on(nullptr) != null0 && scratch_on(per_thread) != mine);
+	device = 0;
+	CHECK(scratch_on(nullptr) == null0 && scratch_on(per_thread) == mine);
+	/* a thread hands its own back */
+	std::thread([&] {
+		scratch_on(per_thread);
+		CHECK(ofi_amd_sched_stream_release(per_thread) == 0);
+	}).join();
+	CHECK(scratch_on(per_thread) == mine && ofi_amd_sched_stream_release(per_thread) == 0);
+	return 0;
+}
+
+/*
  * Copy tables by pieces of 8 KiB: every table up to 2^31 - 1 pieces is launched, within the limits of a launch,
  * every entry in one launch and with a wavefront for each of its pieces; larger ones are refused with nothing launched.
  */
@@ -260,7 +308,7 @@ int pieces()
 
 int main(int argc, char **argv)
 {
-	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "pieces", pieces } };
+	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces } };
 	CHECK(argc == 2 && parts.count(argv[1]) && ofi_amd_gpu_init() == 0);
 	const int rc = parts.at(argv[1])();
 	std::printf("%s: %s\n", argv[1], rc == 0 ? "ok" : "failed");

@@ -20,7 +20,7 @@ def driver(tmp_path_factory):
     exe = os.path.join(tmp_path_factory.mktemp("launches"), "launch_driver")
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
                     "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "host", "launch_driver.cpp"),
-                    "-rdynamic", "-L", LIBDIR, "-l:libofi_amd_hotpath.so", "-Wl,-rpath," + LIBDIR, "-Wl,-rpath,/opt/rocm/lib",
+                    "-rdynamic", "-pthread", "-L", LIBDIR, "-l:libofi_amd_hotpath.so", "-Wl,-rpath," + LIBDIR, "-Wl,-rpath,/opt/rocm/lib",
                     "-Wl,--allow-shlib-undefined", "-o", exe], check=True)
     return exe
 
@@ -35,6 +35,11 @@ def test_small_striping_batches_never_meet_a_count_left_by_another(driver):
     different words, a count left in one is gone before its turn comes again, and a batch that is captured
     counts in none."""
     run(driver, "striping")
+
+
+def test_striping_scratch_is_kept_by_stream_and_not_by_handle(driver):
+    """hipStreamPerThread and the null stream are one handle for several streams, whose batches may overlap."""
+    run(driver, "streams")
 
 
 def test_copy_tables_of_many_pieces_stay_within_what_a_launch_can_number(driver):
