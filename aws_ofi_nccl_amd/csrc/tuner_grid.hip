@@ -845,13 +845,15 @@ int ofi_amd_tuner_model_grid(ofi_amd_tuner_plan_t *plan, const ofi_amd_tuner_var
 	try {
 		if (plan->h_variants.size() != n_variants ||
 		    std::memcmp(plan->h_variants.data(), variants, sizeof(*variants) * n_variants) != 0) {
-			plan->h_variants.assign(variants, variants + n_variants);
-			OFI_AMD_HIP_TRY(hipMemcpyAsync(plan->d_variants, plan->h_variants.data(),
-						       sizeof(*variants) * n_variants, hipMemcpyHostToDevice, s));
-			/* the source is pageable host memory owned by the plan: wait until it has been read */
+			plan->h_variants.clear(); /* stays empty if the upload fails: the next call uploads again */
+			OFI_AMD_HIP_TRY(hipMemcpyAsync(plan->d_variants, variants, sizeof(*variants) * n_variants,
+						       hipMemcpyHostToDevice, s));
+			/* the source is the caller's pageable memory: wait until it has been read */
 			OFI_AMD_HIP_TRY(hipStreamSynchronize(s));
+			plan->h_variants.assign(variants, variants + n_variants);
 		}
 	} catch (...) {
+		plan->h_variants.clear();
 		return -ENOMEM;
 	}
 	if (plan->points > (1ull << 31) || plan->cells * n_variants > (1ull << 38) || n_variants > 65535) {

@@ -47,6 +47,7 @@ std::map<const void *, std::string> &kernels()
 std::function<void(const launch_t &)> on_launch = [](const launch_t &) {};
 hipError_t last_error = hipSuccess;
 int device = 0;
+hipError_t copy_answer = hipSuccess, sync_answer = hipSuccess;
 hipError_t capture_answer = hipSuccess;
 hipStreamCaptureStatus capture_status = hipStreamCaptureStatusNone;
 struct config_t {
@@ -66,7 +67,10 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n);
 hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t)
+{
+	return copy_answer == hipSuccess ? hipMemcpy(d, s, n, k) : copy_answer;
+}
 hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int *d) { *d = device; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
@@ -78,7 +82,7 @@ hipError_t hipGetLastError()
 	last_error = hipSuccess;
 	return e;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return sync_answer; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = reinterpret_cast<hipStream_t>(0x70); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipGetSymbolAddress(void **p, const void *)
@@ -304,11 +308,41 @@ int pieces()
 	return 0;
 }
 
+/* A list of variants or platforms that did not reach the GPU is sent again by the next call with the same list. */
+int uploads()
+{
+	const int32_t colls[] = { 4 }, algos[] = { 1 };
+	const uint64_t sizes[] = { 1 << 20 }, nodes[] = { 4 };
+	const uint32_t ppn[] = { 8 };
+	ofi_amd_tuner_plan_t *plan = nullptr;
+	CHECK(ofi_amd_tuner_plan_create(colls, 1, sizes, 1, nodes, 1, ppn, 1, algos, 1, &plan) == 0);
+	double cost[3];
+	int8_t choice[4];
+	ofi_amd_tuner_variant_t v = { 0, 1, 8, 3 };
+	int launches = 0;
+	on_launch = [&](const launch_t &l) {
+		CHECK(std::memcmp(l.arg<void *>(1), &v, sizeof(v)) == 0); /* what the kernel reads */
+		launches++;
+	};
+	auto grid = [&] { return ofi_amd_tuner_model_grid(plan, &v, 1, cost, choice, nullptr); };
+	CHECK(grid() == 0 && launches == 1);
+	for (hipError_t *answer : { &copy_answer, &sync_answer }) {
+		v.pipe_ops++;
+		*answer = hipErrorUnknown;
+		CHECK(grid() == -EIO && launches == 1);
+		*answer = hipSuccess;
+		CHECK(grid() == 0);
+		launches = 1;
+	}
+	CHECK(ofi_amd_tuner_plan_destroy(plan) == 0);
+	return 0;
+}
+
 } // namespace
 
 int main(int argc, char **argv)
 {
-	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces } };
+	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces }, { "uploads", uploads } };
 	CHECK(argc == 2 && parts.count(argv[1]) && ofi_amd_gpu_init() == 0);
 	const int rc = parts.at(argv[1])();
 	std::printf("%s: %s\n", argv[1], rc == 0 ? "ok" : "failed");

@@ -46,3 +46,9 @@ def test_copy_tables_of_many_pieces_stay_within_what_a_launch_can_number(driver)
     """A launch holds fewer than 2^32 work-items: tables beyond go in several, up to the documented 2^31 - 1
     pieces, and every entry is in exactly one of them."""
     run(driver, "pieces")
+
+
+def test_an_upload_that_failed_is_made_again(driver):
+    """The tuner's grids send a list only when it differs from the last one: one that failed on the way does not
+    count as sent."""
+    run(driver, "uploads")
