@@ -308,6 +308,40 @@ int pieces()
 	return 0;
 }
 
+/* The tiles of a region grid follow its axes: on short ones too, most lanes have a point. */
+int tiles()
+{
+	const int32_t colls[] = { 4, 2 }, algos[] = { 1 };
+	const uint32_t ppn[] = { 8, 2, 1 };
+	const int32_t platforms[] = { 0, 1, 2, 3 };
+	const uint32_t shapes[][2] = { { 1, 20000 }, { 2, 20000 }, { 3, 20000 }, { 5, 20000 }, { 20000, 1 }, { 20000, 2 }, { 20000, 3 },
+				       { 20000, 5 }, { 1, 90000 }, { 90000, 1 }, { 560, 38 }, { 2000, 17 }, { 17, 2000 } };
+	for (const auto &shape : shapes) {
+		std::vector<uint64_t> sizes(shape[0]), nodes(shape[1]);
+		for (size_t i = 0; i < sizes.size(); i++) {
+			sizes[i] = 1000 * i;
+		}
+		for (size_t i = 0; i < nodes.size(); i++) {
+			nodes[i] = i + 1;
+		}
+		ofi_amd_tuner_plan_t *plan = nullptr;
+		CHECK(ofi_amd_tuner_plan_create(colls, 2, sizes.data(), shape[0], nodes.data(), shape[1], ppn, 3, algos, 1, &plan) == 0);
+		uint64_t lanes = 0;
+		on_launch = [&](const launch_t &l) { lanes += (uint64_t)l.grid.x * l.grid.y * l.block.x; };
+		alignas(4) int8_t choice[4];
+		CHECK(ofi_amd_tuner_region_grid(plan, platforms, 4, choice, nullptr) == 0);
+		const uint64_t points = 4 * ofi_amd_tuner_plan_points(plan);
+		CHECK(lanes >= points);
+		if (lanes > points * 2) {
+			std::printf("%u sizes x %u node counts: %llu lanes for %llu points\n", shape[0], shape[1],
+				    (unsigned long long)lanes, (unsigned long long)points);
+			return 1;
+		}
+		CHECK(ofi_amd_tuner_plan_destroy(plan) == 0);
+	}
+	return 0;
+}
+
 /* A list of variants or platforms that did not reach the GPU is sent again by the next call with the same list. */
 int uploads()
 {
@@ -342,7 +376,7 @@ int uploads()
 
 int main(int argc, char **argv)
 {
-	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces }, { "uploads", uploads } };
+	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces }, { "tiles", tiles }, { "uploads", uploads } };
 	CHECK(argc == 2 && parts.count(argv[1]) && ofi_amd_gpu_init() == 0);
 	const int rc = parts.at(argv[1])();
 	std::printf("%s: %s\n", argv[1], rc == 0 ? "ok" : "failed");

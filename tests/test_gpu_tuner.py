@@ -257,6 +257,25 @@ def test_region_tiles_of_every_size(lib, oracle, gpu, repeats, n_sizes, n_nodes)
     lib.ofi_amd_tuner_plan_destroy(plan)
 
 
+@pytest.mark.parametrize("n_sizes,n_nodes", [(1, 130), (2, 67), (3, 70), (5, 70), (130, 1), (130, 2), (70, 3), (1, 3), (3, 1), (2, 2)])
+def test_region_tiles_on_short_axes(lib, oracle, gpu, n_sizes, n_nodes):
+    """Where an axis is shorter than a large tile, the tile's other axis is longer: 64 or 16 points by one, two or four,
+    both ways round, with remainders; the smallest tiles lie half outside.  Points on polygon edges among them, shuffled axes."""
+    rng = np.random.default_rng(1000 * n_sizes + n_nodes)
+    nodes = rng.permutation(np.resize(np.array([16, 4, 3, 8, 32, 64, 128, 1, 2, 5, 100, 512], dtype=np.uint64), n_nodes)
+                            + np.arange(n_nodes, dtype=np.uint64) // np.uint64(12))
+    sizes = rng.permutation(np.resize(np.array([8 << 20, 1 << 15, 196608, 1 << 30, 32 << 20, 1, 31457280, 4 << 20, 107374182400],
+                                               dtype=np.uint64), n_sizes) + np.arange(n_sizes, dtype=np.uint64) // np.uint64(9))
+    colls, ppn = np.array([4, 2, 3], dtype=np.int32), np.array([8, 1, 2], dtype=np.uint32)
+    plan = make_plan(lib, colls, sizes, nodes, ppn, np.array([1], dtype=np.int32))
+    want = oracle_region_grid(oracle, [0, 1, 2, 3], colls, sizes, nodes, ppn)
+    for times in (1, 8, 200):
+        got = run_region(lib, plan, [0, 1, 2, 3] * times, (4 * times, 3, n_sizes, n_nodes, 3))
+        mism = np.argwhere((got != np.concatenate([want] * times)).any(axis=-1))
+        assert len(mism) == 0, (times, mism[:10])
+    lib.ofi_amd_tuner_plan_destroy(plan)
+
+
 def test_region_grid_on_changing_platform_lists(lib, oracle, gpu):
     """One plan, platform lists that grow, shrink and change in place: the launch order the plan keeps
     for a list (which entry, chunk and ranks-per-node value each workgroup takes) is rebuilt whenever

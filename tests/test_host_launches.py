@@ -48,6 +48,11 @@ def test_copy_tables_of_many_pieces_stay_within_what_a_launch_can_number(driver)
     run(driver, "pieces")
 
 
+def test_region_tiles_fit_short_axes(driver):
+    """A region grid of one size and many node counts, or the other way round, is not paid for by the square."""
+    run(driver, "tiles")
+
+
 def test_an_upload_that_failed_is_made_again(driver):
     """The tuner's grids send a list only when it differs from the last one: one that failed on the way does not
     count as sent."""
