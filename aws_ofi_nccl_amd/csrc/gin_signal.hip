@@ -5,9 +5,10 @@
  * The reference updates each counter from a CPU worker thread through GDRCopy -- a PCIe
  * read and a PCIe write per slot (apply_signal_work, src/rdma/gin/nccl_ofi_gin.cpp:
  * 1193-1256) -- and therefore folds a batch by slot first to save round trips
- * (apply_and_complete, :1425-1479).  Here a workgroup folds its items in an LDS table keyed
- * by the counter's address and adds each sum once: additions are commutative, so every
- * counter ends at the value that N single adds leave.
+ * (apply_and_complete, :1425-1479).  Here a workgroup whose items crowd on few lines of counters
+ * folds them in an LDS table keyed by the counter's address and adds each sum once; the others
+ * add item by item.  Additions are commutative, so every counter ends at the value that N single
+ * adds leave.
  *
  * What bounds it: adds to one 64-byte line of counters follow each other at 12 ns, whatever
  * their XCD, so a batch on few counters is a queue at the memory (262,144 items on one counter
@@ -34,22 +35,39 @@ struct regions_t {
 template <uint32_t kSlots> struct fold_t {
 	unsigned long long key[kSlots]; /* address of a counter; 0: free */
 	unsigned long long sum[kSlots];
+	uint32_t used; /* whether anything went into it */
 	uint64_t base[kMaxRegions], size[kMaxRegions];
 	uint64_t *counters[kMaxRegions];
 };
 
-/* before any item; the caller waits for the workgroup afterwards */
+/* Before any item, by the whole workgroup; `fold`: whether items may go into the fold.  The regions (a single
+ * one stays in scalar registers) are written by the first four wavefronts, each a quarter of them, from scalars: a
+ * lane's own index into the kernel's arguments is a vector load from host memory, a link's round trip of 0.7 us. */
 template <uint32_t kSlots>
-__device__ __forceinline__ void fold_begin(fold_t<kSlots> &f, const regions_t &regions, uint32_t threads)
+__device__ __forceinline__ void begin(fold_t<kSlots> &f, const regions_t &regions, bool fold, uint32_t threads)
 {
-	for (uint32_t i = threadIdx.x; i < kSlots; i += threads) {
-		f.key[i] = 0;
-		f.sum[i] = 0;
+	if (fold) {
+		for (uint32_t i = threadIdx.x; i < kSlots; i += threads) {
+			f.key[i] = 0;
+			f.sum[i] = 0;
+		}
+		if (threadIdx.x == 0) {
+			f.used = 0;
+		}
 	}
-	if (threadIdx.x < kMaxRegions) {
-		f.base[threadIdx.x] = regions.base[threadIdx.x];
-		f.size[threadIdx.x] = regions.size[threadIdx.x];
-		f.counters[threadIdx.x] = regions.counters[threadIdx.x];
+	if (regions.n > 1 && (threadIdx.x & 63u) == 0) {
+		const uint32_t wave = threadIdx.x >> 6;
+#pragma unroll
+		for (uint32_t r = 0; r < kMaxRegions; r++) {
+			if (r / 4 == wave && r < regions.n) {
+				f.base[r] = regions.base[r];
+				f.size[r] = regions.size[r];
+				f.counters[r] = regions.counters[r];
+			}
+		}
+	}
+	if (fold || regions.n > 1) {
+		__syncthreads();
 	}
 }
 
@@ -66,6 +84,11 @@ template <uint32_t kSlots>
 __device__ __forceinline__ uint64_t *slot_of(const fold_t<kSlots> &f, const regions_t &regions, uint64_t base,
 					     uint64_t offset)
 {
+	if (regions.n == 1) {
+		const uint64_t size = regions.size[0];
+		const bool ok = base == regions.base[0] && (offset & 7u) == 0 && offset <= size && size - offset >= 8;
+		return ok ? regions.counters[0] + (offset >> 3) : nullptr;
+	}
 	uint32_t r = kMaxRegions;
 #pragma unroll
 	for (int k = (int)kMaxRegions - 1; k >= 0; k--) {
@@ -86,20 +109,16 @@ __device__ __forceinline__ uint64_t *slot_of(const fold_t<kSlots> &f, const regi
 	}
 }
 
-/* One item into the fold; past kProbes entries taken by other counters it goes to its own
- * directly.  Relaxed: ordering against the payload is the put-before-signal protocol's business
- * (the reference uses a relaxed fetch_add on its host path for the same reason, :1209). */
-template <uint32_t kSlots>
-__device__ __forceinline__ void fold_item(fold_t<kSlots> &f, const regions_t &regions, uint64_t base, uint64_t offset,
-					  uint64_t value, uint32_t *__restrict__ rejected)
+/* Relaxed: ordering against the payload is the put-before-signal protocol's business (the reference uses a relaxed
+ * fetch_add on its host path for the same reason, :1209). */
+__device__ __forceinline__ void add_directly(uint64_t *slot, uint64_t value)
 {
-	uint64_t *slot = slot_of(f, regions, base, offset);
-	if (slot == nullptr) {
-		if (rejected) {
-			atomicAdd(rejected, 1u);
-		}
-		return;
-	}
+	__hip_atomic_fetch_add(slot, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* One item into the fold; past kProbes entries taken by other counters it goes to its own directly. */
+template <uint32_t kSlots> __device__ __forceinline__ void add_to_fold(fold_t<kSlots> &f, uint64_t *slot, uint64_t value)
+{
 	const unsigned long long key = (unsigned long long)reinterpret_cast<uintptr_t>(slot);
 	uint32_t h = ((uint32_t)(key >> 3) * 0x9e3779b1u) >> (32 - __builtin_ctz(kSlots));
 	for (uint32_t probe = 0; probe < kProbes; probe++) {
@@ -115,23 +134,75 @@ __device__ __forceinline__ void fold_item(fold_t<kSlots> &f, const regions_t &re
 		}
 		h = (h + 1) & (kSlots - 1);
 	}
-	__hip_atomic_fetch_add(slot, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	add_directly(slot, value);
 }
 
-/* the sums onto the counters; after the workgroup has met behind its last item */
-template <uint32_t kSlots> __device__ __forceinline__ void fold_end(fold_t<kSlots> &f, uint32_t threads)
+/*
+ * Whether the items of a wavefront crowd on few lines of counters: how many of them share a line with lane 0's, 21's
+ * or 42's.  The fold costs a workgroup 0.7-1 us (256 items in HBM on 8192 counters: 2.44 us without, 3.18 with),
+ * and what it saves is the queue at a line, 12 ns for each of the batch's items on it, of which those lanes are a
+ * sample: it pays from about 24576 / n lanes on (crowd_of), a few more than the three themselves at the least.
+ */
+constexpr uint32_t kMostCrowded = 3 * 64;
+__device__ __forceinline__ bool crowded(const uint64_t *slot, uint32_t crowd)
 {
+	const uint32_t line = (uint32_t)(reinterpret_cast<uintptr_t>(slot) >> 6);
+	const uint64_t with_item = __ballot(slot != nullptr);
+	uint32_t same = 0;
+#pragma unroll
+	for (int lane = 0; lane < 63; lane += 21) {
+		same += (uint32_t)__popcll(with_item & __ballot(line == (uint32_t)__builtin_amdgcn_readlane((int)line, lane)));
+	}
+	return same >= crowd;
+}
+static uint32_t crowd_of(uint32_t n)
+{
+	return n < 4096u ? 24576u / n : 6u;
+}
+
+/* The item of every lane that has one, by a whole wavefront; `folds` becomes and stays true with the first crowd. */
+template <uint32_t kSlots>
+__device__ __forceinline__ void add_items(fold_t<kSlots> &f, const regions_t &regions, uint64_t base, uint64_t offset,
+					  uint64_t value, bool live, uint32_t crowd, bool &folds,
+					  uint32_t *__restrict__ rejected)
+{
+	uint64_t *slot = nullptr;
+	if (live) {
+		slot = slot_of(f, regions, base, offset);
+		if (slot == nullptr && rejected) {
+			atomicAdd(rejected, 1u);
+		}
+	}
+	if (!folds && crowded(slot, crowd)) {
+		folds = true;
+		f.used = 1;
+	}
+	if (slot != nullptr) {
+		if (folds) {
+			add_to_fold(f, slot, value);
+		} else {
+			add_directly(slot, value);
+		}
+	}
+}
+
+/* Behind the last item, by the whole workgroup: the sums onto the counters.  `folds`: this wavefront's. */
+template <uint32_t kSlots> __device__ __forceinline__ void end(fold_t<kSlots> &f, bool folds, uint32_t threads)
+{
+	__syncthreads();
+	if (!folds && f.used == 0) {
+		return;
+	}
 	for (uint32_t i = threadIdx.x; i < kSlots; i += threads) {
 		if (f.key[i] != 0) {
-			__hip_atomic_fetch_add(reinterpret_cast<uint64_t *>(f.key[i]), (uint64_t)f.sum[i], __ATOMIC_RELAXED,
-					       __HIP_MEMORY_SCOPE_AGENT);
+			add_directly(reinterpret_cast<uint64_t *>(f.key[i]), (uint64_t)f.sum[i]);
 		}
 	}
 }
 
 template <uint32_t kThreads, uint32_t kItems, uint32_t kSlots>
 __global__ __launch_bounds__(kThreads) void gin_signal_apply_kernel(
-	const ofi_amd_gin_signal_work_t *__restrict__ work, uint32_t n, regions_t regions,
+	const ofi_amd_gin_signal_work_t *__restrict__ work, uint32_t n, regions_t regions, uint32_t crowd,
 	uint32_t *__restrict__ rejected)
 {
 	__shared__ __align__(16) fold_t<kSlots> f;
@@ -144,37 +215,61 @@ __global__ __launch_bounds__(kThreads) void gin_signal_apply_kernel(
 		offset[k] = w->offset;
 		value[k] = w->value;
 	}
-	fold_begin(f, regions, kThreads);
-	__syncthreads();
+	const bool may_fold = crowd <= kMostCrowded;
+	begin(f, regions, may_fold, kThreads);
+	bool folds = crowd == 0;
+	if (folds) {
+		f.used = 1;
+	}
 #pragma unroll
 	for (uint32_t k = 0; k < kItems; k++) {
-		if (first + k * kThreads < n) {
-			fold_item(f, regions, base[k], offset[k], value[k], rejected);
-		}
+		add_items(f, regions, base[k], offset[k], value[k], first + k * kThreads < n, crowd, folds, rejected);
 	}
-	__syncthreads();
-	fold_end(f, kThreads);
+	if (may_fold) {
+		end(f, folds, kThreads);
+	}
 }
 
 /* The adds of a batch and the flush read behind them in one launch of one workgroup: every
  * thread's adds have been performed at the memory before the workgroup meets, and only then is
  * the flush buffer read back into the host's slots -- what two launches order by the kernel
- * boundary between them. */
+ * boundary between them.
+ * Bound by the trips for the items, 256 at a time, which is why the next ones are asked for before the last ones
+ * are added.  In us, items in host memory, every item added by itself / every item folded / as it is:
+ *   1 item                         4.5 / 5.3 / 4.4
+ *   256 items, 8192 counters       4.9 / 6.0 / 4.9
+ *   1024 items, 8192 counters      12.5 / 15.0 / 9.2
+ *   4096 items, 1 counter          95 / 31 / 24
+ *   65536 items, 64 counters       870 / 441 / 330 */
 constexpr uint32_t kPostThreads = 256, kPostSlots = 1024;
 __global__ __launch_bounds__(kPostThreads) void gin_signal_apply_post_kernel(
-	const ofi_amd_gin_signal_work_t *__restrict__ work, uint32_t n, regions_t regions,
+	const ofi_amd_gin_signal_work_t *__restrict__ work, uint32_t n, regions_t regions, uint32_t crowd,
 	uint32_t *__restrict__ rejected, const uint64_t *__restrict__ flush_buf, uint64_t *__restrict__ slots,
 	uint32_t num_rails)
 {
 	__shared__ __align__(16) fold_t<kPostSlots> f;
 	if (n != 0) {
-		fold_begin(f, regions, kPostThreads);
-		__syncthreads();
-		for (uint32_t i = threadIdx.x; i < n; i += kPostThreads) {
-			fold_item(f, regions, work[i].base, work[i].offset, work[i].value, rejected);
+		uint64_t base, offset, value;
+		auto load = [&](uint32_t at) {
+			const ofi_amd_gin_signal_work_t *w = work + min(at + threadIdx.x, n - 1u);
+			base = w->base;
+			offset = w->offset;
+			value = w->value;
+		};
+		load(0); /* on its way while the fold is prepared */
+		const bool may_fold = crowd <= kMostCrowded;
+		bool folds = false;
+		begin(f, regions, may_fold, kPostThreads);
+		for (uint32_t at = 0; at < n; at += kPostThreads) {
+			const uint64_t b = base, o = offset, v = value;
+			if (at + kPostThreads < n) {
+				load(at + kPostThreads);
+			}
+			add_items(f, regions, b, o, v, at + threadIdx.x < n, crowd, folds, rejected);
 		}
-		__syncthreads();
-		fold_end(f, kPostThreads);
+		if (may_fold) {
+			end(f, folds, kPostThreads);
+		}
 	}
 	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
 	__syncthreads();
@@ -239,9 +334,12 @@ extern "C" int ofi_amd_gin_signal_apply(const ofi_amd_gin_signal_work_t *d_work,
 	 *   262144 items in HBM, 64 counters                311 / 166  90   25.9 16.5
 	 *   262144 items in HBM, 8192 counters             16.8 / 16.0 15.8 16.5 18.0
 	 *   262144 items in HBM, 262144 counters           14.3 / 14.6 14.6 16.5 18.0
-	 * so 256 up to 4096 items, then 512, and 2048 or 4096 for long batches on few counters (one to 64 items or more).  Long
-	 * batches in host memory take those too: the link is read faster from 64 CUs than from all of
-	 * them (262144 items over 8192 counters 187 / 188 187 179 160). */
+	 * so 256 up to 4096 items, then 512, and 2048 or 4096 for long batches on few counters (one to 64 items or more).
+	 * Batches up to 32768 items are not told apart by their counters, which costs the fourth line's 1.2 us.
+	 * Long batches in host memory take the large workgroups too: the link is read faster from 64 CUs than
+	 * from all of them (262144 items over 8192 counters 187 / 188 187 179 160).  The times are of workgroups
+	 * that all fold; since only crowded ones do (crowd_of), 1000 items in host memory on 8192 counters take
+	 * 3.8 instead of 4.6, 16384 in HBM 3.4 instead of 3.9, 1000 in HBM on one counter 3.1 instead of 2.9. */
 	uint64_t counters = 0;
 	for (uint32_t i = 0; i < n_regions; i++) {
 		counters += r.size[i] / 8;
@@ -249,7 +347,7 @@ extern "C" int ofi_amd_gin_signal_apply(const ofi_amd_gin_signal_work_t *d_work,
 	const bool large = n > 32768u && (counters <= n / 64u || in_host_memory(d_work));
 	auto launch = [&](auto kernel, uint32_t threads, uint32_t items) {
 		hipLaunchKernelGGL(kernel, dim3((n - 1u) / (threads * items) + 1u), dim3(threads), 0, as_stream(stream),
-				   d_work, n, r, d_rejected);
+				   d_work, n, r, large ? 0u : crowd_of(n), d_rejected);
 	};
 	if (n <= 4096u) {
 		launch(gin_signal_apply_kernel<256, 1, 512>, 256, 1);
@@ -284,8 +382,8 @@ extern "C" int ofi_amd_gin_signal_apply_post(const ofi_amd_gin_signal_work_t *d_
 	if (n != 0 && (!d_work || pack_regions(regions, n_regions, &r) != 0)) {
 		return -EINVAL;
 	}
-	hipLaunchKernelGGL(gin_signal_apply_post_kernel, dim3(1), dim3(256), 0, as_stream(stream), d_work, n, r,
-			   d_rejected, static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
+	hipLaunchKernelGGL(gin_signal_apply_post_kernel, dim3(1), dim3(kPostThreads), 0, as_stream(stream), d_work, n, r,
+			   n != 0 ? crowd_of(n) : 0u, d_rejected, static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
 			   num_rails);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;

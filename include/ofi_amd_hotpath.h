@@ -682,8 +682,8 @@ typedef struct {
 /*
  * Applies a batch of work items to the signal counters in HBM, replacing the reference's
  * GDRCopy read-modify-write over PCIe (apply_signal_work, nccl_ofi_gin.cpp:1193-1256) and
- * its per-batch same-slot fold (apply_and_complete, :1425-1479): one thread per item, one
- * 64-bit device-scope atomic add each, so items hitting one slot combine in the L2.
+ * its per-batch same-slot fold (apply_and_complete, :1425-1479): 64-bit device-scope atomic
+ * adds, one per item or, where a workgroup's items crowd on few counters, one per counter.
  * d_work is device-accessible (pinned host or HBM); regions is a host array (<= 16).
  * Items that match no region or are misaligned are skipped and counted in *d_rejected
  * (device-accessible u32, may be NULL).

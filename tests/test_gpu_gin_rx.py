@@ -331,6 +331,54 @@ def test_adds_and_the_flush_read_behind_them_in_one_launch(lib, oracle, gpu, n, 
     _gpu.sync()
 
 
+@pytest.mark.parametrize("pinned", [False, True])
+@pytest.mark.parametrize("n", [1, 64, 127, 128, 129, 256, 257, 1000, 4095, 4096, 4097, 20000])
+def test_wavefronts_that_crowd_beside_some_that_do_not(lib, gpu, n, pinned):
+    """Both entry points on batches of which some wavefronts have all their items on one counter or on one line, others
+    on more counters than a fold has entries, others half and half or no counter at all: crowds come
+    first, last and in the middle.  Sums modulo 2^64 and the count of refused items are exact."""
+    slots = 9000
+    for regions, kinds in ((1, (0, 1, 2, 3)), (1, (2, 0, 4, 1)), (3, (1, 1, 3, 2)), (16, (4, 2, 0, 3))):
+        rng = np.random.default_rng(n + regions)
+        kind = np.array(kinds)[(np.arange(n) // 64) % 4]
+        anywhere = rng.integers(0, slots, n)
+        slot = np.select([kind == 0, kind == 1, kind == 2], [np.full(n, 77), 8 + np.arange(n) % 8, anywhere],
+                         np.where(np.arange(n) % 2, 4001, anywhere))
+        work = np.zeros(n, dtype=work_array([]).dtype)
+        # windows of slots counters each, one behind the other in the work items' addresses or far apart
+        apart = 8 * slots if regions == 3 else 1 << 32
+        window = rng.integers(0, regions, n)
+        work["base"] = np.uint64(SIG_BASE) + window.astype(np.uint64) * np.uint64(apart)
+        work["offset"] = 8 * slot
+        work["value"] = rng.integers(0, 1 << 63, n).astype(np.uint64) * np.uint64(2) + np.uint64(1)
+        work["run_len"] = 1
+        ok = (kind != 4) & (rng.integers(0, 16, n) != 0)
+        work["offset"][~ok] += np.uint64(4)                       # not a counter's address
+        want = rng.integers(0, 1 << 63, regions * slots).astype(np.uint64)
+        start = want.copy()
+        with np.errstate(over="ignore"):
+            np.add.at(want, (window * slots + slot)[ok], work["value"][ok])
+        words = torch.from_numpy(work.view(np.int64))
+        d_work = words.pin_memory() if pinned else words.cuda()
+        d_flush = torch.full((8,), 77, dtype=torch.int64, device="cuda")
+        slots_host = torch.zeros(4 * 8, dtype=torch.int64, pin_memory=True)
+        for post in (False, True):
+            d_cnt = _gpu.to_dev(start)
+            regs = (m.GinSignalRegion * regions)(*[
+                m.GinSignalRegion(SIG_BASE + r * apart, 8 * slots, d_cnt.data_ptr() + 8 * slots * r) for r in range(regions)])
+            rejected = torch.zeros(1, dtype=torch.int32, device="cuda")
+            if post:
+                rc = lib.ofi_amd_gin_signal_apply_post(d_work.data_ptr(), n, regs, regions, rejected.data_ptr(),
+                                                       d_flush.data_ptr(), slots_host.data_ptr(), 2, _gpu.stream())
+            else:
+                rc = lib.ofi_amd_gin_signal_apply(d_work.data_ptr(), n, regs, regions, rejected.data_ptr(), _gpu.stream())
+            assert rc == 0
+            _gpu.sync()
+            assert np.array_equal(_gpu.to_host(d_cnt, np.uint64), want), (regions, post)
+            assert int(rejected.item()) == int((~ok).sum())
+        assert (slots_host.numpy()[:16] == 77).all() and not slots_host.numpy()[16:].any()
+
+
 def test_apply_post_arguments(lib, gpu):
     d = torch.zeros(64, dtype=torch.int64, device="cuda")
     slots_host = torch.zeros(32, dtype=torch.int64, pin_memory=True)
