@@ -839,7 +839,7 @@ int main(int argc, char **argv)
 		int n = 0;
 		for (int tries = 0; n == 0 && tries < 100; tries++) {
 			n = r_ops.cq_read(r_ops.end, cqe, 4);
-			device_tick(4);
+			CHECK(ofi_amd_gpu_stream_synchronize(nullptr) == 0); /* what that has queued, on whichever thread */
 		}
 		CHECK(n == 1 && cqe[0].kind == OFI_AMD_NET_CQ_EAGER && cqe[0].len == 100);
 		CHECK(r_ops.repost_rx(r_ops.end, cqe[0].rx_cookie) == 0);
