@@ -136,7 +136,7 @@ __device__ __forceinline__ uint32_t contribution(uint64_t size, const params_t &
 /* Inclusive sum over the 64 lanes with lane-to-lane moves inside the vector unit: shifts by 1,
  * 2, 4 and 8 lanes within each row of 16 (a lane shifted in from outside the row reads 0), then
  * lane 15 of rows 0 and 2 added to rows 1 and 3, then lane 31 added to rows 2 and 3. */
-__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, uint32_t)
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v)
 {
 	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false); /* row_shr:1 */
 	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false); /* row_shr:2 */
@@ -155,7 +155,7 @@ __device__ __forceinline__ uint32_t residues(uint32_t packed, uint32_t num_rails
 
 __device__ __forceinline__ uint32_t wave_sum_of(uint32_t v)
 {
-	v = wave_inclusive_scan(v, 0);
+	v = wave_inclusive_scan(v);
 	return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
@@ -339,7 +339,7 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	acc = wave_sum_of(acc);
 	uint32_t k = 0;
 	const uint32_t c = live ? contribution(size, p, k) : 0;
-	const uint32_t inc = wave_inclusive_scan(c, lane);
+	const uint32_t inc = wave_inclusive_scan(c);
 	if (lane == 0) {
 		seed_sum[wave] = acc;
 	}
@@ -528,7 +528,7 @@ int new_scratch(hipStream_t s, uint32_t **out)
  * code object (which starts at zero), held until the process ends.  In host code the
  * array's name is only a handle for hipGetSymbolAddress; kernels get the address it returns.
  */
-constexpr uint64_t kNoAllocMaxBatch = 1ull << 26;
+constexpr uint64_t kNoAllocMaxBatch = 1ull << 26; /* what the entry point promises; the scratch would do for any batch */
 static __device__ __align__(256) __attribute__((used)) uint32_t scratch[kScratchWords];
 
 constexpr int kMaxDevices = 64;
@@ -725,7 +725,7 @@ int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *
 		return -EINVAL;
 	}
 	if (n > kNoAllocMaxBatch) {
-		return -E2BIG; /* more messages than the fixed scratch has tiles for */
+		return -E2BIG;
 	}
 	if (n == 0) {
 		return 0;
@@ -738,7 +738,8 @@ int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *
 		return -ENXIO; /* ofi_amd_gpu_init() allocates it; this call must not */
 	}
 	scratch_t *scratch = nullptr;
-	rc = cached_scratch_of_current_device(&scratch); /* -ENXIO: ofi_amd_gpu_init() looks the address up; this call must not */
+	/* -ENXIO: ofi_amd_gpu_init() looks the address up; this call must not */
+	rc = cached_scratch_of_current_device(&scratch);
 	if (rc != 0) {
 		return rc;
 	}

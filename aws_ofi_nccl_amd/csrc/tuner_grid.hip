@@ -172,7 +172,6 @@ struct region_run_t {
 	int32_t platform;
 };
 
-
 /* What a whole tile knows about one edge of its polygon set */
 struct tile_edge_t {
 	bool crossed;  /* the ray of every point of the tile crosses it, and certainly so (crossing_certain) */
@@ -260,8 +259,8 @@ __device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64
  * point, with quotients, took 40-42 us for 1.02 M points of four platforms (560 sizes, 38 node counts),
  * this takes 10.8, a part of it the handing out of 16,896 wavefronts (kMostRegionWaves), the rest the time of the
  * tiles with the most edges, which is why their turns count instructions (two edges a turn, for
- * shorter chains of dependent operations, was slower: 13.3 against then 12.0).  A grid of few points is the time of such a
- * tile alone, and takes smaller ones (pick_tiling).
+ * shorter chains of dependent operations, was slower: 13.3 against then 12.0).  A grid of few points is the
+ * time of such a tile alone, and takes smaller ones (pick_tiling).
  *
  * In the output the ranks-per-node index runs fastest, so a wavefront's records lie 4 x
  * n_ppn bytes apart and the records between them belong to the same tile's other
@@ -271,16 +270,16 @@ __device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64
  * records, the rest lines that tiles side by side share; with the workgroups of a tile on different XCDs every
  * L2 wrote its quarter of each line, 18.9 MB).
  */
-__global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(grid_dims_t g, tiling_t t, const int32_t *__restrict__ polys,
-							    const double *__restrict__ bboxes,
-							    const edge_t *__restrict__ edges, pt_t far_point,
-							    const region_run_t *__restrict__ runs,
-							    uint32_t points_per_platform, int8_t *__restrict__ choice)
+__global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(
+	grid_dims_t g, tiling_t t, const int32_t *__restrict__ polys, const double *__restrict__ bboxes,
+	const edge_t *__restrict__ edges, pt_t far_point, const region_run_t *__restrict__ runs,
+	uint32_t points_per_platform, int8_t *__restrict__ choice)
 {
 	/* blockIdx.y names a run, blockIdx.x = 8 * group + x the tiles 8 * group .. 8 * group + 7 of it, of
 	 * which XCD x takes one (workgroups are dealt to the XCDs in launch order, and gridDim.x is a
-	 * multiple of 8); a second wavefront takes its tile from the other half of the groups.  The host lists the runs by falling cost (edges of the pair's set): the long
-	 * workgroups start first and the short ones fill the end of the launch. */
+	 * multiple of 8); a second wavefront takes its tile from the other half of the groups.  The host lists the
+	 * runs by falling cost (edges of the pair's set): the long workgroups start first and the short ones fill
+	 * the end of the launch. */
 	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const region_run_t run = runs[blockIdx.y];
 	/* which of a group's eight tiles an XCD takes rotates with the platform entry: the tiles

@@ -243,8 +243,9 @@ static double log2_count(uint64_t v)
 /*
  * Takes the answers as they arrive instead of waiting for the launch to retire, which the host hears of
  * 5 us later (16 questions: 11.4 us for the call instead of 16.7, 259: 16.5 instead of 21.1; from 600 on,
- * where the host's own work per question is what counts, it is the same).  A launch that has retired without all of its answers has failed: the stream is asked
- * now and then, so the wait ends with the launch in any case.
+ * where the host's own work per question is what counts, it is the same).  A launch that has retired without
+ * all of its answers has failed: the stream is asked now and then, so the wait ends with the launch in any
+ * case.
  */
 static int collect_answers(const staging_t &stage, uint32_t n, uint32_t call, ofi_amd_tuner_answer_t *answers)
 {

@@ -146,7 +146,8 @@ def test_graph_of_hot_path_launches_replays_exactly(lib, oracle, gpu):
 def test_batch_first_called_while_its_stream_is_captured(lib, oracle, gpu):
     """The scratch of a stream is made by the call that the stream is being captured in (a capture mode that lets a
     call allocate): batches called before the first replay, the replay and batches after it all match the oracle,
-    whatever the memory held.  1000 messages is the one-launch form, whose workgroups count themselves."""
+    whatever the memory held.  1000 messages are one launch when called, whose workgroups count themselves in the
+    scratch, and two when captured."""
     s = torch.cuda.Stream()
     sp = ctypes.c_void_p(s.cuda_stream)
     assert lib.ofi_amd_sched_stream_release(sp) == 0
@@ -168,10 +169,13 @@ def test_batch_first_called_while_its_stream_is_captured(lib, oracle, gpu):
         return lib.ofi_amd_sched_batch(d_state.data_ptr(), d_sizes.data_ptr(), n, 128, d_num.data_ptr(), d_xf.data_ptr(), sp)
 
     g = torch.cuda.CUDAGraph()
+    probe = ctypes.c_void_p()
     with torch.cuda.graph(g, stream=s, capture_error_mode="relaxed"):
+        can_allocate = lib.ofi_amd_gpu_mem_alloc(ctypes.byref(probe), 1 << 20) == 0
         rc = call()
-    if rc != 0:
-        pytest.skip("this runtime refuses allocations during a capture: %d" % rc)
+    if not can_allocate:
+        pytest.skip("this runtime refuses allocations during a capture")
+    assert rc == 0 and lib.ofi_amd_gpu_mem_free(probe) == 0
     seeds = (2, 1)
     for step in ("call", "replay", "call", "replay"):
         if step == "call":

@@ -188,10 +188,9 @@ def test_bad_arguments(lib, gpu):
 
 @pytest.mark.parametrize("rails,seeds", [(4, (3, 2)), (3, (1, 2))])
 def test_batches_beyond_the_inline_prefix_limit(lib, oracle, gpu, rails, seeds):
-    """Batches up to 2^21 messages use 512-message tiles, larger ones 1024-message tiles; beyond 4096
-    tiles the tile seeds come from the separate scan launch.  One message below and one above each
-    boundary must chain exactly like the small form."""
-    # ... and 9 << 19, from where the XCDs take runs of 16 tiles instead of single tiles in turn
+    """Batches of 2^21 to 9,000,011 messages, on both sides of numbers of tiles that are powers of two and of 6 Mi
+    messages, from where tiles are of 1024 messages and their seeds come from block totals: all must chain
+    exactly like the small form."""
     for n in ((1 << 21), (1 << 21) + 1, 4096 * 1024, 4096 * 1024 + 1, (9 << 19) - 1, 9 << 19, (9 << 19) + 16 * 1024 * 8 + 5,
               4096 * 2048 + 1, 9_000_011):
         sizes = synthetic.stripe_sizes(n + rails, n)

@@ -1,6 +1,6 @@
 """GPU parity of the striping entry point that allocates nothing (ofi_amd_sched_batch_noalloc)
-against ofi_amd_sched_batch and the CPU oracle: two calls in a row on the same scratch, the
-second with a smaller input, then a batch large enough for the separate scan launch."""
+against ofi_amd_sched_batch and the CPU oracle: calls in a row on the same scratch in each of the three launch
+forms (up to 6144 messages, up to 6 Mi, and beyond in parts of 2^24), smaller ones after larger ones."""
 import ctypes
 
 import numpy as np
@@ -32,9 +32,10 @@ def run(fn, d_state, d_sizes, n):
 
 def test_noalloc_matches_allocating_entry_point(lib, oracle, gpu):
     assert lib.ofi_amd_gpu_init() == 0
-    # second call smaller than the first (stale totals of the first stay in the scratch),
-    # third call beyond 4096 tiles of 1024 messages: the scan launch and the prefix half
-    for seed, n in ((11, 300007), (12, 1234), (13, (1 << 23) + 4099)):
+    # stale totals of the larger calls stay in the scratch of the smaller ones; tiles with block totals, then
+    # a second part of one tile and a bit
+    for seed, n in ((11, 300007), (12, 1234), (13, (1 << 23) + 4099), (14, 6144), (15, 6145), (16, 6 << 20),
+                    (17, (6 << 20) + 1), (18, (1 << 24) + 1027), (19, 777)):
         sizes = synthetic.stripe_sizes(seed, n)
         sizes[::7] = sizes[::7] % np.uint64(150)
         d_sizes = _gpu.to_dev(sizes)
@@ -50,7 +51,8 @@ def test_noalloc_matches_allocating_entry_point(lib, oracle, gpu):
 
 
 def test_noalloc_at_its_largest_batch(lib, gpu):
-    """2^26 messages use every tile word of the fixed scratch (65,536 tiles of 1,024).  Compared on
+    """2^26 messages are four parts, each of which uses every tile word of the fixed scratch (16,384
+    tiles of 1,024).  Compared on
     the device with the allocating entry point's output for the same batch (6.4 GB of rows each),
     and through what does not depend on the size: every message's stripes add up to its size."""
     assert lib.ofi_amd_gpu_init() == 0
@@ -78,20 +80,20 @@ def test_noalloc_at_its_largest_batch(lib, gpu):
 def test_noalloc_calls_leave_free_device_memory_where_it_was(lib, gpu):
     """What the entry point is for: after ofi_amd_gpu_init() (which records the scratch array's
     address on every GPU) a call takes no device memory -- the runtime's count of free bytes
-    (hipMemGetInfo) is the same before and after calls of several sizes, the larger ones through
-    the separate scan launch, on a stream that has never been used with the allocating entry
-    point (that one would allocate its per-stream scratch on such a stream)."""
+    (hipMemGetInfo) is the same before and after calls of several sizes in all three launch forms, on a
+    stream that has never been used with the allocating entry point (that one would allocate its
+    per-stream scratch on such a stream)."""
     assert lib.ofi_amd_gpu_init() == 0
     side = torch.cuda.Stream()
     stream = ctypes.c_void_p(side.cuda_stream)
-    big = (1 << 22) + 777
+    big = (6 << 20) + 777
     d_sizes = _gpu.to_dev(synthetic.stripe_sizes(21, big))
     d_state = dev_state(4, 131072, 64, (0, 0))
     d_num = torch.zeros(big, dtype=torch.int32, device="cuda")
     d_xf = torch.zeros(big * 12, dtype=torch.int64, device="cuda")
     call = lambda n: lib.ofi_amd_sched_batch_noalloc(d_state.data_ptr(), d_sizes.data_ptr(), n, 128, d_num.data_ptr(),
                                                      d_xf.data_ptr(), stream)
-    assert call(1000) == 0 and call(big) == 0              # code objects of every kernel are on the device now
+    assert call(1000) == 0 and call(300007) == 0 and call(big) == 0   # code objects of every kernel are on the device now
     torch.cuda.synchronize()
     free_before, _ = torch.cuda.mem_get_info()
     for n in (1, 513, 300007, big, 1234, 3_000_000):
