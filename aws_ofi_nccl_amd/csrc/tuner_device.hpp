@@ -287,6 +287,9 @@ __device__ __forceinline__ pt_t vsub(pt_t a, pt_t b) { return pt_t{ a.x - b.x, a
 __device__ __forceinline__ double vdot(pt_t a, pt_t b) { return a.x * b.x + a.y * b.y; }
 __device__ __forceinline__ double vcross(pt_t a, pt_t b) { return a.x * b.y - a.y * b.x; }
 
+/* ... where only the sign counts, and only when it is certain */
+__device__ __forceinline__ double vcross_sign(pt_t a, pt_t b) { return __builtin_fma(a.x, b.y, -(a.y * b.x)); }
+
 /* intersect, src/tuner/nccl_ofi_regions.cpp:77-109 */
 __device__ inline int intersect(pt_t x0, pt_t x1, pt_t y0, pt_t y1, double eps, pt_t *sect)
 {
@@ -513,7 +516,8 @@ inline region_set_t region_set(const region_tables_t &t, int platform, int coll,
 	return t.set[platform][shape][coll];
 }
 
-/* The nChannels override of the chosen region (:2135-2153), -1 when there is none. */
+/* The nChannels override of the chosen region (:2135-2153), -1 when there is none; only P6 has any. */
+__host__ __device__ inline bool platform_sets_channels(int platform) { return platform == OFI_AMD_PLATFORM_P6; }
 __device__ __forceinline__ int region_channels(int platform, uint64_t size, uint64_t ranks, uint64_t nodes,
 						int algorithm, int protocol)
 {

@@ -154,10 +154,11 @@ __global__ __launch_bounds__(256) void model_grid_kernel(grid_dims_t g,
 }
 
 constexpr int kMaxSetEdges = 64; /* of one (platform, shape, collective) set: one per lane */
-/* Wavefronts per workgroup of the region kernel: two in launches of more than kMostTiles tiles, whose workgroups
- * take as long to hand out as to work off (560 sizes x 38 node counts of four platforms 11.2 -> 10.8 us, 280 x 38 9.6
- * -> 9.0; four wavefronts 10.9), one in smaller ones, where two gain nothing. */
+/* Wavefronts per workgroup of the region kernel: two in launches of more than kPairedTiles tiles, whose workgroups
+ * take as long to hand out as to work off (560 sizes x 38 node counts of four platforms 9.5 -> 8.9 us, 280 x 38 7.3
+ * -> 7.1; four wavefronts 9.2 and 7.2), one in smaller ones, where two gain nothing. */
 constexpr uint32_t kMostRegionWaves = 2;
+constexpr uint64_t kPairedTiles = 6000;
 constexpr uint64_t kMostRuns = 65535; /* of one launch: gridDim.y */
 constexpr uint32_t kXcds = 8;         /* workgroup w of a launch runs on XCD w mod 8, each with its own L2 */
 static_assert(kMaxSetEdges <= 64, "one lane per edge of a set");
@@ -172,59 +173,50 @@ struct region_run_t {
 	int32_t platform;
 };
 
-/* What a whole tile knows about one edge of its polygon set */
+/* What a whole tile knows about one edge of its polygon set: which of the sides of edge_sides are the same, and
+ * certainly so, for every point of it, on which side its centre is, and whether a point of it may lie on the edge */
 struct tile_edge_t {
-	bool crossed;  /* the ray of every point of the tile crosses it, and certainly so (crossing_certain) */
-	bool by_point; /* some points' rays may cross it and some may not: each point looks for itself */
-	bool near;     /* a point of the tile may lie on it */
+	bool a_sure, b_sure, p_sure;
+	bool a_pos, b_pos, p_pos;
+	bool near;
 };
 
 /*
- * Edge e against the tile [lo.x, hi.x] x [lo.y, hi.y].  The sides of edge_sides are affine in the
- * point, so over the tile each lies between its values at the four corners: when those are all beyond
- * kTileSure on one side, every point's certain answer is the same.  The ends of most edges lie
- * outside the narrow fan of rays between a tile and the far point.
+ * Edge e against the tile of points with centre `mid` and half extents `half`.  The sides of edge_sides are
+ * affine in the point, so over the tile each stays within a reach, worked out from the extents, of its value at
+ * the centre: when all of that is beyond kTileSure on one side, every point's certain answer is the same.  The
+ * ends of most edges lie outside the narrow fan of rays between a tile and the far point.
  */
 constexpr double kTileSure = 1e-3; /* > kSure */
-__device__ __forceinline__ tile_edge_t tile_edge(const edge_t &e, pt_t lo, pt_t hi, pt_t far, double side_f)
+__device__ __forceinline__ tile_edge_t tile_edge(const edge_t &e, pt_t mid, pt_t half, pt_t far)
 {
-	const pt_t d = vsub(e.b, e.a), fa = vsub(e.a, far), fb = vsub(e.b, far);
-	bool a_pos = true, a_neg = true, b_pos = true, b_neg = true, p_pos = true, p_neg = true;
-	const double beside = kTileSure * (1.0 + fabs(d.x) + fabs(d.y));
-	bool left = true, right = true; /* the whole tile on one side of the edge's line, and not close to it */
-#pragma unroll
-	for (int k = 0; k < 4; k++) {
-		const pt_t c = { (k & 1) ? hi.x : lo.x, (k & 2) ? hi.y : lo.y };
-		const pt_t fc = vsub(c, far);
-		const double sa = vcross(fc, fa), sb = vcross(fc, fb), sp = vcross(vsub(c, e.a), d);
-		a_pos &= sa > kTileSure, a_neg &= sa < -kTileSure;
-		b_pos &= sb > kTileSure, b_neg &= sb < -kTileSure;
-		p_pos &= sp > kTileSure, p_neg &= sp < -kTileSure;
-		left &= sp > beside, right &= sp < -beside;
-	}
-	const bool f_pos = side_f > kTileSure, f_neg = side_f < -kTileSure;
-	const bool together = (a_pos && b_pos) || (a_neg && b_neg);
-	const bool apart = (a_pos && b_neg) || (a_neg && b_pos);
-	const bool between = (p_pos && f_neg) || (p_neg && f_pos);
-	const bool beyond = (p_pos && f_pos) || (p_neg && f_neg);
+	const pt_t d = vsub(e.b, e.a), fa = vsub(e.a, far), fb = vsub(e.b, far), fm = vsub(mid, far);
+	auto reach = [half](pt_t v) { return __builtin_fma(half.x, fabs(v.y), half.y * fabs(v.x)); };
+	const double sa = vcross_sign(fm, fa), sb = vcross_sign(fm, fb), sp = vcross_sign(vsub(mid, e.a), d), rp = reach(d);
 	tile_edge_t r;
-	r.crossed = apart && between;
-	r.by_point = !(together || (apart && (between || beyond)));
-	bool near = !(left || right); /* &= : no branches between the comparisons */
-	near &= fmin(e.a.x, e.b.x) <= hi.x + kTileSure;
-	near &= fmax(e.a.x, e.b.x) >= lo.x - kTileSure;
-	near &= fmin(e.a.y, e.b.y) <= hi.y + kTileSure;
-	near &= fmax(e.a.y, e.b.y) >= lo.y - kTileSure;
+	r.a_sure = fabs(sa) > reach(fa) + kTileSure, r.a_pos = sa > 0;
+	r.b_sure = fabs(sb) > reach(fb) + kTileSure, r.b_pos = sb > 0;
+	r.p_sure = fabs(sp) > rp + kTileSure, r.p_pos = sp > 0;
+	/* with the whole tile on one side of the edge's line, and not close to it, no point is near */
+	bool near = fabs(sp) <= rp + kTileSure * (1.0 + fabs(d.x) + fabs(d.y));
+	near &= fmin(e.a.x, e.b.x) <= mid.x + half.x + kTileSure; /* &= : no branches between the comparisons */
+	near &= fmax(e.a.x, e.b.x) >= mid.x - half.x - kTileSure;
+	near &= fmin(e.a.y, e.b.y) <= mid.y + half.y + kTileSure;
+	near &= fmax(e.a.y, e.b.y) >= mid.y - half.y - kTileSure;
 	r.near = near;
 	return r;
 }
 
+__device__ __forceinline__ uint64_t lane_word(uint64_t v, int lane)
+{
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+	return ((uint64_t)hi << 32) | lo;
+}
+
 __device__ __forceinline__ double lane_value(double v, int lane)
 {
-	const uint64_t bits = (uint64_t)__double_as_longlong(v);
-	const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, lane);
-	const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), lane);
-	return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+	return __longlong_as_double((long long)lane_word((uint64_t)__double_as_longlong(v), lane));
 }
 
 /* all lanes when m is not 0, else none */
@@ -233,33 +225,21 @@ __device__ __forceinline__ uint64_t every(uint64_t m)
 	return m != 0 ? ~0ull : 0ull;
 }
 
-/* The points of a wavefront against one edge, a bit per point: whether its ray crosses the edge, and whether
- * that is certain (crossing, crossing_certain). */
-struct point_edge_t {
-	uint64_t crossing, sure;
-};
-__device__ __forceinline__ point_edge_t point_edge(const edge_sides_t &s, uint64_t f_positive, uint64_t f_sure)
-{
-	const uint64_t apart = __ballot(s.side_a > 0) ^ __ballot(s.side_b > 0);
-	point_edge_t r;
-	r.crossing = apart & (__ballot(s.side_p > 0) ^ f_positive);
-	r.sure = __ballot(fabs(s.side_a) > kSure) & __ballot(fabs(s.side_b) > kSure) &
-		 (~apart | (__ballot(fabs(s.side_p) > kSure) & f_sure));
-	return r;
-}
-
 /*
  * One thread per point.  A wavefront works on a tile of neighbouring sizes and node
  * counts of one (collective, ranks per node) pair, because the polygon set depends on that pair
  * alone.  The launch is bound by arithmetic (chains of fp64 operations), so a wavefront first
  * works out, one edge per lane, what its whole tile has in common about each edge of the set
- * (tile_edge); the points then only look at the edges about which they differ -- those with an end in the
- * fan of rays from the tile to the far point, and those the tile touches -- read out of the
- * lanes that hold them.  A tile has one such edge at the median and 20 at the most; every edge for every
- * point, with quotients, took 40-42 us for 1.02 M points of four platforms (560 sizes, 38 node counts),
- * this takes 10.8, a part of it the handing out of 16,896 wavefronts (kMostRegionWaves), the rest the time of the
- * tiles with the most edges, which is why their turns count instructions (two edges a turn, for
- * shorter chains of dependent operations, was slower: 13.3 against then 12.0).  A grid of few points is the
+ * (tile_edge); the points then only look at what they differ about, read out of the lanes that hold it: the
+ * vertices in the fan of rays from the tile to the far point, one side each, and the edges whose line runs
+ * through the tile, three sides each.  More than half of a sweep's tiles lie apart from every polygon, the mean
+ * tile has 0.1 such vertices and 0.5 such edges, but those along a border that points at the far point have up
+ * to 14 and 19, and the launch lasts as long as they do, which is why their turns count instructions: 1.02 M points
+ * of four platforms (560 sizes, 38 node counts) 8.9-9.7 us by where the sizes lie, 10.9 with three sides of every edge with an end in
+ * the fan and the tile's four corners against each edge, 40-42 with every edge for every point and quotients;
+ * 4.6 without any polygon, the launch and the handing out of 16,896 wavefronts (kMostRegionWaves).  Measured and
+ * slower: the sides a tile knows left out one by one (branches on scalars: 12.4), two points a lane, half the
+ * wavefronts (11.6: the longest tile counts), two edges a turn.  A grid of few points is the
  * time of such a tile alone, and takes smaller ones (pick_tiling).
  *
  * In the output the ranks-per-node index runs fastest, so a wavefront's records lie 4 x
@@ -309,84 +289,115 @@ __global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(
 		/* lane e's edge; lanes beyond the set's edges take its last one and are masked out below */
 		const edge_t mine = edges[run.first_edge + min(lane, n_edges - 1u)];
 		const uint64_t nodes = g.nodes[ni];
-		const uint64_t size = g.sizes[si];
 		const pt_t at = { g.log2_sizes[si], g.log2_ranks[ni * g.n_ppn + run.pi] };
 		const double2 sx = t.size_span[ts], sy = t.rank_span[tn * g.n_ppn + run.pi];
 
-		const double eps = 1e-10;
-		const double mine_f = vcross(vsub(far_point, mine.a), vsub(mine.b, mine.a));
-		const double mine_reach = touch_reach(mine.a, mine.b);
-		const tile_edge_t te = tile_edge(mine, pt_t{ sx.x, sy.x }, pt_t{ sx.y, sy.y }, far_point, mine_f);
-		/* From here on conditions are masks of lanes in scalar registers -- lanes standing for edges, polygons
-		 * or points -- and the logic between them is scalar: no branch over lanes but the rare ones. */
-		const uint64_t all = edge_lanes(0, (int)n_edges);
-		const uint64_t crossed = __ballot(te.crossed) & all, by_point = __ballot(te.by_point) & all,
-			       near = __ballot(te.near) & all;
-		const uint64_t f_positive = __ballot(mine_f > 0), f_sure = __ballot(fabs(mine_f) > kSure);
 		/* The reference looks for a point on an edge first (result 0) and rejects by bounding
 		 * box second (result -1).  A point more than 1e-6 outside the box cannot be within
 		 * 1e-10 of an edge -- edges lie inside the box, and the foot of the perpendicular may
-		 * leave the segment by at most eps times its length -- so for such a point the second
+		 * leave the segment by at most eps times its length -- so for a tile of such points the second
 		 * answer is known without looking at the edges. */
 		const double margin = 1e-6;
 		const uint64_t apart_polys = __ballot(sx.x > box.y + margin) | __ballot(sx.y < box.x - margin) |
 					     __ballot(sy.x > box.w + margin) | __ballot(sy.y < box.z - margin);
 		const uint64_t whole_polys = __ballot(sx.x >= box.x) & __ballot(sx.y <= box.y) & __ballot(sy.x >= box.z) &
 					     __ballot(sy.y <= box.w);
-		const pt_t ray = vsub(far_point, at);
+		uint64_t todo = edge_lanes(0, (int)n_polys) & ~apart_polys;
 		uint64_t open = __ballot(live) & __ballot(nodes > 2); /* the points still without a region */
-		for (uint64_t todo = edge_lanes(0, (int)n_polys) & ~apart_polys; todo != 0 && open != 0; todo &= todo - 1) {
+
+		const double eps = 1e-10;
+		const double mine_f = vcross(vsub(far_point, mine.a), vsub(mine.b, mine.a));
+		const uint64_t mine_lanes = edge_lanes(pw.z - (int)run.first_edge, pw.w); /* of this lane's polygon */
+		const pt_t mid = { 0.5 * (sx.x + sx.y), 0.5 * (sy.x + sy.y) }, half = { 0.5 * (sx.y - sx.x), 0.5 * (sy.y - sy.x) };
+		const tile_edge_t te = tile_edge(mine, mid, half, far_point);
+		/* points with a |side_p| up to this may lie on the edge */
+		const double mine_reach = te.near ? touch_reach(mine.a, mine.b) : -1.0;
+		/* From here on conditions are masks of lanes in scalar registers -- lanes standing for edges, polygons
+		 * or points -- and the logic between them is scalar: no branch over lanes but the rare ones. */
+		const uint64_t all = edge_lanes(0, (int)n_edges);
+		const uint64_t a_sure = __ballot(te.a_sure), b_sure = __ballot(te.b_sure);
+		const uint64_t a_pos = __ballot(te.a_pos), ends_apart = a_pos ^ __ballot(te.b_pos);
+		const uint64_t f_pos = __ballot(mine_f > 0), f_sure = __ballot(fabs(mine_f) > kSure);
+		/* Edges between whose line's sides every point and the far point certainly lie, or certainly do not: a ray
+		 * crosses the former (`between`) when their ends lie apart, the latter never.  For the points to look
+		 * at are left the ends in the fan of rays of edges between, and the edges whose line runs through the tile. */
+		const uint64_t near = __ballot(te.near), line_sure = __ballot(te.p_sure) & f_sure & ~near;
+		const uint64_t between = all & line_sure & (__ballot(te.p_pos) ^ f_pos);
+		const uint64_t through = all & (near | ~(line_sure | (a_sure & b_sure & ~ends_apart)));
+		for (; todo != 0 && open != 0; todo &= todo - 1) {
 			const int i = __builtin_ctzll(todo);
-			uint64_t asks = open, in_box = ~0ull;
-			if (!((whole_polys >> i) & 1u)) {
-				const double x0 = lane_value(box.x, i), x1 = lane_value(box.y, i);
-				const double y0 = lane_value(box.z, i), y1 = lane_value(box.w, i);
-				asks &= __ballot(at.x >= x0 - margin) & __ballot(at.x <= x1 + margin) & __ballot(at.y >= y0 - margin) &
-					__ballot(at.y <= y1 + margin);
-				in_box = __ballot(at.x >= x0) & __ballot(at.x <= x1) & __ballot(at.y >= y0) & __ballot(at.y <= y1);
-				if (asks == 0) {
-					continue;
-				}
+			const uint64_t of_poly = lane_word(mine_lanes, i);
+			/* The rays' crossings with the edges between, counted by vertex: an edge counts its first vertex when
+			 * that lies on the positive side of the ray, and its second likewise, so that a vertex (bit e: the
+			 * first of edge e) counts for the edges that meet in it, for neither when both are between. */
+			const uint64_t c = between & of_poly;
+			const uint64_t c_before = ((c << 1) & of_poly) | (((c >> (63 - __builtin_clzll(of_poly))) & 1u) << __builtin_ctzll(of_poly));
+			const uint64_t counts = c ^ c_before;
+			uint64_t odd = every((uint64_t)(__popcll(counts & a_sure & a_pos) & 1)); /* points with an odd number of crossings */
+			uint64_t vertices = (c | c_before) & ~a_sure;
+			uint64_t left = through & of_poly;
+			if ((odd | vertices | left) == 0) {
+				continue;
 			}
-			const uint64_t of_poly = edge_lanes(__builtin_amdgcn_readlane(pw.z, i) - (int)run.first_edge,
-							    __builtin_amdgcn_readlane(pw.w, i));
-			uint64_t odd = (__popcll(crossed & of_poly) & 1) ? ~0ull : 0ull; /* points with an odd number of crossings */
-			uint64_t touching = 0;
-			for (uint64_t left = (by_point | near) & of_poly; left != 0; left &= left - 1) {
+			uint64_t in_box = open;
+			if (!((whole_polys >> i) & 1u)) {
+				in_box &= __ballot(at.x >= lane_value(box.x, i)) & __ballot(at.x <= lane_value(box.y, i)) &
+					  __ballot(at.y >= lane_value(box.z, i)) & __ballot(at.y <= lane_value(box.w, i));
+			}
+			const pt_t ray = vsub(far_point, at);
+			/* a far point close to an edge's line (no polygon has such an edge) leaves it to the exact code */
+			uint64_t unsure = every(left & ~f_sure), touching = 0;
+			for (; vertices != 0; vertices &= vertices - 1) {
+				const int e = __builtin_ctzll(vertices);
+				const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
+				const double side = vcross_sign(vsub(a, at), ray);
+				unsure |= __ballot(fabs(side) <= kSure);
+				odd ^= __ballot(side > 0) & every((counts >> e) & 1u);
+			}
+			for (; left != 0; left &= left - 1) {
 				const int e = __builtin_ctzll(left);
-				const uint64_t bit = left & -left;
 				const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
 				const pt_t b = { lane_value(mine.b.x, e), lane_value(mine.b.y, e) };
-				const edge_sides_t s = edge_sides(at, ray, a, b);
-				uint64_t unsure = 0, reached = 0;
-				if ((by_point & bit) != 0) {
-					const point_edge_t pe = point_edge(s, every(f_positive & bit), every(f_sure & bit));
-					unsure = asks & ~pe.sure;
-					odd ^= pe.crossing & ~unsure;
-				}
-				if ((near & bit) != 0) {
-					reached = asks & __ballot(fabs(s.side_p) <= lane_value(mine_reach, e));
-				}
-				if ((unsure | reached) != 0) {
-					bool c = false, t = false;
-					if ((unsure >> lane) & 1u) {
-						c = intersects(at, far_point, a, b, eps);
-					}
+				const pt_t pa = vsub(a, at), pb = vsub(b, at);
+				const edge_sides_t s = { vcross_sign(pa, ray), vcross_sign(pb, ray), vcross_sign(pb, pa) };
+				const uint64_t apart = __ballot(s.side_a > 0) ^ __ballot(s.side_b > 0);
+				unsure |= __ballot(fabs(s.side_a) <= kSure) | __ballot(fabs(s.side_b) <= kSure) |
+					  (apart & __ballot(fabs(s.side_p) <= kSure));
+				odd ^= apart & (__ballot(s.side_p > 0) ^ every((f_pos >> e) & 1u));
+				const uint64_t reached = open & __ballot(fabs(s.side_p) <= lane_value(mine_reach, e));
+				if (reached != 0) {
+					bool t = false;
 					if ((reached >> lane) & 1u) {
 						t = touches_edge(at, a, b, s, eps);
 					}
-					odd ^= __ballot(c);
 					touching |= __ballot(t);
 				}
 			}
-			const uint64_t hit = asks & (touching | (odd & in_box));
+			unsure &= in_box & ~touching;
+			if (unsure != 0) {
+				/* for these points, whose ray or themselves come close to a vertex or an edge, the exact code on
+				 * the edges that the tile does not know about */
+				uint64_t exact = every((uint64_t)(__popcll(c & a_sure & b_sure & ends_apart) & 1));
+				for (uint64_t ask = (c & ~(a_sure & b_sure)) | (through & of_poly); ask != 0; ask &= ask - 1) {
+					const int e = __builtin_ctzll(ask);
+					const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
+					const pt_t b = { lane_value(mine.b.x, e), lane_value(mine.b.y, e) };
+					bool crosses = false;
+					if ((unsure >> lane) & 1u) {
+						crosses = intersects(at, far_point, a, b, eps);
+					}
+					exact ^= __ballot(crosses);
+				}
+				odd = (odd & ~unsure) | (exact & unsure);
+			}
+			const uint64_t hit = open & (touching | (odd & in_box));
 			const int a = __builtin_amdgcn_readlane(pw.x, i), pr = __builtin_amdgcn_readlane(pw.y, i);
 			algorithm = (hit >> lane) & 1u ? a : algorithm;
 			protocol = (hit >> lane) & 1u ? pr : protocol;
 			open &= ~hit;
 		}
-		if (algorithm >= 0) {
-			nchannels = region_channels(run.platform, size, nodes * run.ppn, nodes, algorithm, protocol);
+		if (algorithm >= 0 && platform_sets_channels(run.platform)) {
+			nchannels = region_channels(run.platform, g.sizes[si], nodes * run.ppn, nodes, algorithm, protocol);
 		}
 	}
 	if (!live) {
@@ -503,17 +514,18 @@ void tile_shifts(uint32_t n_sizes, uint32_t n_nodes, uint32_t shift_n[kTilings],
 }
 
 /*
- * The smallest tiles that make at most kMostTiles, which the chip holds at once.  Times in us with tiles of 64 / 16 /
- * 8 / 4 points and, in brackets, the tiles these make (3 collectives, 4 values of ranks per node):
- *   35 sizes, 11 node counts, 4 platforms      14.2 / 10.2 / 8.4 / 7.4  [ 480, 1296, 2592, 5184]
- *   70 sizes, 11 node counts, 2 platforms      14.4 /  8.2 / 7.0 / 6.2  [ 432, 1296, 2592, 5040]
- *   140 sizes, 27 node counts, 1 platform       8.1 /  6.2 / 5.7 / 5.9  [ 840, 2940, 5880, 11760]
- *   35 sizes, 38 node counts, 4 platforms      11.8 /  8.7 / 9.4 / 9.8  [1200, 4320, 8208, 16416]
- *   140 sizes, 11 node counts, 4 platforms     10.6 /  8.4 / 7.8 / 9.7  [1728, 5040, 10080, 20160]
- *   160 sizes, 27 node counts, 3 platforms      5.3 /  6.5 / 7.1 / 13   [2880, 10080, 20160, 40320]
- *   140 sizes, 38 node counts, 4 platforms      9.0 / 10.9 / 12.7 / 23  [4320, 16800, 31920, 63840]
+ * The smallest tiles that make at most kMostTiles: beyond, handing out the wavefronts costs more than their shorter
+ * turns save.  Times in us with tiles of 64 / 16 / 8 / 4 points and, in brackets, the tiles these make (3
+ * collectives, 4 values of ranks per node):
+ *   35 sizes, 11 node counts, 4 platforms      16.0 / 8.9 / 7.0 / 5.6   [ 480, 1296, 2592, 5184]
+ *   70 sizes, 11 node counts, 2 platforms      13.7 / 7.0 / 5.3 / 4.8   [ 432, 1296, 2592, 5040]
+ *   140 sizes, 27 node counts, 1 platform       7.7 / 6.1 / 5.3 / 4.8   [ 840, 2940, 5880, 11760]
+ *   35 sizes, 38 node counts, 4 platforms      11.2 / 7.9 / 6.8 / 7.1   [1200, 4320, 8208, 16416]
+ *   140 sizes, 11 node counts, 4 platforms     10.1 / 6.8 / 6.3 / 7.4   [1728, 5040, 10080, 20160]
+ *   160 sizes, 27 node counts, 3 platforms      7.8 / 6.6 / 7.7 / 12    [2880, 10080, 20160, 40320]
+ *   140 sizes, 38 node counts, 4 platforms      7.9 / 8.0 / 10.4 / 18   [4320, 16800, 31920, 63840]
  */
-constexpr uint64_t kMostTiles = 6000;
+constexpr uint64_t kMostTiles = 12000;
 uint64_t tiling_tiles(const tiling_t &t)
 {
 	return (uint64_t)t.tiles_n * t.tiles_s;
@@ -963,7 +975,7 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 		plan->h_platforms.clear();
 		return -ENOMEM;
 	}
-	const uint32_t waves = n_runs * tiling_tiles(tiling) > kMostTiles ? kMostRegionWaves : 1;
+	const uint32_t waves = n_runs * tiling_tiles(tiling) > kPairedTiles ? kMostRegionWaves : 1;
 	const uint32_t grid_x = (uint32_t)((groups + waves - 1) / waves * kXcds);
 	for (uint64_t at = 0; at < n_runs; at += kMostRuns) {
 		const uint32_t here = (uint32_t)(n_runs - at < kMostRuns ? n_runs - at : kMostRuns);

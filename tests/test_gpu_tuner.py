@@ -276,6 +276,24 @@ def test_region_tiles_on_short_axes(lib, oracle, gpu, n_sizes, n_nodes):
     lib.ofi_amd_tuner_plan_destroy(plan)
 
 
+@pytest.mark.parametrize("n_sizes,n_nodes,first", [(1500, 24, 3), (700, 9, 4), (300, 41, 3)])
+def test_region_tiles_along_borders(lib, oracle, gpu, n_sizes, n_nodes, first):
+    """Sizes so close together that tiles lie along the polygons' borders, with many vertices and edges in the fan of
+    rays from a tile to the far point and rays that pass within the certain answers' margin of a vertex; in tiles of 64
+    points and, one platform at a time, in smaller ones."""
+    rng = np.random.default_rng(n_sizes)
+    sizes = np.unique((2.0 ** rng.uniform(12, 36, n_sizes)).astype(np.uint64))
+    nodes = np.unique(np.round(first * 2.0 ** np.linspace(0, 8, n_nodes)).astype(np.uint64))
+    colls, ppn = np.array([4, 2, 3], dtype=np.int32), np.array([8, 1, 2], dtype=np.uint32)
+    plan = make_plan(lib, colls, sizes, nodes, ppn, np.array([1], dtype=np.int32))
+    want = oracle_region_grid(oracle, [0, 1, 2, 3], colls, sizes, nodes, ppn)
+    for platforms in ([0, 1, 2, 3], [1], [3]):
+        got = run_region(lib, plan, platforms, (len(platforms), 3, len(sizes), len(nodes), 3))
+        mism = np.argwhere((got != want[platforms]).any(axis=-1))
+        assert len(mism) == 0, (platforms, mism[:10])
+    lib.ofi_amd_tuner_plan_destroy(plan)
+
+
 def test_region_grid_on_changing_platform_lists(lib, oracle, gpu):
     """One plan, platform lists that grow, shrink and change in place: the launch order the plan keeps
     for a list (which entry, chunk and ranks-per-node value each workgroup takes) is rebuilt whenever
