@@ -76,7 +76,7 @@ inline void apply_ack(ofi_amd_gin_comm_t *c, uint32_t wire_rx_consumed)
  * size is a power of two (the defaults: 4 rails, 128 KiB), so the modular steps are masks.
  */
 template <bool POW2>
-inline int derive(ofi_amd_gin_comm_t *c, const ofi_amd_gin_mr_t *mrs, uint32_t n_mrs,
+__attribute__((always_inline)) inline int derive(ofi_amd_gin_comm_t *c, const ofi_amd_gin_mr_t *mrs, uint32_t n_mrs,
 		  const ofi_amd_gin_desc_t *d, ofi_amd_gin_wire_t *out)
 {
 	const uint32_t sop = d->signal_op;

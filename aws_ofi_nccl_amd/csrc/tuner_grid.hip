@@ -235,12 +235,12 @@ __device__ __forceinline__ uint64_t every(uint64_t m)
  * through the tile, three sides each.  More than half of a sweep's tiles lie apart from every polygon, the mean
  * tile has 0.1 such vertices and 0.5 such edges, but those along a border that points at the far point have up
  * to 14 and 19, and the launch lasts as long as they do, which is why their turns count instructions: 1.02 M points
- * of four platforms (560 sizes, 38 node counts) 8.9-9.7 us by where the sizes lie, 10.9 with three sides of every edge with an end in
- * the fan and the tile's four corners against each edge, 40-42 with every edge for every point and quotients;
- * 4.6 without any polygon, the launch and the handing out of 16,896 wavefronts (kMostRegionWaves).  Measured and
- * slower: the sides a tile knows left out one by one (branches on scalars: 12.4), two points a lane, half the
- * wavefronts (11.6: the longest tile counts), two edges a turn.  A grid of few points is the
- * time of such a tile alone, and takes smaller ones (pick_tiling).
+ * of four platforms (560 sizes, 38 node counts) take 8.9-9.7 us by where the sizes lie, 10.9 with three sides of
+ * every edge with an end in the fan and the tile's four corners against each edge, 40-42 with every edge for every
+ * point and quotients; 4.6 without any polygon, the launch and the handing out of 16,896 wavefronts
+ * (kMostRegionWaves).  Measured and slower: the sides a tile knows left out one by one (branches on scalars: 12.4),
+ * two points a lane and half the wavefronts (11.6: the longest tile counts), two edges a turn.  A grid of few points
+ * is the time of such a tile alone, and takes smaller ones (pick_tiling).
  *
  * In the output the ranks-per-node index runs fastest, so a wavefront's records lie 4 x
  * n_ppn bytes apart and the records between them belong to the same tile's other

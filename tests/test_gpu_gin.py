@@ -213,6 +213,68 @@ def test_proxy_stops_at_a_descriptor_with_a_handle_outside_the_table(lib, gpu):
         lib.ofi_amd_gin_rings_destroy(rings)
 
 
+@pytest.mark.parametrize("nctx,ops,threads,shift,bad", [(140, 15, 2, 0, None), (140, 16, 2, 0, 3), (130, 17, 2, 8, None),
+                                                        (70, 33, 2, 0, 32), (20, 250, 3, 0, 128), (3, 1, 4, 0, None),
+                                                        (2, 129, 1, 0, 127), (140, 16, 2, 8, 15)])
+def test_proxy_groups_and_bursts(lib, oracle, gpu, nctx, ops, threads, shift, bad):
+    """Descriptors derived by groups of 16 and bursts of 128 (rings of 256), with remainders, gets among the puts, and
+    an output array on a 16-byte boundary (records of several threads go past the caches) or 8 bytes off one: record by
+    record the oracle's.  `bad`: that descriptor of every context has a handle outside the table; the records before it
+    are there, its own is zero, the ones behind it are not touched and the communicator is where the last good one left it."""
+    rng = np.random.default_rng(nctx * 1000 + ops)
+    table = np.zeros((nctx, ops, 8), dtype=np.uint64)
+    table[:, :, 0] = rng.integers(0, 1 << 30, (nctx, ops))
+    table[:, :, 1] = rng.integers(0, 1 << 30, (nctx, ops))
+    table[:, :, 2] = (2 ** rng.uniform(0, 21, (nctx, ops))).astype(np.uint64)
+    table[:, :, 2][rng.random((nctx, ops)) < 0.05] = 0                       # signal only, or nothing at all
+    sop = (rng.random((nctx, ops)) < 0.2).astype(np.uint64)
+    get = (rng.random((nctx, ops)) < 0.1) & (table[:, :, 2] > 0)
+    sop[get] = 0
+    table[:, :, 3] = 8 * rng.integers(0, 16, (nctx, ops))
+    table[:, :, 5] = np.uint64(1) | (sop << np.uint64(32))
+    table[:, :, 6] = rng.integers(0, 2, (nctx, ops))
+    table[:, :, 7] = np.where(get, np.uint64(2 | (0xFFFF << 32) | (3 << 48)),
+                              np.uint64(1 << 16) | np.where(sop > 0, np.uint64((2 << 32) | (2 << 48)),
+                                                            np.uint64((0xFFFF << 32) | (1 << 48))))
+    if bad is not None:
+        table[:, bad, 2] = 4096
+        table[:, bad, 5] = 1
+        table[:, bad, 7] = 7 | (1 << 16) | (0xFFFF << 32) | (1 << 48)
+    d_table = _gpu.to_dev(table)
+    rings = make_rings(lib, nctx, 256)
+    comms = (m.GinComm * nctx)()
+    for c in range(nctx):
+        assert lib.ofi_amd_gin_comm_init(ctypes.byref(comms[c]), c, 4, 131072, 64, 1) == 0
+    pmrs, omrs = _oracle.default_mrs(m.GinMr), _oracle.default_mrs()
+    raw = np.full(nctx * ops * 28 + 8, 0x5A5A5A5A5A5A5A5A, dtype=np.uint64)
+    lead = ((-raw.ctypes.data) % 16 + shift) // 8
+    assert lib.ofi_amd_gin_produce_table(rings, d_table.data_ptr(), ops, 1, 0, _gpu.stream()) == 0
+    if ops <= 256:
+        _gpu.sync()
+    stats = m.GinProxyStats()
+    rc = lib.ofi_amd_gin_proxy_drain_mt(rings, ops, 2, None, ctypes.cast(comms, ctypes.c_void_p),
+                                        ctypes.cast(pmrs, ctypes.c_void_p), 3, raw.ctypes.data + 8 * lead, 5000, threads,
+                                        ctypes.byref(stats))
+    _gpu.sync()
+    assert rc == (0 if bad is None else -errno.EINVAL)
+    good = ops if bad is None else bad
+    assert (raw[:lead] == 0x5A5A5A5A5A5A5A5A).all() and (raw[lead + nctx * ops * 28:] == 0x5A5A5A5A5A5A5A5A).all()
+    wires = raw[lead:lead + nctx * ops * 28].reshape(nctx, ops, 28)
+    for c in range(nctx if bad is None else 1):           # a thread ends with its first context that has a bad one
+        oc = _oracle.GinComm()
+        oracle.oracle_gin_comm_init(ctypes.byref(oc), c, 4, 131072, 64, 1)
+        for i in range(good):
+            d = _oracle.GinDesc.from_buffer_copy(table[c, i].tobytes())
+            w = _oracle.GinWire()
+            fn = oracle.oracle_gin_iget if d.kind == 3 else oracle.oracle_gin_iput_signal
+            assert fn(ctypes.byref(oc), omrs, ctypes.byref(d), ctypes.byref(w)) == 0
+            assert bytes(w) == wires[c, i].tobytes(), (c, i)
+        if bad is not None:
+            assert (wires[c, bad] == 0).all() and (wires[c, bad + 1:] == 0x5A5A5A5A5A5A5A5A).all()
+        assert bytes(oc) == bytes(comms[c]), c
+    lib.ofi_amd_gin_rings_destroy(rings)
+
+
 def test_proxy_thread_count_does_not_change_the_result(lib, oracle, gpu):
     """Several proxy threads, each owning a range of contexts: wire records, per-context comm
     state and the checksum equal the single-thread run (and so the oracle's)."""
