@@ -35,6 +35,40 @@ def sizes_for_test(rng, n):
     return out
 
 
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 15, 16, 17, 63, 64, 65, 255, 257, 300, 1025])
+def test_query_batches_around_the_line_size(lib, oracle, gpu, n):
+    """Eight answers make a line: batches with every kind of remainder, of questions of all three kinds side by side,
+    answered as the oracle answers them one by one, nothing written behind the last one."""
+    rng = np.random.default_rng(n)
+    a, p, ch, out = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_uint64()
+    arr, want = (m.TunerQuery * n)(), []
+    for i in range(n):
+        size, plat, coll = int(2 ** rng.uniform(0, 37)), int(rng.integers(0, 4)), int(rng.choice([4, 2, 3, 2147483647]))
+        nodes = int(rng.choice([3, 4, 8, 16, 100]))
+        ranks = nodes * int(rng.choice([1, 2, 8]))
+        mask, pipe, kind = int(rng.integers(0, ALL + 1)) | 1 << 31, int(rng.integers(1, 1000000)), (i + n) % 3
+        algo, proto = (0, 1) if i % 2 else (6, 2)
+        arr[i] = m.TunerQuery(plat, kind, coll, pipe, 8 + i % 3, 3, algo, proto, mask, 77, size, ranks, nodes)
+        a.value = p.value = ch.value = -1
+        out.value = 0
+        if kind == 0:
+            oracle.oracle_region_decide_masked(plat, coll, size, ranks, nodes, mask, ctypes.byref(a), ctypes.byref(p),
+                                               ctypes.byref(ch))
+        elif kind == 1 and plat < 2:
+            oracle.oracle_model_decide_v2(plat, coll, pipe, size, ranks, nodes, 8 + i % 3, 3, (mask >> 17) & 1,
+                                          ctypes.byref(a), ctypes.byref(p))
+        elif kind == 2 and not oracle.oracle_region_chunk_size(plat, coll, size, algo, proto, ranks, nodes, ctypes.byref(out)):
+            out.value = 0
+        want.append((a.value, p.value, ch.value, 0, out.value))
+    raw = np.full(16 * (n + 1), 0x5A, dtype=np.uint8)
+    for _ in range(2):
+        assert lib.ofi_amd_tuner_query(arr, n, raw.ctypes.data) == 0
+        ans = (m.TunerAnswer * n).from_buffer_copy(raw[:16 * n].tobytes())
+        got = [(x.algo, x.proto, x.nchannels, x.pad, x.chunk_size) for x in ans]
+        assert [(i, got[i], want[i]) for i in range(n) if got[i] != want[i]] == []
+        assert (raw[16 * n:] == 0x5A).all()
+
+
 def test_query_batch_matches_oracle(lib, oracle, gpu):
     rng = np.random.default_rng(11)
     qs, want = [], []
