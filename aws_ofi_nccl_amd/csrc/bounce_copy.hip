@@ -40,9 +40,9 @@
  * bytes, one per lane, so that nothing outside [dst, dst+len) is written and the
  * last, partial unit is written by one instruction.
  *
- * Flush: the wave waits until its own stores have left the CU (they are
- * write-through to the L2 of its XCD), then lane 0 re-reads the first 4 bytes
- * of the destination from that L2 and writes them to d_flush[i].  No wider
+ * Flush: behind its stores (they are write-through to the L2 of the XCD) the wave,
+ * or the last one of its workgroup for all of them, re-reads the first 4 bytes
+ * of the destination through that L2 and writes them to d_flush[i].  No wider
  * fence is used: on a multi-XCD part a device-scope release per buffer would
  * write back the whole L2 each time; device-wide visibility of the copied
  * bytes comes with the end of the kernel, as for any other kernel output.
@@ -67,13 +67,12 @@ struct __attribute__((packed, aligned(4))) dword_aligned_u32x4 {
 
 /* Buffers (= wavefronts) per workgroup and consecutive workgroups that share an XCD, swept over
  * thousands of launches in a row on 65,536 buffers.  Bounce copy: 8 wavefronts per workgroup with
- * runs of 4 workgroups (32 buffers) per XCD was the fastest (91.1 us per launch; 4 x 8: 91.8,
- * 2 x 16: 92.5, 16 x 2: 92.6, 8 x 8: 91.7).  The eager copy, whose sources are rx buffers in
+ * runs of 32 buffers per XCD was the fastest (91.1 us per launch; 4 wavefronts: 91.8,
+ * 2: 92.5, 16: 92.6; runs of 64 buffers 91.7).  The eager copy, whose sources are rx buffers in
  * arrival order, prefers single-wavefront workgroups (1 x 32: 97.8 us, 4 x 8: 98.4, 8 x 4: 101.6,
  * 16 x 2: 108.6), and so does the table copy (1: 419.9 us per GiB, 4: 439.5, 8: 430.3). */
-constexpr int kWavesPerBlock = 8;
-constexpr int kBlock = 64 * kWavesPerBlock;
-constexpr uint32_t kGroup = 4;
+constexpr int kBounceWaves = 8;
+constexpr uint32_t kBounceRun = 32;
 constexpr int kEagerWaves = 1;
 constexpr uint32_t kEagerGroup = 32;
 constexpr int kTableWaves = 1;
@@ -87,7 +86,8 @@ __device__ __forceinline__ u32x4 load16_dword_aligned(const uint8_t *p)
 }
 
 /*
- * Every access to a destination carries the same cache policy, the streaming one: the 16-byte
+ * Every access to a destination carries the same cache policy, the streaming one, but in batches that fit the L2s
+ * (kKeepBytes): the 16-byte
  * stores of the rows, the single head and tail bytes and the read-back of the flush.  With the
  * rows streaming and the tail bytes and the read-back as ordinary accesses, the same batch
  * launched over and over on the same buffers slowed down by 6 % within 2,000 launches (91 ->
@@ -103,9 +103,10 @@ __device__ __forceinline__ void store_byte_streaming(uint8_t *p, uint8_t v)
 /*
  * One trip: R rows from s (4-byte aligned; the data starts `shift` bytes in) to d (16-byte
  * aligned).  nvec = 16-byte words left, 64*(R-1) < nvec <= 64*R unless FULL, where all R rows
- * are complete.  SHIFTED = false: shift is 0 and the source words are used as they are.
+ * are complete.  SHIFTED = false: shift is 0 and the source words are used as they are.  KEEP: the
+ * first row is stored by ordinary stores, for the read-back that follows (kKeepBytes).
  */
-template <int R, bool SHIFTED, bool FULL>
+template <int R, bool SHIFTED, bool FULL, bool KEEP>
 __device__ __forceinline__ void copy_rows(const uint8_t *__restrict__ s, uint8_t *__restrict__ d,
 					  uint32_t nvec, uint32_t shift, uint32_t lane)
 {
@@ -149,50 +150,97 @@ __device__ __forceinline__ void copy_rows(const uint8_t *__restrict__ s, uint8_t
 			o.z = __builtin_amdgcn_alignbyte(v[k].w, v[k].z, shift);
 			o.w = __builtin_amdgcn_alignbyte(x[k], v[k].w, shift);
 		}
-		__builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(d + ((uint64_t)j << 4)));
+		u32x4 *to = reinterpret_cast<u32x4 *>(d + ((uint64_t)j << 4));
+		if (KEEP && k == 0) {
+			*to = o;
+		} else {
+			__builtin_nontemporal_store(o, to);
+		}
 	}
 }
 
-template <bool SHIFTED>
+template <bool SHIFTED, bool KEEP>
 __device__ __forceinline__ void copy_words(const uint8_t *__restrict__ s, uint8_t *__restrict__ d,
 					   uint32_t nvec, uint32_t shift, uint32_t lane)
 {
 	while (nvec > kTripVec) { /* buffers beyond 8 KiB: whole trips first */
-		copy_rows<kRows, SHIFTED, true>(s, d, kTripVec, shift, lane);
+		copy_rows<kRows, SHIFTED, true, KEEP>(s, d, kTripVec, shift, lane);
 		s += (uint64_t)kTripVec << 4;
 		d += (uint64_t)kTripVec << 4;
 		nvec -= kTripVec;
 	}
 	switch ((nvec + 63u) >> 6) { /* wave-uniform */
-	case 1: copy_rows<1, SHIFTED, false>(s, d, nvec, shift, lane); break;
-	case 2: copy_rows<2, SHIFTED, false>(s, d, nvec, shift, lane); break;
-	case 3: copy_rows<3, SHIFTED, false>(s, d, nvec, shift, lane); break;
-	case 4: copy_rows<4, SHIFTED, false>(s, d, nvec, shift, lane); break;
-	case 5: copy_rows<5, SHIFTED, false>(s, d, nvec, shift, lane); break;
-	case 6: copy_rows<6, SHIFTED, false>(s, d, nvec, shift, lane); break;
-	case 7: copy_rows<7, SHIFTED, false>(s, d, nvec, shift, lane); break;
-	case 8: copy_rows<8, SHIFTED, false>(s, d, nvec, shift, lane); break;
+	case 1: copy_rows<1, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
+	case 2: copy_rows<2, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
+	case 3: copy_rows<3, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
+	case 4: copy_rows<4, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
+	case 5: copy_rows<5, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
+	case 6: copy_rows<6, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
+	case 7: copy_rows<7, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
+	case 8: copy_rows<8, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
 	default: break; /* nvec == 0 */
 	}
 }
 
-__global__ __launch_bounds__(kBlock) void bounce_scatter_kernel(
+/*
+ * The flush words of a workgroup's buffers, streamed ones: the wavefront whose copy is done last reads all of them back, in one
+ * instruction, so that the others' places are free for the next buffers meanwhile -- a read of a line that has just
+ * been written takes longer than the copy of a short buffer.  Every wavefront says where its word is and then
+ * adds itself to `arrived` behind a workgroup fence, so the last one's loads follow all of the stores.
+ * 20,000 buffers of up to 4 KiB 17.9 -> 17.0 us, 65,536 of up to 8 KiB launched over and over 88.3 -> 82.2.
+ */
+template <int WAVES> struct read_backs_t {
+	uint64_t at[WAVES]; /* 0: none */
+	uint32_t arrived;
+};
+
+template <int WAVES> __device__ __forceinline__ void begin_read_backs(read_backs_t<WAVES> &r)
+{
+	if (threadIdx.x == 0) {
+		r.arrived = 0;
+	}
+	__syncthreads();
+}
+
+/* By a wavefront behind its copy; true in the last of `here`, with everyone's entries in view. */
+template <int WAVES>
+__device__ __forceinline__ bool arrive(read_backs_t<WAVES> &r, uint32_t wave, uint32_t lane, const uint8_t *d, uint32_t here)
+{
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+	uint32_t before = 0;
+	if (lane == 0) {
+		r.at[wave] = (uint64_t)reinterpret_cast<uintptr_t>(d);
+		before = __hip_atomic_fetch_add(&r.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+	}
+	before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+	return before == here - 1u;
+}
+
+template <int WAVES, bool KEEP>
+__global__ __launch_bounds__(64 * WAVES) void bounce_scatter_kernel(
 	const uint8_t *__restrict__ src, uint64_t src_bytes, uint8_t *__restrict__ arena, uint64_t arena_bytes,
 	const uint64_t *__restrict__ src_off, const uint64_t *__restrict__ dst_off,
 	const uint32_t *__restrict__ len, uint32_t n, uint32_t *__restrict__ flush,
 	uint32_t *__restrict__ err)
 {
+	__shared__ read_backs_t<WAVES> back;
+	constexpr uint32_t kGroup = kBounceRun / WAVES;
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	/* Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Runs of kGroup
-	 * consecutive workgroups' worth of buffers go to one XCD, so that neighbouring buffers
+	const bool together = !KEEP && flush != nullptr;
+	if (together) {
+		begin_read_backs(back);
+	}
+	/* Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Runs of kBounceRun
+	 * consecutive buffers go to one XCD, so that neighbouring buffers
 	 * -- which share a cache line of the packed source at their boundary -- mostly meet in
 	 * the same L2, while every XCD still sees an even sample of the whole batch whatever
 	 * order the lengths come in. */
 	const uint32_t xcd = blockIdx.x % kXcds;
 	const uint32_t turn = blockIdx.x / kXcds;
 	const uint32_t wg = ((turn / kGroup) * kXcds + xcd) * kGroup + turn % kGroup;
-	const uint32_t buf = wg * kWavesPerBlock + wave;
+	const uint32_t first = wg * WAVES, buf = first + wave;
 	if (buf >= n) {
 		return;
 	}
@@ -203,18 +251,16 @@ __global__ __launch_bounds__(kBlock) void bounce_scatter_kernel(
 	/* precondition check: skip (and report) instead of reading or writing out of range; the
 	 * read-back takes four bytes at the destination whatever the length */
 	const uint64_t need = (flush != nullptr && bytes < 4u) ? 4u : bytes;
-	if ((doff & 63u) != 0 || doff > arena_bytes || need > arena_bytes - doff || soff > src_bytes ||
-	    bytes > src_bytes - soff) {
-		if (lane == 0) {
-			atomicOr(err, ofi_amd::ASYNC_ERR_BOUNCE_RANGE);
-		}
-		return;
+	const bool in_range = (doff & 63u) == 0 && doff <= arena_bytes && need <= arena_bytes - doff && soff <= src_bytes &&
+			      bytes <= src_bytes - soff;
+	if (!in_range && lane == 0) {
+		atomicOr(err, ofi_amd::ASYNC_ERR_BOUNCE_RANGE);
 	}
 
 	const uint8_t *s = src + soff;
 	uint8_t *d = arena + doff;
 
-	if (bytes != 0) {
+	if (in_range && bytes != 0) {
 		/* whole 64-byte units as 16-byte words, the rest (up to 63 bytes) singly, one per
 		 * lane: the last, partial unit of memory is then written by one instruction rather
 		 * than by the end of a row and by the tail.  Tail bytes first, so their latency
@@ -226,17 +272,22 @@ __global__ __launch_bounds__(kBlock) void bounce_scatter_kernel(
 
 		const uint32_t shift = (uint32_t)(reinterpret_cast<uintptr_t>(s) & 3u);
 		if (shift == 0) {
-			copy_words<false>(s, d, nvec, 0, lane);
+			copy_words<false, KEEP>(s, d, nvec, 0, lane);
 		} else {
-			copy_words<true>(s - shift, d, nvec, shift, lane);
+			copy_words<true, KEEP>(s - shift, d, nvec, shift, lane);
 		}
 		store_byte_streaming(d + tail_at, tail_byte);
 	}
 
-	if (flush != nullptr) {
+	if (together) {
+		const uint32_t here = min(n - first, (uint32_t)WAVES);
+		if (arrive(back, wave, lane, in_range ? d : nullptr, here) && lane < here && back.at[lane] != 0) {
+			flush[first + lane] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(back.at[lane]));
+		}
+	} else if (flush != nullptr) {
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-		if (lane == 0) {
-			flush[buf] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(d));
+		if (lane == 0 && in_range) {
+			flush[buf] = *reinterpret_cast<const uint32_t *>(d);
 		}
 	}
 }
@@ -250,6 +301,7 @@ __global__ __launch_bounds__(kBlock) void bounce_scatter_kernel(
  * (measured on 65,536 buffers: 99.7 us with rows on 16-byte boundaries, 95.7 us on 64- or
  * 128-byte ones).  Wave-collective.
  */
+template <bool KEEP = false>
 __device__ __forceinline__ void copy_any(const uint8_t *__restrict__ s, uint8_t *__restrict__ d,
 					 uint32_t bytes, uint32_t lane)
 {
@@ -269,13 +321,17 @@ __device__ __forceinline__ void copy_any(const uint8_t *__restrict__ s, uint8_t 
 		const uint8_t tail_byte = s2[tail_at];
 		const uint32_t shift = (uint32_t)(reinterpret_cast<uintptr_t>(s2) & 3u);
 		if (shift == 0) {
-			copy_words<false>(s2, d2, nvec, 0, lane);
+			copy_words<false, KEEP>(s2, d2, nvec, 0, lane);
 		} else {
-			copy_words<true>(s2 - shift, d2, nvec, shift, lane);
+			copy_words<true, KEEP>(s2 - shift, d2, nvec, shift, lane);
 		}
 		store_byte_streaming(d2 + tail_at, tail_byte);
 	}
-	store_byte_streaming(d + head_at, head_byte);
+	if (KEEP) {
+		d[head_at] = head_byte;
+	} else {
+		store_byte_streaming(d + head_at, head_byte);
+	}
 }
 
 /*
@@ -283,6 +339,7 @@ __device__ __forceinline__ void copy_any(const uint8_t *__restrict__ s, uint8_t 
  * payload, which goes to a receive buffer at any alignment, truncated to that buffer's
  * length (rdma_eager_copy_req::post, src/nccl_ofi_rdma.cpp:2729-2776).
  */
+template <bool KEEP>
 __global__ __launch_bounds__(64 * kEagerWaves) void eager_copy_kernel(
 	const uint8_t *__restrict__ rx_base, const uint64_t *__restrict__ rx_off,
 	const uint32_t *__restrict__ recv_len, uint8_t *__restrict__ dst_base,
@@ -305,7 +362,7 @@ __global__ __launch_bounds__(64 * kEagerWaves) void eager_copy_kernel(
 		copied[buf] = bytes;
 	}
 
-	copy_any(s, d, bytes, lane);
+	copy_any<KEEP>(s, d, bytes, lane);
 
 	if (flush != nullptr) {
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -314,7 +371,8 @@ __global__ __launch_bounds__(64 * kEagerWaves) void eager_copy_kernel(
 		 * then the four are combined inside the quad */
 		uint32_t word = 0;
 		if (lane < min(bytes, 4u)) {
-			word = (uint32_t)__builtin_nontemporal_load(d + lane) << (8u * lane);
+			const uint32_t byte = KEEP ? d[lane] : __builtin_nontemporal_load(d + lane);
+			word = byte << (8u * lane);
 		}
 		word |= __shfl_xor(word, 1, 64);
 		word |= __shfl_xor(word, 2, 64);
@@ -480,6 +538,41 @@ struct ofi_amd_devcopy_region {
 constexpr size_t kCpuStoreMax = 2u << 20;
 constexpr size_t kCpuLoadMax = 256;
 
+/*
+ * Batches that fit the L2s (8 x 4 MiB) with room to spare keep the first row of every buffer in them instead of
+ * streaming it: the read-back behind it then finds its line there.  The bytes of a bounce batch are the packed source's,
+ * those of an eager batch are not known beyond 8 KiB a buffer.  Times in us on other buffers at every launch / on the
+ * same ones, streamed and then kept:
+ *   4000 bounce buffers of up to 8 KiB      8.5 / 7.3    7.5 / 6.4
+ *   8000 of up to 8 KiB                    14.5 / 13.2  13.7 / 12.0
+ *   65,536 of up to 500 B                  26.2 / 22.5  20.9 / 19.4
+ *   10,000 of up to 8 KiB                  17.1 / 16.0  18.0 / 15.4  (together: 16.5 / 15.3)
+ *   20,000 of up to 8 KiB                  29.9 / 29.7  35.4 / 26.9
+ *   8000 eager buffers of up to 8 KiB      16.1 / 14.9  14.8 / 12.4
+ *   12,000 of up to 8 KiB                  21.6 / 21.1  21.2 / 18.3
+ *   16,000 of up to 8 KiB                  27.5 / 26.0  32.2 / 23.0
+ */
+constexpr uint64_t kKeepBytes = 32ull << 20;
+constexpr uint32_t kKeepEager = 12000;
+/*
+ * Large batches of long buffers go with 24 wavefronts a CU instead of 32: reads and writes of 65,536 buffers take turns
+ * at the memory, and the fewer of them are under way the longer the turns are (other buffers at every launch / the same
+ * ones over and over, us):
+ *   65,536 of up to 8 KiB         32 by eights 112.7 / 82.0   24 by fours 108.4 / 86.8   16 by eights 109.6 / 91.1
+ *   32,768 of up to 8 KiB                       57.4 / 42.5                55.9 / 43.6
+ *   65,536 of up to 6000 B                      83.5 / 61.4                81.6 / 65.5
+ *   65,536 of up to 4 KiB                       59.5 / 44.9                63.2 / 53.1
+ * (all of them with the read-backs together; each by itself, 32 by eights, 111.4 / 88.4 in the first line).  Below,
+ * short buffers want every wavefront there is, to have enough under way.  The limit is set by the LDS a workgroup
+ * claims: six of four wavefronts fit a CU.
+ */
+constexpr uint64_t kFewerWavesBytes = 100ull << 20;
+constexpr uint64_t kFewerWavesLength = 2900; /* on average */
+constexpr int kFewerWaves = 4;
+constexpr uint32_t kFewerWavesLds = 27000;
+static_assert(6 * (kFewerWavesLds + sizeof(read_backs_t<kFewerWaves>)) <= 160 * 1024 &&
+	      7 * kFewerWavesLds > 160 * 1024, "six workgroups to a CU");
+
 using namespace ofi_amd;
 
 extern "C" {
@@ -502,12 +595,19 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 	if (!err) {
 		return -ENOMEM;
 	}
-	uint32_t blocks = (n + kWavesPerBlock - 1) / kWavesPerBlock;
-	const uint32_t round = kXcds * kGroup; /* whole rounds over the XCDs */
-	blocks = (blocks + round - 1) / round * round;
-	hipLaunchKernelGGL(bounce_scatter_kernel, dim3(blocks), dim3(kBlock), 0, as_stream(stream),
-			   static_cast<const uint8_t *>(d_src), src_bytes, static_cast<uint8_t *>(d_arena),
-			   arena_bytes, d_src_off, d_dst_off, d_len, n, d_flush, err);
+	const uint32_t runs = (n + kXcds * kBounceRun - 1) / (kXcds * kBounceRun); /* whole rounds over the XCDs */
+	auto launch = [&](auto kernel, uint32_t waves, uint32_t lds) {
+		hipLaunchKernelGGL(kernel, dim3(runs * kXcds * (kBounceRun / waves)), dim3(64 * waves), lds, as_stream(stream),
+				   static_cast<const uint8_t *>(d_src), src_bytes, static_cast<uint8_t *>(d_arena), arena_bytes,
+				   d_src_off, d_dst_off, d_len, n, d_flush, err);
+	};
+	if (d_flush && src_bytes <= kKeepBytes) {
+		launch(bounce_scatter_kernel<kBounceWaves, true>, kBounceWaves, 0);
+	} else if (src_bytes >= kFewerWavesBytes && src_bytes / n >= kFewerWavesLength) {
+		launch(bounce_scatter_kernel<kFewerWaves, false>, kFewerWaves, kFewerWavesLds);
+	} else {
+		launch(bounce_scatter_kernel<kBounceWaves, false>, kBounceWaves, 0);
+	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }
@@ -529,9 +629,16 @@ int ofi_amd_eager_copy_batch(const void *rx_base, const uint64_t *d_rx_off, cons
 	uint32_t blocks = (n + kEagerWaves - 1) / kEagerWaves;
 	const uint32_t round = kXcds * kEagerGroup;
 	blocks = (blocks + round - 1) / round * round;
-	hipLaunchKernelGGL(eager_copy_kernel, dim3(blocks), dim3(64 * kEagerWaves), 0, as_stream(stream),
-			   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len,
-			   static_cast<uint8_t *>(dst_base), d_dst_off, d_dst_len, n, d_copied, d_flush);
+	auto launch = [&](auto kernel) {
+		hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kEagerWaves), 0, as_stream(stream),
+				   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base),
+				   d_dst_off, d_dst_len, n, d_copied, d_flush);
+	};
+	if (d_flush && n <= kKeepEager) {
+		launch(eager_copy_kernel<true>);
+	} else {
+		launch(eager_copy_kernel<false>);
+	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -92,6 +92,48 @@ def test_lengths_beyond_one_trip_and_every_row_count(lib, oracle, gpu):
     assert _gpu.fetch_async_errors(lib) == 0
 
 
+@pytest.mark.parametrize("src_mib", [1, 32, 33, 99, 101])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 9, 333])
+@pytest.mark.parametrize("flush", [True, False])
+def test_forms_by_the_size_of_the_source(lib, oracle, gpu, src_mib, n, flush):
+    """The first row kept in the L2 or streamed, the flush words of a workgroup read back together, fewer wavefronts a CU:
+    by the bytes of the packed source.  Batches that fill a workgroup in part, short and long buffers side by side at any
+    source alignment, every fifth one outside the arena or the source: skipped and reported, its flush word untouched,
+    and the others of its workgroup complete."""
+    rng = np.random.default_rng(100 * src_mib + n)
+    src_bytes = (src_mib << 20) + 13
+    pick = np.array([0, 1, 2, 3, 4, 5, 63, 64, 65, 127, 128, 1000, 1023, 1024, 1025, 4096, 8191, 8192, 8193, 20000], dtype=np.uint32)
+    length = np.resize(rng.permutation(pick), n)
+    slot = 20032
+    dst_off = rng.permutation(n).astype(np.uint64) * np.uint64(slot)
+    src_off = rng.integers(0, src_bytes - 20000, n).astype(np.uint64)
+    bad = np.arange(n) % 5 == 4
+    bad_dst, bad_src = bad & (np.arange(n) % 2 == 0), bad & (np.arange(n) % 2 == 1)
+    dst_off_given, src_off_given = dst_off.copy(), src_off.copy()
+    dst_off_given[bad_dst] = np.uint64(n * slot + 64)
+    src_off_given[bad_src] = np.uint64(src_bytes + 1)
+    d_src = torch.randint(0, 256, (src_bytes,), dtype=torch.uint8, device="cuda", generator=torch.Generator("cuda").manual_seed(n))
+    src = d_src.cpu().numpy()
+    want = np.full(n * slot, 0x77, dtype=np.uint8)
+    want_flush = np.full(n, 0xFFFFFFFF, dtype=np.uint32)
+    for i in np.flatnonzero(~bad):
+        at, k, o = int(dst_off[i]), int(length[i]), int(src_off[i])
+        want[at:at + k] = src[o:o + k]
+        want_flush[i] = int.from_bytes(want[at:at + 4].tobytes(), "little")
+    d = [_gpu.to_dev(x) for x in (src_off_given, dst_off_given, length)]
+    for _ in range(2):
+        arena = torch.full((n * slot,), 0x77, dtype=torch.uint8, device="cuda")
+        d_flush = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+        assert lib.ofi_amd_bounce_scatter(d_src.data_ptr(), src_bytes, arena.data_ptr(), n * slot, d[0].data_ptr(),
+                                          d[1].data_ptr(), d[2].data_ptr(), n, d_flush.data_ptr() if flush else None,
+                                          _gpu.stream()) == 0
+        _gpu.sync()
+        assert np.array_equal(arena.cpu().numpy(), want)
+        if flush:
+            assert np.array_equal(_gpu.to_host(d_flush, np.uint32), want_flush)
+    assert bool(_gpu.fetch_async_errors(lib)) == bool(bad.any())
+
+
 def test_empty_batch_and_all_zero_lengths(lib, oracle, gpu):
     arena = torch.full((4096,), 9, dtype=torch.uint8, device="cuda")
     assert lib.ofi_amd_bounce_scatter(arena.data_ptr(), 4096, arena.data_ptr(), 4096, None, None, None, 0,

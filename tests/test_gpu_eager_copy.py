@@ -106,6 +106,22 @@ def test_every_short_length_at_every_alignment(lib, oracle, gpu):
         assert np.array_equal(g, w)
 
 
+@pytest.mark.parametrize("n", [11999, 12000, 12001])
+def test_short_payloads_in_batches_of_both_forms(lib, oracle, gpu, n):
+    """Lengths 0..130 at every destination alignment in batches that keep the first row of a buffer in the L2 and in
+    larger ones that stream it: bytes, counts and flush words."""
+    rng = np.random.default_rng(n)
+    recv_len = (np.arange(n) % 131).astype(np.uint32)
+    rx_off = rng.permutation(n).astype(np.uint64) * np.uint64(160) + rng.integers(0, 16, n).astype(np.uint64)
+    starts = rng.permutation(n).astype(np.uint64) * np.uint64(256) + (np.arange(n) // 131 % 64).astype(np.uint64)
+    rx = rng.integers(0, 256, n * 160 + 64, dtype=np.uint8)
+    d_rx = _gpu.to_dev(rx)
+    want = expected(oracle, rx, rx_off, recv_len, starts, recv_len, n * 256, 0x3C)
+    got = run_gpu(lib, d_rx.data_ptr(), rx_off, recv_len, starts, recv_len, n * 256, 0x3C)
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+
+
 def test_unaligned_rx_buffers_and_large_payloads(lib, oracle, gpu):
     """The format only fixes payload = buffer + 8; buffers themselves may sit at any byte
     (a test of the source-side funnel shift), and payloads may exceed one 8 KiB trip."""
