@@ -22,8 +22,24 @@ using namespace ofi_amd_tuner;
 
 namespace {
 
+/* Quotients of numbers below 2^31 by a number fixed at plan time: with 2^(l-1) < d <= 2^l and m = ceil(2^(31+l) / d),
+ * x / d = x * m >> (31 + l), because m * d exceeds 2^(31+l) by less than d <= 2^l */
+struct divisor_t {
+	uint32_t d, m, l;
+};
+divisor_t divisor(uint32_t d)
+{
+	const uint32_t l = d <= 1 ? 0 : 32 - (uint32_t)__builtin_clz(d - 1);
+	return { d, (uint32_t)(((1ull << (31 + l)) + d - 1) / d), l };
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t x, const divisor_t &by)
+{
+	return __umulhi(x << 1, by.m) >> by.l;
+}
+
 struct grid_dims_t {
 	uint32_t n_colls, n_sizes, n_nodes, n_ppn, n_algos;
+	divisor_t by_ppn, by_nodes, by_coll; /* by_coll: the points of a collective */
 	const int32_t *colls;
 	const uint64_t *sizes;
 	const uint64_t *nodes;
@@ -41,25 +57,90 @@ struct tiling_t {
 	const double2 *rank_span; /* per (tile column, ppn): smallest and largest log2_ranks */
 };
 
+/* Model workgroups have 256 threads and, from 48 MB of costs on, claim enough LDS that six of them share a CU instead of
+ * eight, from 96 MB on 1024 threads: the fewer and longer the runs under way, the better they suit the memory.  Times in
+ * us with eight and with six of 256, and with 1024 threads: 27 MB 7.0 / 7.4 / -, 40 MB 8.0 / 8.6 / 9.9, 60 MB 12.5 /
+ * 12.0 / -, 85 MB 16.6 / 16.3 / 16.8, 133 MB 25.9 / - / 25.1, 266 MB 52.3 / - / 49.6, 495 MB 96.5 / 96.1 / 92.5. */
+constexpr uint32_t kModelThreads = 256, kModelThreadsLarge = 1024;
+constexpr uint64_t kModelSixBytes = 48ull << 20, kModelLargeBytes = 96ull << 20;
+constexpr size_t kModelSixLds = 27000;
+constexpr size_t kModelLds = 64 * 1024; /* at most, for the larger ones */
+
+/* `cells` doubles at `out`, cell(k) each, by a workgroup: two to a lane and store, 1 KiB per wavefront
+ * instruction, where the address allows it */
+template <uint32_t kThreads, typename F> __device__ __forceinline__ void write_cells(double *__restrict__ out, uint32_t cells, F cell)
+{
+	if ((reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
+		typedef double double2_t __attribute__((ext_vector_type(2)));
+		double2_t *to = reinterpret_cast<double2_t *>(out);
+		for (uint32_t k = threadIdx.x; k < cells / 2; k += kThreads) {
+			const double2_t v = { cell(2 * k), cell(2 * k + 1) };
+			__builtin_nontemporal_store(v, &to[k]);
+		}
+		if ((cells & 1u) && threadIdx.x == 0) {
+			out[cells - 1] = cell(cells - 1);
+		}
+	} else {
+		for (uint32_t k = threadIdx.x; k < cells; k += kThreads) {
+			__builtin_nontemporal_store(cell(k), &out[k]);
+		}
+	}
+}
+
+__device__ __forceinline__ void write_choice(int8_t *__restrict__ choice, uint64_t point, int algo, int proto)
+{
+	const uint64_t at = point * 2u;
+	if ((reinterpret_cast<uintptr_t>(choice) & 1u) == 0) {
+		*reinterpret_cast<uint16_t *>(choice + at) =
+			(uint16_t)((uint8_t)(int8_t)algo | ((uint32_t)(uint8_t)(int8_t)proto << 8));
+	} else {
+		choice[at + 0] = (int8_t)algo;
+		choice[at + 1] = (int8_t)proto;
+	}
+}
+
 /*
  * One thread per decision point; blockIdx.y is the variant.  The thread evaluates the
  * n_algos x 3 cost cells of its point -- contiguous in the output -- and its decision.  Cells
- * are staged in LDS so that the workgroup writes its 256 x cells-per-point doubles as one
+ * are staged in LDS, as the floats they are, so that the workgroup writes its points' doubles as one
  * contiguous run (a lane-per-point store would touch 64 cache lines per instruction).
+ * Bound by that write, which goes at 5.4 TB/s from 60 MB on, and below by its own instructions: a workgroup without a
+ * modelled point (two collectives in three, and platforms without a model) writes its -1s and is done, indices are
+ * taken apart by multiplications, and floats make half the LDS traffic of doubles.  140 sizes x 11 node counts: 30 grids
+ * 9.9 -> 8.0 us, 64 grids 16.5 -> 16.3.
  */
-template <bool COST, bool CHOICE>
-__global__ __launch_bounds__(256) void model_grid_kernel(grid_dims_t g,
+template <bool COST, bool CHOICE, uint32_t kThreads = kModelThreads>
+__global__ __launch_bounds__(kThreads) void model_grid_kernel(grid_dims_t g,
 							 const ofi_amd_tuner_variant_t *__restrict__ variants,
 							 uint32_t points_per_variant, double *__restrict__ cost,
 							 int8_t *__restrict__ choice)
 {
-	extern __shared__ double stage[]; /* [256][cells per point] when COST */
+	extern __shared__ float stage[]; /* [kThreads][cells per point] when COST */
 	__shared__ int32_t column_of[NUM_ALGOS]; /* the plan's column of an algorithm, -1: none */
 	const uint32_t cpp = g.n_algos * NUM_PROTOS;
-	const uint32_t first = blockIdx.x * 256u;
+	const uint32_t first = blockIdx.x * kThreads, valid = min(kThreads, points_per_variant - first);
 	const uint32_t p = first + threadIdx.x;
 	const ofi_amd_tuner_variant_t v = variants[blockIdx.y];
-	const bool live = p < points_per_variant;
+	const bool live = threadIdx.x < valid;
+	const uint64_t variant_at = (uint64_t)blockIdx.y * points_per_variant;
+	double *out = COST ? cost + (variant_at + first) * cpp : nullptr;
+
+	bool modelled = false; /* any point of the workgroup */
+	if (platform_has_model(v.platform)) {
+		const uint32_t last_coll = quotient(first + valid - 1u, g.by_coll);
+		for (uint32_t c = quotient(first, g.by_coll); c <= last_coll; c++) {
+			modelled |= g.colls[c] == FUNC_ALLREDUCE;
+		}
+	}
+	if (!modelled) {
+		if (COST) {
+			write_cells<kThreads>(out, valid * cpp, [](uint32_t) { return -1.0; });
+		}
+		if (CHOICE && live) {
+			write_choice(choice, variant_at + p, -1, -1);
+		}
+		return;
+	}
 	if (COST && CHOICE) {
 		if (threadIdx.x < NUM_ALGOS) {
 			int32_t col = -1;
@@ -71,29 +152,24 @@ __global__ __launch_bounds__(256) void model_grid_kernel(grid_dims_t g,
 		__syncthreads();
 	}
 	if (live) {
-		uint32_t r = p;
-		const uint32_t pi = r % g.n_ppn; r /= g.n_ppn;
-		const uint32_t ni = r % g.n_nodes; r /= g.n_nodes;
-		const uint32_t si = r % g.n_sizes; r /= g.n_sizes;
-		const uint32_t ci = r;
+		const uint32_t ci = quotient(p, g.by_coll), of_coll = p - ci * g.by_coll.d;
+		const uint32_t row = quotient(of_coll, g.by_ppn), pi = of_coll - row * g.n_ppn;
+		const uint32_t si = quotient(row, g.by_nodes), ni = row - si * g.n_nodes;
 		const uint64_t nodes = g.nodes[ni];
 		const uint64_t per_node = g.ppn[pi];
 		const uint64_t ranks = nodes * per_node;
 		if (COST) {
-			const bool modelled = platform_has_model(v.platform);
 			const float size_f = (float)g.sizes[si];
 			const int coll = g.colls[ci];
 			const double log2_nodes = g.log2_nodes[ni];
 			for (uint32_t ai = 0; ai < g.n_algos; ai++) {
-				float c[NUM_PROTOS] = { -1.0f, -1.0f, -1.0f };
-				if (modelled) {
-					/* ranks = nodes * per_node, so ranks / nodes is per_node */
-					model_cost_protos(v.platform, coll, g.algos[ai], v.pipe_ops, size_f, ranks, nodes, per_node,
-							  log2_nodes, v.num_channels, v.net_comp_overhead, c);
-				}
+				float c[NUM_PROTOS];
+				/* ranks = nodes * per_node, so ranks / nodes is per_node */
+				model_cost_protos(v.platform, coll, g.algos[ai], v.pipe_ops, size_f, ranks, nodes, per_node,
+						  log2_nodes, v.num_channels, v.net_comp_overhead, c);
 #pragma unroll
 				for (uint32_t proto = 0; proto < NUM_PROTOS; proto++) {
-					stage[threadIdx.x * cpp + ai * NUM_PROTOS + proto] = (double)c[proto];
+					stage[threadIdx.x * cpp + ai * NUM_PROTOS + proto] = c[proto];
 				}
 			}
 		}
@@ -103,13 +179,13 @@ __global__ __launch_bounds__(256) void model_grid_kernel(grid_dims_t g,
 				/* the cells the decision looks at have just been worked out: it reads this thread's
 				 * row of the stage instead of evaluating the model again, and goes to the model
 				 * only for an algorithm the plan has no column for */
-				const double *cells = &stage[threadIdx.x * cpp];
+				const float *cells = &stage[threadIdx.x * cpp];
 				model_choose_with(
 					v.platform, g.colls[ci], g.sizes[si], ranks, nodes, kAllAllowed,
 					[&](int a, int pr) -> float {
 						const int32_t col = column_of[a];
 						if (col >= 0) {
-							return (float)cells[col * NUM_PROTOS + pr]; /* exact: it was a float */
+							return cells[col * NUM_PROTOS + pr];
 						}
 						return model_cost(v.platform, g.colls[ci], a, pr, v.pipe_ops, g.sizes[si], ranks,
 								  nodes, g.log2_nodes[ni], v.num_channels, v.net_comp_overhead);
@@ -119,37 +195,12 @@ __global__ __launch_bounds__(256) void model_grid_kernel(grid_dims_t g,
 				model_choose(v.platform, g.colls[ci], g.sizes[si], ranks, nodes, g.log2_nodes[ni], v.pipe_ops,
 					     v.num_channels, v.net_comp_overhead, kAllAllowed, algo, proto);
 			}
-			const uint64_t at = ((uint64_t)blockIdx.y * points_per_variant + p) * 2u;
-			if ((reinterpret_cast<uintptr_t>(choice) & 1u) == 0) {
-				*reinterpret_cast<uint16_t *>(choice + at) =
-					(uint16_t)((uint8_t)(int8_t)algo | ((uint32_t)(uint8_t)(int8_t)proto << 8));
-			} else {
-				choice[at + 0] = (int8_t)algo;
-				choice[at + 1] = (int8_t)proto;
-			}
+			write_choice(choice, variant_at + p, algo, proto);
 		}
 	}
 	if (COST) {
 		__syncthreads();
-		const uint32_t valid = min(256u, points_per_variant - first);
-		double *out = cost + ((uint64_t)blockIdx.y * points_per_variant + first) * cpp;
-		const uint32_t cells = valid * cpp;
-		if ((reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
-			/* two cells per lane and store: 1 KiB per wavefront instruction */
-			typedef double double2_t __attribute__((ext_vector_type(2)));
-			const double2_t *from = reinterpret_cast<const double2_t *>(stage);
-			double2_t *to = reinterpret_cast<double2_t *>(out);
-			for (uint32_t k = threadIdx.x; k < cells / 2; k += 256u) {
-				__builtin_nontemporal_store(from[k], &to[k]);
-			}
-			if ((cells & 1u) && threadIdx.x == 0) {
-				out[cells - 1] = stage[cells - 1];
-			}
-		} else {
-			for (uint32_t k = threadIdx.x; k < cells; k += 256u) {
-				__builtin_nontemporal_store(stage[k], &out[k]);
-			}
-		}
+		write_cells<kThreads>(out, valid * cpp, [&](uint32_t k) { return (double)stage[k]; });
 	}
 }
 
@@ -816,6 +867,9 @@ int ofi_amd_tuner_plan_create(const int32_t *colls, uint32_t n_colls, const uint
 	g.n_nodes = n_nodes;
 	g.n_ppn = n_ppn;
 	g.n_algos = n_algos;
+	g.by_ppn = divisor(n_ppn);
+	g.by_nodes = divisor(n_nodes);
+	g.by_coll = divisor((uint32_t)std::min<uint64_t>((uint64_t)n_sizes * n_nodes * n_ppn, 1u << 31));
 	g.colls = reinterpret_cast<const int32_t *>(d_axes + at_colls);
 	g.sizes = reinterpret_cast<const uint64_t *>(d_axes + at_sizes);
 	g.nodes = reinterpret_cast<const uint64_t *>(d_axes + at_nodes);
@@ -888,17 +942,21 @@ int ofi_amd_tuner_model_grid(ofi_amd_tuner_plan_t *plan, const ofi_amd_tuner_var
 		return -EINVAL;
 	}
 	const uint32_t points = (uint32_t)plan->points;
-	const dim3 grid((points + 255u) / 256u, n_variants);
-	const size_t lds = (size_t)256 * plan->g.n_algos * NUM_PROTOS * sizeof(double);
+	const size_t row = (size_t)plan->g.n_algos * NUM_PROTOS * sizeof(float); /* of the stage */
+	const uint64_t bytes = d_cost ? plan->cells * n_variants * sizeof(double) : 0;
+	const bool large = bytes > kModelLargeBytes && row * kModelThreadsLarge <= kModelLds;
+	const uint32_t threads = large ? kModelThreadsLarge : kModelThreads;
+	const size_t lds = std::max(row * threads, !large && bytes > kModelSixBytes ? kModelSixLds : 0);
+	auto launch = [&](auto kernel) {
+		hipLaunchKernelGGL(kernel, dim3((points + threads - 1) / threads, n_variants), dim3(threads), d_cost ? lds : 0, s,
+				   plan->g, plan->d_variants, points, d_cost, d_choice);
+	};
 	if (d_cost && d_choice) {
-		hipLaunchKernelGGL((model_grid_kernel<true, true>), grid, dim3(256), lds, s, plan->g,
-				   plan->d_variants, points, d_cost, d_choice);
+		large ? launch(model_grid_kernel<true, true, kModelThreadsLarge>) : launch(model_grid_kernel<true, true>);
 	} else if (d_cost) {
-		hipLaunchKernelGGL((model_grid_kernel<true, false>), grid, dim3(256), lds, s, plan->g,
-				   plan->d_variants, points, d_cost, d_choice);
+		large ? launch(model_grid_kernel<true, false, kModelThreadsLarge>) : launch(model_grid_kernel<true, false>);
 	} else if (d_choice) {
-		hipLaunchKernelGGL((model_grid_kernel<false, true>), grid, dim3(256), 0, s, plan->g,
-				   plan->d_variants, points, d_cost, d_choice);
+		launch(model_grid_kernel<false, true>);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;

@@ -133,6 +133,39 @@ def test_model_grid_on_wide_and_narrow_axes(lib, oracle, gpu, n_nodes, n_ppn):
     lib.ofi_amd_tuner_plan_destroy(plan)
 
 
+@pytest.mark.parametrize("n_sizes,n_nodes,n_ppn,n_variants,odd", [(1, 1, 1, 1, 0), (7, 13, 3, 3, 1), (64, 4, 1, 2, 0), (129, 1, 2, 5, 1),
+                                                                  (97, 11, 4, 640, 0), (96, 11, 4, 640, 1)])
+def test_model_grid_points_and_workgroups(lib, oracle, gpu, n_sizes, n_nodes, n_ppn, n_variants, odd):
+    """Workgroups with no modelled point, with some and with nothing else (collectives of fewer, as many and more points
+    than a workgroup, in an order that puts modelled ones at both ends), outputs on any 8-byte and 1-byte boundary, and
+    more than 96 MiB of costs, which larger workgroups write.  The oracle's bits."""
+    rng = np.random.default_rng(n_sizes)
+    colls = np.array([4, 2, 0, 4], dtype=np.int32)
+    sizes = np.unique((2 ** rng.uniform(0, 36, n_sizes)).astype(np.uint64))
+    nodes = np.arange(1, n_nodes + 1, dtype=np.uint64) * np.uint64(2)
+    ppn = np.array([1, 2, 4, 8], dtype=np.uint32)[:n_ppn]
+    algos = np.array([1, 0, 6], dtype=np.int32)
+    plan = make_plan(lib, colls, sizes, nodes, ppn, algos)
+    distinct = [m.TunerVariant(i % 3, 1 + i % 4, 4 + i % 5, 3) for i in range(min(n_variants, 5))]
+    want_cost, want_choice = oracle_model_grid(oracle, distinct, colls, sizes, nodes, ppn, algos)
+    cells, points = lib.ofi_amd_tuner_plan_cells(plan), lib.ofi_amd_tuner_plan_points(plan)
+    arr = (m.TunerVariant * n_variants)(*[distinct[i % len(distinct)] for i in range(n_variants)])
+    d_cost = torch.full((n_variants * cells + 2,), 7.0, dtype=torch.float64, device="cuda")
+    d_choice = torch.full((n_variants * points * 2 + 2,), 99, dtype=torch.int8, device="cuda")
+    assert lib.ofi_amd_tuner_model_grid(plan, arr, n_variants, d_cost.data_ptr() + 8 * odd, d_choice.data_ptr() + odd,
+                                        _gpu.stream()) == 0
+    _gpu.sync()
+    cost, choice = d_cost.cpu().numpy(), d_choice.cpu().numpy()
+    assert (cost[:odd] == 7.0).all() and (cost[odd + n_variants * cells:] == 7.0).all()
+    assert (choice[:odd] == 99).all() and (choice[odd + n_variants * points * 2:] == 99).all()
+    cost = cost[odd:odd + n_variants * cells].reshape((n_variants,) + want_cost.shape[1:])
+    choice = choice[odd:odd + n_variants * points * 2].reshape((n_variants,) + want_choice.shape[1:])
+    for i in range(n_variants):
+        assert np.array_equal(cost[i].astype(np.float32).view(np.uint32), want_cost[i % len(distinct)].view(np.uint32)), i
+        assert np.array_equal(choice[i], want_choice[i % len(distinct)]), i
+    lib.ofi_amd_tuner_plan_destroy(plan)
+
+
 def oracle_region_grid(oracle, platforms, colls, sizes, nodes, ppn):
     out = np.zeros((len(platforms), len(colls), len(sizes), len(nodes), len(ppn), 3), np.int32)
     a, p, ch = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
