@@ -206,8 +206,8 @@ __global__ __launch_bounds__(kThreads) void model_grid_kernel(grid_dims_t g,
 
 constexpr int kMaxSetEdges = 64; /* of one (platform, shape, collective) set: one per lane */
 /* Wavefronts per workgroup of the region kernel: two in launches of more than kPairedTiles tiles, whose workgroups
- * take as long to hand out as to work off (560 sizes x 38 node counts of four platforms 9.5 -> 8.9 us, 280 x 38 7.3
- * -> 7.1; four wavefronts 9.2 and 7.2), one in smaller ones, where two gain nothing. */
+ * take as long to hand out as to work off (560 sizes x 38 node counts of four platforms 9.3 -> 8.9 us, 280 x 38 7.65
+ * -> 7.5; four wavefronts 9.3 and 7.7), one in smaller ones, where two gain nothing. */
 constexpr uint32_t kMostRegionWaves = 2;
 constexpr uint64_t kPairedTiles = 6000;
 constexpr uint64_t kMostRuns = 65535; /* of one launch: gridDim.y */
@@ -395,16 +395,37 @@ __global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(
 				in_box &= __ballot(at.x >= lane_value(box.x, i)) & __ballot(at.x <= lane_value(box.y, i)) &
 					  __ballot(at.y >= lane_value(box.z, i)) & __ballot(at.y <= lane_value(box.w, i));
 			}
+			left &= near | every(in_box);
+			if (in_box == 0 && left == 0) {
+				continue; /* of the points still open none is in the box or on an edge */
+			}
 			const pt_t ray = vsub(far_point, at);
-			/* a far point close to an edge's line (no polygon has such an edge) leaves it to the exact code */
-			uint64_t unsure = every(left & ~f_sure), touching = 0;
+			uint64_t close = 0, touching = 0; /* close: a vertex may lie on the ray */
 			for (; vertices != 0; vertices &= vertices - 1) {
 				const int e = __builtin_ctzll(vertices);
 				const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
 				const double side = vcross_sign(vsub(a, at), ray);
-				unsure |= __ballot(fabs(side) <= kSure);
+				close |= __ballot(fabs(side) <= kSure);
 				odd ^= __ballot(side > 0) & every((counts >> e) & 1u);
 			}
+			close &= in_box;
+			if (close != 0) {
+				/* for these points the exact code on the edges between that have an end in the fan */
+				uint64_t exact = every((uint64_t)(__popcll(c & a_sure & b_sure & ends_apart) & 1));
+				for (uint64_t ask = c & ~(a_sure & b_sure); ask != 0; ask &= ask - 1) {
+					const int e = __builtin_ctzll(ask);
+					const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
+					const pt_t b = { lane_value(mine.b.x, e), lane_value(mine.b.y, e) };
+					bool crosses = false;
+					if ((close >> lane) & 1u) {
+						crosses = intersects(at, far_point, a, b, eps);
+					}
+					exact ^= __ballot(crosses);
+				}
+				odd = (odd & ~close) | (exact & close);
+			}
+			/* where the far point is close to the line of an edge, the exact code, too */
+			const uint64_t f_close = every(left & ~f_sure);
 			for (; left != 0; left &= left - 1) {
 				const int e = __builtin_ctzll(left);
 				const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
@@ -412,34 +433,21 @@ __global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(
 				const pt_t pa = vsub(a, at), pb = vsub(b, at);
 				const edge_sides_t s = { vcross_sign(pa, ray), vcross_sign(pb, ray), vcross_sign(pb, pa) };
 				const uint64_t apart = __ballot(s.side_a > 0) ^ __ballot(s.side_b > 0);
-				unsure |= __ballot(fabs(s.side_a) <= kSure) | __ballot(fabs(s.side_b) <= kSure) |
-					  (apart & __ballot(fabs(s.side_p) <= kSure));
-				odd ^= apart & (__ballot(s.side_p > 0) ^ every((f_pos >> e) & 1u));
+				const uint64_t unsure = in_box & (__ballot(fabs(s.side_a) <= kSure) | __ballot(fabs(s.side_b) <= kSure) |
+								  (apart & (__ballot(fabs(s.side_p) <= kSure) | f_close)));
+				odd ^= apart & (__ballot(s.side_p > 0) ^ every((f_pos >> e) & 1u)) & ~unsure;
 				const uint64_t reached = open & __ballot(fabs(s.side_p) <= lane_value(mine_reach, e));
-				if (reached != 0) {
-					bool t = false;
-					if ((reached >> lane) & 1u) {
-						t = touches_edge(at, a, b, s, eps);
-					}
-					touching |= __ballot(t);
-				}
-			}
-			unsure &= in_box & ~touching;
-			if (unsure != 0) {
-				/* for these points, whose ray or themselves come close to a vertex or an edge, the exact code on
-				 * the edges that the tile does not know about */
-				uint64_t exact = every((uint64_t)(__popcll(c & a_sure & b_sure & ends_apart) & 1));
-				for (uint64_t ask = (c & ~(a_sure & b_sure)) | (through & of_poly); ask != 0; ask &= ask - 1) {
-					const int e = __builtin_ctzll(ask);
-					const pt_t a = { lane_value(mine.a.x, e), lane_value(mine.a.y, e) };
-					const pt_t b = { lane_value(mine.b.x, e), lane_value(mine.b.y, e) };
-					bool crosses = false;
+				if ((unsure | reached) != 0) {
+					bool crosses = false, t = false;
 					if ((unsure >> lane) & 1u) {
 						crosses = intersects(at, far_point, a, b, eps);
 					}
-					exact ^= __ballot(crosses);
+					if ((reached >> lane) & 1u) {
+						t = touches_edge(at, a, b, s, eps);
+					}
+					odd ^= __ballot(crosses);
+					touching |= __ballot(t);
 				}
-				odd = (odd & ~unsure) | (exact & unsure);
 			}
 			const uint64_t hit = open & (touching | (odd & in_box));
 			const int a = __builtin_amdgcn_readlane(pw.x, i), pr = __builtin_amdgcn_readlane(pw.y, i);
@@ -542,9 +550,9 @@ uint32_t log2_ceil(uint32_t v)
  * tile.  The points of a smaller tile differ about fewer edges, so its wavefront is done sooner, at the price of
  * more wavefronts, each of which costs 0.2 ns of dispatch and works out its edges' sides anew.
  * On an axis shorter than the tile, what is left over of the two largest goes to the other axis: one size and
- * 200,000 node counts of four platforms take 49 us in tiles of 64 node counts, 304 in squares with 7 of 8 lanes
- * idle, 3 sizes and 20,000 node counts 62 and 120.  The smallest tiles stay short there, which is what they are for (35
- * sizes at one node count: 5.5 us in pairs of points, 7.0 in fours).
+ * 200,000 node counts of four platforms take 46 us in tiles of 64 node counts, 270 in squares with 7 of 8 lanes
+ * idle, 3 sizes and 20,000 node counts 42 and 81.  The smallest tiles stay short there, which is what they are for (35
+ * sizes at one node count: 4.1 us in pairs of points, 5.4 in fours).
  */
 constexpr int kTilings = 4;
 void tile_shifts(uint32_t n_sizes, uint32_t n_nodes, uint32_t shift_n[kTilings], uint32_t shift_s[kTilings])
@@ -568,15 +576,17 @@ void tile_shifts(uint32_t n_sizes, uint32_t n_nodes, uint32_t shift_n[kTilings],
  * The smallest tiles that make at most kMostTiles: beyond, handing out the wavefronts costs more than their shorter
  * turns save.  Times in us with tiles of 64 / 16 / 8 / 4 points and, in brackets, the tiles these make (3
  * collectives, 4 values of ranks per node):
- *   35 sizes, 11 node counts, 4 platforms      16.0 / 8.9 / 7.0 / 5.6   [ 480, 1296, 2592, 5184]
- *   70 sizes, 11 node counts, 2 platforms      13.7 / 7.0 / 5.3 / 4.8   [ 432, 1296, 2592, 5040]
- *   140 sizes, 27 node counts, 1 platform       7.7 / 6.1 / 5.3 / 4.8   [ 840, 2940, 5880, 11760]
- *   35 sizes, 38 node counts, 4 platforms      11.2 / 7.9 / 6.8 / 7.1   [1200, 4320, 8208, 16416]
- *   140 sizes, 11 node counts, 4 platforms     10.1 / 6.8 / 6.3 / 7.4   [1728, 5040, 10080, 20160]
- *   160 sizes, 27 node counts, 3 platforms      7.8 / 6.6 / 7.7 / 12    [2880, 10080, 20160, 40320]
- *   140 sizes, 38 node counts, 4 platforms      7.9 / 8.0 / 10.4 / 18   [4320, 16800, 31920, 63840]
+ *   35 sizes, 11 node counts, 4 platforms      14.9 / 8.8 / 7.5 / 6.1   [ 480, 1296, 2592, 5184]
+ *   70 sizes, 11 node counts, 2 platforms      13.7 / 6.8 / 5.8 / 4.9   [ 432, 1296, 2592, 5040]
+ *   140 sizes, 27 node counts, 1 platform       7.0 / 5.6 / 5.1 / 4.9   [ 840, 2940, 5880, 11760]
+ *   35 sizes, 38 node counts, 4 platforms      10.8 / 7.2 / 7.3 / 7.1   [1200, 4320, 8208, 16416]
+ *   140 sizes, 11 node counts, 4 platforms      9.8 / 7.1 / 6.4 / 7.5   [1728, 5040, 10080, 20160]
+ *   160 sizes, 27 node counts, 3 platforms      7.4 / 6.6 / 7.6 / 12    [2880, 10080, 20160, 40320]
+ *   140 sizes, 38 node counts, 4 platforms      7.6 / 8.1 / 10.1 / 18   [4320, 16800, 31920, 63840]
+ * Two sizes far apart, whose tiles see every edge of a set, want fewer: 2000 node counts, 1 and 4 platforms 9.4 and 11.7
+ * (3000 tiles of 16, 3024 of 64), 11.2 and 16.3 with four times as many.
  */
-constexpr uint64_t kMostTiles = 12000;
+constexpr uint64_t kMostTiles = 10500;
 uint64_t tiling_tiles(const tiling_t &t)
 {
 	return (uint64_t)t.tiles_n * t.tiles_s;
