@@ -12,7 +12,7 @@
  *
  * Three forms, by the size of the batch:
  *   up to kDirectBatch messages, one launch: every workgroup adds up the messages before
- *   its tile by itself, from their sizes (at most 48 KiB out of the L2); beyond one tile not in a
+ *   its tile by itself, from their sizes (at most 78 KiB out of the L2); beyond one tile not in a
  *   batch that is being captured into a graph (launch_batch says why);
  *   up to kSmallBatch, two launches: stripe_count_kernel leaves each tile's totals of
  *   (small count, stripe count), reduced mod R (only the residues matter), and
@@ -22,7 +22,7 @@
  *   beyond, the same two launches with larger tiles, and a level of totals above the tiles', for
  *   every kPart messages.
  * The count launch snapshots the two counters of *state as the batch's seed, the workgroup of the
- * last tile writes the new ones back; in the one-launch form the workgroup that is done last does.
+ * last tile writes the new ones back; in the one-launch form the workgroup that reads them last does.
  *
  * HBM traffic per message: 8 B read twice (once in the one-launch form) + 4 B + 96 B written.
  */
@@ -38,12 +38,12 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-/* One-launch form: tiles of 256 messages.  Between 6000 and 7000 messages the workgroups' own look at
- * everything before them comes to cost what the second launch does (4.3 against 6.2 us at 1000 messages, 4.8
- * against 5.7 at 4000, 6.2 against 5.7 at 8000). */
-constexpr uint32_t kDirectTile = 256;
-constexpr uint64_t kDirectBatch = 6144;
-static_assert(4 * kDirectBatch <= 65536, "packed sums of a whole batch: up to 4 stripes a message, and the seed");
+/* One-launch form: tiles of 256 messages up to two of them, of 512 beyond, whose twice as many threads share the look
+ * at everything before the tile (in us, tiles of 256 / 512 / 1024: 3000 messages 4.7 / 4.3 / 5.1, 6144 5.9 / 4.9 / 5.4).
+ * That look grows until it costs what the second launch does: 7000 messages 5.2 against 7.6 us in two launches, 9900 5.7
+ * and 7.7, 12,000 6.2 and 7.6.  (The tests of the launches hold 10,000 to two.) */
+constexpr uint32_t kDirectTile = 256, kDirectTileLarge = 512;
+constexpr uint64_t kDirectBatch = 9984;
 /* Two-launch form: tiles of 512 messages, counted by 256 threads and written by 512 (21.5 us per 1,000,000
  * messages, 39.0 per 2,000,000; 256 threads twice 21.6 and 40.2, 128 threads four times 23.9 and 43.5). */
 constexpr uint32_t kTile = 512;
@@ -282,8 +282,9 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	const bool live = i < n;
 	const uint64_t size = live ? __builtin_nontemporal_load(&sizes[i]) : 0;
 	uint32_t acc = 0;
-	/* DIRECT: the first messages before the tile, requested along with its own */
-	constexpr uint32_t kAhead = 16;
+	/* DIRECT: the first messages before the tile, requested along with its own (8 at a time: 6144 messages 4.93 us,
+	 * 12 or 16 at a time 4.9-5.0, 5000 4.73, 4.80 and 4.92) */
+	constexpr uint32_t kAhead = THREADS == kDirectTile ? 1 : 8;
 	uint64_t before[kAhead];
 	auto look_ahead = [&](uint32_t i0) {
 #pragma unroll
@@ -341,14 +342,14 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	const uint32_t c = live ? contribution(size, p, k) : 0;
 	const uint32_t inc = wave_inclusive_scan(c);
 	if (lane == 0) {
-		seed_sum[wave] = acc;
+		/* the one reader of the counters in a workgroup of the one-launch form: behind the barrier they have been read */
+		seed_sum[wave] = acc + (FORM == DIRECT && wave == 0 ? batch_seed(state, R) : 0u);
 	}
 	if (lane == 63) {
 		wave_sum[wave] = inc;
 	}
-	const uint32_t seed = FORM == DIRECT ? batch_seed(state, R) : *seed0;
+	uint32_t before_tile = FORM == DIRECT ? 0u : *seed0, off = 0, tot = 0;
 	__syncthreads();
-	uint32_t before_tile = seed, off = 0, tot = 0;
 #pragma unroll
 	for (uint32_t w = 0; w < kWaves; w++) {
 		const uint32_t ws = wave_sum[w];
@@ -357,6 +358,21 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 		before_tile += seed_sum[w];
 	}
 	const uint32_t carry_small = (before_tile >> 16) % R, carry_big = (before_tile & 0xffffu) % R;
+	const uint32_t after_small = mod_rails(carry_small + (tot >> 16), p);
+	const uint32_t after_big = mod_rails(carry_big + (tot & 0xffffu), p);
+	/* Every workgroup reads the counters, so they may only be moved on when all have: each adds itself to the
+	 * batch's arrival word (low half), the last tile's with the carries behind it (high half), as soon as it has
+	 * read them, and whoever is last puts them in place and leaves the word at zero.  The answer is there when the
+	 * rows are written (behind the rows the add took 0.25 us of the launch).
+	 * A later batch's word is cleared on the way, whatever is in it (kArrivalWords). */
+	uint32_t arrived = 0;
+	if (FORM == DIRECT && num_tiles > 1 && threadIdx.x == 0) {
+		if (tile == 0) {
+			__hip_atomic_store(arrival_ahead, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		}
+		const uint32_t mine = 1u + (tile == num_tiles - 1 ? (after_small << 16) | (after_big << 20) : 0u);
+		arrived = mine + __hip_atomic_fetch_add(seed0, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
 	const uint32_t excl = off + inc - c;
 
 	/* set_schedule_by_threshold, src/nccl_ofi_scheduler.cpp:77-133 */
@@ -412,22 +428,11 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	if (threadIdx.x != 0) {
 		return;
 	}
-	const uint32_t after_small = mod_rails(carry_small + (tot >> 16), p);
-	const uint32_t after_big = mod_rails(carry_big + (tot & 0xffffu), p);
 	if (FORM == DIRECT && num_tiles > 1) {
-		/* Every workgroup has read the counters, so they may only be moved on when all are done:
-		 * each adds itself to the batch's arrival word (low half), the last tile's with the carries
-		 * behind it (high half), and whoever is last puts them in place and leaves the word at zero.
-		 * A later batch's word is cleared on the way, whatever is in it (kArrivalWords). */
-		if (tile == 0) {
-			__hip_atomic_store(arrival_ahead, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		}
-		const uint32_t mine = 1u + (tile == num_tiles - 1 ? (after_small << 16) | (after_big << 20) : 0u);
-		const uint32_t all = mine + __hip_atomic_fetch_add(seed0, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		if ((all & 0xffffu) == num_tiles) {
+		if ((arrived & 0xffffu) == num_tiles) {
 			__hip_atomic_store(seed0, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			state->rr_small_counter = (all >> 16) & 3u;
-			state->rr_counter = (all >> 20) & 3u;
+			state->rr_small_counter = (arrived >> 16) & 3u;
+			state->rr_counter = (arrived >> 20) & 3u;
 		}
 	} else if (tile == num_tiles - 1) {
 		/* the carries after the last tile are the counters the next batch starts from;
@@ -587,11 +592,19 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 	uint32_t *words = scratch.words;
 	uint32_t *seed0 = words + kSeedWord, *blocks = words + kBlockWords, *totals = words + kTileWords;
 	if (total <= kDirectTile || (total <= kDirectBatch && !being_captured(s))) {
-		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kDirectTile);
+		const bool large = total > 2 * kDirectTile;
+		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, large ? kDirectTileLarge : kDirectTile);
 		const uint32_t turn = tiles > 1 ? scratch.turn.fetch_add(1, std::memory_order_relaxed) : 0u;
-		hipLaunchKernelGGL((stripe_emit_kernel<DIRECT, kDirectTile>), dim3(tiles), dim3(kDirectTile), 0, s, d_sizes, n,
-				   d_state, align, nullptr, nullptr, words + turn % kArrivalWords,
-				   words + (turn + kArrivalWords / 2) % kArrivalWords, tiles, d_num_xfers, d_xfers, err);
+		auto launch = [&](auto kernel, uint32_t threads) {
+			hipLaunchKernelGGL(kernel, dim3(tiles), dim3(threads), 0, s, d_sizes, n, d_state, align, nullptr, nullptr,
+					   words + turn % kArrivalWords, words + (turn + kArrivalWords / 2) % kArrivalWords, tiles,
+					   d_num_xfers, d_xfers, err);
+		};
+		if (large) {
+			launch(stripe_emit_kernel<DIRECT, kDirectTileLarge>, kDirectTileLarge);
+		} else {
+			launch(stripe_emit_kernel<DIRECT, kDirectTile>, kDirectTile);
+		}
 		return;
 	}
 	if (total <= kSmallBatch) {

@@ -89,6 +89,33 @@ def test_batches_around_the_forms_of_the_launch(lib, oracle, gpu, n, rails, min_
         assert (st.rr_small_counter, st.rr_counter) == seeds
 
 
+@pytest.mark.parametrize("n", [256, 257, 512, 513, 1024, 1025, 1537, 4096, 4097, 4608, 4609, 5121, 8705, 9983, 9984, 9985])
+@pytest.mark.parametrize("rails,max_small", [(4, 64), (3, 5000), (1, 0)])
+def test_tiles_of_the_one_launch_form(lib, oracle, gpu, n, rails, max_small):
+    """Tiles of 256 messages up to two of them and of 512 beyond, with remainders, one and more turns of the look at the
+    messages before a tile, the form's largest batch and the next one; five in a row without a wait between them, so
+    that each starts from the counters the one before has moved on."""
+    sizes = [synthetic.stripe_sizes(n * 7 + rails + k, n) for k in range(5)]
+    d_state = dev_state(rails, 100000, max_small, (rails - 1, 0))
+    seeds, out = (rails - 1, 0), []
+    d_sizes = [_gpu.to_dev(s) for s in sizes]
+    for k in range(5):
+        d_num = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+        d_xf = torch.full((n * 12,), -1, dtype=torch.int64, device="cuda")
+        out.append((d_num, d_xf))
+    for k in range(5):
+        assert lib.ofi_amd_sched_batch(d_state.data_ptr(), d_sizes[k].data_ptr(), n, 128, out[k][0].data_ptr(),
+                                       out[k][1].data_ptr(), _gpu.stream()) == 0
+    _gpu.sync()
+    for k in range(5):
+        want_num, want_xf, ost = _oracle.sched_batch(oracle, sizes[k], rails, 100000, max_small, seeds)
+        seeds = (ost.rr_small_counter, ost.rr_counter)
+        assert np.array_equal(_gpu.to_host(out[k][0], np.uint32), want_num), k
+        assert np.array_equal(_gpu.to_host(out[k][1], np.uint64).reshape(n, 4, 3), want_xf), k
+    st = read_state(d_state)
+    assert (st.rr_small_counter, st.rr_counter) == seeds
+
+
 @pytest.mark.parametrize("min_stripe", [1, (1 << 62) - 1, 1 << 62, (1 << 63) + 5, (1 << 64) - 1])
 def test_stripe_sizes_whose_multiples_do_not_fit_64_bits(lib, oracle, gpu, min_stripe):
     sizes = np.array([0, 1, 2, 3, 4, 5, 64, (1 << 62) - 1, 1 << 62, (1 << 62) + 1, (1 << 63) - 1, 1 << 63, (1 << 63) + 6,
