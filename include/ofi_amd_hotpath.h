@@ -127,7 +127,7 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
  * A caller that destroys a stream, or a thread that ends after calls on hipStreamPerThread, hands
  * the scratch back first: waits for the stream, frees.
  * A batch captured into a graph keeps the scratch of the stream it was captured on: replays are
- * ordered with each other and with that stream's batches of more than 6144 messages. */
+ * ordered with each other and with that stream's batches of more than 9984 messages. */
 int ofi_amd_sched_stream_release(void *stream);
 
 /*

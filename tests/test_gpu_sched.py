@@ -71,7 +71,7 @@ def test_parity_random(lib, oracle, gpu, n, rails, min_stripe, max_small, seeds)
 @pytest.mark.parametrize("n", [255, 257, 4097, 6143, 6144, 6145, 6656, 6 << 20, (6 << 20) + 1, (6 << 20) + 4097, (1 << 24) + 1])
 @pytest.mark.parametrize("rails,min_stripe,max_small", [(4, 131072, 64), (3, 100000, 5000)])
 def test_batches_around_the_forms_of_the_launch(lib, oracle, gpu, n, rails, min_stripe, max_small):
-    """Batches of the one-launch form up to its largest (6144), of the form with tiles of 512 up to its largest
+    """Batches of the one-launch form, of the form with tiles of 512 up to its largest
     (6 Mi) and the smallest ones of the next, with whole and ragged tiles and blocks of tiles and a second
     part of one message; twice in a row, so that the second one starts from what the first left in the
     state and in the scratch."""

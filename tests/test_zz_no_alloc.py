@@ -1,6 +1,6 @@
 """GPU parity of the striping entry point that allocates nothing (ofi_amd_sched_batch_noalloc)
 against ofi_amd_sched_batch and the CPU oracle: calls in a row on the same scratch in each of the three launch
-forms (up to 6144 messages, up to 6 Mi, and beyond in parts of 2^24), smaller ones after larger ones."""
+forms (up to 9984 messages, up to 6 Mi, and beyond in parts of 2^24), smaller ones after larger ones."""
 import ctypes
 
 import numpy as np
