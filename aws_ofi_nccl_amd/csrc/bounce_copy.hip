@@ -87,8 +87,7 @@ __device__ __forceinline__ u32x4 load16_dword_aligned(const uint8_t *p)
 
 /*
  * Every access to a destination carries the same cache policy, the streaming one, but for the first rows of batches
- * that fit the L2s (kKeepBytes): the 16-byte
- * stores of the rows, the single head and tail bytes and the read-back of the flush.  With the
+ * that fit the L2s (kKeepBytes): the 16-byte stores of the rows, the single head and tail bytes and the read-back of the flush.  With the
  * rows streaming and the tail bytes and the read-back as ordinary accesses, the same batch
  * launched over and over on the same buffers slowed down by 6 % within 2,000 launches (91 ->
  * 97 us; fewer and fewer of those ordinary lines leave the L2 between launches, and a read
@@ -163,22 +162,41 @@ template <bool SHIFTED, bool KEEP>
 __device__ __forceinline__ void copy_words(const uint8_t *__restrict__ s, uint8_t *__restrict__ d,
 					   uint32_t nvec, uint32_t shift, uint32_t lane)
 {
-	while (nvec > kTripVec) { /* buffers beyond 8 KiB: whole trips first */
-		copy_rows<kRows, SHIFTED, true, KEEP>(s, d, kTripVec, shift, lane);
+	auto part = [&](uint32_t n) { /* at most a trip */
+		switch ((n + 63u) >> 6) { /* wave-uniform */
+		case 1: copy_rows<1, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		case 2: copy_rows<2, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		case 3: copy_rows<3, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		case 4: copy_rows<4, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		case 5: copy_rows<5, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		case 6: copy_rows<6, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		case 7: copy_rows<7, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		case 8: copy_rows<8, SHIFTED, false, KEEP>(s, d, n, shift, lane); break;
+		default: break; /* n == 0 */
+		}
+	};
+	auto whole = [&] {
+		copy_rows<kRows, SHIFTED, true, false>(s, d, kTripVec, shift, lane);
 		s += (uint64_t)kTripVec << 4;
 		d += (uint64_t)kTripVec << 4;
 		nvec -= kTripVec;
-	}
-	switch ((nvec + 63u) >> 6) { /* wave-uniform */
-	case 1: copy_rows<1, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	case 2: copy_rows<2, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	case 3: copy_rows<3, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	case 4: copy_rows<4, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	case 5: copy_rows<5, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	case 6: copy_rows<6, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	case 7: copy_rows<7, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	case 8: copy_rows<8, SHIFTED, false, KEEP>(s, d, nvec, shift, lane); break;
-	default: break; /* nvec == 0 */
+	};
+	if constexpr (KEEP) {
+		/* the trip that is less than whole is the first, so that one row of a buffer is kept however long it
+		 * is (12,000 eager buffers of up to 16 KiB with a row of every trip kept 50.4 us, streamed 43.5) */
+		const uint32_t n = nvec != 0 ? (nvec - 1u) % kTripVec + 1u : 0u;
+		part(n);
+		s += (uint64_t)n << 4;
+		d += (uint64_t)n << 4;
+		nvec -= n;
+		while (nvec != 0) {
+			whole();
+		}
+	} else {
+		while (nvec > kTripVec) { /* buffers beyond 8 KiB: whole trips first */
+			whole();
+		}
+		part(nvec);
 	}
 }
 
@@ -540,20 +558,23 @@ constexpr size_t kCpuLoadMax = 256;
 
 /*
  * Batches that fit the L2s (8 x 4 MiB) with room to spare keep the first row of every buffer in them instead of
- * streaming it: the read-back behind it then finds its line there.  The bytes of a bounce batch are the packed source's,
- * those of an eager batch are not known beyond 8 KiB a buffer.  Times in us on other buffers at every launch / on the
+ * streaming it: the read-back behind it then finds its line there.  The bytes of a bounce batch are at most the
+ * source's where that is packed; where it is a pool that the batch takes a part of, and in an eager batch, the number
+ * of buffers, which are mostly up to 8 KiB, has to do.  Times in us on other buffers at every launch / on the
  * same ones, streamed and then kept:
  *   4000 bounce buffers of up to 8 KiB      8.5 / 7.3    7.5 / 6.4
  *   8000 of up to 8 KiB                    14.5 / 13.2  13.7 / 12.0
+ *   8000 of up to 1000 B                    5.2 / 4.8    4.7 / 4.3   (each read back by itself: 4.9 / 4.5)
  *   65,536 of up to 500 B                  26.2 / 22.5  20.9 / 19.4
  *   10,000 of up to 8 KiB                  17.1 / 16.0  18.0 / 15.4  (together: 16.5 / 15.3)
  *   20,000 of up to 8 KiB                  29.9 / 29.7  35.4 / 26.9
- *   8000 eager buffers of up to 8 KiB      16.1 / 14.9  14.8 / 12.4
- *   12,000 of up to 8 KiB                  21.6 / 21.1  21.2 / 18.3
+ *   8000 eager buffers of up to 8 KiB      14.9 / 13.7  14.1 / 12.2
+ *   9000 of up to 8 KiB                    16.2 / 15.4  16.3 / 13.5
+ *   12,000 of up to 8 KiB                  20.0 / 19.9  21.6 / 17.7
  *   16,000 of up to 8 KiB                  27.5 / 26.0  32.2 / 23.0
  */
 constexpr uint64_t kKeepBytes = 32ull << 20;
-constexpr uint32_t kKeepEager = 12000;
+constexpr uint32_t kKeepBounce = 8000, kKeepEager = 9000;
 /*
  * Large batches of long buffers go with 24 wavefronts a CU instead of 32: reads and writes of 65,536 buffers take turns
  * at the memory, and the fewer of them are under way the longer the turns are (other buffers at every launch / the same
@@ -567,7 +588,10 @@ constexpr uint32_t kKeepEager = 12000;
  * claims: six of four wavefronts fit a CU.
  */
 constexpr uint64_t kFewerWavesBytes = 100ull << 20;
-constexpr uint64_t kFewerWavesLength = 2900; /* on average */
+constexpr uint64_t kFewerWavesLength = 2900; /* on average ... */
+/* ... and less than this: a source that holds more for every buffer is rather a pool that the batch takes a part of,
+ * and its buffers may be short (65,536 of up to 1000 B out of 1 GiB 27.0 us with 32 wavefronts, 35.1 with 24). */
+constexpr uint64_t kFewerWavesMost = 8192;
 constexpr int kFewerWaves = 4;
 constexpr uint32_t kFewerWavesLds = 27000;
 static_assert(6 * (kFewerWavesLds + sizeof(read_backs_t<kFewerWaves>)) <= 160 * 1024 &&
@@ -601,9 +625,9 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 				   static_cast<const uint8_t *>(d_src), src_bytes, static_cast<uint8_t *>(d_arena), arena_bytes,
 				   d_src_off, d_dst_off, d_len, n, d_flush, err);
 	};
-	if (d_flush && src_bytes <= kKeepBytes) {
+	if (d_flush && (src_bytes <= kKeepBytes || n <= kKeepBounce)) {
 		launch(bounce_scatter_kernel<kBounceWaves, true>, kBounceWaves, 0);
-	} else if (src_bytes >= kFewerWavesBytes && src_bytes / n >= kFewerWavesLength) {
+	} else if (src_bytes >= kFewerWavesBytes && src_bytes / n >= kFewerWavesLength && src_bytes / n < kFewerWavesMost) {
 		launch(bounce_scatter_kernel<kFewerWaves, false>, kFewerWaves, kFewerWavesLds);
 	} else {
 		launch(bounce_scatter_kernel<kBounceWaves, false>, kBounceWaves, 0);

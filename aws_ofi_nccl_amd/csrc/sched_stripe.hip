@@ -44,6 +44,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
  * and 7.7, 12,000 6.2 and 7.6.  (The tests of the launches hold 10,000 to two.) */
 constexpr uint32_t kDirectTile = 256, kDirectTileLarge = 512;
 constexpr uint64_t kDirectBatch = 9984;
+static_assert(4 * kDirectBatch < 65536 - 8, "packed sums of a whole batch: up to 4 stripes a message, and the seed");
 /* Two-launch form: tiles of 512 messages, counted by 256 threads and written by 512 (21.5 us per 1,000,000
  * messages, 39.0 per 2,000,000; 256 threads twice 21.6 and 40.2, 128 threads four times 23.9 and 43.5). */
 constexpr uint32_t kTile = 512;
