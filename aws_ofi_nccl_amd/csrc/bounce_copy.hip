@@ -87,9 +87,9 @@ __device__ __forceinline__ u32x4 load16_dword_aligned(const uint8_t *p)
 
 /*
  * Every access to a destination carries the same cache policy, the streaming one, but for the first rows of batches
- * that fit the L2s (kKeepBytes): the 16-byte stores of the rows, the single head and tail bytes and the read-back of the flush.  With the
- * rows streaming and the tail bytes and the read-back as ordinary accesses, the same batch
- * launched over and over on the same buffers slowed down by 6 % within 2,000 launches (91 ->
+ * that fit the L2s (kKeepBytes): the 16-byte stores of the rows, the single head and tail bytes and the
+ * read-back of the flush.  With the rows streaming and the tail bytes and the read-back as ordinary
+ * accesses, the same batch launched over and over on the same buffers slowed down by 6 % within 2,000 launches (91 ->
  * 97 us; fewer and fewer of those ordinary lines leave the L2 between launches, and a read
  * sweep of 16 MiB of other memory brought the first rate back); with one policy the rate does
  * not move (91 us from the first launch to the 20,000th).
