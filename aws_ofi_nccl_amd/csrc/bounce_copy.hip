@@ -207,12 +207,12 @@ __device__ __forceinline__ void copy_words(const uint8_t *__restrict__ s, uint8_
  * adds itself to `arrived` behind a workgroup fence, so the last one's loads follow all of the stores.
  * 20,000 buffers of up to 4 KiB 17.9 -> 17.0 us, 65,536 of up to 8 KiB launched over and over 88.3 -> 82.2.
  */
-template <int WAVES> struct read_backs_t {
-	uint64_t at[WAVES]; /* 0: none */
+struct read_backs_t {
+	uint64_t at[kBounceWaves]; /* 0: none */
 	uint32_t arrived;
 };
 
-template <int WAVES> __device__ __forceinline__ void begin_read_backs(read_backs_t<WAVES> &r)
+__device__ __forceinline__ void begin_read_backs(read_backs_t &r)
 {
 	if (threadIdx.x == 0) {
 		r.arrived = 0;
@@ -221,8 +221,7 @@ template <int WAVES> __device__ __forceinline__ void begin_read_backs(read_backs
 }
 
 /* By a wavefront behind its copy; true in the last of `here`, with everyone's entries in view. */
-template <int WAVES>
-__device__ __forceinline__ bool arrive(read_backs_t<WAVES> &r, uint32_t wave, uint32_t lane, const uint8_t *d, uint32_t here)
+__device__ __forceinline__ bool arrive(read_backs_t &r, uint32_t wave, uint32_t lane, const uint8_t *d, uint32_t here)
 {
 	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
 	uint32_t before = 0;
@@ -235,15 +234,15 @@ __device__ __forceinline__ bool arrive(read_backs_t<WAVES> &r, uint32_t wave, ui
 	return before == here - 1u;
 }
 
-template <int WAVES, bool KEEP>
-__global__ __launch_bounds__(64 * WAVES) void bounce_scatter_kernel(
+template <bool KEEP>
+__global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
 	const uint8_t *__restrict__ src, uint64_t src_bytes, uint8_t *__restrict__ arena, uint64_t arena_bytes,
 	const uint64_t *__restrict__ src_off, const uint64_t *__restrict__ dst_off,
 	const uint32_t *__restrict__ len, uint32_t n, uint32_t *__restrict__ flush,
 	uint32_t *__restrict__ err)
 {
-	__shared__ read_backs_t<WAVES> back;
-	constexpr uint32_t kGroup = kBounceRun / WAVES;
+	__shared__ read_backs_t back;
+	constexpr uint32_t kGroup = kBounceRun / kBounceWaves;
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const bool together = !KEEP && flush != nullptr;
@@ -258,7 +257,7 @@ __global__ __launch_bounds__(64 * WAVES) void bounce_scatter_kernel(
 	const uint32_t xcd = blockIdx.x % kXcds;
 	const uint32_t turn = blockIdx.x / kXcds;
 	const uint32_t wg = ((turn / kGroup) * kXcds + xcd) * kGroup + turn % kGroup;
-	const uint32_t first = wg * WAVES, buf = first + wave;
+	const uint32_t first = wg * kBounceWaves, buf = first + wave;
 	if (buf >= n) {
 		return;
 	}
@@ -298,7 +297,7 @@ __global__ __launch_bounds__(64 * WAVES) void bounce_scatter_kernel(
 	}
 
 	if (together) {
-		const uint32_t here = min(n - first, (uint32_t)WAVES);
+		const uint32_t here = min(n - first, (uint32_t)kBounceWaves);
 		if (arrive(back, wave, lane, in_range ? d : nullptr, here) && lane < here && back.at[lane] != 0) {
 			flush[first + lane] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(back.at[lane]));
 		}
@@ -576,26 +575,12 @@ constexpr size_t kCpuLoadMax = 256;
 constexpr uint64_t kKeepBytes = 32ull << 20;
 constexpr uint32_t kKeepBounce = 8000, kKeepEager = 9000;
 /*
- * Large batches of long buffers go with 24 wavefronts a CU instead of 32: reads and writes of 65,536 buffers take turns
- * at the memory, and the fewer of them are under way the longer the turns are (other buffers at every launch / the same
- * ones over and over, us):
- *   65,536 of up to 8 KiB         32 by eights 112.7 / 82.0   24 by fours 108.4 / 86.8   16 by eights 109.6 / 91.1
- *   32,768 of up to 8 KiB                       57.4 / 42.5                55.9 / 43.6
- *   65,536 of up to 6000 B                      83.5 / 61.4                81.6 / 65.5
- *   65,536 of up to 4 KiB                       59.5 / 44.9                63.2 / 53.1
- * (all of them with the read-backs together; each by itself, 32 by eights, 111.4 / 88.4 in the first line).  Below,
- * short buffers want every wavefront there is, to have enough under way.  The limit is set by the LDS a workgroup
- * claims: six of four wavefronts fit a CU.
+ * Fewer wavefronts a CU for large batches of long buffers -- reads and writes take turns at the memory, and the fewer
+ * buffers are open the longer the turns are -- were measured and are not used: 65,536 of up to 8 KiB 110.9 us with 32
+ * wavefronts, 109.0 with 24 and 107.2 with 20 (limited by the LDS a workgroup claims) on other buffers at every launch, but
+ * 81.1, 84.1 and 86.5 on the same ones over and over, and short buffers starve (65,536 of up to 1000 B 25.2 / 31.2 /
+ * 34.8).  The host has no lengths to choose by: src_bytes is the range the batch's offsets lie in, a pool as a rule.
  */
-constexpr uint64_t kFewerWavesBytes = 100ull << 20;
-constexpr uint64_t kFewerWavesLength = 2900; /* on average ... */
-/* ... and less than this: a source that holds more for every buffer is rather a pool that the batch takes a part of,
- * and its buffers may be short (65,536 of up to 1000 B out of 1 GiB 27.0 us with 32 wavefronts, 35.1 with 24). */
-constexpr uint64_t kFewerWavesMost = 8192;
-constexpr int kFewerWaves = 4;
-constexpr uint32_t kFewerWavesLds = 27000;
-static_assert(6 * (kFewerWavesLds + sizeof(read_backs_t<kFewerWaves>)) <= 160 * 1024 &&
-	      7 * kFewerWavesLds > 160 * 1024, "six workgroups to a CU");
 
 using namespace ofi_amd;
 
@@ -620,17 +605,15 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 		return -ENOMEM;
 	}
 	const uint32_t runs = (n + kXcds * kBounceRun - 1) / (kXcds * kBounceRun); /* whole rounds over the XCDs */
-	auto launch = [&](auto kernel, uint32_t waves, uint32_t lds) {
-		hipLaunchKernelGGL(kernel, dim3(runs * kXcds * (kBounceRun / waves)), dim3(64 * waves), lds, as_stream(stream),
-				   static_cast<const uint8_t *>(d_src), src_bytes, static_cast<uint8_t *>(d_arena), arena_bytes,
-				   d_src_off, d_dst_off, d_len, n, d_flush, err);
+	auto launch = [&](auto kernel) {
+		hipLaunchKernelGGL(kernel, dim3(runs * kXcds * (kBounceRun / kBounceWaves)), dim3(64 * kBounceWaves), 0,
+				   as_stream(stream), static_cast<const uint8_t *>(d_src), src_bytes, static_cast<uint8_t *>(d_arena),
+				   arena_bytes, d_src_off, d_dst_off, d_len, n, d_flush, err);
 	};
 	if (d_flush && (src_bytes <= kKeepBytes || n <= kKeepBounce)) {
-		launch(bounce_scatter_kernel<kBounceWaves, true>, kBounceWaves, 0);
-	} else if (src_bytes >= kFewerWavesBytes && src_bytes / n >= kFewerWavesLength && src_bytes / n < kFewerWavesMost) {
-		launch(bounce_scatter_kernel<kFewerWaves, false>, kFewerWaves, kFewerWavesLds);
+		launch(bounce_scatter_kernel<true>);
 	} else {
-		launch(bounce_scatter_kernel<kBounceWaves, false>, kBounceWaves, 0);
+		launch(bounce_scatter_kernel<false>);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;

@@ -33,6 +33,7 @@ namespace {
 struct launch_t {
 	std::string kernel; /* demangled, with its template arguments */
 	dim3 grid, block;
+	size_t shared;
 	void **args;
 	hipStream_t stream;
 	template <typename T> T arg(int i) const { return *static_cast<T *>(args[i]); }
@@ -117,13 +118,13 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
 	*grid = pushed.grid, *block = pushed.block, *shared = pushed.shared, *stream = pushed.stream;
 	return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t, hipStream_t stream)
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t shared, hipStream_t stream)
 {
 	/* what HIP supports: fewer than 2^32 work-items along each dimension */
 	if ((uint64_t)grid.x * block.x >> 32 || (uint64_t)grid.y * block.y >> 32 || (uint64_t)grid.z * block.z >> 32) {
 		return last_error = hipErrorInvalidConfiguration;
 	}
-	on_launch({ kernels()[f], grid, block, args, stream });
+	on_launch({ kernels()[f], grid, block, shared, args, stream });
 	return hipSuccess;
 }
 
@@ -308,6 +309,38 @@ int pieces()
 	return 0;
 }
 
+/*
+ * The bytes of a bounce batch's source are the range its offsets lie in, a pool as a rule, and say nothing about how long
+ * the buffers are: beyond what the L2s hold the launch is the same whatever they are.
+ */
+int bounce()
+{
+	uint8_t *const src = reinterpret_cast<uint8_t *>(0x1000000), *const arena = reinterpret_cast<uint8_t *>(0x80000000000);
+	uint64_t *const off = reinterpret_cast<uint64_t *>(0x70000000000);
+	uint32_t *const len = reinterpret_cast<uint32_t *>(0x71000000000), *const words = reinterpret_cast<uint32_t *>(0x72000000000);
+	for (uint32_t *flush : { words, static_cast<uint32_t *>(nullptr) }) {
+		for (uint32_t n : { 8001u, 20000u, 65536u, 200000u }) {
+			std::string kernel;
+			dim3 block;
+			size_t shared = 0;
+			for (uint64_t mib : { 33ull, 64ull, 101ull, 130ull, 256ull, 512ull, 1024ull, 1ull << 16 }) {
+				int launches = 0;
+				on_launch = [&](const launch_t &l) {
+					if (kernel.empty()) {
+						kernel = l.kernel, block = l.block, shared = l.shared;
+					}
+					CHECK(l.kernel == kernel && l.block.x == block.x && l.shared == shared);
+					CHECK((uint64_t)l.grid.x * l.block.x >= 64ull * n && l.arg<uint64_t>(1) == mib << 20);
+					launches++;
+				};
+				CHECK(ofi_amd_bounce_scatter(src, mib << 20, arena, 1ull << 40, off, off, len, n, flush, nullptr) == 0);
+				CHECK(launches == 1);
+			}
+		}
+	}
+	return 0;
+}
+
 /* The tiles of a region grid follow its axes: on short ones too, most lanes have a point. */
 int tiles()
 {
@@ -376,7 +409,8 @@ int uploads()
 
 int main(int argc, char **argv)
 {
-	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces }, { "tiles", tiles }, { "uploads", uploads } };
+	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces },
+							       { "bounce", bounce }, { "tiles", tiles }, { "uploads", uploads } };
 	CHECK(argc == 2 && parts.count(argv[1]) && ofi_amd_gpu_init() == 0);
 	const int rc = parts.at(argv[1])();
 	std::printf("%s: %s\n", argv[1], rc == 0 ? "ok" : "failed");

@@ -96,9 +96,8 @@ def test_lengths_beyond_one_trip_and_every_row_count(lib, oracle, gpu):
                                         (99, 13001), (101, 8003), (101, 13001), (101, 13003), (101, 36700)])
 @pytest.mark.parametrize("flush", [True, False])
 def test_forms_by_the_size_of_the_source(lib, oracle, gpu, src_mib, n, flush):
-    """The first row kept in the L2 or streamed, the flush words of a workgroup read back together, fewer wavefronts a CU:
-    by the bytes of the source and the number of buffers.  Batches that fill a workgroup in part, short and long buffers side by side at any
-    source alignment, every fifth one outside the arena or the source: skipped and reported, its flush word untouched,
+    """The first row kept in the L2 or streamed, the flush words of a workgroup read back together: by the bytes of the
+    source and the number of buffers.  Batches that fill a workgroup in part, short and long buffers side by side at any source alignment, every fifth one outside the arena or the source: skipped and reported, its flush word untouched,
     and the others of its workgroup complete."""
     rng = np.random.default_rng(100 * src_mib + n)
     src_bytes = (src_mib << 20) + 13

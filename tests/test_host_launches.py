@@ -48,6 +48,12 @@ def test_copy_tables_of_many_pieces_stay_within_what_a_launch_can_number(driver)
     run(driver, "pieces")
 
 
+def test_a_bounce_batch_is_launched_alike_whatever_the_size_of_the_pool(driver):
+    """The bytes of the source are no measure of the buffers' lengths: short buffers out of a pool are not taken for
+    long ones."""
+    run(driver, "bounce")
+
+
 def test_region_tiles_fit_short_axes(driver):
     """A region grid of one size and many node counts, or the other way round, is not paid for by the square."""
     run(driver, "tiles")
