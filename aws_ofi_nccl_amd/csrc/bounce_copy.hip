@@ -41,7 +41,7 @@
  * last, partial unit is written by one instruction.
  *
  * Flush: behind its stores (they are write-through to the L2 of the XCD) the wave,
- * or the last one of its workgroup for all of them, re-reads the first 4 bytes
+ * or one of its workgroup for all of them, re-reads the first 4 bytes
  * of the destination through that L2 and writes them to d_flush[i].  No wider
  * fence is used: on a multi-XCD part a device-scope release per buffer would
  * write back the whole L2 each time; device-wide visibility of the copied
@@ -200,84 +200,39 @@ __device__ __forceinline__ void copy_words(const uint8_t *__restrict__ s, uint8_
 	}
 }
 
-/*
- * The flush words of a workgroup's buffers, streamed ones: the wavefront whose copy is done last reads all of them
- * back, in one instruction, so that the others' places are free for the next buffers meanwhile -- a read of a line
- * that has just been streamed takes longer than the copy of a short buffer.  Every wavefront says where its word is and then
- * adds itself to `arrived` behind a workgroup fence, so the last one's loads follow all of the stores.
- * 20,000 buffers of up to 4 KiB 17.9 -> 17.0 us, 65,536 of up to 8 KiB launched over and over 88.3 -> 82.2.
- */
-struct read_backs_t {
-	uint64_t at[kBounceWaves]; /* 0: none */
-	uint32_t arrived;
-};
+/* The flush words: no output for them, each buffer's read back by its own wavefront (kept rows), or a workgroup's
+ * together (streamed ones). */
+enum read_back_t { NO_READ_BACK, BY_ITSELF, TOGETHER };
 
-__device__ __forceinline__ void begin_read_backs(read_backs_t &r)
+constexpr uint64_t kNoOffset = ~0ull;
+
+/* Copies buffer buf of the batch; its place in the arena, or kNoOffset (skipped and reported) when it is out of range. */
+template <read_back_t BACK>
+__device__ __forceinline__ uint64_t bounce_buffer(const uint8_t *__restrict__ src, uint64_t src_bytes,
+						  uint8_t *__restrict__ arena, uint64_t arena_bytes,
+						  const uint64_t *__restrict__ src_off, const uint64_t *__restrict__ dst_off,
+						  const uint32_t *__restrict__ len, uint32_t buf, uint32_t lane,
+						  uint32_t *__restrict__ err)
 {
-	if (threadIdx.x == 0) {
-		r.arrived = 0;
-	}
-	__syncthreads();
-}
-
-/* By a wavefront behind its copy; true in the last of `here`, with everyone's entries in view. */
-__device__ __forceinline__ bool arrive(read_backs_t &r, uint32_t wave, uint32_t lane, const uint8_t *d, uint32_t here)
-{
-	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-	uint32_t before = 0;
-	if (lane == 0) {
-		r.at[wave] = (uint64_t)reinterpret_cast<uintptr_t>(d);
-		before = __hip_atomic_fetch_add(&r.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-	}
-	before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
-	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-	return before == here - 1u;
-}
-
-template <bool KEEP>
-__global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
-	const uint8_t *__restrict__ src, uint64_t src_bytes, uint8_t *__restrict__ arena, uint64_t arena_bytes,
-	const uint64_t *__restrict__ src_off, const uint64_t *__restrict__ dst_off,
-	const uint32_t *__restrict__ len, uint32_t n, uint32_t *__restrict__ flush,
-	uint32_t *__restrict__ err)
-{
-	__shared__ read_backs_t back;
-	constexpr uint32_t kGroup = kBounceRun / kBounceWaves;
-	const uint32_t lane = threadIdx.x & 63u;
-	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	const bool together = !KEEP && flush != nullptr;
-	if (together) {
-		begin_read_backs(back);
-	}
-	/* Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Runs of kBounceRun
-	 * consecutive buffers go to one XCD, so that neighbouring buffers
-	 * -- which share a cache line of the packed source at their boundary -- mostly meet in
-	 * the same L2, while every XCD still sees an even sample of the whole batch whatever
-	 * order the lengths come in. */
-	const uint32_t xcd = blockIdx.x % kXcds;
-	const uint32_t turn = blockIdx.x / kXcds;
-	const uint32_t wg = ((turn / kGroup) * kXcds + xcd) * kGroup + turn % kGroup;
-	const uint32_t first = wg * kBounceWaves, buf = first + wave;
-	if (buf >= n) {
-		return;
-	}
-
+	constexpr bool KEEP = BACK == BY_ITSELF;
 	const uint64_t doff = dst_off[buf];
 	const uint32_t bytes = len[buf];
 	const uint64_t soff = src_off[buf];
 	/* precondition check: skip (and report) instead of reading or writing out of range; the
 	 * read-back takes four bytes at the destination whatever the length */
-	const uint64_t need = (flush != nullptr && bytes < 4u) ? 4u : bytes;
-	const bool in_range = (doff & 63u) == 0 && doff <= arena_bytes && need <= arena_bytes - doff && soff <= src_bytes &&
-			      bytes <= src_bytes - soff;
-	if (!in_range && lane == 0) {
-		atomicOr(err, ofi_amd::ASYNC_ERR_BOUNCE_RANGE);
+	const uint64_t need = (BACK != NO_READ_BACK && bytes < 4u) ? 4u : bytes;
+	if ((doff & 63u) != 0 || doff > arena_bytes || need > arena_bytes - doff || soff > src_bytes ||
+	    bytes > src_bytes - soff) {
+		if (lane == 0) {
+			atomicOr(err, ofi_amd::ASYNC_ERR_BOUNCE_RANGE);
+		}
+		return kNoOffset;
 	}
 
 	const uint8_t *s = src + soff;
 	uint8_t *d = arena + doff;
 
-	if (in_range && bytes != 0) {
+	if (bytes != 0) {
 		/* whole 64-byte units as 16-byte words, the rest (up to 63 bytes) singly, one per
 		 * lane: the last, partial unit of memory is then written by one instruction rather
 		 * than by the end of a row and by the tail.  Tail bytes first, so their latency
@@ -295,16 +250,60 @@ __global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
 		}
 		store_byte_streaming(d + tail_at, tail_byte);
 	}
+	return doff;
+}
 
-	if (together) {
-		const uint32_t here = min(n - first, (uint32_t)kBounceWaves);
-		if (arrive(back, wave, lane, in_range ? d : nullptr, here) && lane < here && back.at[lane] != 0) {
-			flush[first + lane] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(back.at[lane]));
+/*
+ * TOGETHER: one wavefront reads the words of its workgroup's eight buffers back, in one instruction, behind a barrier,
+ * and the other seven are done: a read of a line that has just been streamed takes longer than the copy of a short
+ * buffer.  Each by itself and together, on other buffers at every launch / on the same ones over and over, us:
+ *   65,536 of up to 8 KiB                116.4 / 88.0  117.0 / 83.1
+ *   20,000 of up to 4 KiB                 17.0 / 16.5   16.1 / 15.6
+ *   65,536 of up to 1000 B out of a pool  25.7 / 25.4   24.0 / 23.8
+ *   65,536 of up to 60 B out of a pool    18.8 / 15.5   19.2 / 16.2
+ *   1,000,000 of up to 60 B out of a pool 222 / 219     229 / 221
+ * (Counting the wavefronts in an LDS word, for the last one to read back without a barrier, needs a barrier in front of
+ * the copies all the same, and is slower nearly everywhere: 117.0 / 83.0, 16.2 / 15.6, 24.3 / 24.0, 20.3 / 17.6, 232 / 229.)
+ * NO_READ_BACK is a kernel of its own because one that claims LDS starts later: 65,536 of up to 60 B 11.2 us with
+ * the claim, 9.8 without.
+ */
+template <read_back_t BACK>
+__global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
+	const uint8_t *__restrict__ src, uint64_t src_bytes, uint8_t *__restrict__ arena, uint64_t arena_bytes,
+	const uint64_t *__restrict__ src_off, const uint64_t *__restrict__ dst_off,
+	const uint32_t *__restrict__ len, uint32_t n, uint32_t *__restrict__ flush,
+	uint32_t *__restrict__ err)
+{
+	constexpr uint32_t kGroup = kBounceRun / kBounceWaves;
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	/* Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Runs of kBounceRun
+	 * consecutive buffers go to one XCD, so that neighbouring buffers
+	 * -- which share a cache line of the packed source at their boundary -- mostly meet in
+	 * the same L2, while every XCD still sees an even sample of the whole batch whatever
+	 * order the lengths come in. */
+	const uint32_t xcd = blockIdx.x % kXcds;
+	const uint32_t turn = blockIdx.x / kXcds;
+	const uint32_t wg = ((turn / kGroup) * kXcds + xcd) * kGroup + turn % kGroup;
+	const uint32_t first = wg * kBounceWaves, buf = first + wave;
+
+	uint64_t at = kNoOffset;
+	if (buf < n) {
+		at = bounce_buffer<BACK>(src, src_bytes, arena, arena_bytes, src_off, dst_off, len, buf, lane, err);
+	}
+	if constexpr (BACK == TOGETHER) {
+		__shared__ uint64_t back[kBounceWaves];
+		if (lane == 0) {
+			back[wave] = at;
 		}
-	} else if (flush != nullptr) {
+		__syncthreads(); /* the copies, too, are in front of it */
+		if (threadIdx.x < kBounceWaves && back[lane] != kNoOffset) {
+			flush[first + lane] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(arena + back[lane]));
+		}
+	} else if constexpr (BACK == BY_ITSELF) {
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-		if (lane == 0 && in_range) {
-			flush[buf] = *reinterpret_cast<const uint32_t *>(d);
+		if (lane == 0 && at != kNoOffset) {
+			flush[buf] = *reinterpret_cast<const uint32_t *>(arena + at);
 		}
 	}
 }
@@ -610,10 +609,12 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 				   as_stream(stream), static_cast<const uint8_t *>(d_src), src_bytes, static_cast<uint8_t *>(d_arena),
 				   arena_bytes, d_src_off, d_dst_off, d_len, n, d_flush, err);
 	};
-	if (d_flush && (src_bytes <= kKeepBytes || n <= kKeepBounce)) {
-		launch(bounce_scatter_kernel<true>);
+	if (!d_flush) {
+		launch(bounce_scatter_kernel<NO_READ_BACK>);
+	} else if (src_bytes <= kKeepBytes || n <= kKeepBounce) {
+		launch(bounce_scatter_kernel<BY_ITSELF>);
 	} else {
-		launch(bounce_scatter_kernel<false>);
+		launch(bounce_scatter_kernel<TOGETHER>);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;

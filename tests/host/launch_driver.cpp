@@ -311,13 +311,15 @@ int pieces()
 
 /*
  * The bytes of a bounce batch's source are the range its offsets lie in, a pool as a rule, and say nothing about how long
- * the buffers are: beyond what the L2s hold the launch is the same whatever they are.
+ * the buffers are: beyond what the L2s hold the launch is the same whatever they are.  A batch without flush words has a
+ * kernel of its own, which does none of their work.
  */
 int bounce()
 {
 	uint8_t *const src = reinterpret_cast<uint8_t *>(0x1000000), *const arena = reinterpret_cast<uint8_t *>(0x80000000000);
 	uint64_t *const off = reinterpret_cast<uint64_t *>(0x70000000000);
 	uint32_t *const len = reinterpret_cast<uint32_t *>(0x71000000000), *const words = reinterpret_cast<uint32_t *>(0x72000000000);
+	std::set<std::string> with[2];
 	for (uint32_t *flush : { words, static_cast<uint32_t *>(nullptr) }) {
 		for (uint32_t n : { 8001u, 20000u, 65536u, 200000u }) {
 			std::string kernel;
@@ -331,12 +333,16 @@ int bounce()
 					}
 					CHECK(l.kernel == kernel && l.block.x == block.x && l.shared == shared);
 					CHECK((uint64_t)l.grid.x * l.block.x >= 64ull * n && l.arg<uint64_t>(1) == mib << 20);
+					with[flush != nullptr].insert(l.kernel);
 					launches++;
 				};
 				CHECK(ofi_amd_bounce_scatter(src, mib << 20, arena, 1ull << 40, off, off, len, n, flush, nullptr) == 0);
 				CHECK(launches == 1);
 			}
 		}
+	}
+	for (const std::string &kernel : with[0]) {
+		CHECK(with[1].count(kernel) == 0);
 	}
 	return 0;
 }
