@@ -200,58 +200,36 @@ __device__ __forceinline__ void copy_words(const uint8_t *__restrict__ s, uint8_
 	}
 }
 
+/* bytes, at least one, from s to a 64-byte-aligned d; KEEP: the line at d is left to ordinary stores */
+template <bool KEEP>
+__device__ __forceinline__ void copy_to_aligned(const uint8_t *__restrict__ s, uint8_t *__restrict__ d, uint32_t bytes,
+						uint32_t lane)
+{
+	/* whole 64-byte units as 16-byte words, the rest (up to 63 bytes) singly, one per
+	 * lane: the last, partial unit of memory is then written by one instruction rather
+	 * than by the end of a row and by the tail.  Tail bytes first, so their latency
+	 * overlaps the body; unpredicated (lanes without a tail byte re-copy the buffer's
+	 * last byte) to stay branch-free */
+	const uint32_t nvec = (bytes >> 6) << 2;
+	const uint32_t tail_at = min((nvec << 4) + lane, bytes - 1u);
+	const uint8_t tail_byte = s[tail_at];
+
+	const uint32_t shift = (uint32_t)(reinterpret_cast<uintptr_t>(s) & 3u);
+	if (shift == 0) {
+		copy_words<false, KEEP>(s, d, nvec, 0, lane);
+	} else {
+		copy_words<true, KEEP>(s - shift, d, nvec, shift, lane);
+	}
+	if (KEEP && nvec == 0) { /* no row: the tail's line is the one read back */
+		d[tail_at] = tail_byte;
+	} else {
+		store_byte_streaming(d + tail_at, tail_byte);
+	}
+}
+
 /* The flush words: no output for them, each buffer's read back by its own wavefront (kept rows), or a workgroup's
  * together (streamed ones). */
 enum read_back_t { NO_READ_BACK, BY_ITSELF, TOGETHER };
-
-constexpr uint64_t kNoOffset = ~0ull;
-
-/* Copies buffer buf of the batch; its place in the arena, or kNoOffset (skipped and reported) when it is out of range. */
-template <read_back_t BACK>
-__device__ __forceinline__ uint64_t bounce_buffer(const uint8_t *__restrict__ src, uint64_t src_bytes,
-						  uint8_t *__restrict__ arena, uint64_t arena_bytes,
-						  const uint64_t *__restrict__ src_off, const uint64_t *__restrict__ dst_off,
-						  const uint32_t *__restrict__ len, uint32_t buf, uint32_t lane,
-						  uint32_t *__restrict__ err)
-{
-	constexpr bool KEEP = BACK == BY_ITSELF;
-	const uint64_t doff = dst_off[buf];
-	const uint32_t bytes = len[buf];
-	const uint64_t soff = src_off[buf];
-	/* precondition check: skip (and report) instead of reading or writing out of range; the
-	 * read-back takes four bytes at the destination whatever the length */
-	const uint64_t need = (BACK != NO_READ_BACK && bytes < 4u) ? 4u : bytes;
-	if ((doff & 63u) != 0 || doff > arena_bytes || need > arena_bytes - doff || soff > src_bytes ||
-	    bytes > src_bytes - soff) {
-		if (lane == 0) {
-			atomicOr(err, ofi_amd::ASYNC_ERR_BOUNCE_RANGE);
-		}
-		return kNoOffset;
-	}
-
-	const uint8_t *s = src + soff;
-	uint8_t *d = arena + doff;
-
-	if (bytes != 0) {
-		/* whole 64-byte units as 16-byte words, the rest (up to 63 bytes) singly, one per
-		 * lane: the last, partial unit of memory is then written by one instruction rather
-		 * than by the end of a row and by the tail.  Tail bytes first, so their latency
-		 * overlaps the body; unpredicated (lanes without a tail byte re-copy the buffer's
-		 * last byte) to stay branch-free */
-		const uint32_t nvec = (bytes >> 6) << 2;
-		const uint32_t tail_at = min((nvec << 4) + lane, bytes - 1u);
-		const uint8_t tail_byte = s[tail_at];
-
-		const uint32_t shift = (uint32_t)(reinterpret_cast<uintptr_t>(s) & 3u);
-		if (shift == 0) {
-			copy_words<false, KEEP>(s, d, nvec, 0, lane);
-		} else {
-			copy_words<true, KEEP>(s - shift, d, nvec, shift, lane);
-		}
-		store_byte_streaming(d + tail_at, tail_byte);
-	}
-	return doff;
-}
 
 /*
  * TOGETHER: one wavefront reads the words of its workgroup's eight buffers back, in one instruction, behind a barrier,
@@ -259,11 +237,11 @@ __device__ __forceinline__ uint64_t bounce_buffer(const uint8_t *__restrict__ sr
  * buffer.  Each by itself and together, on other buffers at every launch / on the same ones over and over, us:
  *   65,536 of up to 8 KiB                116.4 / 88.0  117.0 / 83.1
  *   20,000 of up to 4 KiB                 17.0 / 16.5   16.1 / 15.6
- *   65,536 of up to 1000 B out of a pool  25.7 / 25.4   24.0 / 23.8
- *   65,536 of up to 60 B out of a pool    18.8 / 15.5   19.2 / 16.2
+ *   65,536 of up to 1000 B out of a pool  25.7 / 25.4   24.3 / 24.0
+ *   65,536 of up to 60 B out of a pool    18.8 / 15.5   19.2 / 16.3
  *   1,000,000 of up to 60 B out of a pool 222 / 219     229 / 221
  * (Counting the wavefronts in an LDS word, for the last one to read back without a barrier, needs a barrier in front of
- * the copies all the same, and is slower nearly everywhere: 117.0 / 83.0, 16.2 / 15.6, 24.3 / 24.0, 20.3 / 17.6, 232 / 229.)
+ * the copies all the same: no faster for long buffers, the last two lines 20.3 / 17.6 and 232 / 229.)
  * NO_READ_BACK is a kernel of its own because one that claims LDS starts later: 65,536 of up to 60 B 11.2 us with
  * the claim, 9.8 without.
  */
@@ -286,24 +264,48 @@ __global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
 	const uint32_t turn = blockIdx.x / kXcds;
 	const uint32_t wg = ((turn / kGroup) * kXcds + xcd) * kGroup + turn % kGroup;
 	const uint32_t first = wg * kBounceWaves, buf = first + wave;
-
-	uint64_t at = kNoOffset;
-	if (buf < n) {
-		at = bounce_buffer<BACK>(src, src_bytes, arena, arena_bytes, src_off, dst_off, len, buf, lane, err);
+	if (BACK != TOGETHER && buf >= n) {
+		return;
 	}
+
+	uint8_t *d = nullptr; /* until there is something to read back */
+	if (BACK != TOGETHER || buf < n) { /* all of a workgroup come to the barrier of TOGETHER */
+		const uint64_t doff = dst_off[buf];
+		const uint32_t bytes = len[buf];
+		const uint64_t soff = src_off[buf];
+		/* precondition check: skip (and report) instead of reading or writing out of range; the
+		 * read-back takes four bytes at the destination whatever the length */
+		const uint64_t need = (BACK != NO_READ_BACK && bytes < 4u) ? 4u : bytes;
+		if ((doff & 63u) != 0 || doff > arena_bytes || need > arena_bytes - doff || soff > src_bytes ||
+		    bytes > src_bytes - soff) {
+			if (lane == 0) {
+				atomicOr(err, ofi_amd::ASYNC_ERR_BOUNCE_RANGE);
+			}
+			if (BACK != TOGETHER) {
+				return;
+			}
+		} else {
+			const uint8_t *s = src + soff;
+			d = arena + doff;
+			if (bytes != 0) {
+				copy_to_aligned<BACK == BY_ITSELF>(s, d, bytes, lane);
+			}
+		}
+	}
+
 	if constexpr (BACK == TOGETHER) {
-		__shared__ uint64_t back[kBounceWaves];
+		__shared__ uint8_t *back[kBounceWaves]; /* nullptr: none */
 		if (lane == 0) {
-			back[wave] = at;
+			back[wave] = d;
 		}
 		__syncthreads(); /* the copies, too, are in front of it */
-		if (threadIdx.x < kBounceWaves && back[lane] != kNoOffset) {
-			flush[first + lane] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(arena + back[lane]));
+		if (threadIdx.x < kBounceWaves && back[lane] != nullptr) {
+			flush[first + lane] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(back[lane]));
 		}
 	} else if constexpr (BACK == BY_ITSELF) {
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-		if (lane == 0 && at != kNoOffset) {
-			flush[buf] = *reinterpret_cast<const uint32_t *>(arena + at);
+		if (lane == 0) {
+			flush[buf] = *reinterpret_cast<const uint32_t *>(d);
 		}
 	}
 }
@@ -556,23 +558,28 @@ constexpr size_t kCpuLoadMax = 256;
 
 /*
  * Batches that fit the L2s (8 x 4 MiB) with room to spare keep the first row of every buffer in them instead of
- * streaming it: the read-back behind it then finds its line there.  The bytes of a bounce batch are at most the
- * source's where that is packed; where it is a pool that the batch takes a part of, and in an eager batch, the number
- * of buffers, which are mostly up to 8 KiB, has to do.  Times in us on other buffers at every launch / on the
- * same ones, streamed and then kept:
- *   4000 bounce buffers of up to 8 KiB      8.5 / 7.3    7.5 / 6.4
- *   8000 of up to 8 KiB                    14.5 / 13.2  13.7 / 12.0
- *   8000 of up to 1000 B                    5.2 / 4.8    4.7 / 4.3   (each read back by itself: 4.9 / 4.5)
- *   65,536 of up to 500 B                  26.2 / 22.5  20.9 / 19.4
- *   10,000 of up to 8 KiB                  17.1 / 16.0  18.0 / 15.4  (together: 16.5 / 15.3)
- *   20,000 of up to 8 KiB                  29.9 / 29.7  35.4 / 26.9
+ * streaming it (a buffer without a row, its tail): the read-back behind it then finds its line there.  The bytes of a
+ * bounce batch are at most the source's where that is packed; where it is a pool that the batch takes a part of, and in an
+ * eager batch, the number of buffers, which are mostly up to 8 KiB, has to do.  However short the buffers are, each keeps a
+ * line, and from some hundred thousand on these no longer fit (kKeepLines).  Times in us on other buffers at
+ * every launch / on the same ones, streamed (bounce: read back together) and then kept:
+ *   6000 bounce buffers of up to 8 KiB     10.9 / 10.2   9.7 / 9.2
+ *   8000 of up to 8 KiB                    13.7 / 12.2  13.1 / 12.0  (out of a pool 13.6 / 12.2  13.8 / 12.3)
+ *   10,000 of up to 8 KiB                  16.5 / 15.3  18.0 / 15.4
+ *   16,000 of up to 4 KiB                  13.6 / 12.6  12.8 / 12.0
+ *   60,000 of up to 1000 B                 22.8 / 22.2  18.5 / 17.9
+ *   65,536 of up to 60 B                   17.5 / 15.9  17.0 / 14.8  (its tail streamed: 18.9 / 14.9)
+ *   200,000 of up to 100 B                   62 / 55      48 / 48
+ *   450,000 of up to 60 B                   113 / 105     85 / 85
+ *   500,000 of up to 60 B                   123 / 117    113 / 93    (flush words in HBM 104 / 98  110 / 90)
+ *   700,000 of up to 60 B                   163 / 162    174 / 128
  *   8000 eager buffers of up to 8 KiB      14.9 / 13.7  14.1 / 12.2
  *   9000 of up to 8 KiB                    16.2 / 15.4  16.3 / 13.5
  *   12,000 of up to 8 KiB                  20.0 / 19.9  21.6 / 17.7
  *   16,000 of up to 8 KiB                  27.5 / 26.0  32.2 / 23.0
  */
 constexpr uint64_t kKeepBytes = 32ull << 20;
-constexpr uint32_t kKeepBounce = 8000, kKeepEager = 9000;
+constexpr uint32_t kKeepBounce = 8000, kKeepLines = 450000, kKeepEager = 9000;
 /*
  * Fewer wavefronts a CU for large batches of long buffers -- reads and writes take turns at the memory, and the fewer
  * buffers are open the longer the turns are -- were measured and are not used: 65,536 of up to 8 KiB 110.9 us with 32
@@ -611,7 +618,7 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 	};
 	if (!d_flush) {
 		launch(bounce_scatter_kernel<NO_READ_BACK>);
-	} else if (src_bytes <= kKeepBytes || n <= kKeepBounce) {
+	} else if (n <= kKeepBounce || (n <= kKeepLines && src_bytes <= kKeepBytes)) {
 		launch(bounce_scatter_kernel<BY_ITSELF>);
 	} else {
 		launch(bounce_scatter_kernel<TOGETHER>);

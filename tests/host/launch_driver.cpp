@@ -344,6 +344,14 @@ int bounce()
 	for (const std::string &kernel : with[0]) {
 		CHECK(with[1].count(kernel) == 0);
 	}
+	/* however short the buffers of a small source are, the lines of so many do not stay in the L2s */
+	auto kernel_of = [&](uint32_t n, uint64_t mib) {
+		std::string kernel;
+		on_launch = [&](const launch_t &l) { kernel = l.kernel; };
+		CHECK(ofi_amd_bounce_scatter(src, mib << 20, arena, 1ull << 40, off, off, len, n, words, nullptr) == 0);
+		return kernel;
+	};
+	CHECK(kernel_of(100000, 16) != kernel_of(100000, 33) && kernel_of(1000000, 16) == kernel_of(1000000, 33));
 	return 0;
 }
 

@@ -133,6 +133,24 @@ def test_forms_by_the_size_of_the_source(lib, oracle, gpu, src_mib, n, flush):
     assert bool(_gpu.fetch_async_errors(lib)) == bool(bad.any())
 
 
+@pytest.mark.parametrize("n", [449_999, 450_001])
+def test_many_buffers_without_a_row(lib, oracle, gpu, n):
+    """Buffers of up to 63 bytes are their tails, read back from the lines these leave: kept ones up to 450,000 buffers,
+    streamed ones beyond."""
+    rng = np.random.default_rng(n)
+    length = rng.integers(0, 64, n).astype(np.uint32)
+    src_off = (np.cumsum(length) - length).astype(np.uint64)
+    dst_off = rng.permutation(n).astype(np.uint64) * np.uint64(64)
+    src = synthetic.random_bytes(n, int(length.sum()) + 16)
+    want = np.full(n * 64, 0x3C, dtype=np.uint8)
+    want_flush = oracle_scatter(oracle, src, want, src_off, dst_off, length)
+    arena = torch.full((n * 64,), 0x3C, dtype=torch.uint8, device="cuda")
+    flush = scatter(lib, src, arena, src_off, dst_off, length)
+    assert np.array_equal(arena.cpu().numpy(), want)
+    assert np.array_equal(flush, want_flush)
+    assert _gpu.fetch_async_errors(lib) == 0
+
+
 def test_empty_batch_and_all_zero_lengths(lib, oracle, gpu):
     arena = torch.full((4096,), 9, dtype=torch.uint8, device="cuda")
     assert lib.ofi_amd_bounce_scatter(arena.data_ptr(), 4096, arena.data_ptr(), 4096, None, None, None, 0,
