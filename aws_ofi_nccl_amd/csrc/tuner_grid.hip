@@ -57,13 +57,23 @@ struct tiling_t {
 	const double2 *rank_span; /* per (tile column, ppn): smallest and largest log2_ranks */
 };
 
-/* Model workgroups have 256 threads and, from 48 MB of costs on, claim enough LDS that six of them share a CU instead of
- * eight, from 96 MB on 1024 threads: the fewer and longer the runs under way, the better they suit the memory.  Times in
- * us with eight and with six of 256, and with 1024 threads: 27 MB 7.0 / 7.4 / -, 40 MB 8.0 / 8.6 / 9.9, 60 MB 12.5 /
- * 12.0 / -, 85 MB 16.6 / 16.3 / 16.8, 133 MB 25.9 / - / 25.1, 266 MB 52.3 / - / 49.6, 495 MB 96.5 / 96.1 / 92.5. */
+/* Model workgroups have 256 threads and, from 48 MiB of costs on (68 where every point is modelled: 64 MB 13.0 us with
+ * eight and 14.3 with five, 76 MB 16.0 and 16.1, 82 MB 17.4 and 16.8), claim enough LDS that five of them share a CU instead
+ * of eight: the fewer and longer the runs under way, the better they suit the memory.  From 150 MiB on, 1024 threads write
+ * longer runs still, but they also evaluate the model all at once and then write all at once, so that they are
+ * the slower way where more than half of the points are modelled.  Times in us with eight and with five of 256, and with 1024
+ * threads, by the share of modelled points:
+ *           a third              half                 two thirds           all
+ *    45 MB   8.6 / 8.9 / 10.0     8.7 / 9.7 / 10.3     9.2 / 10.1 / 10.5   10.4 / 11.2 / 13.1
+ *    60 MB  12.5 / 12.0 / 12.0   12.3 / 12.4 / 13.0   13.5 / 12.0 / 13.5   13.2 / 13.9 / 15.1
+ *    85 MB  16.4 / 15.9 / 16.6   16.2 / 16.6 / 17.4   17.0 / 16.7 / 17.8   18.6 / 17.6 / 19.6
+ *   120 MB  23.0 / 22.6 / 22.8   23.0 / 23.0 / 23.9   23.8 / 23.2 / 24.3   24.8 / 23.2 / 25.3
+ *   180 MB  34.9 / 34.5 / 33.6   34.8 / 35.2 / 34.9   35.4 / 34.6 / 35.1   34.8 / 32.3 / 34.3
+ *   250 MB  47.9 / 47.4 / 46.2   48.4 / 48.0 / 48.1   48.3 / 47.8 / 48.0   47.5 / 43.2 / 45.9
+ *   480 MB  91.6 / 91.2 / 88.0   94.2 / 93.4 / 90.5   90.8 / 90.5 / 91.3   90.5 / 79.3 / 84.2 */
 constexpr uint32_t kModelThreads = 256, kModelThreadsLarge = 1024;
-constexpr uint64_t kModelSixBytes = 48ull << 20, kModelLargeBytes = 96ull << 20;
-constexpr size_t kModelSixLds = 27000;
+constexpr uint64_t kModelFewerBytes = 48ull << 20, kModelFewerBytesAll = 68ull << 20, kModelLargeBytes = 150ull << 20;
+constexpr size_t kModelFewerLds = 27000;
 constexpr size_t kModelLds = 64 * 1024; /* at most, for the larger ones */
 
 /* `cells` doubles at `out`, cell(k) each, by a workgroup: two to a lane and store, 1 KiB per wavefront
@@ -954,9 +964,19 @@ int ofi_amd_tuner_model_grid(ofi_amd_tuner_plan_t *plan, const ofi_amd_tuner_var
 	const uint32_t points = (uint32_t)plan->points;
 	const size_t row = (size_t)plan->g.n_algos * NUM_PROTOS * sizeof(float); /* of the stage */
 	const uint64_t bytes = d_cost ? plan->cells * n_variants * sizeof(double) : 0;
-	const bool large = bytes > kModelLargeBytes && row * kModelThreadsLarge <= kModelLds;
+	/* modelled points: AllReduce's, of the platforms that have a model */
+	uint64_t reduces = 0, with_model = 0;
+	for (int32_t coll : plan->h_colls) {
+		reduces += coll == FUNC_ALLREDUCE;
+	}
+	for (uint32_t i = 0; i < n_variants; i++) {
+		with_model += platform_has_model(variants[i].platform);
+	}
+	const uint64_t modelled = reduces * with_model, all = plan->h_colls.size() * (uint64_t)n_variants; /* in collectives */
+	const bool large = bytes > kModelLargeBytes && 2 * modelled <= all && row * kModelThreadsLarge <= kModelLds;
 	const uint32_t threads = large ? kModelThreadsLarge : kModelThreads;
-	const size_t lds = std::max(row * threads, !large && bytes > kModelSixBytes ? kModelSixLds : 0);
+	const bool fewer = !large && bytes > (modelled == all ? kModelFewerBytesAll : kModelFewerBytes);
+	const size_t lds = std::max(row * threads, fewer ? kModelFewerLds : 0);
 	auto launch = [&](auto kernel) {
 		hipLaunchKernelGGL(kernel, dim3((points + threads - 1) / threads, n_variants), dim3(threads), d_cost ? lds : 0, s,
 				   plan->g, plan->d_variants, points, d_cost, d_choice);

@@ -389,6 +389,59 @@ int tiles()
 	return 0;
 }
 
+/*
+ * Workgroups of 1024 threads are for large cost grids most of whose points are only written: never where more than half of
+ * the points are modelled, AllReduce's on a platform with a model.  Where all are, fewer workgroups a CU pay later, too.
+ */
+int model()
+{
+	std::vector<uint64_t> sizes(140), nodes(11);
+	for (size_t i = 0; i < sizes.size(); i++) {
+		sizes[i] = 1000 * i;
+	}
+	for (size_t i = 0; i < nodes.size(); i++) {
+		nodes[i] = 1ull << i;
+	}
+	const uint32_t ppn[] = { 1, 2, 4, 8 };
+	const int32_t algos[] = { 1, 0, 6 };
+	struct grid_t {
+		std::vector<int32_t> colls;
+		int32_t platforms[2];
+		bool large;
+	};
+	const grid_t grids[] = { { { 4 }, { 0, 1 }, false },	 { { 4, 2, 3 }, { 0, 1 }, true }, { { 4, 4, 2 }, { 0, 1 }, false },
+				 { { 4, 2 }, { 0, 1 }, true },	 { { 4 }, { 0, 2 }, true },	  { { 4 }, { 2, 3 }, true },
+				 { { 4, 4, 2 }, { 0, 2 }, true } };
+	for (const grid_t &grid : grids) {
+		ofi_amd_tuner_plan_t *plan = nullptr;
+		CHECK(ofi_amd_tuner_plan_create(grid.colls.data(), (uint32_t)grid.colls.size(), sizes.data(), 140, nodes.data(), 11,
+						ppn, 4, algos, 3, &plan) == 0);
+		const uint64_t cells = ofi_amd_tuner_plan_cells(plan);
+		for (uint64_t mb : { 1, 40, 60, 120, 180, 500, 2000 }) {
+			std::vector<ofi_amd_tuner_variant_t> v((size_t)(mb * 1000000 / (16 * cells)) * 2 + 2);
+			for (size_t i = 0; i < v.size(); i++) {
+				v[i] = { grid.platforms[i % 2], 1, 8, 3 };
+			}
+			double cost[1];
+			alignas(2) int8_t choice[2];
+			int launches = 0;
+			on_launch = [&](const launch_t &l) {
+				const bool large = grid.large && mb >= 180;
+				CHECK(l.block.x == (large ? 1024 : 256) && l.grid.y == v.size());
+				CHECK((uint64_t)l.grid.x * l.block.x >= ofi_amd_tuner_plan_points(plan));
+				CHECK(l.shared >= 36u * l.block.x && l.shared <= 65536);
+				CHECK(large || (l.shared > 9216) == (mb >= (grid.colls.size() == 1 && grid.platforms[1] == 1 ? 120 : 60)));
+				launches++;
+			};
+			CHECK(ofi_amd_tuner_model_grid(plan, v.data(), (uint32_t)v.size(), cost, choice, nullptr) == 0);
+			CHECK(ofi_amd_tuner_model_grid(plan, v.data(), (uint32_t)v.size(), cost, nullptr, nullptr) == 0);
+			CHECK(launches == 2);
+		}
+		CHECK(ofi_amd_tuner_plan_destroy(plan) == 0);
+	}
+	return 0;
+}
+
 /* A list of variants or platforms that did not reach the GPU is sent again by the next call with the same list. */
 int uploads()
 {
@@ -424,7 +477,7 @@ int uploads()
 int main(int argc, char **argv)
 {
 	const std::map<std::string, int (*)()> parts = { { "striping", striping }, { "streams", streams }, { "pieces", pieces },
-							       { "bounce", bounce }, { "tiles", tiles }, { "uploads", uploads } };
+							       { "bounce", bounce }, { "model", model }, { "tiles", tiles }, { "uploads", uploads } };
 	CHECK(argc == 2 && parts.count(argv[1]) && ofi_amd_gpu_init() == 0);
 	const int rc = parts.at(argv[1])();
 	std::printf("%s: %s\n", argv[1], rc == 0 ? "ok" : "failed");

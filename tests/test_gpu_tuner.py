@@ -138,7 +138,7 @@ def test_model_grid_on_wide_and_narrow_axes(lib, oracle, gpu, n_nodes, n_ppn):
 def test_model_grid_points_and_workgroups(lib, oracle, gpu, n_sizes, n_nodes, n_ppn, n_variants, odd):
     """Workgroups with no modelled point, with some and with nothing else (collectives of fewer, as many and more points
     than a workgroup, in an order that puts modelled ones at both ends), outputs on any 8-byte and 1-byte boundary, and
-    more than 96 MiB of costs, which larger workgroups write.  The oracle's bits."""
+    so many costs that larger workgroups write them.  The oracle's bits."""
     rng = np.random.default_rng(n_sizes)
     colls = np.array([4, 2, 0, 4], dtype=np.int32)
     sizes = np.unique((2 ** rng.uniform(0, 36, n_sizes)).astype(np.uint64))

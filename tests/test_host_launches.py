@@ -54,6 +54,11 @@ def test_a_bounce_batch_is_launched_alike_whatever_the_size_of_the_pool(driver):
     run(driver, "bounce")
 
 
+def test_model_grids_that_are_mostly_evaluated_stay_with_small_workgroups(driver):
+    """The form for large outputs suits grids that are mostly written."""
+    run(driver, "model")
+
+
 def test_region_tiles_fit_short_axes(driver):
     """A region grid of one size and many node counts, or the other way round, is not paid for by the square."""
     run(driver, "tiles")
