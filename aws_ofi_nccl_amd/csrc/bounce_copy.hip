@@ -583,7 +583,7 @@ constexpr uint32_t kKeepBounce = 8000, kKeepLines = 450000, kKeepEager = 9000;
 /*
  * Fewer wavefronts a CU for large batches of long buffers -- reads and writes take turns at the memory, and the fewer
  * buffers are open the longer the turns are -- were measured and are not used: 65,536 of up to 8 KiB 110.9 us with 32
- * wavefronts, 109.0 with 24 and 107.2 with 20 (limited by the LDS a workgroup claims) on other buffers at every launch, but
+ * wavefronts, 109.0 with 24 and 107.2 with 20 (held by the LDS a workgroup claims) on other buffers at every launch, but
  * 81.1, 84.1 and 86.5 on the same ones over and over, and short buffers starve (65,536 of up to 1000 B 25.2 / 31.2 /
  * 34.8).  The host has no lengths to choose by: src_bytes is the range the batch's offsets lie in, a pool as a rule.
  */

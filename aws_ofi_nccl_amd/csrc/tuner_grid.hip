@@ -73,7 +73,11 @@ struct tiling_t {
  *   480 MB  91.6 / 91.2 / 88.0   94.2 / 93.4 / 90.5   90.8 / 90.5 / 91.3   90.5 / 79.3 / 84.2 */
 constexpr uint32_t kModelThreads = 256, kModelThreadsLarge = 1024;
 constexpr uint64_t kModelFewerBytes = 48ull << 20, kModelFewerBytesAll = 68ull << 20, kModelLargeBytes = 150ull << 20;
+/* LDS is handed out in units of 1280 bytes, 128 of them to a CU: with column_of this is 22 units, five times and not six */
 constexpr size_t kModelFewerLds = 27000;
+constexpr size_t kLdsUnit = 1280, kLdsUnits = 128;
+static_assert(kLdsUnits / ((kModelFewerLds + kLdsUnit - 1) / kLdsUnit) == 5 &&
+	      kLdsUnits / ((kModelFewerLds + NUM_ALGOS * sizeof(int32_t) + kLdsUnit - 1) / kLdsUnit) == 5, "workgroups to a CU");
 constexpr size_t kModelLds = 64 * 1024; /* at most, for the larger ones */
 
 /* `cells` doubles at `out`, cell(k) each, by a workgroup: two to a lane and store, 1 KiB per wavefront
