@@ -306,6 +306,18 @@ def test_proxy_thread_count_does_not_change_the_result(lib, oracle, gpu):
     lib.ofi_amd_gin_rings_destroy(rings)
 
 
+@pytest.mark.parametrize("ops", [1 << 62, (1 << 64) - 1])
+def test_drain_until_nothing_comes(lib, gpu, ops):
+    """A count that no ring will ever see drains what there is and times out, however the counts of the contexts add up."""
+    rings = make_rings(lib, 4, 256)
+    assert lib.ofi_amd_gin_produce_seeded(rings, SEED, 100, 1, 64, 1, 1, 0, _gpu.stream()) == 0
+    _gpu.sync()
+    stats = m.GinProxyStats()
+    rc = lib.ofi_amd_gin_proxy_drain_mt(rings, ops, 0, None, None, None, 0, None, 20, 4, ctypes.byref(stats))
+    assert rc == -errno.ETIMEDOUT and stats.descriptors == 400
+    lib.ofi_amd_gin_rings_destroy(rings)
+
+
 def drain_descs(lib, rings, nctx, ops, timeout_ms=10000):
     descs = (m.GinDesc * (nctx * ops))()
     stats = m.GinProxyStats()
