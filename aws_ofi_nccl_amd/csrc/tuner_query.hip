@@ -264,8 +264,7 @@ static double log2_count(uint64_t v)
  * all of its answers has failed: the stream is asked now and then, so the wait ends with the launch in any
  * case.
  */
-static int collect_answers(const staging_t &stage, const ofi_amd_tuner_query_t *queries, uint32_t n, uint32_t call,
-			   ofi_amd_tuner_answer_t *answers)
+static int collect_answers(const staging_t &stage, uint32_t n, uint32_t call, ofi_amd_tuner_answer_t *answers)
 {
 	constexpr uint32_t kAskEvery = 4096; /* polls of one answer, some 50 us */
 	bool retired = false;
@@ -291,7 +290,7 @@ static int collect_answers(const staging_t &stage, const ofi_amd_tuner_query_t *
 			}
 			__builtin_ia32_pause();
 		}
-		const bool chunk = queries[i].kind == 2;
+		const bool chunk = stage.q[i].kind == 2; /* the caller's questions may lie where the answers go */
 		const uint32_t low = (uint32_t)word, decision = chunk ? ~0u : low;
 		ofi_amd_tuner_answer_t &a = answers[i];
 		a.algo = (int8_t)decision;
@@ -381,5 +380,5 @@ extern "C" int ofi_amd_tuner_query(const ofi_amd_tuner_query_t *queries, uint32_
 				   static_cast<uint64_t *>(g_stage.da) + at);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
-	return collect_answers(g_stage, queries, n, call, answers);
+	return collect_answers(g_stage, n, call, answers);
 }

@@ -69,6 +69,18 @@ def test_query_batches_around_the_line_size(lib, oracle, gpu, n):
         assert (raw[16 * n:] == 0x5A).all()
 
 
+@pytest.mark.parametrize("n", [1, 5, 64, 259])
+def test_query_answers_may_take_the_place_of_the_questions(lib, gpu, n):
+    """An answer depends on its question, not on what has become of the caller's array by the time it arrives."""
+    rng = np.random.default_rng(n)
+    arr = (m.TunerQuery * n)(*[m.TunerQuery(int(rng.integers(0, 4)), int(rng.integers(0, 3)), 4, 1, 8, 3, 0, 2, ALL, 0,
+                                            int(2 ** rng.uniform(0, 35)), 256, 32) for _ in range(n)])
+    want, place = np.zeros(16 * n, dtype=np.uint8), np.frombuffer(bytes(arr), dtype=np.uint8).copy()
+    assert lib.ofi_amd_tuner_query(arr, n, want.ctypes.data) == 0
+    assert lib.ofi_amd_tuner_query(ctypes.cast(place.ctypes.data, ctypes.POINTER(m.TunerQuery)), n, place.ctypes.data) == 0
+    assert np.array_equal(place[:16 * n], want)
+
+
 def test_query_batch_matches_oracle(lib, oracle, gpu):
     rng = np.random.default_rng(11)
     qs, want = [], []
