@@ -70,6 +70,28 @@ burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_
 		     ofi_amd_gin_wire_t *staged, bool fold_wires, uint64_t *hash, ofi_amd_gin_proxy_stats_t *st)
 {
 	ofi_amd_gin_comm_t c = *comm;
+	uint32_t tail = 0, pending = 0;
+	/* What an ACK changes is taken up with every group and given back only where the derivation changed it: the thread
+	 * that receives ACKs may apply one meanwhile (ofi_amd_gin_apply_ack), also while there is nothing to derive. */
+	auto take_acks = [&] {
+		c.tx_tail = tail = __atomic_load_n(&comm->tx_tail, __ATOMIC_RELAXED);
+		c.has_pending_ack_request = pending = __atomic_load_n(&comm->has_pending_ack_request, __ATOMIC_RELAXED);
+	};
+	auto give_back = [&] {
+		comm->sched = c.sched;
+		comm->tx_head = c.tx_head;
+		comm->consecutive_puts_without_ack = c.consecutive_puts_without_ack;
+		comm->last_ack_requested_seq = c.last_ack_requested_seq;
+		comm->pinned_rail_id = c.pinned_rail_id;
+		comm->pinned_rail_run = c.pinned_rail_run;
+		comm->next_rail_id = c.next_rail_id;
+		if (c.tx_tail != tail) {
+			__atomic_store_n(&comm->tx_tail, c.tx_tail, __ATOMIC_RELAXED);
+		}
+		if (c.has_pending_ack_request != pending) {
+			__atomic_store_n(&comm->has_pending_ack_request, c.has_pending_ack_request, __ATOMIC_RELAXED);
+		}
+	};
 	uint64_t h = *hash, signals = 0, writes = 0;
 	burst_t b = { 0, 0 };
 	while (b.done < limit && b.rc == 0) {
@@ -82,6 +104,7 @@ burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_
 		if (ready == 0) {
 			break;
 		}
+		take_acks();
 		uint32_t k = 0;
 		for (; k < ready; k++) {
 			const uint32_t at = start + b.done + k;
@@ -94,9 +117,9 @@ burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_
 			if (__builtin_expect(d->kind != OFI_AMD_GIN_KIND_GET, 1)) {
 				b.rc = ofi_amd_gin::derive<true>(&c, mrs, n_mrs, d, wire);
 			} else {
-				*comm = c;
+				comm->sched = c.sched; /* all that a get changes */
 				b.rc = ofi_amd_gin_iget(comm, mrs, n_mrs, d, wire);
-				c = *comm;
+				c.sched = comm->sched;
 			}
 			if (b.rc != 0) {
 				break;
@@ -109,6 +132,7 @@ burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_
 				h = fold_words(h, reinterpret_cast<const uint64_t *>(wire), (int)(sizeof(*wire) / 8));
 			}
 		}
+		give_back();
 		if (STREAM) {
 			/* the record of a descriptor that failed, which is all zero, too */
 			stream_records(out + b.done, staged, k + (b.rc != 0));
@@ -118,7 +142,6 @@ burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_
 			break;
 		}
 	}
-	*comm = c;
 	*hash = h;
 	st->signals += signals;
 	st->writes += writes;

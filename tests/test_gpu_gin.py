@@ -306,6 +306,30 @@ def test_proxy_thread_count_does_not_change_the_result(lib, oracle, gpu):
     lib.ofi_amd_gin_rings_destroy(rings)
 
 
+def test_acks_applied_beside_a_drain_stay(lib, gpu):
+    """The thread that receives ACKs applies them while a proxy thread waits for descriptors, before and between bursts:
+    none of them is undone by what the drain keeps of the communicator."""
+    rings, ops = make_rings(lib, 1, 256), 200
+    comms, mrs, stats = (m.GinComm * 1)(), (m.GinMr * 3)(), m.GinProxyStats()
+    assert lib.ofi_amd_gin_comm_init(ctypes.byref(comms[0]), 1, 4, 131072, 64, 0) == 0
+    rc = []
+    thread = threading.Thread(target=lambda: rc.append(lib.ofi_amd_gin_proxy_drain(
+        rings, ops, 2, None, comms, mrs, 3, None, 20000, ctypes.byref(stats))))
+    thread.start()
+    lost = 0
+    for i in range(1, 8001):                     # each of them moves the tail on by one
+        lib.ofi_amd_gin_apply_ack(ctypes.byref(comms[0]), i)
+        lost += comms[0].tx_tail != i
+        comms[0].tx_tail = i
+    comms[0].tx_tail = 0
+    assert lib.ofi_amd_gin_produce_seeded(rings, SEED, ops, 1, 64, 1, 1, 0, _gpu.stream()) == 0
+    thread.join()
+    _gpu.sync()
+    assert rc == [0] and stats.descriptors == ops and comms[0].tx_tail == 0
+    assert lost == 0
+    lib.ofi_amd_gin_rings_destroy(rings)
+
+
 @pytest.mark.parametrize("ops", [1 << 62, (1 << 64) - 1])
 def test_drain_until_nothing_comes(lib, gpu, ops):
     """A count that no ring will ever see drains what there is and times out, however the counts of the contexts add up."""
