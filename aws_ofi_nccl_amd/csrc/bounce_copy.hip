@@ -67,8 +67,8 @@ struct __attribute__((packed, aligned(4))) dword_aligned_u32x4 {
 
 /* Buffers (= wavefronts) per workgroup and consecutive workgroups that share an XCD, swept over
  * thousands of launches in a row on 65,536 buffers.  Bounce copy: 8 wavefronts per workgroup with
- * runs of 32 buffers per XCD was the fastest (91.1 us per launch; 4 wavefronts: 91.8,
- * 2: 92.5, 16: 92.6; runs of 64 buffers 91.7).  The eager copy, whose sources are rx buffers in
+ * runs of 32 buffers per XCD was the fastest (91.1 us per launch, every wavefront reading its own
+ * word back; 4 wavefronts: 91.8, 2: 92.5, 16: 92.6; runs of 64 buffers 91.7).  The eager copy, whose sources are rx buffers in
  * arrival order, prefers single-wavefront workgroups (1 x 32: 97.8 us, 4 x 8: 98.4, 8 x 4: 101.6,
  * 16 x 2: 108.6), and so does the table copy (1: 419.9 us per GiB, 4: 439.5, 8: 430.3). */
 constexpr int kBounceWaves = 8;
@@ -92,7 +92,7 @@ __device__ __forceinline__ u32x4 load16_dword_aligned(const uint8_t *p)
  * accesses, the same batch launched over and over on the same buffers slowed down by 6 % within 2,000 launches (91 ->
  * 97 us; fewer and fewer of those ordinary lines leave the L2 between launches, and a read
  * sweep of 16 MiB of other memory brought the first rate back); with one policy the rate does
- * not move (91 us from the first launch to the 20,000th).
+ * not move (91 us from the first launch to the 20,000th; 84.7 since workgroups read their words back together).
  */
 __device__ __forceinline__ void store_byte_streaming(uint8_t *p, uint8_t v)
 {

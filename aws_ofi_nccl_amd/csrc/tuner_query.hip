@@ -107,8 +107,8 @@ __device__ __forceinline__ void region_choose_wave(const int4 *__restrict__ poly
  * instruction (a word per lane, one line), a region set's edges lie in the lanes and every polygon's verdict
  * comes out of the same pass over them, the cells of the model are evaluated side by side, one per
  * lane.  With a thread per question each lane walked the polygons by itself through global memory,
- * a trip for the polygon, its bounds and every four edges: 30.6 us for 259 questions, now
- * 5.6.  From some hundred questions on it is the answers that bound it: the link takes a write of 8 bytes as
+ * a trip for the polygon, its bounds and every four edges: the kernel took 30.6 us for 259 questions,
+ * and takes 5.7.  From some hundred questions on it is the answers that bound it: the link takes a write of 8 bytes as
  * slowly as one of 64, so the eight answers of a workgroup, 8 bytes each, meet in LDS and leave as a line
  * (the call for 1200 questions, with two writes of 8 bytes each and questions of a line and a half 37.6 us, now 18.6;
  * for 259 questions 15.7 and 13.0; in workgroups of one question 23.1 and 13.0).

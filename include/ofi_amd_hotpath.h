@@ -499,10 +499,11 @@ int ofi_amd_gin_proxy_drain(ofi_amd_gin_rings_t *rings, uint64_t ops_per_context
 			    uint32_t timeout_ms, ofi_amd_gin_proxy_stats_t *stats);
 
 /*
- * The same loop on up to n_threads proxy threads (the caller's included; no more than one for every
- * 2000 descriptors the call is to drain), each owning a contiguous range of contexts -- NCCL runs up
- * to NCCL_GIN_MAX_CONNECTIONS = 4 GIN proxy threads (nccl/net.h:38).  Contexts are independent (own ring, own comm state), so the per-context
- * results, and the checksum summed over contexts, do not depend on n_threads.  1..64.
+ * The same loop on up to n_threads proxy threads (the caller's included; one more for every 2000
+ * descriptors the call is to drain), each owning a contiguous range of contexts -- NCCL runs up to
+ * NCCL_GIN_MAX_CONNECTIONS = 4 GIN proxy threads (nccl/net.h:38).  Contexts are independent (own
+ * ring, own comm state), so the per-context results, and the checksum summed over contexts, do not
+ * depend on n_threads.  1..64.
  */
 int ofi_amd_gin_proxy_drain_mt(ofi_amd_gin_rings_t *rings, uint64_t ops_per_context, int mode,
 			       ofi_amd_gin_desc_t *out_desc, ofi_amd_gin_comm_t *comms,
