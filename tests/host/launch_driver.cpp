@@ -179,7 +179,7 @@ int striping()
 		auto small = [&](uint64_t n) { CHECK(batch(&state, sizes, n, 128, num, xfers, stream) == 0); };
 		/* no two of 512 batches in a row count in one word, and each finds its own at zero */
 		for (int i = 0; i < 5000; i++) {
-			small(257 + (i * 97) % 5888);
+			small(257 + (i * 97) % 9728); /* up to 9984, the most in one launch */
 		}
 		CHECK(seen.words.size() == 5000 && seen.spoiled == 0 && seen.two_launch == 0);
 		for (size_t i = 0; i + 512 <= seen.words.size(); i++) {
@@ -202,13 +202,14 @@ int striping()
 		capture_status = hipStreamCaptureStatusActive;
 		small(257);
 		small(6144);
+		small(9984);
 		capture_status = hipStreamCaptureStatusNone;
 		capture_answer = hipErrorStreamCaptureImplicit;
 		small(1000);
 		capture_answer = hipSuccess;
-		CHECK(seen.words.size() == before && seen.two_launch == 3);
+		CHECK(seen.words.size() == before && seen.two_launch == 4);
 		small(256); /* one tile */
-		CHECK(seen.words.size() == before && seen.two_launch == 3);
+		CHECK(seen.words.size() == before && seen.two_launch == 4);
 	}
 	CHECK(ofi_amd_sched_stream_release(stream) == 0);
 	return 0;
