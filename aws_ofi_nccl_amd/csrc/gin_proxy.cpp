@@ -3,6 +3,7 @@
  * include/nccl_ofi_mpsc_ring.h:56-163 and the proxy loop that drains all rings and
  * hands each descriptor to the wire derivation of gin_wire.cpp.
  */
+#include <algorithm>
 #include <cerrno>
 #include <chrono>
 #include <thread>
@@ -11,25 +12,23 @@
 
 #include <emmintrin.h>
 
-#include "gin_derive.hpp"
+#include "gin_derive8.hpp"
 #include "gin_rings.hpp"
 
 namespace {
 
 inline uint64_t rotl64(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }
 
+inline uint64_t fold_sum(uint64_t h, uint64_t x) { return (rotl64(h, 5) ^ x) * 0x100000001B3ull; }
+
 /* Order-sensitive fold of n 64-bit words into a running per-context hash. */
 inline uint64_t fold_words(uint64_t h, const uint64_t *w, int n)
 {
-	static const uint64_t K[8] = {
-		0x9E3779B97F4A7C15ull, 0xBF58476D1CE4E5B9ull, 0x94D049BB133111EBull, 0xD6E8FEB86659FD93ull,
-		0xCA5A826395121157ull, 0x2545F4914F6CDD1Dull, 0xA0761D6478BD642Full, 0xE7037ED1A0B428DBull,
-	};
 	uint64_t x = 0;
 	for (int k = 0; k < n; k++) {
-		x += (w[k] + (uint64_t)(k + 1)) * K[k & 7];
+		x += (w[k] + (uint64_t)(k + 1)) * ofi_amd_gin::kFoldKeys[k & 7];
 	}
-	return (rotl64(h, 5) ^ x) * 0x100000001B3ull;
+	return fold_sum(h, x);
 }
 
 /* n records past the caches, in order; both 16-byte aligned */
@@ -45,8 +44,26 @@ inline void stream_records(ofi_amd_gin_wire_t *to, const ofi_amd_gin_wire_t *fro
 	}
 }
 
+/* ... by whole lines of `to`, but for its ends */
+OFI_AMD_WIDE inline void stream_records_wide(ofi_amd_gin_wire_t *to, const ofi_amd_gin_wire_t *from, uint32_t n)
+{
+	const char *s = reinterpret_cast<const char *>(from);
+	char *d = reinterpret_cast<char *>(to), *const end = d + n * sizeof(*to);
+	auto words = [&](char *until) {
+		for (; d < until; d += 16, s += 16) {
+			_mm_stream_si128(reinterpret_cast<__m128i *>(d), _mm_load_si128(reinterpret_cast<const __m128i *>(s)));
+		}
+	};
+	words(std::min(end, d + ((64 - (reinterpret_cast<uintptr_t>(d) & 63)) & 63)));
+	for (; end - d >= 64; d += 64, s += 64) {
+		_mm512_stream_si512(reinterpret_cast<__m512i *>(d), _mm512_loadu_si512(s));
+	}
+	words(end);
+}
+
 constexpr uint32_t kGroup = 16;  /* descriptors looked at and handed on together */
 constexpr uint32_t kStaged = 64; /* records of a thread's own array, 14 KiB */
+constexpr uint64_t kCachedRecords = 20000; /* 4.5 MB */
 
 struct burst_t {
 	uint32_t done; /* descriptors derived */
@@ -55,16 +72,17 @@ struct burst_t {
 
 /*
  * Derives up to `limit` published descriptors of one ring, from position `start` on, to the records at `out`, or round
- * `staged` when there is no `out`.  What bounds it is the core: some 250 instructions a descriptor, two of their
- * branches by its size, and the descriptor's line, which comes from memory.  The communicator lives in a copy whose
- * address goes nowhere, so that its fields are registers or stack words, not loads and stores through a pointer that may
- * alias the records, and the derivation is inlined (four threads, no output array: 16.8 -> 14.4 ns a descriptor).
+ * `staged` when there is no `out`.  What bounds it is the core: some 250 instructions a descriptor one by one, two of their
+ * branches by its size, and the descriptor's line, which comes from memory.  WIDE: eight at a time (derive8), and one by one
+ * only the groups that it hands back; one thread, no output array 12.5 -> 5.5 ns a descriptor.  The communicator lives in a
+ * copy: one by one its address goes nowhere, so that its fields are registers or stack words, not loads and stores
+ * through a pointer that may alias the records, and the derivation is inlined (four threads, no output array: 16.8 -> 14.4 ns).
  * STREAM: records are made in `staged`, which stays in the first-level cache, and leave by groups past the caches: an
  * ordinary store fetches every line of the array first, from memory or from whichever core read it last.  256,000
- * records (57 MB) on four threads 1.3-1.6 -> 1.05-1.1 ms; 32,000 (7 MB) that another thread reads between the
- * calls 461 -> 175 us.
+ * records (57 MB) on four threads, descriptors produced ahead: ordinary 1.3-1.6 ms one by one, streamed 1.03, WIDE 0.61
+ * (the stores alone take four threads 0.36); 32,000 (7 MB) that another thread reads between the calls 461 -> 175 us one by one.
  */
-template <bool STREAM>
+template <bool STREAM, bool WIDE>
 burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_t mask, uint32_t start, uint32_t limit,
 		     ofi_amd_gin_comm_t *comm, const ofi_amd_gin_mr_t *mrs, uint32_t n_mrs, ofi_amd_gin_wire_t *out,
 		     ofi_amd_gin_wire_t *staged, bool fold_wires, uint64_t *hash, ofi_amd_gin_proxy_stats_t *st)
@@ -105,10 +123,30 @@ burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_
 			break;
 		}
 		take_acks();
-		uint32_t k = 0;
-		for (; k < ready; k++) {
+		uint32_t k = 0, singly = 0; /* singly: those before it are derived one by one */
+		while (k < ready) {
 			const uint32_t at = start + b.done + k;
 			const ofi_amd_gin_desc_t *d = &rec[at & mask];
+			if (WIDE && k >= singly) {
+				/* up to the ring's end */
+				const uint32_t m = std::min({ ready - k, ofi_amd_gin::kLanes, mask + 1 - (at & mask) });
+				for (uint32_t j = 0; j < m; j++) {
+					__builtin_prefetch(&rec[(at + kGroup + j) & mask]);
+				}
+				ofi_amd_gin_wire_t *wires = STREAM || !out ? &staged[k] : &out[b.done + k];
+				ofi_amd_gin::derived8_t sums;
+				if (ofi_amd_gin::derive8(&c, mrs, n_mrs, d, m, wires, &sums)) {
+					__asm__ volatile("" : : "r"(wires) : "memory"); /* as below */
+					for (uint32_t j = 0; j < m; j++) {
+						h = fold_sum(h, sums.folds[j]);
+					}
+					signals += sums.signals;
+					writes += sums.writes;
+					k += m;
+					continue;
+				}
+				singly = k + m;
+			}
 			__builtin_prefetch(&rec[(at + kGroup) & mask]);
 			/* the slot is handed back only after this burst, so the record is read in place */
 			ofi_amd_gin_wire_t *wire = STREAM ? &staged[k] : (out ? &out[b.done + k] : &staged[at % kStaged]);
@@ -131,11 +169,12 @@ burst_t derive_burst(const uint32_t *seq, const ofi_amd_gin_desc_t *rec, uint32_
 			if (fold_wires) {
 				h = fold_words(h, reinterpret_cast<const uint64_t *>(wire), (int)(sizeof(*wire) / 8));
 			}
+			k++;
 		}
 		give_back();
 		if (STREAM) {
 			/* the record of a descriptor that failed, which is all zero, too */
-			stream_records(out + b.done, staged, k + (b.rc != 0));
+			(WIDE ? stream_records_wide : stream_records)(out + b.done, staged, k + (b.rc != 0));
 		}
 		b.done += k;
 		if (ready < most) {
@@ -203,15 +242,15 @@ int ofi_amd_gin_ring_pop(ofi_amd_gin_rings_t *r, uint32_t context, ofi_amd_gin_d
 
 /*
  * A call has one thread more for every so many descriptors, up to the number asked for: starting threads takes some 20 us.  Us
- * for a call on four threads and on those this allows, descriptors produced ahead, without / with an output array:
- *   200 descriptors   27 / 27   6 / 6
- *   800               34 / 22  15 / 15
- *   1000              35 / 25  17 / 18
- *   2000 (two)        27 / 38  26 / 31
- *   4000 (three)      42 / 38  40 / 44
- *   6000 (all four)   38 / 54  39 / 54
+ * for a call that may have four, with one for every 2000 / for every 3000, descriptors produced ahead, without an output
+ * array and with one:
+ *    2400 descriptors   35 and 35 (two threads)    17 and 19 (one)
+ *    4800               40 and 41 (three)          36 and 38 (two)
+ *    8000               55 and 57 (four)           52 and 57 (three)
+ *   12,800              63 and 74 (four)           63 and 74 (four)
+ * Derived one by one, 2000 are worth a thread: 6000 on all four 38 and 54, 4000 on three 40 and 44, on four 42 and 38.
  */
-static constexpr uint64_t kOpsPerThread = 2000;
+static constexpr uint64_t kOpsPerThread = 3000, kOpsPerThreadSingly = 2000;
 
 /* One proxy thread's share: contexts [c_begin, c_end). */
 static int drain_contexts(ofi_amd_gin_rings_t *r, uint32_t c_begin, uint32_t c_end,
@@ -237,10 +276,13 @@ static int drain_contexts(ofi_amd_gin_rings_t *r, uint32_t c_begin, uint32_t c_e
 	/* without an output array the records go round this one (it stays in the core's cache), where a post step would
 	 * pick them up */
 	alignas(64) ofi_amd_gin_wire_t staged[kStaged];
-	/* A thread that is the only one of its call stores through the caches: 13.4 ns a descriptor, streamed 14.6, and with
-	 * four threads in calls of their own 14.4 and 14.6.  The line fetches that streaming saves cost most when another core
-	 * has read the array since (30-50 ns against 15), which is not known here. */
-	const bool stream = out_wire && !alone && (reinterpret_cast<uintptr_t>(out_wire) & 15u) == 0;
+	/* A thread that is the only one of its call stores through the caches while they hold the records: 2.9 MB of them WIDE 84-100
+	 * us, streamed 94, 3.6 MB 108-118 and 126, 5.4 MB 203-217 and 183-193, 14 MB 607 and 440; one by one at every size 13.4 ns a
+	 * descriptor, streamed 14.6.  (The line fetches that streaming saves cost most when another core has read the array
+	 * since, 30-50 ns against 15, which is not known here.) */
+	const bool wide = mode == 2 && ofi_amd_gin::cpu_has_wide();
+	const bool fits = !wide || ops_per_context <= kCachedRecords / nctx;
+	const bool stream = out_wire && !(alone && fits) && (reinterpret_cast<uintptr_t>(out_wire) & 15u) == 0;
 
 	ofi_amd_gin_proxy_stats_t st;
 	std::memset(&st, 0, sizeof(st));
@@ -268,7 +310,8 @@ static int drain_contexts(ofi_amd_gin_rings_t *r, uint32_t c_begin, uint32_t c_e
 			/* whether the fast form applies is constant over the burst: the derivation keeps the counters below
 			 * the rail count */
 			if (mode >= 2 && ofi_amd_gin::derive_fast_path(&comms[c])) {
-				const burst_t b = (stream ? derive_burst<true> : derive_burst<false>)(
+				const burst_t b = (wide ? (stream ? derive_burst<true, true> : derive_burst<false, true>)
+							: (stream ? derive_burst<true, false> : derive_burst<false, false>))(
 					seq, rec, mask, start, limit, &comms[c], mrs, n_mrs, out_wire ? out_wire + first : nullptr, staged,
 					mode == 3, &h, &st);
 				pos = start + b.done;
@@ -355,8 +398,9 @@ int ofi_amd_gin_proxy_drain_mt(ofi_amd_gin_rings_t *r, uint64_t ops_per_context,
 	}
 	const uint32_t nctx = r->n_contexts;
 	uint32_t workers = n_threads < nctx ? n_threads : nctx;
-	if (ops_per_context < kOpsPerThread) { /* each context is not worth a thread by itself */
-		const uint64_t worth = nctx * ops_per_context / kOpsPerThread + 1;
+	const uint64_t per_thread = mode == 2 && ofi_amd_gin::cpu_has_wide() ? kOpsPerThread : kOpsPerThreadSingly;
+	if (ops_per_context < per_thread) { /* each context is not worth a thread by itself */
+		const uint64_t worth = nctx * ops_per_context / per_thread + 1;
 		workers = worth < workers ? (uint32_t)worth : workers;
 	}
 	std::vector<ofi_amd_gin_proxy_stats_t> part(workers);

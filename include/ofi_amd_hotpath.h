@@ -499,8 +499,8 @@ int ofi_amd_gin_proxy_drain(ofi_amd_gin_rings_t *rings, uint64_t ops_per_context
 			    uint32_t timeout_ms, ofi_amd_gin_proxy_stats_t *stats);
 
 /*
- * The same loop on up to n_threads proxy threads (the caller's included; one more for every 2000
- * descriptors the call is to drain), each owning a contiguous range of contexts -- NCCL runs up to
+ * The same loop on up to n_threads proxy threads (the caller's included; one more for every 3000
+ * descriptors the call is to drain, 2000 where it derives them one by one), each owning a contiguous range of contexts -- NCCL runs up to
  * NCCL_GIN_MAX_CONNECTIONS = 4 GIN proxy threads (nccl/net.h:38).  Contexts are independent (own
  * ring, own comm state), so the per-context results, and the checksum summed over contexts, do not
  * depend on n_threads.  1..64.
