@@ -247,10 +247,9 @@ enum read_back_t { NO_READ_BACK, BY_ITSELF, TOGETHER };
  */
 template <read_back_t BACK>
 __global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
-	const uint8_t *__restrict__ src, uint64_t src_bytes, uint8_t *__restrict__ arena, uint64_t arena_bytes,
-	const uint64_t *__restrict__ src_off, const uint64_t *__restrict__ dst_off,
-	const uint32_t *__restrict__ len, uint32_t n, uint32_t *__restrict__ flush,
-	uint32_t *__restrict__ err)
+	const uint8_t *__restrict__ src, uint64_t src_bytes, const uint64_t *__restrict__ src_off,
+	const uint64_t *__restrict__ dst_off, const uint32_t *__restrict__ len, uint32_t n, uint8_t *__restrict__ arena,
+	uint64_t arena_bytes, uint32_t *__restrict__ flush, uint32_t *__restrict__ err)
 {
 	constexpr uint32_t kGroup = kBounceRun / kBounceWaves;
 	const uint32_t lane = threadIdx.x & 63u;
@@ -373,9 +372,14 @@ __global__ __launch_bounds__(64 * kEagerWaves) void eager_copy_kernel(
 	if (buf >= n) {
 		return;
 	}
-	const uint8_t *s = rx_base + rx_off[buf] + 8u; /* skip nccl_ofi_eager_msg_header_t */
-	uint8_t *d = dst_base + dst_off[buf];
-	const uint32_t bytes = min(recv_len[buf], dst_len[buf]);
+	const uint64_t from = rx_off[buf], to = dst_off[buf];
+	const uint32_t received = recv_len[buf], room = dst_len[buf];
+	/* all of the entry is in hand from here on: the compiler would ask for the source only once the length is known (us, other
+	 * buffers at every launch: 2000 of up to 8 KiB 5.9 -> 5.6, 65,536 of up to 4000 B 67.9 -> 66.4, of up to 500 B 28.5 -> 27.6) */
+	__asm__ volatile("" : : "s"(from), "s"(to), "s"(received), "s"(room), "s"(copied), "s"(flush));
+	const uint8_t *s = rx_base + from + 8u; /* skip nccl_ofi_eager_msg_header_t */
+	uint8_t *d = dst_base + to;
+	const uint32_t bytes = min(received, room);
 	if (copied != nullptr && lane == 0) {
 		copied[buf] = bytes;
 	}
@@ -613,8 +617,8 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 	const uint32_t runs = (n + kXcds * kBounceRun - 1) / (kXcds * kBounceRun); /* whole rounds over the XCDs */
 	auto launch = [&](auto kernel) {
 		hipLaunchKernelGGL(kernel, dim3(runs * kXcds * (kBounceRun / kBounceWaves)), dim3(64 * kBounceWaves), 0,
-				   as_stream(stream), static_cast<const uint8_t *>(d_src), src_bytes, static_cast<uint8_t *>(d_arena),
-				   arena_bytes, d_src_off, d_dst_off, d_len, n, d_flush, err);
+				   as_stream(stream), static_cast<const uint8_t *>(d_src), src_bytes, d_src_off, d_dst_off, d_len, n,
+				   static_cast<uint8_t *>(d_arena), arena_bytes, d_flush, err);
 	};
 	if (!d_flush) {
 		launch(bounce_scatter_kernel<NO_READ_BACK>);

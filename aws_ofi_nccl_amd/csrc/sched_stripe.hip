@@ -180,11 +180,19 @@ __global__ __launch_bounds__(kCountThreads) void stripe_count_kernel(
 	uint64_t size_of[kPer];
 #pragma unroll
 	for (uint32_t j = 0; j < kPer; j++) {
-		const uint32_t i = base + j * kCountThreads + threadIdx.x;
-		size_of[j] = i < n ? sizes[i] : 0;
+		size_of[j] = sizes[min(base + j * kCountThreads + threadIdx.x, n - 1u)];
 	}
 	params_t p;
-	if (!load_params(state, align, p)) {
+	const bool usable = load_params(state, align, p);
+	uint32_t acc = 0;
+#pragma unroll
+	for (uint32_t j = 0; j < kPer; j++) {
+		uint32_t k;
+		const uint32_t c = contribution(size_of[j], p, k);
+		acc += base + j * kCountThreads + threadIdx.x < n ? c : 0u;
+	}
+	__asm__ volatile("" : "+v"(acc)); /* the sizes are not asked for behind the test of the state only */
+	if (!usable) {
 		if (blockIdx.x == 0 && threadIdx.x == 0) {
 			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE);
 		}
@@ -192,13 +200,6 @@ __global__ __launch_bounds__(kCountThreads) void stripe_count_kernel(
 	}
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		*seed0 = batch_seed(state, p.num_rails);
-	}
-	uint32_t acc = 0;
-#pragma unroll
-	for (uint32_t j = 0; j < kPer; j++) {
-		uint32_t k;
-		const uint32_t c = contribution(size_of[j], p, k);
-		acc += base + j * kCountThreads + threadIdx.x < n ? c : 0u;
 	}
 	acc = wave_sum_of(acc);
 	if ((threadIdx.x & 63u) == 0) {
@@ -225,11 +226,19 @@ __global__ __launch_bounds__(64 * kBlockTiles) void stripe_count_big_kernel(
 	uint64_t size_of[kPer];
 #pragma unroll
 	for (uint32_t j = 0; j < kPer; j++) {
-		const uint64_t i = base + j * 64u + lane;
-		size_of[j] = i < n ? sizes[i] : 0;
+		size_of[j] = sizes[min((uint32_t)base + j * 64u + lane, n - 1u)];
 	}
 	params_t p;
-	if (!load_params(state, align, p)) {
+	const bool usable = load_params(state, align, p);
+	uint32_t acc = 0;
+#pragma unroll
+	for (uint32_t j = 0; j < kPer; j++) {
+		uint32_t k;
+		const uint32_t c = contribution(size_of[j], p, k);
+		acc += base + j * 64u + lane < n ? c : 0u;
+	}
+	__asm__ volatile("" : "+v"(acc)); /* the sizes are not asked for behind the test of the state only */
+	if (!usable) {
 		if (blockIdx.x == 0 && threadIdx.x == 0) {
 			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE);
 		}
@@ -237,13 +246,6 @@ __global__ __launch_bounds__(64 * kBlockTiles) void stripe_count_big_kernel(
 	}
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		*seed0 = batch_seed(state, p.num_rails);
-	}
-	uint32_t acc = 0;
-#pragma unroll
-	for (uint32_t j = 0; j < kPer; j++) {
-		uint32_t k;
-		const uint32_t c = contribution(size_of[j], p, k);
-		acc += base + j * 64u + lane < n ? c : 0u;
 	}
 	acc = residues(wave_sum_of(acc), p.num_rails);
 	if (lane == 0) {
@@ -281,8 +283,9 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 	const uint32_t tile = blockIdx.x, base = tile * THREADS, i = base + threadIdx.x;
 	const bool live = i < n;
-	const uint64_t size = live ? __builtin_nontemporal_load(&sizes[i]) : 0;
-	uint32_t acc = 0;
+	/* Everything a tile reads is asked for before it waits for anything: its sizes, what is before it, the state and the
+	 * seed.  What is beyond an end is read inside it and masked out, rather than left out by a branch. */
+	const uint64_t size_read = __builtin_nontemporal_load(&sizes[min(i, n - 1u)]);
 	/* DIRECT: the first messages before the tile, requested along with its own (8 at a time: 6144 messages 4.93 us,
 	 * 12 or 16 at a time 4.9-5.0, 5000 4.73, 4.80 and 4.92) */
 	constexpr uint32_t kAhead = THREADS == kDirectTile ? 1 : 8;
@@ -294,36 +297,42 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 			before[j] = at < base ? sizes[at] : 0;
 		}
 	};
+	/* TILES: the first words of the totals.  BLOCKS: at most kMaxBlocks words, one 16-byte load a thread, and those of the
+	 * block's own tiles */
+	const uint32_t blocks = tile / kBlockTiles;
+	u32x4 block_words;
+	uint32_t total = 0;
 	if (FORM == DIRECT) {
 		look_ahead(0);
-	} else {
-		/* sums of residues: packed halves, below 2^14 words of at most 3 each */
-		if (FORM == TILES) {
-			/* A word a thread and turn: the later a tile, the later its workgroup starts to write, and
-			 * the launch is faster for it (1,000,000 messages: 21.6 us; with four 16-byte loads in
-			 * flight, so that all start at once, 22.8). */
-			for (uint32_t t = threadIdx.x; t < tile; t += THREADS) {
-				acc += totals[t];
-			}
-		}
-		if (FORM == BLOCKS) {
-			/* at most kMaxBlocks words: one 16-byte load a thread, the words beyond the last masked out */
-			const uint32_t blocks = tile / kBlockTiles, at = threadIdx.x * 4u;
-			if (at < blocks) {
-				const u32x4 v = *reinterpret_cast<const u32x4 *>(block_totals + at);
-				acc = v.x + (at + 1 < blocks ? v.y : 0) + (at + 2 < blocks ? v.z : 0) + (at + 3 < blocks ? v.w : 0);
-			}
-			acc += threadIdx.x < tile % kBlockTiles ? totals[blocks * kBlockTiles + threadIdx.x] : 0;
-		}
 	}
+	if (FORM == TILES) {
+		total = totals[min(threadIdx.x, tile)];
+	}
+	if (FORM == BLOCKS) {
+		static_assert(FORM != BLOCKS || THREADS * 4 == kMaxBlocks, "a load a thread is within the block totals");
+		block_words = *reinterpret_cast<const u32x4 *>(block_totals + threadIdx.x * 4u);
+		total = totals[blocks * kBlockTiles + threadIdx.x % kBlockTiles];
+	}
+	const uint32_t seed = FORM == DIRECT ? 0u : *seed0;
 	params_t p;
-	if (!load_params(state, align, p)) {
-		if (FORM == DIRECT && tile == 0 && threadIdx.x == 0) {
-			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE);
-		}
-		return;
-	}
+	const bool usable = load_params(state, align, p);
 	const uint32_t R = p.num_rails;
+	/* sums of residues: packed halves, below 2^14 words of at most 3 each */
+	uint32_t acc = 0;
+	if (FORM == TILES) {
+		/* A word a thread and turn: the later a tile, the later its workgroup starts to write, and
+		 * the launch is faster for it (1,000,000 messages: 21.6 us; with four 16-byte loads in
+		 * flight, so that all start at once, 22.8). */
+		acc = threadIdx.x < tile ? total : 0u;
+		for (uint32_t t = threadIdx.x + THREADS; t < tile; t += THREADS) {
+			acc += totals[t];
+		}
+	}
+	if (FORM == BLOCKS) {
+		const uint32_t at = threadIdx.x * 4u;
+		acc = (at < blocks ? block_words.x : 0u) + (at + 1 < blocks ? block_words.y : 0u) + (at + 2 < blocks ? block_words.z : 0u) +
+		      (at + 3 < blocks ? block_words.w : 0u) + (threadIdx.x < tile % kBlockTiles ? total : 0u);
+	}
 	if (FORM == DIRECT) {
 		for (uint32_t i0 = 0; i0 < base;) {
 #pragma unroll
@@ -338,6 +347,15 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 			}
 		}
 	}
+	const uint64_t size = live ? size_read : 0;
+	/* in hand from here on: the compiler would move their loads behind the test of the state */
+	__asm__ volatile("" : "+v"(acc) : "v"(size), "s"(seed));
+	if (!usable) {
+		if (FORM == DIRECT && tile == 0 && threadIdx.x == 0) {
+			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE);
+		}
+		return;
+	}
 	acc = wave_sum_of(acc);
 	uint32_t k = 0;
 	const uint32_t c = live ? contribution(size, p, k) : 0;
@@ -349,7 +367,7 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	if (lane == 63) {
 		wave_sum[wave] = inc;
 	}
-	uint32_t before_tile = FORM == DIRECT ? 0u : *seed0, off = 0, tot = 0;
+	uint32_t before_tile = seed, off = 0, tot = 0;
 	__syncthreads();
 #pragma unroll
 	for (uint32_t w = 0; w < kWaves; w++) {

@@ -124,10 +124,9 @@ __device__ __forceinline__ void write_choice(int8_t *__restrict__ choice, uint64
  * 9.9 -> 8.0 us, 64 grids 16.5 -> 16.3.
  */
 template <bool COST, bool CHOICE, uint32_t kThreads = kModelThreads>
-__global__ __launch_bounds__(kThreads) void model_grid_kernel(grid_dims_t g,
+__global__ __launch_bounds__(kThreads) void model_grid_kernel(double *__restrict__ cost,
 							 const ofi_amd_tuner_variant_t *__restrict__ variants,
-							 uint32_t points_per_variant, double *__restrict__ cost,
-							 int8_t *__restrict__ choice)
+							 int8_t *__restrict__ choice, uint32_t points_per_variant, grid_dims_t g)
 {
 	extern __shared__ float stage[]; /* [kThreads][cells per point] when COST */
 	__shared__ int32_t column_of[NUM_ALGOS]; /* the plan's column of an algorithm, -1: none */
@@ -316,9 +315,9 @@ __device__ __forceinline__ uint64_t every(uint64_t m)
  * L2 wrote its quarter of each line, 18.9 MB).
  */
 __global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(
-	grid_dims_t g, tiling_t t, const int32_t *__restrict__ polys, const double *__restrict__ bboxes,
-	const edge_t *__restrict__ edges, pt_t far_point, const region_run_t *__restrict__ runs,
-	uint32_t points_per_platform, int8_t *__restrict__ choice)
+	const region_run_t *__restrict__ runs, const int32_t *__restrict__ polys, const double *__restrict__ bboxes,
+	const edge_t *__restrict__ edges, int8_t *__restrict__ choice, uint32_t points_per_platform, pt_t far_point, tiling_t t,
+	grid_dims_t g)
 {
 	/* blockIdx.y names a run, blockIdx.x = 8 * group + x the tiles 8 * group .. 8 * group + 7 of it, of
 	 * which XCD x takes one (workgroups are dealt to the XCDs in launch order, and gridDim.x is a
@@ -983,7 +982,7 @@ int ofi_amd_tuner_model_grid(ofi_amd_tuner_plan_t *plan, const ofi_amd_tuner_var
 	const size_t lds = std::max(row * threads, fewer ? kModelFewerLds : 0);
 	auto launch = [&](auto kernel) {
 		hipLaunchKernelGGL(kernel, dim3((points + threads - 1) / threads, n_variants), dim3(threads), d_cost ? lds : 0, s,
-				   plan->g, plan->d_variants, points, d_cost, d_choice);
+				   d_cost, plan->d_variants, d_choice, points, plan->g);
 	};
 	if (d_cost && d_choice) {
 		large ? launch(model_grid_kernel<true, true, kModelThreadsLarge>) : launch(model_grid_kernel<true, true>);
@@ -1071,9 +1070,8 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 	const uint32_t grid_x = (uint32_t)((groups + waves - 1) / waves * kXcds);
 	for (uint64_t at = 0; at < n_runs; at += kMostRuns) {
 		const uint32_t here = (uint32_t)(n_runs - at < kMostRuns ? n_runs - at : kMostRuns);
-		hipLaunchKernelGGL(region_choice_kernel, dim3(grid_x, here), dim3(64 * waves), 0, s, plan->g,
-				   tiling, plan->t.poly, plan->t.bbox, plan->t.edges, plan->t.far_point, plan->d_runs + at, points,
-				   d_choice);
+		hipLaunchKernelGGL(region_choice_kernel, dim3(grid_x, here), dim3(64 * waves), 0, s, plan->d_runs + at,
+				   plan->t.poly, plan->t.bbox, plan->t.edges, d_choice, points, plan->t.far_point, tiling, plan->g);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
