@@ -10,10 +10,11 @@
  *   small_rail_i = (rr_small + #{j < i : size_j <  max_small}) mod R
  *   start_rail_i = (rr      + sum{j < i : size_j >= max_small} n_j) mod R
  *
- * Three forms, by the size of the batch:
+ * Four forms, by the size of the batch:
  *   up to kDirectBatch messages, one launch: every workgroup adds up the messages before
- *   its tile by itself, from their sizes (at most 78 KiB out of the L2); beyond one tile not in a
- *   batch that is being captured into a graph (launch_batch says why);
+ *   its tile by itself, from their sizes (at most 78 KiB out of the L2);
+ *   from kTwoLaunchBatch up to kOnceBatch, one launch whose workgroups publish the totals of their tiles and add up those
+ *   of the tiles before them (stripe_once_kernel);
  *   up to kSmallBatch, two launches: stripe_count_kernel leaves each tile's totals of
  *   (small count, stripe count), reduced mod R (only the residues matter), and
  *   stripe_emit_kernel, whose workgroups add up the totals of the tiles before them (at most
@@ -21,6 +22,7 @@
  *   stores;
  *   beyond, the same two launches with larger tiles, and a level of totals above the tiles', for
  *   every kPart messages.
+ * Beyond one tile a batch that is being captured into a graph takes the two launches (launch_batch says why).
  * The count launch snapshots the two counters of *state as the batch's seed, the workgroup of the
  * last tile writes the new ones back; in the one-launch form the workgroup that reads them last does.
  *
@@ -45,6 +47,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kDirectTile = 256, kDirectTileLarge = 512;
 constexpr uint64_t kDirectBatch = 9984;
 static_assert(4 * kDirectBatch < 65536 - 8, "packed sums of a whole batch: up to 4 stripes a message, and the seed");
+constexpr uint64_t kTwoLaunchBatch = 10240; /* from kDirectBatch up to here two launches, as the tests hold 10,000 to */
 /* Two-launch form: tiles of 512 messages, counted by 256 threads and written by 512 (21.5 us per 1,000,000
  * messages, 39.0 per 2,000,000; 256 threads twice 21.6 and 40.2, 128 threads four times 23.9 and 43.5). */
 constexpr uint32_t kTile = 512;
@@ -265,6 +268,93 @@ __global__ __launch_bounds__(64 * kBlockTiles) void stripe_count_big_kernel(
 	}
 }
 
+/*
+ * The rows of a tile, by its workgroup: this thread's message with its contribution c, its k stripes and what the messages
+ * before it in the tile add up to.  BY_WAVE: `rows` has room for half of them.
+ */
+template <bool BY_WAVE, uint32_t THREADS>
+__device__ __forceinline__ void write_rows(uint64_t size, bool live, uint32_t c, uint32_t k, uint32_t excl, uint32_t carry_small,
+					   uint32_t carry_big, const params_t &p, uint32_t n, uint32_t base, u32x4 *rows,
+					   uint32_t *__restrict__ num_xfers, u32x4 *__restrict__ xfers)
+{
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, R = p.num_rails;
+	/* set_schedule_by_threshold, src/nccl_ofi_scheduler.cpp:77-133 */
+	const bool small = (c >> 16) != 0;
+	uint32_t rail = mod_rails(small ? carry_small + (excl >> 16) : carry_big + (excl & 0xffffu), p);
+	uint64_t max_stripe = size;
+	if (!small) {
+		/* (size - 1) / k: k is 1, 2 or 4 unless there are three rails */
+		uint64_t whole = size == 0 ? 0 : (size - 1) >> (k >> 1);
+		if (R == 3) {
+			whole = k == 3 ? (size == 0 ? 0 : (size - 1) / 3) : whole;
+		}
+		const uint64_t per = size == 0 ? 0 : 1 + whole;
+		max_stripe = div_ceil_by(per, p.align, p.align_shift) * p.align;
+	}
+	/* k stripes of max_stripe cover the message, so `left` is 0 from stripe k on and the
+	 * length of an unused entry comes out as 0 by itself; lanes past the end have k = 0 */
+	uint64_t left = size, offset = 0;
+	uint64_t f[12]; /* 4 x {rail word, offset, msg_size} */
+#pragma unroll
+	for (uint32_t s = 0; s < 4; s++) {
+		const bool used = s < k;
+		const uint64_t stripe = left < max_stripe ? left : max_stripe;
+		f[3 * s + 0] = used ? rail : 0; /* rail_id in the low 16 bits, padding zero */
+		f[3 * s + 1] = used ? offset : 0;
+		f[3 * s + 2] = stripe;
+		offset += stripe;
+		left -= stripe;
+		rail = rail + 1 == R ? 0 : rail + 1;
+	}
+	auto stage_row = [&](u32x4 *row) {
+#pragma unroll
+		for (uint32_t q = 0; q < 6; q++) {
+			u32x4 v;
+			v.x = (uint32_t)f[2 * q];
+			v.y = (uint32_t)(f[2 * q] >> 32);
+			v.z = (uint32_t)f[2 * q + 1];
+			v.w = (uint32_t)(f[2 * q + 1] >> 32);
+			row[q] = v;
+		}
+	};
+	if (live) {
+		num_xfers[base + threadIdx.x] = k;
+	}
+	const uint32_t valid = (n - base) < THREADS ? (n - base) : THREADS;
+	u32x4 *out = xfers + (uint64_t)base * 6;
+	if (BY_WAVE) {
+		/* A wavefront writes its rows by itself, the first and then the second half of its lanes', out of 3 KiB of LDS.  So
+		 * four workgroups share a CU, all the wavefronts it has room for, where three did with every row in LDS, and none
+		 * waits for another wavefront's rows (us, rows of a workgroup / of a wavefront / of half a one: 400,000 messages 12.7 /
+		 * 12.4 / 11.4, 1,000,000 21.7 / 21.1 / 21.2, 2,000,000 39.3 / 38.5 / 37.6, 6,000,000 113.2 / 111.7 / 110.6). */
+		u32x4 *const stage = &rows[wave * (32u * 6u)];
+#pragma unroll
+		for (uint32_t half = 0; half < 2; half++) {
+			if (lane / 32u == half) {
+				stage_row(&stage[lane % 32u * 6u]);
+			}
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+#pragma unroll
+			for (uint32_t q = 0; q < 3; q++) {
+				const uint32_t v = q * 64u + lane, at = (wave * 64u + half * 32u) * 6u + v;
+				if (at < valid * 6) {
+					__builtin_nontemporal_store(stage[v], &out[at]);
+				}
+			}
+			__builtin_amdgcn_wave_barrier(); /* the rows of one half have been read before the other's are written */
+		}
+	} else {
+		/* The rows of the workgroup together: the small batches gain nothing by the other way, and the large ones lose
+		 * the narrow front on which the chip writes (16,000,000 messages 270 and 311 us). */
+		stage_row(&rows[threadIdx.x * 6]);
+		__syncthreads();
+		for (uint32_t v = threadIdx.x; v < valid * 6; v += THREADS) {
+			__builtin_nontemporal_store(rows[v], &out[v]);
+		}
+	}
+}
+
 /* Where a tile's seed comes from: the sizes before it (DIRECT), the totals of the tiles before it (TILES), or
  * the totals of the blocks of tiles before its block and of the tiles before it in its block (BLOCKS) */
 enum stripe_form { DIRECT, TILES, BLOCKS };
@@ -392,83 +482,7 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 		const uint32_t mine = 1u + (tile == num_tiles - 1 ? (after_small << 16) | (after_big << 20) : 0u);
 		arrived = mine + __hip_atomic_fetch_add(seed0, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	}
-	const uint32_t excl = off + inc - c;
-
-	/* set_schedule_by_threshold, src/nccl_ofi_scheduler.cpp:77-133 */
-	const bool small = (c >> 16) != 0;
-	uint32_t rail = mod_rails(small ? carry_small + (excl >> 16) : carry_big + (excl & 0xffffu), p);
-	uint64_t max_stripe = size;
-	if (!small) {
-		/* (size - 1) / k: k is 1, 2 or 4 unless there are three rails */
-		uint64_t whole = size == 0 ? 0 : (size - 1) >> (k >> 1);
-		if (R == 3) {
-			whole = k == 3 ? (size == 0 ? 0 : (size - 1) / 3) : whole;
-		}
-		const uint64_t per = size == 0 ? 0 : 1 + whole;
-		max_stripe = div_ceil_by(per, p.align, p.align_shift) * p.align;
-	}
-	/* k stripes of max_stripe cover the message, so `left` is 0 from stripe k on and the
-	 * length of an unused entry comes out as 0 by itself; lanes past the end have k = 0 */
-	uint64_t left = size, offset = 0;
-	uint64_t f[12]; /* 4 x {rail word, offset, msg_size} */
-#pragma unroll
-	for (uint32_t s = 0; s < 4; s++) {
-		const bool used = s < k;
-		const uint64_t stripe = left < max_stripe ? left : max_stripe;
-		f[3 * s + 0] = used ? rail : 0; /* rail_id in the low 16 bits, padding zero */
-		f[3 * s + 1] = used ? offset : 0;
-		f[3 * s + 2] = stripe;
-		offset += stripe;
-		left -= stripe;
-		rail = rail + 1 == R ? 0 : rail + 1;
-	}
-	auto stage_row = [&](u32x4 *row) {
-#pragma unroll
-		for (uint32_t q = 0; q < 6; q++) {
-			u32x4 v;
-			v.x = (uint32_t)f[2 * q];
-			v.y = (uint32_t)(f[2 * q] >> 32);
-			v.z = (uint32_t)f[2 * q + 1];
-			v.w = (uint32_t)(f[2 * q + 1] >> 32);
-			row[q] = v;
-		}
-	};
-	if (live) {
-		num_xfers[i] = k;
-	}
-	const uint32_t valid = (n - base) < THREADS ? (n - base) : THREADS;
-	u32x4 *out = xfers + (uint64_t)base * 6;
-	if (FORM == TILES) {
-		/* A wavefront writes its rows by itself, the first and then the second half of its lanes', out of 3 KiB of LDS.  So
-		 * four workgroups share a CU, all the wavefronts it has room for, where three did with every row in LDS, and none
-		 * waits for another wavefront's rows (us, rows of a workgroup / of a wavefront / of half a one: 400,000 messages 12.7 /
-		 * 12.4 / 11.4, 1,000,000 21.7 / 21.1 / 21.2, 2,000,000 39.3 / 38.5 / 37.6, 6,000,000 113.2 / 111.7 / 110.6). */
-		u32x4 *const stage = &rows[wave * (32u * 6u)];
-#pragma unroll
-		for (uint32_t half = 0; half < 2; half++) {
-			if (lane / 32u == half) {
-				stage_row(&stage[lane % 32u * 6u]);
-			}
-			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-			__builtin_amdgcn_wave_barrier();
-#pragma unroll
-			for (uint32_t q = 0; q < 3; q++) {
-				const uint32_t v = q * 64u + lane, at = (wave * 64u + half * 32u) * 6u + v;
-				if (at < valid * 6) {
-					__builtin_nontemporal_store(stage[v], &out[at]);
-				}
-			}
-			__builtin_amdgcn_wave_barrier(); /* the rows of one half have been read before the other's are written */
-		}
-	} else {
-		/* The rows of the workgroup together: the small batches gain nothing by the other way, and the large ones lose
-		 * the narrow front on which the chip writes (16,000,000 messages 270 and 311 us). */
-		stage_row(&rows[threadIdx.x * 6]);
-		__syncthreads();
-		for (uint32_t v = threadIdx.x; v < valid * 6; v += THREADS) {
-			__builtin_nontemporal_store(rows[v], &out[v]);
-		}
-	}
+	write_rows<FORM == TILES, THREADS>(size, live, c, k, off + inc - c, carry_small, carry_big, p, n, base, rows, num_xfers, xfers);
 
 	if (threadIdx.x != 0) {
 		return;
@@ -487,6 +501,160 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 	}
 }
 
+/*
+ * The one-launch form for batches whose sizes are too many for every tile to look through: a tile counts its own messages,
+ * publishes the total in a word and adds up the words of the tiles before it, one a thread.  So it waits for other
+ * workgroups, all of which have been handed out before it, and every wait has an end:
+ * - After `looks` looks a tile that still misses words adds up the messages before it by itself, from their sizes.
+ * - The tile that moves the counters on may only do so when they have been read.  Tile 0 reads them before it publishes, and
+ *   says what they were in its word: a tile on its own reads the counters first and that word second, and takes the
+ *   word's if it is there.  The last tile, on its own, waits for that word with the counters; nobody waits for it.
+ * A word carries the batch's number, no other batch's on this scratch, so that nothing has to be cleared, and only ever grows.
+ * Words are read past the L2s, and up to 512 workgroups ask for the same few lines at once: eight copies, of which a tile
+ * reads one, are faster than one (150,000 messages 7.2 and 8.1 us, 300,000 9.2 and 10.3).
+ * Us in two launches / in this one, in a row (two launches of this length are also more than some hosts queue in that time):
+ *    10,300 messages   5.9-7.4 / 5.2
+ *    30,000            6.0-7.2 / 5.3
+ *   100,000            6.7-7.2 / 6.5
+ *   150,000            7.9     / 7.4
+ *   262,144            9.0     / 8.4
+ * Beyond 262,144 (a word a thread) workgroups would start while others write, and the words take longer than the second
+ * launch: 600,000 messages 15.1 / 17.5, 1,000,000 21.7 / 28.9.
+ */
+constexpr uint32_t kOnceTile = 512, kOnceCopies = 8;
+constexpr uint64_t kOnceBatch = (uint64_t)kOnceTile * kOnceTile;
+constexpr uint32_t kOnceLooks = 2048; /* some 2 ms */
+constexpr uint32_t kSeedLooks = 1u << 22;
+constexpr uint32_t kMissing = ~0u;
+__device__ __forceinline__ uint64_t look(const uint64_t *word)
+{
+	return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* a pair of residues, as the packed sums have them, in four bits, and back */
+__device__ __forceinline__ uint32_t four_bits(uint32_t residues)
+{
+	return (residues >> 16) << 2 | (residues & 3u);
+}
+__device__ __forceinline__ uint32_t of_four_bits(uint32_t bits)
+{
+	return (bits >> 2 & 3u) << 16 | (bits & 3u);
+}
+
+/* published: [kOnceCopies][kOnceTile] words, each the batch's number << 8 | tile 0's: the seed << 4 | residues of the tile's
+ * total */
+__global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
+	const uint64_t *__restrict__ sizes, uint32_t n, uint32_t num_tiles, ofi_amd_sched_state_t *__restrict__ state, uint64_t align,
+	uint64_t *published, uint64_t number, uint32_t max_looks, uint32_t *__restrict__ num_xfers, u32x4 *__restrict__ xfers,
+	uint32_t *__restrict__ err)
+{
+	constexpr uint32_t kWaves = kOnceTile / 64;
+	__shared__ u32x4 rows[kOnceTile * 3];
+	__shared__ uint32_t wave_sum[kWaves], seed_sum[kWaves];
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	const uint32_t tile = blockIdx.x, base = tile * kOnceTile, i = base + threadIdx.x;
+	const bool live = i < n;
+	const uint64_t size_read = __builtin_nontemporal_load(&sizes[min(i, n - 1u)]);
+	params_t p;
+	const bool usable = load_params(state, align, p);
+	const uint32_t small_counter = state->rr_small_counter, counter = state->rr_counter;
+	const uint64_t size = live ? size_read : 0;
+	__asm__ volatile("" : : "v"(size), "s"(small_counter), "s"(counter)); /* as in the emit kernel */
+	if (!usable) {
+		if (tile == 0 && threadIdx.x == 0) {
+			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE);
+		}
+		return;
+	}
+	const uint32_t R = p.num_rails, seed_read = (small_counter % R) << 16 | (counter % R);
+	uint32_t k = 0;
+	const uint32_t c = live ? contribution(size, p, k) : 0;
+	const uint32_t inc = wave_inclusive_scan(c);
+	if (lane == 63) {
+		wave_sum[wave] = inc;
+	}
+	__syncthreads();
+	uint32_t off = 0, tot = 0;
+#pragma unroll
+	for (uint32_t w = 0; w < kWaves; w++) {
+		const uint32_t ws = wave_sum[w];
+		off += (w < wave) ? ws : 0;
+		tot += ws;
+	}
+	if (threadIdx.x < kOnceCopies) {
+		const uint32_t seed_bits = tile == 0 ? four_bits(seed_read) << 4 : 0u;
+		__hip_atomic_fetch_max(&published[threadIdx.x * kOnceTile + tile],
+				       number << 8 | seed_bits | four_bits(residues(tot, R)), __ATOMIC_RELAXED,
+				       __HIP_MEMORY_SCOPE_AGENT);
+	}
+
+	const uint64_t *const words = published + tile % kOnceCopies * kOnceTile;
+	uint32_t acc = tile == 0 && wave == 0 ? seed_read : 0u;
+	if (wave * 64u < tile) {
+		acc = kMissing;
+		for (uint32_t looks = 0; looks < max_looks; looks++) {
+			const uint64_t word = threadIdx.x < tile ? look(&words[threadIdx.x]) : number << 8;
+			if (__ballot(word >> 8 != number) == 0) {
+				acc = wave_sum_of(of_four_bits((uint32_t)word & 15u) + of_four_bits((uint32_t)word >> 4 & 15u));
+				break;
+			}
+			__builtin_amdgcn_s_sleep(1);
+		}
+	}
+	if (lane == 0) {
+		seed_sum[wave] = acc;
+	}
+	__syncthreads();
+	uint32_t before_tile = 0;
+	bool missing = false;
+#pragma unroll
+	for (uint32_t w = 0; w < kWaves; w++) {
+		missing |= seed_sum[w] == kMissing;
+		before_tile += seed_sum[w];
+	}
+	if (missing) { /* the same in the whole workgroup */
+		const uint64_t word = look(&words[0]);
+		const uint32_t seed = word >> 8 == number ? of_four_bits((uint32_t)word >> 4 & 15u) : seed_read;
+		uint32_t smalls = 0, stripes = 0;
+		for (uint32_t at = threadIdx.x; at < base; at += kOnceTile) {
+			uint32_t unused;
+			const uint32_t each = contribution(sizes[at], p, unused);
+			smalls += each >> 16;
+			stripes += each & 0xffffu;
+		}
+		__syncthreads(); /* seed_sum has been read */
+		acc = wave_sum_of((smalls % R) << 16 | (stripes % R));
+		if (lane == 0) {
+			seed_sum[wave] = acc;
+		}
+		__syncthreads();
+		before_tile = seed;
+#pragma unroll
+		for (uint32_t w = 0; w < kWaves; w++) {
+			before_tile += seed_sum[w];
+		}
+	}
+	const uint32_t carry_small = (before_tile >> 16) % R, carry_big = (before_tile & 0xffffu) % R;
+	write_rows<true, kOnceTile>(size, live, c, k, off + inc - c, carry_small, carry_big, p, n, base, rows, num_xfers, xfers);
+
+	if (tile == num_tiles - 1 && threadIdx.x == 0) {
+		bool read = true;
+		if (missing) {
+			read = false;
+			for (uint32_t looks = 0; !read && looks < kSeedLooks; looks++) {
+				read = look(&words[0]) >> 8 >= number;
+				__builtin_amdgcn_s_sleep(8);
+			}
+		}
+		if (read) {
+			state->rr_small_counter = mod_rails(carry_small + (tot >> 16), p);
+			state->rr_counter = mod_rails(carry_big + (tot & 0xffffu), p);
+		} else {
+			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE); /* somebody has changed the state under the batch */
+		}
+	}
+}
+
 /* Scratch of the batches of one stream: launches on one stream are ordered, so they can share; launches on
  * different streams may overlap and must not.  Layout in 32-bit words: the arrival words of the one-launch
  * form; the seed word of the others, on a 128-byte line of its own; then the block totals; then the
@@ -501,11 +669,16 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 constexpr uint32_t kArrivalWords = 1024;
 constexpr uint32_t kSeedWord = kArrivalWords, kBlockWords = kSeedWord + 32;
 constexpr uint32_t kTileWords = kBlockWords + kMaxBlocks;
-constexpr uint32_t kScratchWords = kTileWords + kMaxTiles;
-static_assert((kArrivalWords & (kArrivalWords - 1)) == 0 && kBlockWords % 32 == 0, "a ring; block totals on a line");
+constexpr uint32_t kOnceWords = kTileWords + kMaxTiles; /* words of 64 bits */
+constexpr uint32_t kScratchWords = kOnceWords + 2 * kOnceCopies * kOnceTile;
+constexpr uint32_t kClearThreads = 256;
+static_assert((kArrivalWords & (kArrivalWords - 1)) == 0 && kBlockWords % 32 == 0 && kOnceWords % 32 == 0,
+	      "a ring; block totals and published words on a line");
+static_assert(kArrivalWords % kClearThreads == 0 && kOnceCopies * kOnceTile % kClearThreads == 0, "cleared by whole workgroups");
 struct scratch_t {
 	uint32_t *words = nullptr;
-	std::atomic<uint32_t> turn{ 0 }; /* of the next batch that counts arrivals */
+	std::atomic<uint32_t> turn{ 0 };    /* of the next batch that counts arrivals */
+	std::atomic<uint64_t> published{ 0 }; /* batches that published totals: the last one's number */
 };
 /* The stream behind a handle: a created stream has its own, but the null stream's stands for another
  * stream on each GPU, and hipStreamPerThread for another one in each thread besides. */
@@ -524,10 +697,12 @@ int key_of_stream(void *stream, stream_key_t *key)
 std::mutex g_ws_lock;
 std::map<stream_key_t, scratch_t> g_ws_by_stream;
 
-constexpr uint32_t kClearThreads = 256;
+/* The arrival words and the published ones; the others are written before they are read */
+constexpr uint32_t kClearBlocks = (kArrivalWords + 2 * kOnceCopies * kOnceTile) / kClearThreads;
 __global__ __launch_bounds__(kClearThreads) void stripe_scratch_kernel(uint32_t *__restrict__ words)
 {
-	words[blockIdx.x * kClearThreads + threadIdx.x] = 0;
+	const uint32_t at = blockIdx.x * kClearThreads + threadIdx.x;
+	words[at < kArrivalWords ? at : kOnceWords + (at - kArrivalWords)] = 0;
 }
 
 /* also where the runtime cannot say: the null stream while another one is captured */
@@ -550,13 +725,13 @@ int new_scratch(hipStream_t s, uint32_t **out)
 	OFI_AMD_HIP_TRY(hipMalloc((void **)&words, sizeof(uint32_t) * kScratchWords));
 	hipError_t e = hipSuccess;
 	if (!being_captured(s)) {
-		hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kArrivalWords / kClearThreads), dim3(kClearThreads), 0, s, words);
+		hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kClearBlocks), dim3(kClearThreads), 0, s, words);
 		e = hipGetLastError();
 	} else {
 		hipStream_t own = nullptr;
 		e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
 		if (e == hipSuccess) {
-			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kArrivalWords / kClearThreads), dim3(kClearThreads), 0, own,
+			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kClearBlocks), dim3(kClearThreads), 0, own,
 					   words);
 			e = hipGetLastError();
 			const hipError_t waited = hipStreamSynchronize(own);
@@ -629,10 +804,10 @@ uint32_t tiles_of(uint64_t n, uint32_t tile)
 }
 
 /* A batch that is being captured goes the two-launch way from its second tile on, all of whose scratch is
- * written before it is read: a replay would come back to the arrival word it was captured with, and its stream's
- * other batches may meanwhile be anywhere round the ring. */
+ * written before it is read: a replay would come back to the arrival word or the batch number it was captured with, and its
+ * stream's other batches may meanwhile be anywhere round the ring. */
 void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_amd_sched_state_t *d_state, uint64_t align,
-		  scratch_t &scratch, uint32_t *d_num_xfers, u32x4 *d_xfers, uint32_t *err)
+		  scratch_t &scratch, uint32_t *d_num_xfers, u32x4 *d_xfers, uint32_t *err, uint32_t looks = kOnceLooks)
 {
 	uint32_t *words = scratch.words;
 	uint32_t *seed0 = words + kSeedWord, *blocks = words + kBlockWords, *totals = words + kTileWords;
@@ -650,6 +825,13 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 		} else {
 			launch(stripe_emit_kernel<DIRECT, kDirectTile>, kDirectTile);
 		}
+		return;
+	}
+	if (total > kTwoLaunchBatch && total <= kOnceBatch && !being_captured(s)) {
+		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kOnceTile);
+		const uint64_t number = scratch.published.fetch_add(1, std::memory_order_relaxed) + 1;
+		hipLaunchKernelGGL(stripe_once_kernel, dim3(tiles), dim3(kOnceTile), 0, s, d_sizes, n, tiles, d_state, align,
+				   reinterpret_cast<uint64_t *>(words + kOnceWords), number, looks, d_num_xfers, d_xfers, err);
 		return;
 	}
 	if (total <= kSmallBatch) {
@@ -696,9 +878,11 @@ using namespace ofi_amd;
 
 extern "C" {
 
-int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
-			uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
-			void *stream)
+/* ofi_amd_sched_batch with the number of looks that a tile takes at the words of the others, for the tests: after none, every
+ * tile adds up what is before it by itself. */
+int ofi_amd_sched_batch_looks(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
+			      uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
+			      void *stream, uint32_t looks)
 {
 	int rc = require_device();
 	if (rc != 0) {
@@ -736,12 +920,19 @@ int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes,
 				return rc;
 			}
 		}
-		launch_batch(s, d_sizes, n, d_state, align, scratch, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err);
+		launch_batch(s, d_sizes, n, d_state, align, scratch, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err, looks);
 	} catch (...) {
 		return -ENOMEM;
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
+}
+
+int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
+			uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
+			void *stream)
+{
+	return ofi_amd_sched_batch_looks(d_state, d_sizes, n, align, d_num_xfers, d_xfers, stream, kOnceLooks);
 }
 
 int ofi_amd_sched_stream_release(void *stream)
