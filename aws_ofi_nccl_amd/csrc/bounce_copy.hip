@@ -65,16 +65,16 @@ struct __attribute__((packed, aligned(4))) dword_aligned_u32x4 {
 	u32x4 v;
 };
 
-/* Buffers (= wavefronts) per workgroup and consecutive workgroups that share an XCD, swept over
+/* Buffers (= wavefronts) per workgroup and consecutive ones that share an XCD, swept over
  * thousands of launches in a row on 65,536 buffers.  Bounce copy: 8 wavefronts per workgroup with
  * runs of 32 buffers per XCD was the fastest (91.1 us per launch, every wavefront reading its own
  * word back; 4 wavefronts: 91.8, 2: 92.5, 16: 92.6; runs of 64 buffers 91.7).  The eager copy, whose sources are rx buffers in
- * arrival order, prefers single-wavefront workgroups (1 x 32: 97.8 us, 4 x 8: 98.4, 8 x 4: 101.6,
- * 16 x 2: 108.6), and so does the table copy (1: 419.9 us per GiB, 4: 439.5, 8: 430.3). */
+ * arrival order, prefers single-wavefront workgroups while every wavefront reads its own bytes back (runs of 32: 97.8 us, 4
+ * wavefronts 98.4, 8: 101.6, 16: 108.6), four where a workgroup reads them back together (eager_copy_kernel), and the table copy
+ * single ones (1: 419.9 us per GiB, 4: 439.5, 8: 430.3). */
 constexpr int kBounceWaves = 8;
 constexpr uint32_t kBounceRun = 32;
-constexpr int kEagerWaves = 1;
-constexpr uint32_t kEagerGroup = 32;
+constexpr int kEagerWaves = 4; /* of TOGETHER */
 constexpr int kTableWaves = 1;
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kRows = 8;              /* rows of 64 x 16 bytes per trip: 8 KiB per wave */
@@ -355,49 +355,94 @@ __device__ __forceinline__ void copy_any(const uint8_t *__restrict__ s, uint8_t 
  * The same copy for eager arrivals as they sit in rx buffers: an 8-byte header, then the
  * payload, which goes to a receive buffer at any alignment, truncated to that buffer's
  * length (rdma_eager_copy_req::post, src/nccl_ofi_rdma.cpp:2729-2776).
+ *
+ * TOGETHER as in the bounce copy: one wavefront reads the bytes of its workgroup's four buffers back behind a barrier.  Each by
+ * itself in workgroups of one and together in workgroups of four, on other buffers at every launch / on the same ones, us:
+ *   65,536 of up to 8 KiB    120.7 / 95.5  121.0 / 95.8  (two wavefronts 120.9 / 96.4, eight 121.8 / 99.1; runs of 32: 121.0 / 97.2)
+ *   20,000 of up to 8 KiB     38.2 / 32.7   38.3 / 32.0
+ *   65,536 of up to 4000 B    66.3 / 51.1   66.1 / 48.7
+ *   65,536 of up to 500 B     27.7 / 26.9   24.7 / 23.5  (two wavefronts 27.4 / 26.3, eight 25.3 / 24.0; no read-back 17.1)
+ *   20,000 of up to 500 B     11.7 /  8.9   10.5 /  8.5
  */
-template <bool KEEP>
-__global__ __launch_bounds__(64 * kEagerWaves) void eager_copy_kernel(
+constexpr int eager_waves(read_back_t back)
+{
+	return back == TOGETHER ? kEagerWaves : 1;
+}
+constexpr uint32_t eager_run(read_back_t back)
+{
+	return back == TOGETHER ? 64 : 32;
+}
+template <read_back_t BACK>
+__global__ __launch_bounds__(64 * eager_waves(BACK)) void eager_copy_kernel(
 	const uint8_t *__restrict__ rx_base, const uint64_t *__restrict__ rx_off,
 	const uint32_t *__restrict__ recv_len, uint8_t *__restrict__ dst_base,
 	const uint64_t *__restrict__ dst_off, const uint32_t *__restrict__ dst_len, uint32_t n,
 	uint32_t *__restrict__ copied, uint32_t *__restrict__ flush)
 {
+	constexpr int WAVES = eager_waves(BACK);
+	constexpr uint32_t kGroup = eager_run(BACK) / WAVES;
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const uint32_t xcd = blockIdx.x % kXcds;
 	const uint32_t turn = blockIdx.x / kXcds;
-	const uint32_t wg = ((turn / kEagerGroup) * kXcds + xcd) * kEagerGroup + turn % kEagerGroup;
-	const uint32_t buf = wg * kEagerWaves + wave;
-	if (buf >= n) {
+	const uint32_t wg = ((turn / kGroup) * kXcds + xcd) * kGroup + turn % kGroup;
+	const uint32_t first = wg * WAVES, buf = first + wave;
+	if (BACK != TOGETHER && buf >= n) {
 		return;
 	}
-	const uint64_t from = rx_off[buf], to = dst_off[buf];
-	const uint32_t received = recv_len[buf], room = dst_len[buf];
-	/* all of the entry is in hand from here on: the compiler would ask for the source only once the length is known (us, other
-	 * buffers at every launch: 2000 of up to 8 KiB 5.9 -> 5.6, 65,536 of up to 4000 B 67.9 -> 66.4, of up to 500 B 28.5 -> 27.6) */
-	__asm__ volatile("" : : "s"(from), "s"(to), "s"(received), "s"(room), "s"(copied), "s"(flush));
-	const uint8_t *s = rx_base + from + 8u; /* skip nccl_ofi_eager_msg_header_t */
-	uint8_t *d = dst_base + to;
-	const uint32_t bytes = min(received, room);
-	if (copied != nullptr && lane == 0) {
-		copied[buf] = bytes;
+	uint8_t *d = nullptr;
+	uint32_t bytes = 0;
+	if (BACK != TOGETHER || buf < n) {
+		const uint64_t from = rx_off[buf], to = dst_off[buf];
+		const uint32_t received = recv_len[buf], room = dst_len[buf];
+		/* all of the entry is in hand from here on: the compiler would ask for the source only once the length is known (us, other
+		 * buffers at every launch: 2000 of up to 8 KiB 5.9 -> 5.6, 65,536 of up to 4000 B 67.9 -> 66.4, of up to 500 B 28.5 -> 27.6) */
+		__asm__ volatile("" : : "s"(from), "s"(to), "s"(received), "s"(room), "s"(copied), "s"(flush));
+		const uint8_t *s = rx_base + from + 8u; /* skip nccl_ofi_eager_msg_header_t */
+		d = dst_base + to;
+		bytes = min(received, room);
+		if (copied != nullptr && lane == 0) {
+			copied[buf] = bytes;
+		}
+
+		copy_any<BACK == BY_ITSELF>(s, d, bytes, lane);
 	}
 
-	copy_any<KEEP>(s, d, bytes, lane);
-
-	if (flush != nullptr) {
-		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-		/* the first min(4, bytes) destination bytes, little-endian: lanes 0..3 read one byte
-		 * each in one instruction (the destination has no alignment to read a word from),
-		 * then the four are combined inside the quad */
-		uint32_t word = 0;
-		if (lane < min(bytes, 4u)) {
-			const uint32_t byte = KEEP ? d[lane] : __builtin_nontemporal_load(d + lane);
-			word = byte << (8u * lane);
-		}
+	/* The first min(4, bytes) destination bytes, little-endian: a quad of lanes reads one byte
+	 * each in one instruction (the destination has no alignment to read a word from),
+	 * then the four are combined inside the quad. */
+	auto word_of = [](uint32_t byte, uint32_t at) {
+		uint32_t word = byte << (8u * at);
 		word |= __shfl_xor(word, 1, 64);
 		word |= __shfl_xor(word, 2, 64);
+		return word;
+	};
+	if constexpr (BACK == TOGETHER) {
+		__shared__ uint8_t *back[WAVES];
+		__shared__ uint32_t count[WAVES];
+		if (lane == 0) {
+			back[wave] = d;
+			count[wave] = min(bytes, 4u);
+		}
+		__syncthreads(); /* the copies, too, are in front of it */
+		if (threadIdx.x < WAVES * 4) {
+			const uint32_t of = lane >> 2, at = lane & 3u;
+			uint32_t byte = 0;
+			if (at < count[of]) {
+				byte = __builtin_nontemporal_load(back[of] + at);
+			}
+			const uint32_t word = word_of(byte, at);
+			if (at == 0 && first + of < n) {
+				flush[first + of] = word;
+			}
+		}
+	} else if constexpr (BACK == BY_ITSELF) {
+		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+		uint32_t byte = 0;
+		if (lane < min(bytes, 4u)) {
+			byte = d[lane];
+		}
+		const uint32_t word = word_of(byte, lane & 3u);
 		if (lane == 0) {
 			flush[buf] = word;
 		}
@@ -645,18 +690,18 @@ int ofi_amd_eager_copy_batch(const void *rx_base, const uint64_t *d_rx_off, cons
 	if (!rx_base || !d_rx_off || !d_recv_len || !d_dst_off || !d_dst_len || n > (1u << 30)) {
 		return -EINVAL;
 	}
-	uint32_t blocks = (n + kEagerWaves - 1) / kEagerWaves;
-	const uint32_t round = kXcds * kEagerGroup;
-	blocks = (blocks + round - 1) / round * round;
-	auto launch = [&](auto kernel) {
-		hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kEagerWaves), 0, as_stream(stream),
+	auto launch = [&](auto kernel, read_back_t back) {
+		const uint32_t round = kXcds * eager_run(back), waves = (uint32_t)eager_waves(back); /* whole rounds over the XCDs */
+		hipLaunchKernelGGL(kernel, dim3((n + round - 1) / round * (round / waves)), dim3(64 * waves), 0, as_stream(stream),
 				   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base),
 				   d_dst_off, d_dst_len, n, d_copied, d_flush);
 	};
-	if (d_flush && n <= kKeepEager) {
-		launch(eager_copy_kernel<true>);
+	if (!d_flush) {
+		launch(eager_copy_kernel<NO_READ_BACK>, NO_READ_BACK);
+	} else if (n <= kKeepEager) {
+		launch(eager_copy_kernel<BY_ITSELF>, BY_ITSELF);
 	} else {
-		launch(eager_copy_kernel<false>);
+		launch(eager_copy_kernel<TOGETHER>, TOGETHER);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
