@@ -228,8 +228,16 @@ __device__ __forceinline__ void copy_to_aligned(const uint8_t *__restrict__ s, u
 }
 
 /* The flush words: no output for them, each buffer's read back by its own wavefront (kept rows), or a workgroup's
- * together (streamed ones). */
-enum read_back_t { NO_READ_BACK, BY_ITSELF, TOGETHER };
+ * together (streamed ones, or kept ones). */
+enum read_back_t { NO_READ_BACK, BY_ITSELF, TOGETHER, KEPT_TOGETHER };
+constexpr bool keeps_rows(read_back_t back)
+{
+	return back == BY_ITSELF || back == KEPT_TOGETHER;
+}
+constexpr bool by_workgroup(read_back_t back)
+{
+	return back == TOGETHER || back == KEPT_TOGETHER;
+}
 
 /*
  * TOGETHER: one wavefront reads the words of its workgroup's eight buffers back, in one instruction, behind a barrier,
@@ -242,6 +250,14 @@ enum read_back_t { NO_READ_BACK, BY_ITSELF, TOGETHER };
  *   1,000,000 of up to 60 B out of a pool 222 / 219     229 / 221
  * (Counting the wavefronts in an LDS word, for the last one to read back without a barrier, needs a barrier in front of
  * the copies all the same: no faster for long buffers, the last two lines 20.3 / 17.6 and 232 / 229.)
+ * KEPT_TOGETHER: the words are found in the L2, but eight of them still leave in one write, to host memory as a rule.  Each by
+ * itself and together, rows kept, other buffers at every launch / the same ones, us:
+ *   8100 of up to 8 KiB, packed           18.2 / 11.4   18.4 / 11.4   (7000: 16.7 / 10.2  16.8 / 10.3, 4000: 11.0 / 6.2  11.2 / 6.4)
+ *   16,000 of up to 4 KiB                 18.2 / 11.9   18.0 / 11.7
+ *   32,000 of up to 2000 B                21.5 / 13.6   19.6 / 13.0
+ *   65,536 of up to 1000 B                28.9 / 18.1   27.7 / 17.9
+ *   200,000 of up to 100 B                47.3 / 46.7   44.7 / 44.2
+ *   450,000 of up to 60 B                 95.7 / 82.2   91.3 / 80.0
  * NO_READ_BACK is a kernel of its own because one that claims LDS starts later: 65,536 of up to 60 B 11.2 us with
  * the claim, 9.8 without.
  */
@@ -263,12 +279,12 @@ __global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
 	const uint32_t turn = blockIdx.x / kXcds;
 	const uint32_t wg = ((turn / kGroup) * kXcds + xcd) * kGroup + turn % kGroup;
 	const uint32_t first = wg * kBounceWaves, buf = first + wave;
-	if (BACK != TOGETHER && buf >= n) {
+	if (!by_workgroup(BACK) && buf >= n) {
 		return;
 	}
 
 	uint8_t *d = nullptr; /* until there is something to read back */
-	if (BACK != TOGETHER || buf < n) { /* all of a workgroup come to the barrier of TOGETHER */
+	if (!by_workgroup(BACK) || buf < n) { /* all of a workgroup come to the barrier */
 		const uint64_t doff = dst_off[buf];
 		const uint32_t bytes = len[buf];
 		const uint64_t soff = src_off[buf];
@@ -280,26 +296,27 @@ __global__ __launch_bounds__(64 * kBounceWaves) void bounce_scatter_kernel(
 			if (lane == 0) {
 				atomicOr(err, ofi_amd::ASYNC_ERR_BOUNCE_RANGE);
 			}
-			if (BACK != TOGETHER) {
+			if (!by_workgroup(BACK)) {
 				return;
 			}
 		} else {
 			const uint8_t *s = src + soff;
 			d = arena + doff;
 			if (bytes != 0) {
-				copy_to_aligned<BACK == BY_ITSELF>(s, d, bytes, lane);
+				copy_to_aligned<keeps_rows(BACK)>(s, d, bytes, lane);
 			}
 		}
 	}
 
-	if constexpr (BACK == TOGETHER) {
+	if constexpr (by_workgroup(BACK)) {
 		__shared__ uint8_t *back[kBounceWaves]; /* nullptr: none */
 		if (lane == 0) {
 			back[wave] = d;
 		}
 		__syncthreads(); /* the copies, too, are in front of it */
 		if (threadIdx.x < kBounceWaves && back[lane] != nullptr) {
-			flush[first + lane] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(back[lane]));
+			const uint32_t *word = reinterpret_cast<const uint32_t *>(back[lane]);
+			flush[first + lane] = BACK == TOGETHER ? __builtin_nontemporal_load(word) : *word;
 		}
 	} else if constexpr (BACK == BY_ITSELF) {
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -667,8 +684,10 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 	};
 	if (!d_flush) {
 		launch(bounce_scatter_kernel<NO_READ_BACK>);
-	} else if (n <= kKeepBounce || (n <= kKeepLines && src_bytes <= kKeepBytes)) {
+	} else if (n <= kKeepBounce) {
 		launch(bounce_scatter_kernel<BY_ITSELF>);
+	} else if (n <= kKeepLines && src_bytes <= kKeepBytes) {
+		launch(bounce_scatter_kernel<KEPT_TOGETHER>);
 	} else {
 		launch(bounce_scatter_kernel<TOGETHER>);
 	}
