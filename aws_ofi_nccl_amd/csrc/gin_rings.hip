@@ -9,16 +9,15 @@
  * (include/nccl_ofi_gin_base.h:83-91) as a 64-byte record -- into one ring per
  * context that follows the slot protocol of include/nccl_ofi_mpsc_ring.h:56-163.
  *
- * Per 256-op round of a workgroup (= one context):
- *   1. every lane decides whether it has an op; slot positions come from a
- *      wavefront ballot + popcount prefix and a workgroup prefix over the four
- *      wave counts, added to the ring cursor -- no atomic per op;
- *   2. each lane waits until its slot is free (sequence == position), bounded
- *      by spin_limit polls;
- *   3. the wave stages its 64 records in LDS and writes them as 16-byte stores,
- *      1 KiB contiguous per instruction, to the pinned ring;
+ * A workgroup is a context, each of its wavefronts takes every so manieth group of 64 ops and
+ * goes on by itself:
+ *   1. slot positions follow from the ring cursor and the op's number -- no atomic;
+ *   2. the wavefront waits until its last slot is free (sequence == position), bounded by spin_limit
+ *      polls, unless an earlier look further ahead has already seen that;
+ *   3. it stages its 64 records in LDS and writes them as 16-byte stores, 1 KiB contiguous per
+ *      instruction, to the pinned ring;
  *   4. system-scope fence, then each lane publishes sequence = position + 1
- *      with a release store (64 lanes = one contiguous 256-byte write).
+ *      (64 lanes = one contiguous 256-byte write).
  * The ring cursor (device memory, shared with ofi_amd_gin_dev_put) stays in a register for
  * the whole launch and is written back once at the end: this generator owns its context
  * for the duration of a launch.
@@ -34,8 +33,23 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kThreads = 256;
-constexpr uint32_t kWaves = kThreads / 64;
+/*
+ * Wavefronts of a context.  A group is a chain of trips over the host link, some 5 us, so a few contexts want several
+ * groups on their way at once.  The link is shared evenly by all that is, though, and nobody's group has arrived before nearly
+ * everybody's has, while the consumer waits: 256 contexts x 256 records, 4.4 MB, arrive together after some 80 us, x 64
+ * after 20.  Us to produce alone / to produce and drain on four threads with 64, 128 and 256 threads a context, and,
+ * last, with 256 that met at three barriers a round and looked for free slots in every one, which is what this was before:
+ *     1 x 1000    21.2 / 24.9    13.8 / 19.1    12.7 / 18.3    20.2
+ *     8 x 1000    25.8 / 50.6    19.6 / 49.0    19.0 / 49.8    25.1 / 61.2
+ *    16 x 300     14.6 / 44.8    14.2 / 35.8    14.8 / 45.6    17.5
+ *    24 x 1000    38.8 / 94.7    39.1 / 93.2    38.6 / 93.8    44.3
+ *   128 x 1000     170 / 358      171 / 321      170 / 330      171 / 325
+ *   256 x 300      108 / 246      110 / 303      107 / 257      122 / 260
+ *   256 x 1000     335 / 616      339 / 607      337 / 734      342 / 829
+ * (The drain by itself takes up to a fifth longer in one process than in another.  What the producer adds to it, 256 x 1000:
+ * -30 to 25 with 64 threads a context, 12 to 60 with 128, 80 to 140 with 256 and 170 with 1024.)
+ */
+constexpr uint32_t kMostThreads = 256;
 constexpr uint64_t kDefaultSpinLimit = 1ull << 22;
 static_assert(OFI_AMD_GIN_DEV_TIMEOUT_BIT == ofi_amd::ASYNC_ERR_GIN_TIMEOUT,
 	      "the device header and the status reader agree on the timeout bit");
@@ -94,119 +108,112 @@ __device__ __forceinline__ void make_desc(uint64_t seed, uint32_t ctx, uint64_t 
 	       ((uint64_t)kind << 48);
 }
 
-__global__ __launch_bounds__(kThreads) void gin_produce_seeded_kernel(
-	u32x4 *__restrict__ records, uint32_t *__restrict__ sequences,
-	uint32_t *__restrict__ enqueue_pos, uint32_t *__restrict__ status, uint32_t capacity,
-	uint64_t seed, uint64_t ops, uint32_t peer_rank, uint32_t signal_every, uint32_t signal_op,
+__global__ __launch_bounds__(kMostThreads) void gin_produce_seeded_kernel(
+	u32x4 *__restrict__ records, uint32_t *__restrict__ sequences, uint32_t *__restrict__ enqueue_pos, uint32_t capacity,
+	uint64_t seed, uint64_t ops, uint32_t *__restrict__ status, uint32_t peer_rank, uint32_t signal_every, uint32_t signal_op,
 	uint32_t aggregate_mask, uint64_t spin_limit)
 {
-	__shared__ u32x4 stage[kWaves][64 * 4];
-	__shared__ uint32_t wave_count[kWaves];
+	extern __shared__ u32x4 stages[]; /* 64 records of 4 x 16 B for each wavefront */
 
 	const uint32_t ctx = blockIdx.x;
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const uint32_t waves = blockDim.x / 64u;
 	const uint32_t mask = capacity - 1;
-	u32x4 *ring = records + (uint64_t)ctx * capacity * 4;
-	uint32_t *seq = sequences + (uint64_t)ctx * capacity;
+	u32x4 *const ring = records + (uint64_t)ctx * capacity * 4;
+	uint32_t *const seq = sequences + (uint64_t)ctx * capacity;
+	u32x4 *const stage = stages + wave * (64u * 4u);
 
-	uint32_t cursor = __hip_atomic_load(&enqueue_pos[ctx * kGinReserveStride], __ATOMIC_RELAXED,
-					    __HIP_MEMORY_SCOPE_AGENT);
-
-	for (uint64_t round = 0; round < ops; round += kThreads) {
-		const uint64_t i = round + threadIdx.x;
+	const uint32_t cursor = __builtin_amdgcn_readfirstlane(
+		__hip_atomic_load(&enqueue_pos[ctx * kGinReserveStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+	uint32_t horizon = cursor; /* every position before it has been seen free in this launch */
+	bool timed_out = false;
+	for (uint64_t first = wave * 64u; first < ops; first += waves * 64u) {
+		const uint64_t i = first + lane;
 		const bool active = i < ops;
-
-		/* slot reservation: ballot + prefix popcount, then a prefix over the waves */
-		const uint64_t ballot = __ballot(active);
-		const uint32_t lane_prefix = __popcll(ballot & ((1ull << lane) - 1ull));
-		if (lane == 0) {
-			wave_count[wave] = __popcll(ballot);
-		}
-		__syncthreads();
-		uint32_t wave_base = 0, total = 0;
-#pragma unroll
-		for (uint32_t w = 0; w < kWaves; w++) {
-			const uint32_t c = wave_count[w];
-			wave_base += (w < wave) ? c : 0;
-			total += c;
-		}
-		const uint32_t pos = cursor + wave_base + lane_prefix;
-		const uint32_t slot = pos & mask;
+		const uint32_t count = ops - first < 64u ? (uint32_t)(ops - first) : 64u;
+		const uint32_t base = cursor + (uint32_t)first, pos = base + lane;
 
 		uint64_t w[8];
-		if (active) {
-			make_desc(seed, ctx, i, peer_rank, signal_every, signal_op, aggregate_mask, w);
-		}
+		make_desc(seed, ctx, i, peer_rank, signal_every, signal_op, aggregate_mask, w);
 
-		/* Wait for the consumer to have freed the wave's slots one lap ago.  The
-		 * single consumer frees slots in position order, so the slot of the
-		 * wave's highest position being free implies the others are: one lane
-		 * polls one word instead of 64 lanes polling over the host link. */
-		bool timed_out = false;
-		if (ballot != 0) {
-			const uint32_t last = 63u - (uint32_t)__clzll((long long)ballot);
-			const uint32_t last_pos = __shfl(pos, last, 64);
-			if (lane == 0) {
-				uint64_t spins = 0;
-				while (__hip_atomic_load(&seq[last_pos & mask], __ATOMIC_RELAXED,
-							 __HIP_MEMORY_SCOPE_SYSTEM) != last_pos) {
-					if (++spins > spin_limit) {
-						timed_out = true;
-						break;
-					}
-					__builtin_amdgcn_s_sleep(16);
+		/* Wait for the consumer to have freed the wave's slots one lap ago.  The single consumer frees slots in
+		 * position order, so a free slot implies the ones before it, and what has been seen free stays so until it is
+		 * published here: one look over the host link takes in the wave's last slot, one half a lap on and the last of
+		 * the lap that the launch began with. */
+		const uint32_t last = base + count - 1u;
+		if ((int32_t)(last - horizon) >= 0) {
+			const uint32_t look = lane == 0 ? last : (lane == 1 ? last + capacity / 2 : cursor + capacity - 1u);
+			uint64_t spins = 0, seen;
+			for (;;) {
+				uint32_t there = ~look;
+				if (lane < 3u) {
+					there = __hip_atomic_load(&seq[look & mask], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 				}
+				seen = __ballot(there == look && (int32_t)(look - last) >= 0);
+				if (seen != 0) {
+					break;
+				}
+				if (++spins > spin_limit) {
+					timed_out = true;
+					break;
+				}
+				__builtin_amdgcn_s_sleep(16);
 			}
-		}
-		if (__syncthreads_or(timed_out ? 1 : 0)) {
-			if (threadIdx.x == 0) {
-				atomicOr(status, ofi_amd::ASYNC_ERR_GIN_TIMEOUT);
+			if (timed_out) {
+				break;
 			}
-			return; /* every wave leaves here: the grid always drains */
+#pragma unroll
+			for (int l = 0; l < 3; l++) {
+				const uint32_t free_to = (uint32_t)__builtin_amdgcn_readlane((int)look, l) + 1u;
+				horizon = ((seen >> l) & 1u) != 0 && (int32_t)(free_to - horizon) > 0 ? free_to : horizon;
+			}
+			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
 		}
-		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
 
 		/* stage: lane l holds record l of this wave */
-		if (active) {
 #pragma unroll
-			for (uint32_t q = 0; q < 4; q++) {
-				u32x4 v;
-				v.x = (uint32_t)w[2 * q];
-				v.y = (uint32_t)(w[2 * q] >> 32);
-				v.z = (uint32_t)w[2 * q + 1];
-				v.w = (uint32_t)(w[2 * q + 1] >> 32);
-				stage[wave][lane * 4 + q] = v;
-			}
+		for (uint32_t q = 0; q < 4; q++) {
+			u32x4 v;
+			v.x = (uint32_t)w[2 * q];
+			v.y = (uint32_t)(w[2 * q] >> 32);
+			v.z = (uint32_t)w[2 * q + 1];
+			v.w = (uint32_t)(w[2 * q + 1] >> 32);
+			stage[lane * 4 + q] = v;
 		}
-		__syncthreads();
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
 
 		/* write-out: instruction q covers records 16q..16q+15 of the wave, 16 B per lane */
 #pragma unroll
 		for (uint32_t q = 0; q < 4; q++) {
-			const uint32_t rec = q * 16 + (lane >> 2);
-			const uint32_t part = lane & 3u;
-			const uint32_t rec_pos = __shfl(pos, rec, 64);
-			if ((ballot >> rec) & 1ull) {
-				ring[(uint64_t)(rec_pos & mask) * 4 + part] = stage[wave][rec * 4 + part];
+			const uint32_t rec = q * 16 + (lane >> 2), part = lane & 3u;
+			if (rec < count) {
+				ring[(uint64_t)((base + rec) & mask) * 4 + part] = stage[rec * 4 + part];
 			}
 		}
 
 		/* publish */
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
 		if (active) {
-			__hip_atomic_store(&seq[slot], pos + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+			__hip_atomic_store(&seq[pos & mask], pos + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 		}
-		cursor += total;
-		__syncthreads();
+		__builtin_amdgcn_wave_barrier(); /* the records have been read before the next ones are staged */
 	}
 
+	if (timed_out && lane == 0) {
+		atomicOr(status, ofi_amd::ASYNC_ERR_GIN_TIMEOUT);
+	}
+	/* every wave comes here, if only when it has waited as long as it may: the grid always drains */
+	if (__syncthreads_or(timed_out ? 1 : 0)) {
+		return;
+	}
 	if (threadIdx.x == 0) {
 		/* the free-slot horizon of the device-side put follows the cursor: every position
 		 * this kernel filled was seen free first */
-		__hip_atomic_store(&enqueue_pos[ctx * kGinReserveStride + 1], cursor, __ATOMIC_RELAXED,
+		const uint32_t end = cursor + (uint32_t)ops;
+		__hip_atomic_store(&enqueue_pos[ctx * kGinReserveStride + 1], end, __ATOMIC_RELAXED,
 				   __HIP_MEMORY_SCOPE_AGENT);
-		__hip_atomic_store(&enqueue_pos[ctx * kGinReserveStride], cursor, __ATOMIC_RELEASE,
-				   __HIP_MEMORY_SCOPE_AGENT);
+		__hip_atomic_store(&enqueue_pos[ctx * kGinReserveStride], end, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 	}
 }
 
@@ -368,10 +375,10 @@ int ofi_amd_gin_produce_seeded(ofi_amd_gin_rings_t *r, uint64_t seed, uint64_t o
 	if (ops_per_context == 0) {
 		return 0;
 	}
-	hipLaunchKernelGGL(gin_produce_seeded_kernel, dim3(r->n_contexts), dim3(kThreads), 0,
-			   as_stream(stream), reinterpret_cast<u32x4 *>(r->d_records), r->d_sequences,
-			   r->d_reserve, r->d_status, r->capacity, seed, ops_per_context, peer_rank,
-			   signal_every, signal_op, aggregate_mask,
+	const uint32_t threads = r->n_contexts < 16 ? kMostThreads : (r->n_contexts < 32 ? kMostThreads / 2 : 64u);
+	hipLaunchKernelGGL(gin_produce_seeded_kernel, dim3(r->n_contexts), dim3(threads), threads * 64u,
+			   as_stream(stream), reinterpret_cast<u32x4 *>(r->d_records), r->d_sequences, r->d_reserve, r->capacity,
+			   seed, ops_per_context, r->d_status, peer_rank, signal_every, signal_op, aggregate_mask,
 			   spin_limit ? spin_limit : kDefaultSpinLimit);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
