@@ -326,6 +326,11 @@ __global__ __launch_bounds__(64 * kMostRegionWaves) void region_choice_kernel(
 	 * the end of the launch. */
 	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const region_run_t run = runs[blockIdx.y];
+	/* The arguments that are not in registers yet lie on four lines of memory: all are asked for at once, along with the run,
+	 * and not each when its turn comes (us, 1 platform of 120 x 12 4.7 -> 4.4, 4 of 280 x 30 7.5 -> 7.1, 4 of 560 x 44 8.9 ->
+	 * 8.6; model grids lose by the same, 32 of 140 x 11 8.4 -> 8.8: their workgroups then write all at once). */
+	__asm__ volatile("" : : "s"(far_point.x), "s"(far_point.y), "s"(t.size_span), "s"(t.rank_span), "s"(g.nodes), "s"(g.log2_sizes),
+			 "s"(g.log2_ranks), "s"(run.first_poly), "s"(run.pi));
 	/* which of a group's eight tiles an XCD takes rotates with the platform entry: the tiles
 	 * differ in cost (size range), and an XCD that kept the same ones for every
 	 * entry would keep the same share of the long ones */

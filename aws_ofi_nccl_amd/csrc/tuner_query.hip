@@ -112,12 +112,14 @@ __device__ __forceinline__ void region_choose_wave(const int4 *__restrict__ poly
  * slowly as one of 64, so the eight answers of a workgroup, 8 bytes each, meet in LDS and leave as a line
  * (the call for 1200 questions, with two writes of 8 bytes each and questions of a line and a half 37.6 us, now 18.6;
  * for 259 questions 15.7 and 13.0; in workgroups of one question 23.1 and 13.0).
+ * The structure comes first, so that no argument is preloaded: here that is no gain (259 questions 13.1 us, preloaded 13.3; 16
+ * 10.65 and 10.8).
  */
-__global__ __launch_bounds__(64 * kQueryWaves) void tuner_query_kernel(const uint64_t *__restrict__ queries, uint32_t n,
-								       uint32_t call, uint64_t *__restrict__ answers,
-								       const int4 *__restrict__ polys,
+__global__ __launch_bounds__(64 * kQueryWaves) void tuner_query_kernel(pt_t far_point, const int4 *__restrict__ polys,
 								       const double4_t *__restrict__ boxes,
-								       const edge_t *__restrict__ edges, pt_t far_point)
+								       const edge_t *__restrict__ edges,
+								       const uint64_t *__restrict__ queries, uint32_t n,
+								       uint32_t call, uint64_t *__restrict__ answers)
 {
 	__shared__ uint32_t found[kQueryWaves];
 	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -374,9 +376,10 @@ extern "C" int ofi_amd_tuner_query(const ofi_amd_tuner_query_t *queries, uint32_
 		const uint32_t here = n - at < kMostPerLaunch ? n - at : kMostPerLaunch;
 		const uint32_t waves = here < kQueryWaves ? here : kQueryWaves;
 		hipLaunchKernelGGL(tuner_query_kernel, dim3((here + kQueryWaves - 1) / kQueryWaves), dim3(64 * waves), 0,
-				   g_stage.stream, static_cast<const uint64_t *>(g_stage.dq) + (uint64_t)at * kQueryWords, here, call,
-				   static_cast<uint64_t *>(g_stage.da) + at, reinterpret_cast<const int4 *>(tables.poly),
-				   reinterpret_cast<const double4_t *>(tables.bbox), tables.edges, tables.far_point);
+				   g_stage.stream, tables.far_point, reinterpret_cast<const int4 *>(tables.poly),
+				   reinterpret_cast<const double4_t *>(tables.bbox), tables.edges,
+				   static_cast<const uint64_t *>(g_stage.dq) + (uint64_t)at * kQueryWords, here, call,
+				   static_cast<uint64_t *>(g_stage.da) + at);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return collect_answers(g_stage, n, call, answers);
