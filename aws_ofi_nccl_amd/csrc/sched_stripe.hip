@@ -508,7 +508,8 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
  * - After `looks` looks a tile that still misses words adds up the messages before it by itself, from their sizes.
  * - The tile that moves the counters on may only do so when they have been read.  Tile 0 reads them before it publishes, and
  *   says what they were in its word: a tile on its own reads the counters first and that word second, and takes the
- *   word's if it is there.  The last tile, on its own, waits for that word with the counters; nobody waits for it.
+ *   word's if it is there.  The last tile, on its own, waits for that word with the counters; nobody waits for it.  Both look
+ *   at the first copy: of another one the word could still be missing when the counters have been moved on.
  * A word carries the batch's number, no other batch's on this scratch, so that nothing has to be cleared, and only ever grows.
  * Words are read past the L2s, and up to 512 workgroups ask for the same few lines at once: eight copies, of which a tile
  * reads one, are faster than one (150,000 messages 7.2 and 8.1 us, 300,000 9.2 and 10.3).
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
 		before_tile += seed_sum[w];
 	}
 	if (missing) { /* the same in the whole workgroup */
-		const uint64_t word = look(&words[0]);
+		const uint64_t word = look(&published[0]);
 		const uint32_t seed = word >> 8 == number ? of_four_bits((uint32_t)word >> 4 & 15u) : seed_read;
 		uint32_t smalls = 0, stripes = 0;
 		for (uint32_t at = threadIdx.x; at < base; at += kOnceTile) {
@@ -642,7 +643,7 @@ __global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
 		if (missing) {
 			read = false;
 			for (uint32_t looks = 0; !read && looks < kSeedLooks; looks++) {
-				read = look(&words[0]) >> 8 >= number;
+				read = look(&published[0]) >> 8 >= number;
 				__builtin_amdgcn_s_sleep(8);
 			}
 		}
