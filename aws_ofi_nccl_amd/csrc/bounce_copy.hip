@@ -698,7 +698,7 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 	}
 	const uint32_t runs = (n + kXcds * kBounceRun - 1) / (kXcds * kBounceRun); /* whole rounds over the XCDs */
 	auto launch = [&](auto kernel) {
-		hipLaunchKernelGGL(kernel, dim3(runs * kXcds * (kBounceRun / kBounceWaves)), dim3(64 * kBounceWaves), 0,
+		ofi_amd::launch_kernel(kernel, dim3(runs * kXcds * (kBounceRun / kBounceWaves)), dim3(64 * kBounceWaves), 0,
 				   as_stream(stream), static_cast<const uint8_t *>(d_src), src_bytes, d_src_off, d_dst_off, d_len, n,
 				   static_cast<uint8_t *>(d_arena), arena_bytes, d_flush, err);
 	};
@@ -731,7 +731,7 @@ int ofi_amd_eager_copy_batch(const void *rx_base, const uint64_t *d_rx_off, cons
 	}
 	auto launch = [&](auto kernel, read_back_t back) {
 		const uint32_t round = kXcds * eager_run(back), waves = (uint32_t)eager_waves(back); /* whole rounds over the XCDs */
-		hipLaunchKernelGGL(kernel, dim3((n + round - 1) / round * (round / waves)), dim3(64 * waves), 0, as_stream(stream),
+		ofi_amd::launch_kernel(kernel, dim3((n + round - 1) / round * (round / waves)), dim3(64 * waves), 0, as_stream(stream),
 				   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base),
 				   d_dst_off, d_dst_len, n, d_copied, d_flush);
 	};
@@ -759,7 +759,7 @@ int ofi_amd_copy_table(const uint64_t *d_src_addr, const uint64_t *d_dst_addr, c
 	if (!d_src_addr || !d_dst_addr || !d_len || n > (1u << 30)) {
 		return -EINVAL;
 	}
-	hipLaunchKernelGGL(copy_table_kernel, dim3((n + kTableWaves - 1) / kTableWaves), dim3(64 * kTableWaves), 0,
+	ofi_amd::launch_kernel(copy_table_kernel, dim3((n + kTableWaves - 1) / kTableWaves), dim3(64 * kTableWaves), 0,
 			   as_stream(stream), d_src_addr, d_dst_addr, d_len, n);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
@@ -794,7 +794,7 @@ int ofi_amd_copy_table_pieces(const uint64_t *d_src_addr, const uint64_t *d_dst_
 		const piece_map_t map = copy_pieces_map((uint32_t)pieces_per_entry, here * pieces_per_entry);
 		const uint64_t round = (uint64_t)kXcds * map.run_blocks * kPieceWaves; /* whole rounds over the XCDs */
 		const uint64_t blocks = ((uint64_t)here * map.per + round - 1) / round * (kXcds * map.run_blocks);
-		hipLaunchKernelGGL(copy_table_pieces_kernel, dim3((uint32_t)blocks), dim3(64 * kPieceWaves), 0,
+		ofi_amd::launch_kernel(copy_table_pieces_kernel, dim3((uint32_t)blocks), dim3(64 * kPieceWaves), 0,
 				   as_stream(stream), d_src_addr + at, d_dst_addr + at, d_len + at, here, map, max_len, err);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
@@ -814,7 +814,7 @@ int ofi_amd_flush_read(const void *d_arena, const uint64_t *d_dst_off, uint32_t 
 	if (!d_arena || !d_dst_off || !d_flush) {
 		return -EINVAL;
 	}
-	hipLaunchKernelGGL(flush_read_kernel, dim3((n + 255u) / 256u), dim3(256), 0,
+	ofi_amd::launch_kernel(flush_read_kernel, dim3((n + 255u) / 256u), dim3(256), 0,
 			   as_stream(stream), static_cast<const uint8_t *>(d_arena), d_dst_off, n,
 			   d_flush);
 	OFI_AMD_HIP_TRY(hipGetLastError());
@@ -830,7 +830,7 @@ int ofi_amd_flush_buffer_fill(void *d_flush_buf, uint64_t sentinel, void *stream
 	if (!d_flush_buf || (reinterpret_cast<uintptr_t>(d_flush_buf) & 7u)) {
 		return -EINVAL;
 	}
-	hipLaunchKernelGGL(flush_fill_kernel, dim3(1), dim3(64), 0, as_stream(stream),
+	ofi_amd::launch_kernel(flush_fill_kernel, dim3(1), dim3(64), 0, as_stream(stream),
 			   static_cast<uint64_t *>(d_flush_buf), sentinel);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
@@ -846,7 +846,7 @@ int ofi_amd_flush_post(const void *d_flush_buf, void *slots_dev, uint32_t num_ra
 	    (reinterpret_cast<uintptr_t>(d_flush_buf) & 7u) || (reinterpret_cast<uintptr_t>(slots_dev) & 7u)) {
 		return -EINVAL;
 	}
-	hipLaunchKernelGGL(flush_post_kernel, dim3(1), dim3(64), 0, as_stream(stream),
+	ofi_amd::launch_kernel(flush_post_kernel, dim3(1), dim3(64), 0, as_stream(stream),
 			   static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
 			   num_rails);
 	OFI_AMD_HIP_TRY(hipGetLastError());

@@ -346,7 +346,7 @@ extern "C" int ofi_amd_gin_signal_apply(const ofi_amd_gin_signal_work_t *d_work,
 	}
 	const bool large = n > 32768u && (counters <= n / 64u || in_host_memory(d_work));
 	auto launch = [&](auto kernel, uint32_t threads, uint32_t items) {
-		hipLaunchKernelGGL(kernel, dim3((n - 1u) / (threads * items) + 1u), dim3(threads), 0, as_stream(stream),
+		ofi_amd::launch_kernel(kernel, dim3((n - 1u) / (threads * items) + 1u), dim3(threads), 0, as_stream(stream),
 				   d_work, n, r, large ? 0u : crowd_of(n), d_rejected);
 	};
 	if (n <= 4096u) {
@@ -382,7 +382,7 @@ extern "C" int ofi_amd_gin_signal_apply_post(const ofi_amd_gin_signal_work_t *d_
 	if (n != 0 && (!d_work || pack_regions(regions, n_regions, &r) != 0)) {
 		return -EINVAL;
 	}
-	hipLaunchKernelGGL(gin_signal_apply_post_kernel, dim3(1), dim3(kPostThreads), 0, as_stream(stream), d_work, n, r,
+	ofi_amd::launch_kernel(gin_signal_apply_post_kernel, dim3(1), dim3(kPostThreads), 0, as_stream(stream), d_work, n, r,
 			   n != 0 ? crowd_of(n) : 0u, d_rejected, static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
 			   num_rails);
 	OFI_AMD_HIP_TRY(hipGetLastError());

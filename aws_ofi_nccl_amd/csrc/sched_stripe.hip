@@ -726,13 +726,13 @@ int new_scratch(hipStream_t s, uint32_t **out)
 	OFI_AMD_HIP_TRY(hipMalloc((void **)&words, sizeof(uint32_t) * kScratchWords));
 	hipError_t e = hipSuccess;
 	if (!being_captured(s)) {
-		hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kClearBlocks), dim3(kClearThreads), 0, s, words);
+		ofi_amd::launch_kernel(stripe_scratch_kernel, dim3(kClearBlocks), dim3(kClearThreads), 0, s, words);
 		e = hipGetLastError();
 	} else {
 		hipStream_t own = nullptr;
 		e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
 		if (e == hipSuccess) {
-			hipLaunchKernelGGL(stripe_scratch_kernel, dim3(kClearBlocks), dim3(kClearThreads), 0, own,
+			ofi_amd::launch_kernel(stripe_scratch_kernel, dim3(kClearBlocks), dim3(kClearThreads), 0, own,
 					   words);
 			e = hipGetLastError();
 			const hipError_t waited = hipStreamSynchronize(own);
@@ -817,7 +817,7 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, large ? kDirectTileLarge : kDirectTile);
 		const uint32_t turn = tiles > 1 ? scratch.turn.fetch_add(1, std::memory_order_relaxed) : 0u;
 		auto launch = [&](auto kernel, uint32_t threads) {
-			hipLaunchKernelGGL(kernel, dim3(tiles), dim3(threads), 0, s, d_sizes, n, d_state, align, nullptr, nullptr,
+			ofi_amd::launch_kernel(kernel, dim3(tiles), dim3(threads), 0, s, d_sizes, n, d_state, align, nullptr, nullptr,
 					   words + turn % kArrivalWords, words + (turn + kArrivalWords / 2) % kArrivalWords, tiles,
 					   d_num_xfers, d_xfers, err);
 		};
@@ -831,23 +831,23 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 	if (total > kTwoLaunchBatch && total <= kOnceBatch && !being_captured(s)) {
 		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kOnceTile);
 		const uint64_t number = scratch.published.fetch_add(1, std::memory_order_relaxed) + 1;
-		hipLaunchKernelGGL(stripe_once_kernel, dim3(tiles), dim3(kOnceTile), 0, s, d_sizes, n, tiles, d_state, align,
+		ofi_amd::launch_kernel(stripe_once_kernel, dim3(tiles), dim3(kOnceTile), 0, s, d_sizes, n, tiles, d_state, align,
 				   reinterpret_cast<uint64_t *>(words + kOnceWords), number, looks, d_num_xfers, d_xfers, err);
 		return;
 	}
 	if (total <= kSmallBatch) {
 		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kTile);
-		hipLaunchKernelGGL(stripe_count_kernel, dim3(tiles), dim3(kCountThreads), 0, s, d_sizes, n, d_state, align, totals,
+		ofi_amd::launch_kernel(stripe_count_kernel, dim3(tiles), dim3(kCountThreads), 0, s, d_sizes, n, d_state, align, totals,
 				   seed0, err);
-		hipLaunchKernelGGL((stripe_emit_kernel<TILES, kTile>), dim3(tiles), dim3(kTile), 0, s, d_sizes, n, d_state, align,
+		ofi_amd::launch_kernel((stripe_emit_kernel<TILES, kTile>), dim3(tiles), dim3(kTile), 0, s, d_sizes, n, d_state, align,
 				   totals, nullptr, seed0, nullptr, tiles, d_num_xfers, d_xfers, err);
 		return;
 	}
 	for (uint64_t at = 0; at < total; at += kPart) {
 		const uint32_t n = (uint32_t)(total - at < kPart ? total - at : kPart), tiles = tiles_of(n, kBigTile);
-		hipLaunchKernelGGL(stripe_count_big_kernel, dim3(tiles_of(tiles, kBlockTiles)), dim3(64 * kBlockTiles), 0, s,
+		ofi_amd::launch_kernel(stripe_count_big_kernel, dim3(tiles_of(tiles, kBlockTiles)), dim3(64 * kBlockTiles), 0, s,
 				   d_sizes + at, n, d_state, align, totals, blocks, seed0, err);
-		hipLaunchKernelGGL((stripe_emit_kernel<BLOCKS, kBigTile>), dim3(tiles), dim3(kBigTile), 0, s, d_sizes + at, n,
+		ofi_amd::launch_kernel((stripe_emit_kernel<BLOCKS, kBigTile>), dim3(tiles), dim3(kBigTile), 0, s, d_sizes + at, n,
 				   d_state, align, totals, blocks, seed0, nullptr, tiles, d_num_xfers + at, d_xfers + 6 * at, err);
 	}
 }

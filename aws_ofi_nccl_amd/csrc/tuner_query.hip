@@ -375,7 +375,7 @@ extern "C" int ofi_amd_tuner_query(const ofi_amd_tuner_query_t *queries, uint32_
 	for (uint32_t at = 0; at < n; at += kMostPerLaunch) {
 		const uint32_t here = n - at < kMostPerLaunch ? n - at : kMostPerLaunch;
 		const uint32_t waves = here < kQueryWaves ? here : kQueryWaves;
-		hipLaunchKernelGGL(tuner_query_kernel, dim3((here + kQueryWaves - 1) / kQueryWaves), dim3(64 * waves), 0,
+		ofi_amd::launch_kernel(tuner_query_kernel, dim3((here + kQueryWaves - 1) / kQueryWaves), dim3(64 * waves), 0,
 				   g_stage.stream, tables.far_point, reinterpret_cast<const int4 *>(tables.poly),
 				   reinterpret_cast<const double4_t *>(tables.bbox), tables.edges,
 				   static_cast<const uint64_t *>(g_stage.dq) + (uint64_t)at * kQueryWords, here, call,
