@@ -368,6 +368,17 @@ __device__ __forceinline__ void copy_any(const uint8_t *__restrict__ s, uint8_t 
 	}
 }
 
+/* The first min(4, bytes) destination bytes, little-endian: a quad of lanes reads one byte
+ * each in one instruction (the destination has no alignment to read a word from),
+ * then the four are combined inside the quad. */
+__device__ __forceinline__ uint32_t quad_word(uint32_t byte, uint32_t at)
+{
+	uint32_t word = byte << (8u * at);
+	word |= __shfl_xor(word, 1, 64);
+	word |= __shfl_xor(word, 2, 64);
+	return word;
+}
+
 /*
  * The same copy for eager arrivals as they sit in rx buffers: an 8-byte header, then the
  * payload, which goes to a receive buffer at any alignment, truncated to that buffer's
@@ -425,15 +436,6 @@ __global__ __launch_bounds__(64 * eager_waves(BACK)) void eager_copy_kernel(
 		copy_any<BACK == BY_ITSELF>(s, d, bytes, lane);
 	}
 
-	/* The first min(4, bytes) destination bytes, little-endian: a quad of lanes reads one byte
-	 * each in one instruction (the destination has no alignment to read a word from),
-	 * then the four are combined inside the quad. */
-	auto word_of = [](uint32_t byte, uint32_t at) {
-		uint32_t word = byte << (8u * at);
-		word |= __shfl_xor(word, 1, 64);
-		word |= __shfl_xor(word, 2, 64);
-		return word;
-	};
 	if constexpr (BACK == TOGETHER) {
 		__shared__ uint8_t *back[WAVES];
 		__shared__ uint32_t count[WAVES];
@@ -448,7 +450,7 @@ __global__ __launch_bounds__(64 * eager_waves(BACK)) void eager_copy_kernel(
 			if (at < count[of]) {
 				byte = __builtin_nontemporal_load(back[of] + at);
 			}
-			const uint32_t word = word_of(byte, at);
+			const uint32_t word = quad_word(byte, at);
 			if (at == 0 && first + of < n) {
 				flush[first + of] = word;
 			}
@@ -459,10 +461,76 @@ __global__ __launch_bounds__(64 * eager_waves(BACK)) void eager_copy_kernel(
 		if (lane < min(bytes, 4u)) {
 			byte = d[lane];
 		}
-		const uint32_t word = word_of(byte, lane & 3u);
+		const uint32_t word = quad_word(byte, lane & 3u);
 		if (lane == 0) {
 			flush[buf] = word;
 		}
+	}
+}
+
+/*
+ * The same for rx buffers in host memory, which the link bounds.  It reads 8 KiB each for thousands of wavefronts at 46 GB/s and for
+ * some tens to hundreds at 54, so wavefronts with more than kTurnBytes take turns, one of a workgroup's four at a time, and the
+ * others, whose copies are a few trips and no more, do not.  Neighbours are dealt to the XCDs by fours here: by runs of 32 a few
+ * hundred buffers load them unevenly, and nothing that neighbours share in host memory stays in an L2.  (Eight to a workgroup:
+ * short buffers 0.8 us slower, their pages are looked up CU by CU.  256 wavefronts with a loop over buffers: long ones as
+ * fast, 600 of up to 500 B 8.2.)  By the kernel above / in fours without turns / with turns, us:
+ *     64 of up to 8 KiB   8.6 / 7.9 / 10.1        300 of up to 4000 B   16.1 / 15.0 / 14.5
+ *    150                 16.6 / 14.8 / 14.6      2048                   96.5 / 97 / 83
+ *    300                 30.7 / 27.6 / 26.3       300 of up to 500 B     5.1 / 5.2 / 5.2
+ *   1000                 96 / 96 / 80             600                    7.3 / 7.4 / 7.4
+ *   2048                183 / 183 / 162          2048                   18.0 / 18.1 / 18.1
+ * Asking the runtime where the buffers lie takes the host 0.1 us, so that small batches are left to the kernel above.
+ */
+constexpr uint32_t kHostWaves = 4, kTurnBytes = 1024, kHostBatch = 128;
+template <bool READ_BACK>
+__global__ __launch_bounds__(64 * kHostWaves) void eager_copy_host_kernel(
+	const uint8_t *__restrict__ rx_base, const uint64_t *__restrict__ rx_off,
+	const uint32_t *__restrict__ recv_len, uint8_t *__restrict__ dst_base,
+	const uint64_t *__restrict__ dst_off, const uint32_t *__restrict__ dst_len, uint32_t n,
+	uint32_t *__restrict__ copied, uint32_t *__restrict__ flush)
+{
+	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const uint32_t buf = blockIdx.x * kHostWaves + wave;
+	const uint32_t at = min(buf, n - 1u);
+	const uint64_t from = rx_off[at], to = dst_off[at];
+	const uint32_t received = recv_len[at], room = dst_len[at];
+	__asm__ volatile("" : : "s"(from), "s"(to), "s"(received), "s"(room), "s"(copied), "s"(flush)); /* as above */
+	const uint8_t *s = rx_base + from + 8u;
+	uint8_t *d = dst_base + to;
+	const uint32_t bytes = buf < n ? min(received, room) : 0u;
+	if (copied != nullptr && buf < n && lane == 0) {
+		copied[buf] = bytes;
+	}
+	auto read_back = [&] {
+		if (READ_BACK && buf < n) {
+			__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+			uint32_t byte = 0;
+			if (lane < min(bytes, 4u)) {
+				byte = d[lane];
+			}
+			const uint32_t word = quad_word(byte, lane & 3u);
+			if (lane == 0) {
+				flush[buf] = word;
+			}
+		}
+	};
+	/* kHostWaves - 1 barriers in every wavefront, in front of the copy as many as its turn */
+	const bool waits = bytes > kTurnBytes;
+	if (waits) {
+		for (uint32_t t = 0; t < wave; t++) {
+			__builtin_amdgcn_s_barrier();
+		}
+	}
+	copy_any<READ_BACK>(s, d, bytes, lane); /* its loads have come when its stores leave */
+	if (!waits) {
+		read_back();
+	}
+	for (uint32_t t = waits ? wave + 1u : 1u; t < kHostWaves; t++) {
+		__builtin_amdgcn_s_barrier();
+	}
+	if (waits) {
+		read_back();
 	}
 }
 
@@ -503,7 +571,7 @@ __global__ __launch_bounds__(64 * kTableWaves) void copy_table_kernel(const uint
  *   of 8 B..512 KiB 200 -> 183 us.
  * - The table may lie in host memory, a link's round trip away.  Its three words are asked for together,
  *   not the addresses once the length is known (7 entries of 4-8 KiB: 5.6 -> 4.1 us).
- * All told, tables in host memory, other buffers at every launch: 2048 entries of 8 B..1 MiB 78 -> 76 us, with whole rows between the ends 72 (5.3 of
+ * All told, tables in host memory, other buffers at every launch: 2048 entries of 8 B..1 MiB 78 -> 72 us (5.2 of
  * the 5.4 TB/s read + written of one plain copy of those bytes), 16,384 of 8 B..64 KiB 69 -> 48 us.
  */
 constexpr uint32_t kPieceBytes = kRows * 1024u;
@@ -735,7 +803,14 @@ int ofi_amd_eager_copy_batch(const void *rx_base, const uint64_t *d_rx_off, cons
 				   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base),
 				   d_dst_off, d_dst_len, n, d_copied, d_flush);
 	};
-	if (!d_flush) {
+	if (n >= kHostBatch && in_host_memory(rx_base)) {
+		auto launch_host = [&](auto kernel) {
+			ofi_amd::launch_kernel(kernel, dim3((n + kHostWaves - 1) / kHostWaves), dim3(64 * kHostWaves), 0, as_stream(stream),
+					   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base), d_dst_off,
+					   d_dst_len, n, d_copied, d_flush);
+		};
+		d_flush ? launch_host(eager_copy_host_kernel<true>) : launch_host(eager_copy_host_kernel<false>);
+	} else if (!d_flush) {
 		launch(eager_copy_kernel<NO_READ_BACK>, NO_READ_BACK);
 	} else if (n <= kKeepEager) {
 		launch(eager_copy_kernel<BY_ITSELF>, BY_ITSELF);

@@ -58,6 +58,17 @@ int sched_noalloc_setup();
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
+/* Pinned memory of the host's, as the runtime knows it */
+inline bool in_host_memory(const void *p)
+{
+	hipPointerAttribute_t attr;
+	if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+		(void)hipGetLastError();
+		return false;
+	}
+	return attr.type == hipMemoryTypeHost;
+}
+
 template <typename T> struct as_declared { /* an argument is converted to the kernel's parameter, not deduced from */
 	using type = T;
 };

@@ -300,16 +300,6 @@ static int pack_regions(const ofi_amd_gin_signal_region_t *regions, uint32_t n_r
 	return 0;
 }
 
-static bool in_host_memory(const void *p)
-{
-	hipPointerAttribute_t attr;
-	if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
-		(void)hipGetLastError();
-		return false;
-	}
-	return attr.type == hipMemoryTypeHost;
-}
-
 extern "C" int ofi_amd_gin_signal_apply(const ofi_amd_gin_signal_work_t *d_work, uint32_t n,
 					const ofi_amd_gin_signal_region_t *regions, uint32_t n_regions,
 					uint32_t *d_rejected, void *stream)
