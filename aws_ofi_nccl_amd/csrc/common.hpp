@@ -74,7 +74,8 @@ template <typename T> struct as_declared { /* an argument is converted to the ke
 };
 /* What <<<>>> does, without its detour through a stub that pushes the launch's shape and pops it again, which is 0.15 to 0.35 us
  * of the 2.5 to 3.4 that a launch with ten arguments takes the host (64 eager arrivals in a row 4.11 -> 3.93 us, 1000 striping
- * messages 4.05 -> 3.88, 300 bounce buffers 4.20 -> 3.96, 4 one-sided writes 3.63 -> 3.47).  The error is the runtime's last one, as with <<<>>>. */
+ * messages 4.05 -> 3.88, 300 bounce buffers 4.20 -> 3.96, 4 one-sided writes 3.63 -> 3.47).  The error is the runtime's last
+ * one, as with <<<>>>. */
 template <typename... P>
 inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream,
 			  typename as_declared<P>::type... args)
