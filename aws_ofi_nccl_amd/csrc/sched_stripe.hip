@@ -35,10 +35,12 @@
 
 #include "common.hpp"
 #include "ofi_amd_hotpath.h"
+#include "sched_once.hpp"
 
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+namespace once = ofi_amd_once;
 
 /* One-launch form: tiles of 256 messages up to two of them, of 512 beyond, whose twice as many threads share the look
  * at everything before the tile (in us, tiles of 256 / 512 / 1024: 3000 messages 4.7 / 4.3 / 5.1, 6144 5.9 / 4.9 / 5.4).
@@ -504,12 +506,12 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
 /*
  * The one-launch form for batches whose sizes are too many for every tile to look through: a tile counts its own messages,
  * publishes the total in a word and adds up the words of the tiles before it, one a thread.  So it waits for other
- * workgroups, all of which have been handed out before it, and every wait has an end:
+ * workgroups.  They have been handed out before it as a rule, but on eight XCDs, of which one may be busy with another stream's
+ * kernel; every wait has an end, and none is needed for the result (sched_once.hpp has the words and the rules):
  * - After `looks` looks a tile that still misses words adds up the messages before it by itself, from their sizes.
- * - The tile that moves the counters on may only do so when they have been read.  Tile 0 reads them before it publishes, and
- *   says what they were in its word: a tile on its own reads the counters first and that word second, and takes the
- *   word's if it is there.  The last tile, on its own, waits for that word with the counters; nobody waits for it.  Both look
- *   at the first copy: of another one the word could still be missing when the counters have been moved on.
+ * - The counters are moved on only when every tile has read them or finds the seed in tile 0's word.  A last tile that
+ *   has given up leaves that to tile 0 if tile 0 has not published yet.  Both it and the tiles on their own go by the first
+ *   copy of the word: another one may be there before it.
  * A word carries the batch's number, no other batch's on this scratch, so that nothing has to be cleared, and only ever grows.
  * Words are read past the L2s, and up to 512 workgroups ask for the same few lines at once: eight copies, of which a tile
  * reads one, are faster than one (150,000 messages 7.2 and 8.1 us, 300,000 9.2 and 10.3).
@@ -524,26 +526,20 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
  */
 constexpr uint32_t kOnceTile = 512, kOnceCopies = 8;
 constexpr uint64_t kOnceBatch = (uint64_t)kOnceTile * kOnceTile;
+static_assert(kTwoLaunchBatch >= kOnceTile, "tile 0 and the last one are two");
 constexpr uint32_t kOnceLooks = 2048; /* some 2 ms */
-constexpr uint32_t kSeedLooks = 1u << 22;
 constexpr uint32_t kMissing = ~0u;
 __device__ __forceinline__ uint64_t look(const uint64_t *word)
 {
 	return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* a pair of residues, as the packed sums have them, in four bits, and back */
-__device__ __forceinline__ uint32_t four_bits(uint32_t residues)
+__device__ __forceinline__ uint64_t raise(uint64_t *word, uint64_t to)
 {
-	return (residues >> 16) << 2 | (residues & 3u);
-}
-__device__ __forceinline__ uint32_t of_four_bits(uint32_t bits)
-{
-	return (bits >> 2 & 3u) << 16 | (bits & 3u);
+	return __hip_atomic_fetch_max(word, to, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* published: [kOnceCopies][kOnceTile] words, each the batch's number << 8 | tile 0's: the seed << 4 | residues of the tile's
- * total */
+/* published: [kOnceCopies][kOnceTile] words, and behind them the one in which tile 0 and the last tile meet */
 __global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
 	const uint64_t *__restrict__ sizes, uint32_t n, uint32_t num_tiles, ofi_amd_sched_state_t *__restrict__ state, uint64_t align,
 	uint64_t *published, uint64_t number, uint32_t max_looks, uint32_t *__restrict__ num_xfers, u32x4 *__restrict__ xfers,
@@ -582,11 +578,10 @@ __global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
 		off += (w < wave) ? ws : 0;
 		tot += ws;
 	}
+	uint64_t before = 0;
 	if (threadIdx.x < kOnceCopies) {
-		const uint32_t seed_bits = tile == 0 ? four_bits(seed_read) << 4 : 0u;
-		__hip_atomic_fetch_max(&published[threadIdx.x * kOnceTile + tile],
-				       number << 8 | seed_bits | four_bits(residues(tot, R)), __ATOMIC_RELAXED,
-				       __HIP_MEMORY_SCOPE_AGENT);
+		before = raise(&published[threadIdx.x * kOnceTile + tile],
+			       once::published_word(number, tile == 0 ? seed_read : 0u, residues(tot, R)));
 	}
 
 	const uint64_t *const words = published + tile % kOnceCopies * kOnceTile;
@@ -594,9 +589,9 @@ __global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
 	if (wave * 64u < tile) {
 		acc = kMissing;
 		for (uint32_t looks = 0; looks < max_looks; looks++) {
-			const uint64_t word = threadIdx.x < tile ? look(&words[threadIdx.x]) : number << 8;
-			if (__ballot(word >> 8 != number) == 0) {
-				acc = wave_sum_of(of_four_bits((uint32_t)word & 15u) + of_four_bits((uint32_t)word >> 4 & 15u));
+			const uint64_t word = threadIdx.x < tile ? look(&words[threadIdx.x]) : once::published_word(number, 0, 0);
+			if (__ballot(!once::is_published(word, number)) == 0) {
+				acc = wave_sum_of(once::seed_and_total(word));
 				break;
 			}
 			__builtin_amdgcn_s_sleep(1);
@@ -614,8 +609,7 @@ __global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
 		before_tile += seed_sum[w];
 	}
 	if (missing) { /* the same in the whole workgroup */
-		const uint64_t word = look(&published[0]);
-		const uint32_t seed = word >> 8 == number ? of_four_bits((uint32_t)word >> 4 & 15u) : seed_read;
+		const uint32_t seed = once::seed_by_itself(look(&published[0]), number, seed_read);
 		uint32_t smalls = 0, stripes = 0;
 		for (uint32_t at = threadIdx.x; at < base; at += kOnceTile) {
 			uint32_t unused;
@@ -638,21 +632,24 @@ __global__ __launch_bounds__(kOnceTile) void stripe_once_kernel(
 	const uint32_t carry_small = (before_tile >> 16) % R, carry_big = (before_tile & 0xffffu) % R;
 	write_rows<true, kOnceTile>(size, live, c, k, off + inc - c, carry_small, carry_big, p, n, base, rows, num_xfers, xfers);
 
-	if (tile == num_tiles - 1 && threadIdx.x == 0) {
-		bool read = true;
-		if (missing) {
-			read = false;
-			for (uint32_t looks = 0; !read && looks < kSeedLooks; looks++) {
-				read = look(&published[0]) >> 8 >= number;
-				__builtin_amdgcn_s_sleep(8);
-			}
-		}
-		if (read) {
-			state->rr_small_counter = mod_rails(carry_small + (tot >> 16), p);
-			state->rr_counter = mod_rails(carry_big + (tot & 0xffffu), p);
-		} else {
-			atomicOr(err, ofi_amd::ASYNC_ERR_SCHED_STATE); /* somebody has changed the state under the batch */
-		}
+	if (threadIdx.x != 0) {
+		return;
+	}
+	uint64_t *const meet = &published[kOnceCopies * kOnceTile];
+	bool stores = false;
+	uint32_t counters = 0;
+	if (tile == 0) {
+		__asm__ volatile("" : : "v"(before) : "memory"); /* it has been answered: the word is there before the one below */
+		const uint64_t found = raise(meet, once::first_tile_word(number));
+		stores = once::first_tile_stores(found, number);
+		counters = once::counters_left(found);
+	} else if (tile == num_tiles - 1) {
+		counters = mod_rails(carry_small + (tot >> 16), p) << 16 | mod_rails(carry_big + (tot & 0xffffu), p);
+		stores = !missing || once::last_tile_stores(raise(meet, once::last_tile_word(number, counters)), number);
+	}
+	if (stores) {
+		state->rr_small_counter = counters >> 16;
+		state->rr_counter = counters & 0xffffu;
 	}
 }
 
@@ -671,11 +668,11 @@ constexpr uint32_t kArrivalWords = 1024;
 constexpr uint32_t kSeedWord = kArrivalWords, kBlockWords = kSeedWord + 32;
 constexpr uint32_t kTileWords = kBlockWords + kMaxBlocks;
 constexpr uint32_t kOnceWords = kTileWords + kMaxTiles; /* words of 64 bits */
-constexpr uint32_t kScratchWords = kOnceWords + 2 * kOnceCopies * kOnceTile;
+constexpr uint32_t kMeetWord = kOnceWords + 2 * kOnceCopies * kOnceTile;
+constexpr uint32_t kScratchWords = kMeetWord + 32;
 constexpr uint32_t kClearThreads = 256;
 static_assert((kArrivalWords & (kArrivalWords - 1)) == 0 && kBlockWords % 32 == 0 && kOnceWords % 32 == 0,
 	      "a ring; block totals and published words on a line");
-static_assert(kArrivalWords % kClearThreads == 0 && kOnceCopies * kOnceTile % kClearThreads == 0, "cleared by whole workgroups");
 struct scratch_t {
 	uint32_t *words = nullptr;
 	std::atomic<uint32_t> turn{ 0 };    /* of the next batch that counts arrivals */
@@ -698,12 +695,15 @@ int key_of_stream(void *stream, stream_key_t *key)
 std::mutex g_ws_lock;
 std::map<stream_key_t, scratch_t> g_ws_by_stream;
 
-/* The arrival words and the published ones; the others are written before they are read */
-constexpr uint32_t kClearBlocks = (kArrivalWords + 2 * kOnceCopies * kOnceTile) / kClearThreads;
+/* The arrival words, the published ones and the one behind them; the others are written before they are read */
+constexpr uint32_t kClearWords = kArrivalWords + kScratchWords - kOnceWords;
+constexpr uint32_t kClearBlocks = (kClearWords + kClearThreads - 1) / kClearThreads;
 __global__ __launch_bounds__(kClearThreads) void stripe_scratch_kernel(uint32_t *__restrict__ words)
 {
 	const uint32_t at = blockIdx.x * kClearThreads + threadIdx.x;
-	words[at < kArrivalWords ? at : kOnceWords + (at - kArrivalWords)] = 0;
+	if (at < kClearWords) {
+		words[at < kArrivalWords ? at : kOnceWords + (at - kArrivalWords)] = 0;
+	}
 }
 
 /* also where the runtime cannot say: the null stream while another one is captured */
