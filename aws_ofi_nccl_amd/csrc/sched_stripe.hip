@@ -13,7 +13,7 @@
  * Four forms, by the size of the batch:
  *   up to kDirectBatch messages, one launch: every workgroup adds up the messages before
  *   its tile by itself, from their sizes (at most 78 KiB out of the L2);
- *   from kTwoLaunchBatch up to kOnceBatch, one launch whose workgroups publish the totals of their tiles and add up those
+ *   up to kOnceBatch, one launch whose workgroups publish the totals of their tiles and add up those
  *   of the tiles before them (stripe_once_kernel);
  *   up to kSmallBatch, two launches: stripe_count_kernel leaves each tile's totals of
  *   (small count, stripe count), reduced mod R (only the residues matter), and
@@ -44,12 +44,12 @@ namespace once = ofi_amd_once;
 
 /* One-launch form: tiles of 256 messages up to two of them, of 512 beyond, whose twice as many threads share the look
  * at everything before the tile (in us, tiles of 256 / 512 / 1024: 3000 messages 4.7 / 4.3 / 5.1, 6144 5.9 / 4.9 / 5.4).
- * That look grows until it costs what the second launch does: 7000 messages 5.2 against 7.6 us in two launches, 9900 5.7
- * and 7.7, 12,000 6.2 and 7.6.  (The tests of the launches hold 10,000 to two.) */
+ * The line was drawn where that look costs nearly what a second launch does: 7000 messages 5.2 against 7.6 us in two launches, 9900
+ * 5.7 and 7.7, 12,000 6.2 and 7.6.  The form with published totals, 4.4 us at 9985, is the faster one from some thousands
+ * on. */
 constexpr uint32_t kDirectTile = 256, kDirectTileLarge = 512;
 constexpr uint64_t kDirectBatch = 9984;
 static_assert(4 * kDirectBatch < 65536 - 8, "packed sums of a whole batch: up to 4 stripes a message, and the seed");
-constexpr uint64_t kTwoLaunchBatch = 10240; /* from kDirectBatch up to here two launches, as the tests hold 10,000 to */
 /* Two-launch form: tiles of 512 messages, counted by 256 threads and written by 512 (21.5 us per 1,000,000
  * messages, 39.0 per 2,000,000; 256 threads twice 21.6 and 40.2, 128 threads four times 23.9 and 43.5). */
 constexpr uint32_t kTile = 512;
@@ -516,7 +516,8 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
  * Words are read past the L2s, and up to 512 workgroups ask for the same few lines at once: eight copies, of which a tile
  * reads one, are faster than one (150,000 messages 7.2 and 8.1 us, 300,000 9.2 and 10.3).
  * Us in two launches / in this one, in a row (two launches of this length are also more than some hosts queue in that time):
- *    10,300 messages   5.9-7.4 / 5.2
+ *     9985 messages    6.3-6.6 / 4.4
+ *    10,300            5.9-7.4 / 4.5
  *    30,000            6.0-7.2 / 5.3
  *   100,000            6.7-7.2 / 6.5
  *   150,000            7.9     / 7.4
@@ -526,7 +527,7 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
  */
 constexpr uint32_t kOnceTile = 512, kOnceCopies = 8;
 constexpr uint64_t kOnceBatch = (uint64_t)kOnceTile * kOnceTile;
-static_assert(kTwoLaunchBatch >= kOnceTile, "tile 0 and the last one are two");
+static_assert(kDirectBatch >= kOnceTile, "tile 0 and the last one are two");
 constexpr uint32_t kOnceLooks = 2048; /* some 2 ms */
 constexpr uint32_t kMissing = ~0u;
 __device__ __forceinline__ uint64_t look(const uint64_t *word)
@@ -828,7 +829,7 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 		}
 		return;
 	}
-	if (total > kTwoLaunchBatch && total <= kOnceBatch && !being_captured(s)) {
+	if (total > kDirectBatch && total <= kOnceBatch && !being_captured(s)) {
 		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kOnceTile);
 		const uint64_t number = scratch.published.fetch_add(1, std::memory_order_relaxed) + 1;
 		ofi_amd::launch_kernel(stripe_once_kernel, dim3(tiles), dim3(kOnceTile), 0, s, d_sizes, n, tiles, d_state, align,

@@ -143,7 +143,7 @@ int ofi_amd_sched_stream_release(void *stream);
  * an overlap spoils is the batches that took part in it, not later ones.  A call writes every word of the
  * array before it reads it, but for 1024 words that small batches count in -- those are zero between
  * calls, as they are when the code is loaded, and calls clear them again by turns -- and the words in which the tiles
- * of batches of 10,241 to 262,144 messages publish their totals, which carry the number of their batch.
+ * of batches of 9,985 to 262,144 messages publish their totals, which carry the number of their batch.
  */
 int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
 				uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,

@@ -197,6 +197,12 @@ int striping()
 			small(1000);
 		}
 		CHECK(seen.spoiled == 0);
+		/* one message more has totals to publish, in one launch too */
+		int once = 0;
+		on_launch = [&](const launch_t &l) { once += l.kernel.find("stripe_once_kernel") != std::string::npos ? 1 : 100; };
+		small(9985);
+		CHECK(once == 1);
+		on_launch = std::ref(seen);
 		/* a captured batch comes back to the scratch it was captured with: it counts in no word */
 		const size_t before = seen.words.size();
 		capture_status = hipStreamCaptureStatusActive;
@@ -233,7 +239,7 @@ int streams()
 				totals = l.arg<uint32_t *>(4);
 			}
 		};
-		CHECK(ofi_amd_sched_batch(&state, sizes, 10000, 128, num, xfers, stream) == 0 && totals);
+		CHECK(ofi_amd_sched_batch(&state, sizes, 300000, 128, num, xfers, stream) == 0 && totals);
 		return totals;
 	};
 	auto in_another_thread = [&](void *stream) {

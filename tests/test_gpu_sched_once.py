@@ -56,7 +56,7 @@ class Chain:
 
 # the smallest batches, with whole and ragged last tiles, both sides of a wavefront's share of the words, the largest batch
 # and the one after it
-@pytest.mark.parametrize("n", [10240, 10241, 20 * TILE + 513, 64 * TILE, 64 * TILE + 1, 65 * TILE + 1, TILE * TILE - 1, TILE * TILE,
+@pytest.mark.parametrize("n", [9984, 9985, 10240, 10241, 20 * TILE + 513, 64 * TILE, 64 * TILE + 1, 65 * TILE + 1, TILE * TILE - 1, TILE * TILE,
                                TILE * TILE + 1])
 @pytest.mark.parametrize("rails,max_small", [(4, 64), (3, 5000), (1, 0)])
 def test_batches_of_published_totals(lib, oracle, gpu, n, rails, max_small):
@@ -71,7 +71,7 @@ def test_batches_of_published_totals(lib, oracle, gpu, n, rails, max_small):
 
 
 @pytest.mark.parametrize("looks", [0, 1])
-@pytest.mark.parametrize("n", [10241, 65 * TILE + 1, TILE * TILE])
+@pytest.mark.parametrize("n", [9985, 10241, 65 * TILE + 1, TILE * TILE])
 @pytest.mark.parametrize("rails,max_small", [(4, 64), (3, 5000)])
 def test_tiles_that_do_not_wait_add_up_by_themselves(lib, oracle, gpu, n, rails, max_small, looks):
     """What a tile does that has looked for the others' words in vain, for all of them and for those that one look finds
