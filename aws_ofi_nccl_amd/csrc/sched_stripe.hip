@@ -671,6 +671,7 @@ constexpr uint32_t kTileWords = kBlockWords + kMaxBlocks;
 constexpr uint32_t kOnceWords = kTileWords + kMaxTiles; /* words of 64 bits */
 constexpr uint32_t kMeetWord = kOnceWords + 2 * kOnceCopies * kOnceTile;
 constexpr uint32_t kScratchWords = kMeetWord + 32;
+static_assert(kScratchWords == 29760, "116 KiB, as the header says; the graph tests leave memory of this size dirty");
 constexpr uint32_t kClearThreads = 256;
 static_assert((kArrivalWords & (kArrivalWords - 1)) == 0 && kBlockWords % 32 == 0 && kOnceWords % 32 == 0,
 	      "a ring; block totals and published words on a line");

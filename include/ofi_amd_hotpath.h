@@ -121,7 +121,7 @@ typedef struct {
 int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
 			uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
 			void *stream);
-/* ofi_amd_sched_batch keeps some 150 KiB of device scratch per stream it has been called with
+/* ofi_amd_sched_batch keeps 116 KiB of device scratch per stream it has been called with
  * (the reference's scheduler keeps a freelist per instance, src/nccl_ofi_scheduler.cpp:135-190).
  * The null stream has scratch on each GPU, hipStreamPerThread on each GPU and for each thread.
  * A caller that destroys a stream, or a thread that ends after calls on hipStreamPerThread, hands
@@ -135,7 +135,7 @@ int ofi_amd_sched_stream_release(void *stream);
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
  * reference.  Same arguments, same results and the same kernels; the totals of tiles and
  * of blocks of tiles that ofi_amd_sched_batch keeps in a per-stream allocation live here in a fixed array
- * inside the library's device code (about 150 KiB per GPU, held until the process ends), so the call
+ * inside the library's device code (116 KiB per GPU, held until the process ends), so the call
  * allocates and frees nothing.  n <= 2^26 messages per call, -E2BIG beyond.  Call
  * ofi_amd_gpu_init() once beforehand (it allocates the asynchronous error word and looks up
  * the array's address on every GPU); -ENXIO otherwise.  All calls on one GPU share that GPU's
