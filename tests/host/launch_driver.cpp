@@ -214,6 +214,20 @@ int striping()
 		small(1000);
 		capture_answer = hipSuccess;
 		CHECK(seen.words.size() == before && seen.two_launch == 4);
+		/* nor does it take a number from the batches that publish totals */
+		std::vector<uint64_t> numbers;
+		on_launch = [&](const launch_t &l) {
+			if (l.kernel.find("stripe_once_kernel") != std::string::npos) {
+				numbers.push_back(l.arg<uint64_t>(6));
+			}
+		};
+		small(30001);
+		capture_status = hipStreamCaptureStatusActive;
+		small(30001);
+		capture_status = hipStreamCaptureStatusNone;
+		small(262144);
+		CHECK(numbers.size() == 2 && numbers[1] == numbers[0] + 1);
+		on_launch = std::ref(seen);
 		small(256); /* one tile */
 		CHECK(seen.words.size() == before && seen.two_launch == 4);
 	}
@@ -264,6 +278,22 @@ int streams()
 		CHECK(ofi_amd_sched_stream_release(per_thread) == 0);
 	}).join();
 	CHECK(scratch_on(per_thread) == mine && ofi_amd_sched_stream_release(per_thread) == 0);
+	/* New scratch is cleared as far as a batch reads what it has not written: 1024 words that batches count in, eight copies
+	 * of 512 published words of 64 bits and the one behind them, whichever batch and stream state come first */
+	for (const hipStreamCaptureStatus status : { hipStreamCaptureStatusNone, hipStreamCaptureStatusActive }) {
+		uint64_t cleared = 0, launches = 0;
+		on_launch = [&](const launch_t &l) {
+			if (l.kernel.find("stripe_scratch_kernel") != std::string::npos) {
+				CHECK(launches == 0);
+				cleared += (uint64_t)l.grid.x * l.block.x;
+			}
+			launches++;
+		};
+		capture_status = status;
+		CHECK(ofi_amd_sched_batch(&state, sizes, 30001, 128, num, xfers, reinterpret_cast<void *>(0x48)) == 0);
+		capture_status = hipStreamCaptureStatusNone;
+		CHECK(cleared >= 1024 + 2 * (8 * 512 + 1) && ofi_amd_sched_stream_release(reinterpret_cast<void *>(0x48)) == 0);
+	}
 	return 0;
 }
 

@@ -14,6 +14,7 @@ import aws_ofi_nccl_amd as m
 from aws_ofi_nccl_amd import synthetic
 
 pytestmark = pytest.mark.gpu
+SCRATCH_WORDS = 29_760  # of a stream's striping scratch, kScratchWords in csrc/sched_stripe.hip
 
 
 def test_graph_of_hot_path_launches_replays_exactly(lib, oracle, gpu):
@@ -143,20 +144,20 @@ def test_graph_of_hot_path_launches_replays_exactly(lib, oracle, gpu):
     assert _gpu.fetch_async_errors(lib) == 0
 
 
-def test_batch_first_called_while_its_stream_is_captured(lib, oracle, gpu):
+@pytest.mark.parametrize("n", [1000, 30_001])
+def test_batch_first_called_while_its_stream_is_captured(lib, oracle, gpu, n):
     """The scratch of a stream is made by the call that the stream is being captured in (a capture mode that lets a
     call allocate): batches called before the first replay, the replay and batches after it all match the oracle,
     whatever the memory held.  1000 messages are one launch when called, whose workgroups count themselves in the
-    scratch, and two when captured."""
+    scratch, 30,001 one whose workgroups publish totals there, and both two when captured."""
     s = torch.cuda.Stream()
     sp = ctypes.c_void_p(s.cuda_stream)
     assert lib.ofi_amd_sched_stream_release(sp) == 0
     # memory of the scratch's size, left dirty for the allocator to hand out again
-    dirty = [torch.full((20608,), -1, dtype=torch.int32, device="cuda") for _ in range(8)]
+    dirty = [torch.full((SCRATCH_WORDS,), -1, dtype=torch.int32, device="cuda") for _ in range(8)]
     torch.cuda.synchronize()
     del dirty
     torch.cuda.empty_cache()
-    n = 1000
     sizes = synthetic.stripe_sizes(6, n)
     st = m.SchedState(2, 1, 64, 131072, 4, 0)
     d_state = _gpu.to_dev(np.frombuffer(bytes(st), dtype=np.uint8).copy())
