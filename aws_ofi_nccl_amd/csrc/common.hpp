@@ -13,6 +13,13 @@
 
 #include <hip/hip_runtime.h>
 
+#include "ofi_amd_hotpath.h"
+
+/* Not part of the library's interface, for its tests: ofi_amd_sched_batch with fewer looks (at most as many as it takes) that a
+ * tile takes at the words of the others.  After none, every tile adds up what is before it by itself. */
+extern "C" int ofi_amd_sched_batch_looks(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n, uint64_t align,
+					 uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers, void *stream, uint32_t looks);
+
 namespace ofi_amd {
 
 inline int errno_of(hipError_t e)

@@ -28,6 +28,7 @@
  *
  * HBM traffic per message: 8 B read twice (once in the one-launch form) + 4 B + 96 B written.
  */
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -854,6 +855,54 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 	}
 }
 
+/* A batch on a stream's scratch; looks: at most so many does a tile take at the words of the others. */
+int batch_on_stream(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n, uint64_t align, uint32_t *d_num_xfers,
+		    ofi_amd_xfer_info_t *d_xfers, void *stream, uint32_t looks)
+{
+	int rc = ofi_amd::require_device();
+	if (rc != 0) {
+		return rc;
+	}
+	if (!d_state || align == 0 || n > kMaxBatch) {
+		return -EINVAL;
+	}
+	if (n == 0) {
+		return 0;
+	}
+	if (!d_sizes || !d_num_xfers || !d_xfers) {
+		return -EINVAL;
+	}
+
+	uint32_t *err = ofi_amd::async_error_word();
+	if (!err) {
+		return -ENOMEM;
+	}
+
+	hipStream_t s = ofi_amd::as_stream(stream);
+	stream_key_t key;
+	rc = key_of_stream(stream, &key);
+	if (rc != 0) {
+		return rc;
+	}
+	try {
+		/* held until the launches are queued: two threads submitting to one stream share its
+		 * scratch, and their count/emit pairs must not interleave */
+		std::lock_guard<std::mutex> g(g_ws_lock);
+		scratch_t &scratch = g_ws_by_stream[key];
+		if (!scratch.words) {
+			rc = new_scratch(s, &scratch.words);
+			if (rc != 0) {
+				return rc;
+			}
+		}
+		launch_batch(s, d_sizes, n, d_state, align, scratch, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err, looks);
+	} catch (...) {
+		return -ENOMEM;
+	}
+	OFI_AMD_HIP_TRY(hipGetLastError());
+	return 0;
+}
+
 } // namespace
 
 namespace ofi_amd {
@@ -881,61 +930,18 @@ using namespace ofi_amd;
 
 extern "C" {
 
-/* ofi_amd_sched_batch with the number of looks that a tile takes at the words of the others, for the tests: after none, every
- * tile adds up what is before it by itself. */
-int ofi_amd_sched_batch_looks(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
-			      uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
-			      void *stream, uint32_t looks)
-{
-	int rc = require_device();
-	if (rc != 0) {
-		return rc;
-	}
-	if (!d_state || align == 0 || n > kMaxBatch) {
-		return -EINVAL;
-	}
-	if (n == 0) {
-		return 0;
-	}
-	if (!d_sizes || !d_num_xfers || !d_xfers) {
-		return -EINVAL;
-	}
-
-	uint32_t *err = async_error_word();
-	if (!err) {
-		return -ENOMEM;
-	}
-
-	hipStream_t s = as_stream(stream);
-	stream_key_t key;
-	rc = key_of_stream(stream, &key);
-	if (rc != 0) {
-		return rc;
-	}
-	try {
-		/* held until the launches are queued: two threads submitting to one stream share its
-		 * scratch, and their count/emit pairs must not interleave */
-		std::lock_guard<std::mutex> g(g_ws_lock);
-		scratch_t &scratch = g_ws_by_stream[key];
-		if (!scratch.words) {
-			rc = new_scratch(s, &scratch.words);
-			if (rc != 0) {
-				return rc;
-			}
-		}
-		launch_batch(s, d_sizes, n, d_state, align, scratch, d_num_xfers, reinterpret_cast<u32x4 *>(d_xfers), err, looks);
-	} catch (...) {
-		return -ENOMEM;
-	}
-	OFI_AMD_HIP_TRY(hipGetLastError());
-	return 0;
-}
-
 int ofi_amd_sched_batch(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
 			uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
 			void *stream)
 {
-	return ofi_amd_sched_batch_looks(d_state, d_sizes, n, align, d_num_xfers, d_xfers, stream, kOnceLooks);
+	return batch_on_stream(d_state, d_sizes, n, align, d_num_xfers, d_xfers, stream, kOnceLooks);
+}
+
+int ofi_amd_sched_batch_looks(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
+			      uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
+			      void *stream, uint32_t looks)
+{
+	return batch_on_stream(d_state, d_sizes, n, align, d_num_xfers, d_xfers, stream, std::min(looks, kOnceLooks));
 }
 
 int ofi_amd_sched_stream_release(void *stream)

@@ -20,6 +20,10 @@
 
 #include "ofi_amd_hotpath.h"
 
+/* the tests' own way into the library (csrc/common.hpp) */
+extern "C" int ofi_amd_sched_batch_looks(ofi_amd_sched_state_t *, const uint64_t *, uint64_t, uint64_t, uint32_t *,
+					 ofi_amd_xfer_info_t *, void *, uint32_t looks);
+
 #define CHECK(cond)                                                                  \
 	do {                                                                         \
 		if (!(cond)) {                                                       \
@@ -231,6 +235,18 @@ int striping()
 		small(256); /* one tile */
 		CHECK(seen.words.size() == before && seen.two_launch == 4);
 	}
+	/* no tile looks for longer than those of an ordinary batch, however it is called */
+	std::vector<uint32_t> looks;
+	on_launch = [&](const launch_t &l) {
+		if (l.kernel.find("stripe_once_kernel") != std::string::npos) {
+			looks.push_back(l.arg<uint32_t>(7));
+		}
+	};
+	CHECK(ofi_amd_sched_batch(&state, sizes, 30001, 128, num, xfers, stream) == 0);
+	for (const uint32_t asked : { 0u, 1u, ~0u }) {
+		CHECK(ofi_amd_sched_batch_looks(&state, sizes, 30001, 128, num, xfers, stream, asked) == 0);
+	}
+	CHECK(looks.size() == 4 && looks[0] <= 2048 && looks[1] == 0 && looks[2] == 1 && looks[3] == looks[0]);
 	CHECK(ofi_amd_sched_stream_release(stream) == 0);
 	return 0;
 }
