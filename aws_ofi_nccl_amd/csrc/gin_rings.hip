@@ -37,17 +37,27 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
  * Wavefronts of a context.  A group is a chain of trips over the host link, some 5 us, so a few contexts want several
  * groups on their way at once.  The link is shared evenly by all that is, though, and nobody's group has arrived before nearly
  * everybody's has, while the consumer waits: 256 contexts x 256 records, 4.4 MB, arrive together after some 80 us, x 64
- * after 20.  Us to produce alone / to produce and drain on four threads with 64, 128 and 256 threads a context, and,
- * last, with 256 that met at three barriers a round and looked for free slots in every one, which is what this was before:
- *     1 x 1000    21.2 / 24.9    13.8 / 19.1    12.7 / 18.3    20.2
- *     8 x 1000    25.8 / 50.6    19.6 / 49.0    19.0 / 49.8    25.1 / 61.2
- *    16 x 300     14.6 / 44.8    14.2 / 35.8    14.8 / 45.6    17.5
- *    24 x 1000    38.8 / 94.7    39.1 / 93.2    38.6 / 93.8    44.3
- *   128 x 1000     170 / 358      171 / 321      170 / 330      171 / 325
- *   256 x 300      108 / 246      110 / 303      107 / 257      122 / 260
- *   256 x 1000     335 / 616      339 / 607      337 / 734      342 / 829
- * (The drain by itself takes up to a fifth longer in one process than in another.  What the producer adds to it, 256 x 1000:
- * -30 to 25 with 64 threads a context, 12 to 60 with 128, 80 to 140 with 256 and 170 with 1024.)
+ * after 20.  Us to produce alone with 64 / 128 / 256 threads a context, and with 256 that met at three barriers a round and
+ * looked for free slots in every one:
+ *     1 x 1000    21.2 / 13.8 / 12.7   20.2
+ *     8 x 1000    25.8 / 19.6 / 19.0   25.1
+ *    24 x 1000    38.8 / 39.1 / 38.6   44.3
+ *   128 x 1000     170 /  171 /  170    171
+ *   256 x 300      108 /  110 /  107    122
+ *   256 x 1000     335 /  339 /  337    342
+ * and to produce and drain on four threads, by turns in one process, the middle one of three processes:
+ *    16 x 300       60 /   59 /   60
+ *    24 x 1000     104 /  112 /  113
+ *    32 x 1000     136 /  139 /  137
+ *    64 x 1000     232 /  233 /  235
+ *    96 x 300      140 /  150 /  154
+ *    96 x 1000     309 /  326 /  344
+ *   128 x 1000     425 /  422 /  437
+ *   256 x 300      264 /  274 /  287
+ *   256 x 1000     664 /  661 /  695
+ * (The drain by itself takes up to a quarter longer in one process than in another, so that only times of one process compare.
+ * What the producer adds to it, 256 x 1000: -30 to 25 with 64 threads a context, 12 to 60 with 128, 80 to 140 with 256 and 170
+ * with 1024.)
  */
 constexpr uint32_t kMostThreads = 256;
 constexpr uint64_t kDefaultSpinLimit = 1ull << 22;

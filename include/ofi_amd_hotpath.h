@@ -307,8 +307,8 @@ typedef struct {
 
 typedef struct ofi_amd_gin_rings ofi_amd_gin_rings_t;
 
-/* n_contexts rings of `capacity` descriptors each (a power of two, 256 .. 2^24: a workgroup of
- * the seeded producer reserves 256 slots at a time; -EINVAL otherwise), in pinned host memory:
+/* n_contexts rings of `capacity` descriptors each (a power of two, 256 .. 2^24: up to four
+ * wavefronts of the seeded producer fill 64 slots each at a time; -EINVAL otherwise), in pinned host memory:
  * record array (64 B each) + sequence array (u32 each). */
 int ofi_amd_gin_rings_create(uint32_t n_contexts, uint32_t capacity, ofi_amd_gin_rings_t **out);
 int ofi_amd_gin_rings_destroy(ofi_amd_gin_rings_t *rings);
@@ -323,7 +323,9 @@ int ofi_amd_gin_rings_destroy(ofi_amd_gin_rings_t *rings);
  * host producers and the GPU producers' horizon are set accordingly.  Which ring a producer
  * gave up on is not recorded, so after a reported time-out reset all of them; only that form
  * clears the status ofi_amd_gin_producer_status reports.  The producers re-issue what they
- * could not put; what the consumer had popped before stays delivered.
+ * could not put; what the consumer had popped before stays delivered.  Until then the consumer may pop
+ * what was published in front of the first slot that never was; records behind such a slot, which other
+ * wavefronts may have published, are among the dropped ones.
  */
 #define OFI_AMD_GIN_ALL_CONTEXTS 0xffffffffu
 int ofi_amd_gin_rings_reset(ofi_amd_gin_rings_t *rings, uint32_t context, uint64_t *dropped);
@@ -338,7 +340,9 @@ int ofi_amd_gin_rings_view(ofi_amd_gin_rings_t *rings, void **records, uint32_t 
  * slot's sequence word).  Returns right after the launch; a host proxy must be
  * draining concurrently or the kernel gives up after spin_limit polls of a
  * still-occupied slot (0 = default) and ofi_amd_gin_producer_status reports
- * -ETIMEDOUT.
+ * -ETIMEDOUT.  Descriptors are published in groups of 64 by up to four wavefronts
+ * that do not wait for each other: of a launch that gives up, groups for which slots were
+ * free have been published, also behind one that never will be.
  */
 int ofi_amd_gin_produce_seeded(ofi_amd_gin_rings_t *rings, uint64_t seed,
 			       uint64_t ops_per_context, uint32_t peer_rank,
