@@ -252,9 +252,11 @@ constexpr bool by_workgroup(read_back_t back)
  * the copies all the same: no faster for long buffers, the last two lines 20.3 / 17.6 and 232 / 229.)
  * KEPT_TOGETHER: the words are found in the L2, but eight of them still leave in one write, to host memory as a rule.  Each by
  * itself and together, rows kept, other buffers at every launch / the same ones, us:
- *   8100 of up to 8 KiB, packed           18.2 / 11.4   18.4 / 11.4   (7000: 16.7 / 10.2  16.8 / 10.3, 4000: 11.0 / 6.2  11.2 / 6.4)
- *   16,000 of up to 4 KiB                 18.2 / 11.9   18.0 / 11.7
- *   32,000 of up to 2000 B                21.5 / 13.6   19.6 / 13.0
+ *   8100 of up to 8 KiB, packed           18.1 / 11.4   18.3 / 11.5   (7000: 15.9 / 10.3  16.0 / 10.4, 4000: 11.0 / 6.2  11.2 / 6.4)
+ *   10,000 of up to 6600 B                18.5 / 11.9   18.6 / 11.9   (of up to 60 B and 1000 B alike)
+ *   12,000 of up to 5500 B                19.2 / 12.1   18.7 / 12.1   (kKeepByItself lies between)
+ *   16,000 of up to 4 KiB                 18.8 / 12.0   18.5 / 11.8
+ *   32,000 of up to 2000 B                22.0 / 13.8   19.9 / 13.1
  *   65,536 of up to 1000 B                28.9 / 18.1   27.7 / 17.9
  *   200,000 of up to 100 B                47.3 / 46.7   44.7 / 44.2
  *   450,000 of up to 60 B                 95.7 / 82.2   91.3 / 80.0
@@ -733,7 +735,7 @@ constexpr size_t kCpuLoadMax = 256;
  *   16,000 of up to 8 KiB                  27.5 / 26.0  32.2 / 23.0
  */
 constexpr uint64_t kKeepBytes = 32ull << 20;
-constexpr uint32_t kKeepBounce = 8000, kKeepLines = 450000, kKeepEager = 9000;
+constexpr uint32_t kKeepBounce = 8000, kKeepByItself = 11000, kKeepLines = 450000, kKeepEager = 9000;
 /*
  * Fewer wavefronts a CU for large batches of long buffers -- reads and writes take turns at the memory, and the fewer
  * buffers are open the longer the turns are -- were measured and are not used: 65,536 of up to 8 KiB 110.9 us with 32
@@ -772,7 +774,7 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 	};
 	if (!d_flush) {
 		launch(bounce_scatter_kernel<NO_READ_BACK>);
-	} else if (n <= kKeepBounce) {
+	} else if (n <= kKeepBounce || (n <= kKeepByItself && src_bytes <= kKeepBytes)) {
 		launch(bounce_scatter_kernel<BY_ITSELF>);
 	} else if (n <= kKeepLines && src_bytes <= kKeepBytes) {
 		launch(bounce_scatter_kernel<KEPT_TOGETHER>);
