@@ -252,8 +252,9 @@ constexpr bool by_workgroup(read_back_t back)
  * the copies all the same: no faster for long buffers, the last two lines 20.3 / 17.6 and 232 / 229.)
  * KEPT_TOGETHER: the words are found in the L2, but eight of them still leave in one write, to host memory as a rule.  Each by
  * itself and together, rows kept, other buffers at every launch / the same ones, us:
- *   8100 of up to 8 KiB, packed           18.1 / 11.4   18.3 / 11.5   (7000: 15.9 / 10.3  16.0 / 10.4, 4000: 11.0 / 6.2  11.2 / 6.4)
- *   10,000 of up to 6600 B                18.5 / 11.9   18.6 / 11.9   (of up to 60 B and 1000 B alike)
+ *   7000 of up to 8 KiB, packed           15.9 / 10.3   16.0 / 10.4   (4000: 11.0 / 6.2  11.2 / 6.4)
+ *   8100 of up to 8 KiB, packed           18.1 / 11.4   18.3 / 11.5   (of up to 100 and 1000 B alike)
+ *   10,000 of up to 6600 B                18.5 / 11.9   18.6 / 11.9
  *   12,000 of up to 5500 B                19.2 / 12.1   18.7 / 12.1   (kKeepByItself lies between)
  *   16,000 of up to 4 KiB                 18.8 / 12.0   18.5 / 11.8
  *   32,000 of up to 2000 B                22.0 / 13.8   19.9 / 13.1
@@ -388,7 +389,8 @@ __device__ __forceinline__ uint32_t quad_word(uint32_t byte, uint32_t at)
  *
  * TOGETHER as in the bounce copy: one wavefront reads the bytes of its workgroup's four buffers back behind a barrier.  Each by
  * itself in workgroups of one and together in workgroups of four, on other buffers at every launch / on the same ones, us:
- *   65,536 of up to 8 KiB    120.7 / 95.5  121.0 / 95.8  (two wavefronts 120.9 / 96.4, eight 121.8 / 99.1; runs of 32: 121.0 / 97.2)
+ *   65,536 of up to 8 KiB    120.7 / 95.5  121.0 / 95.8  (two wavefronts 120.9 / 96.4, eight 121.8 / 99.1;
+ *                                                         runs of 32: 121.0 / 97.2)
  *   20,000 of up to 8 KiB     38.2 / 32.7   38.3 / 32.0
  *   65,536 of up to 4000 B    66.3 / 51.1   66.1 / 48.7
  *   65,536 of up to 500 B     27.7 / 26.9   24.7 / 23.5  (two wavefronts 27.4 / 26.3, eight 25.3 / 24.0; no read-back 17.1)
@@ -471,8 +473,8 @@ __global__ __launch_bounds__(64 * eager_waves(BACK)) void eager_copy_kernel(
 }
 
 /*
- * The same for rx buffers in host memory, which the link bounds.  It reads 8 KiB each for thousands of wavefronts at 46 GB/s and for
- * some tens to hundreds at 54, so wavefronts with more than kTurnBytes take turns, one of a workgroup's four at a time, and the
+ * The same for rx buffers in host memory, which the link bounds.  It reads 8 KiB each for thousands of wavefronts at 46 GB/s
+ * and for some tens to hundreds at 54, so wavefronts with more than kTurnBytes take turns, one of a workgroup's four at a time, and the
  * others, whose copies are a few trips and no more, do not.  Neighbours are dealt to the XCDs by fours here: by runs of 32 a few
  * hundred buffers load them unevenly, and nothing that neighbours share in host memory stays in an L2.  (Eight to a workgroup:
  * short buffers 0.8 us slower, their pages are looked up CU by CU.  256 wavefronts with a loop over buffers: long ones as
@@ -769,8 +771,8 @@ int ofi_amd_bounce_scatter(const void *d_src, uint64_t src_bytes, void *d_arena,
 	const uint32_t runs = (n + kXcds * kBounceRun - 1) / (kXcds * kBounceRun); /* whole rounds over the XCDs */
 	auto launch = [&](auto kernel) {
 		ofi_amd::launch_kernel(kernel, dim3(runs * kXcds * (kBounceRun / kBounceWaves)), dim3(64 * kBounceWaves), 0,
-				   as_stream(stream), static_cast<const uint8_t *>(d_src), src_bytes, d_src_off, d_dst_off, d_len, n,
-				   static_cast<uint8_t *>(d_arena), arena_bytes, d_flush, err);
+				       as_stream(stream), static_cast<const uint8_t *>(d_src), src_bytes, d_src_off, d_dst_off, d_len, n,
+				       static_cast<uint8_t *>(d_arena), arena_bytes, d_flush, err);
 	};
 	if (!d_flush) {
 		launch(bounce_scatter_kernel<NO_READ_BACK>);
@@ -802,14 +804,14 @@ int ofi_amd_eager_copy_batch(const void *rx_base, const uint64_t *d_rx_off, cons
 	auto launch = [&](auto kernel, read_back_t back) {
 		const uint32_t round = kXcds * eager_run(back), waves = (uint32_t)eager_waves(back); /* whole rounds over the XCDs */
 		ofi_amd::launch_kernel(kernel, dim3((n + round - 1) / round * (round / waves)), dim3(64 * waves), 0, as_stream(stream),
-				   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base),
-				   d_dst_off, d_dst_len, n, d_copied, d_flush);
+				       static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base),
+				       d_dst_off, d_dst_len, n, d_copied, d_flush);
 	};
 	if (n >= kHostBatch && in_host_memory(rx_base)) {
 		auto launch_host = [&](auto kernel) {
 			ofi_amd::launch_kernel(kernel, dim3((n + kHostWaves - 1) / kHostWaves), dim3(64 * kHostWaves), 0, as_stream(stream),
-					   static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len, static_cast<uint8_t *>(dst_base), d_dst_off,
-					   d_dst_len, n, d_copied, d_flush);
+					       static_cast<const uint8_t *>(rx_base), d_rx_off, d_recv_len,
+					       static_cast<uint8_t *>(dst_base), d_dst_off, d_dst_len, n, d_copied, d_flush);
 		};
 		d_flush ? launch_host(eager_copy_host_kernel<true>) : launch_host(eager_copy_host_kernel<false>);
 	} else if (!d_flush) {
@@ -837,7 +839,7 @@ int ofi_amd_copy_table(const uint64_t *d_src_addr, const uint64_t *d_dst_addr, c
 		return -EINVAL;
 	}
 	ofi_amd::launch_kernel(copy_table_kernel, dim3((n + kTableWaves - 1) / kTableWaves), dim3(64 * kTableWaves), 0,
-			   as_stream(stream), d_src_addr, d_dst_addr, d_len, n);
+			       as_stream(stream), d_src_addr, d_dst_addr, d_len, n);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }
@@ -872,7 +874,7 @@ int ofi_amd_copy_table_pieces(const uint64_t *d_src_addr, const uint64_t *d_dst_
 		const uint64_t round = (uint64_t)kXcds * map.run_blocks * kPieceWaves; /* whole rounds over the XCDs */
 		const uint64_t blocks = ((uint64_t)here * map.per + round - 1) / round * (kXcds * map.run_blocks);
 		ofi_amd::launch_kernel(copy_table_pieces_kernel, dim3((uint32_t)blocks), dim3(64 * kPieceWaves), 0,
-				   as_stream(stream), d_src_addr + at, d_dst_addr + at, d_len + at, here, map, max_len, err);
+				       as_stream(stream), d_src_addr + at, d_dst_addr + at, d_len + at, here, map, max_len, err);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
@@ -892,8 +894,8 @@ int ofi_amd_flush_read(const void *d_arena, const uint64_t *d_dst_off, uint32_t 
 		return -EINVAL;
 	}
 	ofi_amd::launch_kernel(flush_read_kernel, dim3((n + 255u) / 256u), dim3(256), 0,
-			   as_stream(stream), static_cast<const uint8_t *>(d_arena), d_dst_off, n,
-			   d_flush);
+			       as_stream(stream), static_cast<const uint8_t *>(d_arena), d_dst_off, n,
+			       d_flush);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }
@@ -908,7 +910,7 @@ int ofi_amd_flush_buffer_fill(void *d_flush_buf, uint64_t sentinel, void *stream
 		return -EINVAL;
 	}
 	ofi_amd::launch_kernel(flush_fill_kernel, dim3(1), dim3(64), 0, as_stream(stream),
-			   static_cast<uint64_t *>(d_flush_buf), sentinel);
+			       static_cast<uint64_t *>(d_flush_buf), sentinel);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }
@@ -924,8 +926,8 @@ int ofi_amd_flush_post(const void *d_flush_buf, void *slots_dev, uint32_t num_ra
 		return -EINVAL;
 	}
 	ofi_amd::launch_kernel(flush_post_kernel, dim3(1), dim3(64), 0, as_stream(stream),
-			   static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
-			   num_rails);
+			       static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
+			       num_rails);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -79,9 +79,10 @@ inline bool in_host_memory(const void *p)
 template <typename T> struct as_declared { /* an argument is converted to the kernel's parameter, not deduced from */
 	using type = T;
 };
-/* What <<<>>> does, without its detour through a stub that pushes the launch's shape and pops it again, which is 0.15 to 0.35 us
- * of the 2.5 to 3.4 that a launch with ten arguments takes the host (64 eager arrivals in a row 4.11 -> 3.93 us, 1000 striping
- * messages 4.05 -> 3.88, 300 bounce buffers 4.20 -> 3.96, 4 one-sided writes 3.63 -> 3.47).  The error is the runtime's last
+/* What <<<>>> does, without its detour through a stub that pushes the launch's shape and pops it again: 0.1 to 0.2 us of what a
+ * call takes the host.  <<<>>> and this by turns in one process, calls in a row: 64 eager arrivals 4.18 and 3.99 us, 1000 striping
+ * messages 4.07 and 3.92, 300 bounce buffers 4.26 and 4.08, 4 one-sided writes 3.70 and 3.54, 259 tuner questions 12.89 and 12.76,
+ * 16,384 signals 13.1 both ways.  (From process to process such calls differ by up to 0.8.)  The error is the runtime's last
  * one, as with <<<>>>. */
 template <typename... P>
 inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream,

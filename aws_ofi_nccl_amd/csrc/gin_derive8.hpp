@@ -3,8 +3,8 @@
  * lane of the AVX-512 registers, for the proxy's drain loop (gin_proxy.cpp) on CPUs that have them.
  *
  * A descriptor by itself costs some 250 instructions and two branches on its size (12.5 ns on a Zen 5 core, all told); eight
- * together cost 5.5 ns each, 6.6 where a region's words are gathered lane by lane.  What goes from one descriptor to the next -- the scheduler's two counters, the pinned rail
- * with the length of its run, the sequence number -- is a prefix over the lanes.
+ * together cost 5.5 ns each, 6.6 where a region's words are gathered lane by lane.  What goes from one descriptor to the next --
+ * the scheduler's two counters, the pinned rail with the length of its run, the sequence number -- is a prefix over the lanes.
  */
 #ifndef OFI_AMD_GIN_DERIVE8_HPP_
 #define OFI_AMD_GIN_DERIVE8_HPP_
@@ -195,7 +195,8 @@ OFI_AMD_WIDE __attribute__((noinline)) inline bool derive8(ofi_amd_gin_comm_t *c
 	a[3] = _mm512_maskz_mov_epi64(signal, deferred);
 	/* every stripe but the last has the full length; a single one has the message's, aligned or not */
 	const __m512i per = _mm512_add_epi64(one, _mm512_srlv_epi64(last, _mm512_srli_epi64(n, 1)));
-	__m512i stripe = _mm512_and_si512(_mm512_add_epi64(per, _mm512_set1_epi64(kStripeAlign - 1)), _mm512_set1_epi64(-(long long)kStripeAlign));
+	__m512i stripe = _mm512_and_si512(_mm512_add_epi64(per, _mm512_set1_epi64(kStripeAlign - 1)),
+					  _mm512_set1_epi64(-(long long)kStripeAlign));
 	stripe = _mm512_mask_mov_epi64(stripe, single, size);
 	a[4] = src;
 	a[5] = _mm512_min_epu64(size, stripe);

@@ -387,9 +387,9 @@ int ofi_amd_gin_produce_seeded(ofi_amd_gin_rings_t *r, uint64_t seed, uint64_t o
 	}
 	const uint32_t threads = r->n_contexts < 16 ? kMostThreads : (r->n_contexts < 32 ? kMostThreads / 2 : 64u);
 	ofi_amd::launch_kernel(gin_produce_seeded_kernel, dim3(r->n_contexts), dim3(threads), threads * 64u,
-			   as_stream(stream), reinterpret_cast<u32x4 *>(r->d_records), r->d_sequences, r->d_reserve, r->capacity,
-			   seed, ops_per_context, r->d_status, peer_rank, signal_every, signal_op, aggregate_mask,
-			   spin_limit ? spin_limit : kDefaultSpinLimit);
+			       as_stream(stream), reinterpret_cast<u32x4 *>(r->d_records), r->d_sequences, r->d_reserve, r->capacity,
+			       seed, ops_per_context, r->d_status, peer_rank, signal_every, signal_op, aggregate_mask,
+			       spin_limit ? spin_limit : kDefaultSpinLimit);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }
@@ -429,8 +429,8 @@ int ofi_amd_gin_produce_table(ofi_amd_gin_rings_t *r, const ofi_amd_gin_desc_t *
 		return rc;
 	}
 	ofi_amd::launch_kernel(gin_produce_table_kernel, dim3(r->n_contexts * waves_per_context), dim3(64), 0,
-			   as_stream(stream), first, d_table, ops_per_context, waves_per_context,
-			   spin_limit ? spin_limit : kDefaultSpinLimit);
+			       as_stream(stream), first, d_table, ops_per_context, waves_per_context,
+			       spin_limit ? spin_limit : kDefaultSpinLimit);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -337,7 +337,7 @@ extern "C" int ofi_amd_gin_signal_apply(const ofi_amd_gin_signal_work_t *d_work,
 	const bool large = n > 32768u && (counters <= n / 64u || in_host_memory(d_work));
 	auto launch = [&](auto kernel, uint32_t threads, uint32_t items) {
 		ofi_amd::launch_kernel(kernel, dim3((n - 1u) / (threads * items) + 1u), dim3(threads), 0, as_stream(stream),
-				   d_work, n, r, large ? 0u : crowd_of(n), d_rejected);
+				       d_work, n, r, large ? 0u : crowd_of(n), d_rejected);
 	};
 	if (n <= 4096u) {
 		launch(gin_signal_apply_kernel<256, 1, 512>, 256, 1);
@@ -373,8 +373,8 @@ extern "C" int ofi_amd_gin_signal_apply_post(const ofi_amd_gin_signal_work_t *d_
 		return -EINVAL;
 	}
 	ofi_amd::launch_kernel(gin_signal_apply_post_kernel, dim3(1), dim3(kPostThreads), 0, as_stream(stream), d_work, n, r,
-			   n != 0 ? crowd_of(n) : 0u, d_rejected, static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
-			   num_rails);
+			       n != 0 ? crowd_of(n) : 0u, d_rejected, static_cast<const uint64_t *>(d_flush_buf), static_cast<uint64_t *>(slots_dev),
+			       num_rails);
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;
 }

@@ -519,12 +519,12 @@ __global__ __launch_bounds__(THREADS) void stripe_emit_kernel(
  * Us in two launches / in this one, in a row (two launches of this length are also more than some hosts queue in that time):
  *     9985 messages    6.3-6.6 / 4.4
  *    10,300            5.9-7.4 / 4.5
- *    30,000            6.0-7.2 / 5.3
- *   100,000            6.7-7.2 / 6.5
- *   150,000            7.9     / 7.4
- *   262,144            9.0     / 8.4
+ *    30,000            6.0-7.2 / 4.8
+ *   100,000            6.7-7.2 / 6.0
+ *   150,000            7.9     / 7.0
+ *   262,144            9.0     / 8.5
  * Beyond 262,144 (a word a thread) workgroups would start while others write, and the words take longer than the second
- * launch: 600,000 messages 15.1 / 17.5, 1,000,000 21.7 / 28.9.
+ * launch: 600,000 messages 15.1 / 17.5, 1,000,000 21.7 / 28.9 (23.2 in tiles of 1024 to 2048 messages).
  */
 constexpr uint32_t kOnceTile = 512, kOnceCopies = 8;
 constexpr uint64_t kOnceBatch = (uint64_t)kOnceTile * kOnceTile;
@@ -736,7 +736,7 @@ int new_scratch(hipStream_t s, uint32_t **out)
 		e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
 		if (e == hipSuccess) {
 			ofi_amd::launch_kernel(stripe_scratch_kernel, dim3(kClearBlocks), dim3(kClearThreads), 0, own,
-					   words);
+					       words);
 			e = hipGetLastError();
 			const hipError_t waited = hipStreamSynchronize(own);
 			e = e == hipSuccess ? waited : e;
@@ -821,8 +821,8 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 		const uint32_t turn = tiles > 1 ? scratch.turn.fetch_add(1, std::memory_order_relaxed) : 0u;
 		auto launch = [&](auto kernel, uint32_t threads) {
 			ofi_amd::launch_kernel(kernel, dim3(tiles), dim3(threads), 0, s, d_sizes, n, d_state, align, nullptr, nullptr,
-					   words + turn % kArrivalWords, words + (turn + kArrivalWords / 2) % kArrivalWords, tiles,
-					   d_num_xfers, d_xfers, err);
+					       words + turn % kArrivalWords, words + (turn + kArrivalWords / 2) % kArrivalWords, tiles,
+					       d_num_xfers, d_xfers, err);
 		};
 		if (large) {
 			launch(stripe_emit_kernel<DIRECT, kDirectTileLarge>, kDirectTileLarge);
@@ -835,23 +835,23 @@ void launch_batch(hipStream_t s, const uint64_t *d_sizes, uint64_t total, ofi_am
 		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kOnceTile);
 		const uint64_t number = scratch.published.fetch_add(1, std::memory_order_relaxed) + 1;
 		ofi_amd::launch_kernel(stripe_once_kernel, dim3(tiles), dim3(kOnceTile), 0, s, d_sizes, n, tiles, d_state, align,
-				   reinterpret_cast<uint64_t *>(words + kOnceWords), number, looks, d_num_xfers, d_xfers, err);
+				       reinterpret_cast<uint64_t *>(words + kOnceWords), number, looks, d_num_xfers, d_xfers, err);
 		return;
 	}
 	if (total <= kSmallBatch) {
 		const uint32_t n = (uint32_t)total, tiles = tiles_of(n, kTile);
 		ofi_amd::launch_kernel(stripe_count_kernel, dim3(tiles), dim3(kCountThreads), 0, s, d_sizes, n, d_state, align, totals,
-				   seed0, err);
+				       seed0, err);
 		ofi_amd::launch_kernel((stripe_emit_kernel<TILES, kTile>), dim3(tiles), dim3(kTile), 0, s, d_sizes, n, d_state, align,
-				   totals, nullptr, seed0, nullptr, tiles, d_num_xfers, d_xfers, err);
+				       totals, nullptr, seed0, nullptr, tiles, d_num_xfers, d_xfers, err);
 		return;
 	}
 	for (uint64_t at = 0; at < total; at += kPart) {
 		const uint32_t n = (uint32_t)(total - at < kPart ? total - at : kPart), tiles = tiles_of(n, kBigTile);
 		ofi_amd::launch_kernel(stripe_count_big_kernel, dim3(tiles_of(tiles, kBlockTiles)), dim3(64 * kBlockTiles), 0, s,
-				   d_sizes + at, n, d_state, align, totals, blocks, seed0, err);
+				       d_sizes + at, n, d_state, align, totals, blocks, seed0, err);
 		ofi_amd::launch_kernel((stripe_emit_kernel<BLOCKS, kBigTile>), dim3(tiles), dim3(kBigTile), 0, s, d_sizes + at, n,
-				   d_state, align, totals, blocks, seed0, nullptr, tiles, d_num_xfers + at, d_xfers + 6 * at, err);
+				       d_state, align, totals, blocks, seed0, nullptr, tiles, d_num_xfers + at, d_xfers + 6 * at, err);
 	}
 }
 

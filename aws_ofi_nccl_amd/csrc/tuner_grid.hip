@@ -987,7 +987,7 @@ int ofi_amd_tuner_model_grid(ofi_amd_tuner_plan_t *plan, const ofi_amd_tuner_var
 	const size_t lds = std::max(row * threads, fewer ? kModelFewerLds : 0);
 	auto launch = [&](auto kernel) {
 		ofi_amd::launch_kernel(kernel, dim3((points + threads - 1) / threads, n_variants), dim3(threads), d_cost ? lds : 0, s,
-				   d_cost, plan->d_variants, d_choice, points, plan->g);
+				       d_cost, plan->d_variants, d_choice, points, plan->g);
 	};
 	if (d_cost && d_choice) {
 		large ? launch(model_grid_kernel<true, true, kModelThreadsLarge>) : launch(model_grid_kernel<true, true>);
@@ -1076,7 +1076,7 @@ int ofi_amd_tuner_region_grid(ofi_amd_tuner_plan_t *plan, const int32_t *platfor
 	for (uint64_t at = 0; at < n_runs; at += kMostRuns) {
 		const uint32_t here = (uint32_t)(n_runs - at < kMostRuns ? n_runs - at : kMostRuns);
 		ofi_amd::launch_kernel(region_choice_kernel, dim3(grid_x, here), dim3(64 * waves), 0, s, plan->d_runs + at,
-				   plan->t.poly, plan->t.bbox, plan->t.edges, d_choice, points, plan->t.far_point, tiling, plan->g);
+				       plan->t.poly, plan->t.bbox, plan->t.edges, d_choice, points, plan->t.far_point, tiling, plan->g);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return 0;

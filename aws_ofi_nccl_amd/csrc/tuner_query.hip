@@ -376,10 +376,10 @@ extern "C" int ofi_amd_tuner_query(const ofi_amd_tuner_query_t *queries, uint32_
 		const uint32_t here = n - at < kMostPerLaunch ? n - at : kMostPerLaunch;
 		const uint32_t waves = here < kQueryWaves ? here : kQueryWaves;
 		ofi_amd::launch_kernel(tuner_query_kernel, dim3((here + kQueryWaves - 1) / kQueryWaves), dim3(64 * waves), 0,
-				   g_stage.stream, tables.far_point, reinterpret_cast<const int4 *>(tables.poly),
-				   reinterpret_cast<const double4_t *>(tables.bbox), tables.edges,
-				   static_cast<const uint64_t *>(g_stage.dq) + (uint64_t)at * kQueryWords, here, call,
-				   static_cast<uint64_t *>(g_stage.da) + at);
+				       g_stage.stream, tables.far_point, reinterpret_cast<const int4 *>(tables.poly),
+				       reinterpret_cast<const double4_t *>(tables.bbox), tables.edges,
+				       static_cast<const uint64_t *>(g_stage.dq) + (uint64_t)at * kQueryWords, here, call,
+				       static_cast<uint64_t *>(g_stage.da) + at);
 	}
 	OFI_AMD_HIP_TRY(hipGetLastError());
 	return collect_answers(g_stage, n, call, answers);

@@ -142,8 +142,9 @@ int ofi_amd_sched_stream_release(void *stream);
  * array: calls that overlap there -- different streams, or two threads -- race; order them.  What
  * an overlap spoils is the batches that took part in it, not later ones.  A call writes every word of the
  * array before it reads it, but for 1024 words that small batches count in -- those are zero between
- * calls, as they are when the code is loaded, and calls clear them again by turns -- and the words in which the tiles
- * of batches of 9,985 to 262,144 messages publish their totals, which carry the number of their batch.
+ * calls, as they are when the code is loaded, and calls clear them again by turns -- and the words in
+ * which the tiles of batches of 9,985 to 262,144 messages publish their totals and agree on the
+ * counters, which carry the number of their batch.
  */
 int ofi_amd_sched_batch_noalloc(ofi_amd_sched_state_t *d_state, const uint64_t *d_sizes, uint64_t n,
 				uint64_t align, uint32_t *d_num_xfers, ofi_amd_xfer_info_t *d_xfers,
@@ -308,8 +309,8 @@ typedef struct {
 typedef struct ofi_amd_gin_rings ofi_amd_gin_rings_t;
 
 /* n_contexts rings of `capacity` descriptors each (a power of two, 256 .. 2^24: up to four
- * wavefronts of the seeded producer fill 64 slots each at a time; -EINVAL otherwise), in pinned host memory:
- * record array (64 B each) + sequence array (u32 each). */
+ * wavefronts of the seeded producer fill 64 slots each at a time; -EINVAL otherwise), in pinned
+ * host memory: record array (64 B each) + sequence array (u32 each). */
 int ofi_amd_gin_rings_create(uint32_t n_contexts, uint32_t capacity, ofi_amd_gin_rings_t **out);
 int ofi_amd_gin_rings_destroy(ofi_amd_gin_rings_t *rings);
 /*
@@ -505,8 +506,9 @@ int ofi_amd_gin_proxy_drain(ofi_amd_gin_rings_t *rings, uint64_t ops_per_context
 
 /*
  * The same loop on up to n_threads proxy threads (the caller's included; one more for every 3000
- * descriptors the call is to drain, 2000 where it derives them one by one), each owning a contiguous range of contexts -- NCCL runs up to
- * NCCL_GIN_MAX_CONNECTIONS = 4 GIN proxy threads (nccl/net.h:38).  Contexts are independent (own
+ * descriptors the call is to drain, 2000 where it derives them one by one), each owning a contiguous
+ * range of contexts -- NCCL runs up to NCCL_GIN_MAX_CONNECTIONS = 4 GIN proxy threads
+ * (nccl/net.h:38).  Contexts are independent (own
  * ring, own comm state), so the per-context results, and the checksum summed over contexts, do not
  * depend on n_threads.  1..64.
  */

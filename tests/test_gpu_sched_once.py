@@ -56,8 +56,8 @@ class Chain:
 
 # the smallest batches, with whole and ragged last tiles, both sides of a wavefront's share of the words, the largest batch
 # and the one after it
-@pytest.mark.parametrize("n", [9984, 9985, 10240, 10241, 20 * TILE + 513, 64 * TILE, 64 * TILE + 1, 65 * TILE + 1, TILE * TILE - 1, TILE * TILE,
-                               TILE * TILE + 1])
+@pytest.mark.parametrize("n", [9984, 9985, 10240, 10241, 20 * TILE + 513, 64 * TILE, 64 * TILE + 1, 65 * TILE + 1,
+                               TILE * TILE - 1, TILE * TILE, TILE * TILE + 1])
 @pytest.mark.parametrize("rails,max_small", [(4, 64), (3, 5000), (1, 0)])
 def test_batches_of_published_totals(lib, oracle, gpu, n, rails, max_small):
     """Three in a row without a wait between them: each starts from the counters the one before has moved on, and none
