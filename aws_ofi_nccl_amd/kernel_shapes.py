@@ -19,14 +19,16 @@ nothing else of interest, which keeps counter runs short.  The shapes:
                          destinations 4 KiB-aligned and apart: whole entries through
                          ofi_amd_copy_table_pieces (a wavefront per 8 KiB), or with --cut the same
                          bytes as 256 KiB entries through ofi_amd_copy_table (a wavefront per entry)
-  striping  1m | 16m     1,000,000 / 16,000,000 message sizes, 4 rails
+  striping  100k | 1m | 16m  100,000 / 1,000,000 / 16,000,000 message sizes, 4 rails
   model     64 | 256     tuner cost-model grids per launch
   region    64           tuner region grids per launch
+            sweep        four platforms' grids of 560 sizes and the node counts that 44 steps from 1 to 1024 give
   eager     configured   65,536 rx buffers of 8,320 B, payloads 0..8,184 B, taken in a random
                          order of slots, destinations at any byte alignment
             slots        the same with the rx buffers taken in slot order
             align<N>     the same as configured with every destination a multiple of N bytes
                          (N = 16, 64 or 128); "slots+align<N>" combines the two
+            host         2048 rx buffers in pinned host memory
 """
 import argparse
 import ctypes
@@ -132,7 +134,7 @@ def main():
                                                                  len(starts), piece, stream), "copy_table_pieces")
         print("bytes copied per launch: %d in %d table entries" % (entries * each, len(starts)))
     elif args.kernel == "eager":
-        n, stride = 65536, 8320
+        n, stride = 2048 if args.shape == "host" else 65536, 8320
         rng = np.random.default_rng(SEED)
         recv_len = rng.integers(0, 8185, n).astype(np.uint32)
         rx_off = rng.permutation(n).astype(np.uint64) * np.uint64(stride)
@@ -143,9 +145,11 @@ def main():
                 rx_off = np.arange(n, dtype=np.uint64) * np.uint64(stride)
             elif word in ("align16", "align64", "align128"):
                 dst_off &= ~np.uint64(int(word[5:]) - 1)
-            elif word != "configured":
+            elif word not in ("configured", "host"):
                 ap.error("unknown shape")
         d_rx = torch.randint(0, 255, (n * stride,), dtype=torch.uint8, device="cuda")
+        if args.shape == "host":
+            d_rx = d_rx.cpu().pin_memory()
         d_dst = torch.zeros(2 << 30, dtype=torch.uint8, device="cuda")
         d = [dev(x) for x in (rx_off, recv_len, dst_off, recv_len)]
         d_copied = torch.zeros(n, dtype=torch.int32, device="cuda")
@@ -156,7 +160,7 @@ def main():
             n, d_copied.data_ptr(), flush, stream), "eager_copy_batch")
         print("payload bytes per launch: %d" % int(recv_len.sum()))
     elif args.kernel == "striping":
-        n = {"1m": 1_000_000, "16m": 16_000_000}[args.shape or "1m"]
+        n = {"100k": 100_000, "1m": 1_000_000, "16m": 16_000_000}[args.shape or "1m"]
         sizes = synthetic.stripe_sizes(SEED, n)
         st = m.SchedState(0, 0, 64, 131072, 4, 0)
         d_state = dev(np.frombuffer(bytes(st), dtype=np.uint8).copy())
@@ -167,12 +171,16 @@ def main():
                                                        d_num.data_ptr(), d_xf.data_ptr(), stream), "sched_batch")
     else:
         colls, sizes, nodes, ppn, algos = synthetic.tuner_axes()
+        sweep = args.kernel == "region" and args.shape == "sweep"
+        if sweep:
+            sizes = np.array([int(round(2.0 ** ((k + 0.5) / 16))) for k in range(16 * 35)], dtype=np.uint64)
+            nodes = np.unique(np.round(2.0 ** (np.arange(44) * 10.0 / 43)).astype(nodes.dtype))
         plan = ctypes.c_void_p()
         m.check(lib.ofi_amd_tuner_plan_create(colls.ctypes.data, len(colls), sizes.ctypes.data, len(sizes),
                                               nodes.ctypes.data, len(nodes), ppn.ctypes.data, len(ppn),
                                               algos.ctypes.data, len(algos), ctypes.byref(plan)), "plan_create")
         points, cells = lib.ofi_amd_tuner_plan_points(plan), lib.ofi_amd_tuner_plan_cells(plan)
-        nv = int(args.shape or "64")
+        nv = 4 if sweep else int(args.shape or "64")
         if args.kernel == "model":
             variants = (m.TunerVariant * nv)(*[m.TunerVariant(i % 2, 1 + (i // 2) % 32, 8 + i // 64, 3)
                                                for i in range(nv)])
